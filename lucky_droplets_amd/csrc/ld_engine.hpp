@@ -177,6 +177,7 @@ struct Engine final : EngineBase {
     if (evG0) (void)hipEventDestroy(evG0);
     if (evG1) (void)hipEventDestroy(evG1);
     if (evB) (void)hipEventDestroy(evB);
+    if (evR) (void)hipEventDestroy(evR);
     for (void* a : allocs) (void)hipFree(a);
   }
 
@@ -347,6 +348,7 @@ struct Engine final : EngineBase {
     if (const char* e = getenv("LD_SERIAL")) serial = atoi(e) != 0;
     if (const char* e = getenv("LD_YSPLIT")) ysplit = atoi(e) != 0;
     if (const char* e = getenv("LD_LATE_DENSITY")) late_density = atoi(e) != 0;
+    if (const char* e = getenv("LD_ROW_SORT_MIN")) api_sort_min = atoll(e);   // measurement, tests
     if (const char* e = getenv("LD_TRUNCATE")) kc = atoi(e) != 0 ? N / 3 : N / 2;
     if (const char* e = getenv("LD_PSTAGE_LDS")) {
       const int v = atoi(e);
@@ -394,6 +396,7 @@ struct Engine final : EngineBase {
     }
     LD_HIP(hipEventCreateWithFlags(&evA, hipEventDisableTiming));
     LD_HIP(hipEventCreateWithFlags(&evB, hipEventDisableTiming));
+    LD_HIP(hipEventCreateWithFlags(&evR, hipEventDisableTiming));
     // per-realization state and work buffers (one slab per realization)
     arena(uk, 3 * CF); arena(us, 3 * CF); arena(acc, 3 * CF); arena(w6, 6 * CF); arena(wn, 4 * CF);
     arena(ubuf[0], 3 * RF); arena(ubuf[1], 3 * RF); arena(v, 3 * RF);
@@ -950,17 +953,22 @@ struct Engine final : EngineBase {
     hipLaunchKernelGGL((k_bin_count<N>), dim3(pb, 1, B), dim3(256), 0, s, (const double*)x0, (int)np, (int)cap, p.L,
                        dp.invL, dp.inv_dx, pkey, prank, hist, rs);
     LD_LAUNCHED();
+    LD_TRY(scan_bins(s));
+    hipLaunchKernelGGL((k_bin_scatter<PT>), dim3(pb, 1, B), dim3(256), 0, s, (int)np, (int)cap, (const int*)pkey,
+                       (const int*)prank, (const int*)hist, (const double*)x0, (const PT*)v0, (const int64_t*)rid,
+                       x0b, v0b, rid2, rs);
+    LD_LAUNCHED();
+    swap_sorted();
+    return LD_OK;
+  }
+  // bin counts -> bin starts
+  int scan_bins(hipStream_t s) {
     hipLaunchKernelGGL(k_scan_local, dim3(NBS, 1, B), dim3(1024), 0, s, hist, NB, bsum, rs);
     LD_LAUNCHED();
     hipLaunchKernelGGL(k_scan_bsums, dim3(1, 1, B), dim3(1024), 0, s, bsum, NBS, rs);
     LD_LAUNCHED();
     hipLaunchKernelGGL(k_scan_add, dim3((NB + 255) / 256, 1, B), dim3(256), 0, s, hist, NB, (const int*)bsum, rs);
     LD_LAUNCHED();
-    hipLaunchKernelGGL((k_bin_scatter<PT>), dim3(pb, 1, B), dim3(256), 0, s, (int)np, (int)cap, (const int*)pkey,
-                       (const int*)prank, (const int*)hist, (const double*)x0, (const PT*)v0, (const int64_t*)rid,
-                       x0b, v0b, rid2, rs);
-    LD_LAUNCHED();
-    swap_sorted();
     return LD_OK;
   }
   // The sort scatters into the second set of droplet buffers; they become current.
@@ -1023,6 +1031,7 @@ struct Engine final : EngineBase {
   }
 
   int advance(double h, int nsteps) override {
+    LD_TRY(rows_begin());            // the step's scratch may be in use by a row call on another stream
     if (use_graph && prof_id < 0) {
       // steps on the internal stream (a legacy default stream cannot be captured)
       hipStream_t caller = st;
@@ -1081,6 +1090,7 @@ struct Engine final : EngineBase {
 
   int rk4(double h, const void* ukin, void* nio, const double* coord, int64_t n_, void* uknew, void* nnew,
           double* coord_new) override {
+    LD_TRY(rows_begin());
     LD_TRY(state_set(ukin, nio, coord, n_));
     LD_TRY(join(st2, st, evA));
     // rows come in any order: sorted as a step sorts its droplets, so that the
@@ -1117,13 +1127,7 @@ struct Engine final : EngineBase {
     LD_TRY(xrhs(st, ra));
     // the physical-space v the droplets see uses visc as well (forced-dns-sm.py:319-321)
     LD_TRY(velocity(st, vphys, nullptr, (const T*)nin, clip_none, nullptr));
-    LD_TRY(fill<T>(st, fcp, RF, (T)0));
-    if (n_ > 0) {
-      hipLaunchKernelGGL((k_prhs<T, N>), dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, coord, (int)n_,
-                         (const T*)uphys, (const T*)vphys, (const T*)nin, (const double*)clip_none, fcp, kp, rows_a,
-                         wrow, dp);
-      LD_LAUNCHED();
-    }
+    LD_TRY(prhs_rows(coord, n_, uphys, vphys, (const T*)nin, fcp, kp, rows_a, wrow));
     OpZKn<T, N, P1> ok;
     ok.w = wn; ok.fs = CF; ok.scale = inv(); ok.kn_out = (T*)kn;
     ok.n0 = nullptr; ok.nacc = nullptr; ok.nnext = nullptr; ok.wacc = (T)0; ok.anext = (T)0; ok.acc_init = 0;
@@ -1493,9 +1497,112 @@ struct Engine final : EngineBase {
   }
 
   // ------------------------------------------------------------ droplet API
+  // Rows handed to interp / exterp / prhs / full_rhs: sorted by bin first when
+  // that pays for the bin counts and scans (NB bins) and not so many that a
+  // brick's own work no longer spreads over the chip (2 N^3).  The scratch is
+  // the step's (bin keys, ranks and starts, deposit records, the fallback list
+  // for the row numbers), free between steps, so the context's capacity bounds
+  // the rows; more rows take the one-thread-per-row kernels.  Where the line
+  // lies (us per call, sorted / one thread per row):
+  //  * fields of at most 4 MB (up to 32^3) stay in each L2, where scattered
+  //    loads cost little: pRHS 102 / 106 at 12000 rows, 107 / 94 at 3000;
+  //    exterp 145 / 85 at 25000 and 366 / 180 at 60000, interp 60 / 47: never;
+  //  * pRHS otherwise always: 64^3 FP32 106 / 129 at 300 rows, 218 / 1046 at
+  //    200000, 512^3 212 / 353 and 952 / 1889 (590 / 573 at 60000);
+  //  * interp from 1024 rows with four or more components (128^3 FP32, 7
+  //    components: 63 / 149 at 3000; FP64 62 / 63 at 1000) or 131072 values
+  //    (one component: 64 / 31 at 60000, 63 / 91 at 200000);
+  //  * exterp from 16384 rows (128^3: 72 / 57 at 12000, 70 / 94 at 25000) and
+  //    N^3 / 2048 (512^3: 305 / 224 at 25000, 336 / 325 at 60000, 355 / 776 at
+  //    200000: the bricks write every node).
+  enum RowOp { ROW_PRHS, ROW_INTERP, ROW_EXTERP };
+  int64_t api_sort_min = -1;         // >= 0: the line for every call (LD_ROW_SORT_MIN)
+  bool rows_sorted(RowOp op, int64_t n_, int nc = 1) const {
+    if (n_ > cap || n_ > 2 * (int64_t)RF) return false;
+    if (api_sort_min >= 0) return n_ >= api_sort_min;
+    const bool small = 7 * RF * sizeof(T) <= (size_t)4 << 20;
+    if (op == ROW_PRHS) return !small || n_ >= 12288;
+    if (small) return false;
+    if (op == ROW_INTERP) return (nc >= 4 && n_ >= 1024) || n_ * nc >= 131072;
+    return n_ >= 16384 && n_ >= (int64_t)(RF / 2048);
+  }
+  int sort_rows(const double* coord, int64_t n_, const double* w) {
+    LD_TRY(rows_begin());
+    const unsigned pb = (unsigned)((n_ + 255) / 256);
+    LD_TRY(fill<int>(st, hist, NB, 0));
+    hipLaunchKernelGGL((k_row_bin<N>), dim3(pb), dim3(256), 0, st, coord, (int)n_, p.L, dp.inv_dx, pkey, prank, hist);
+    LD_LAUNCHED();
+    LD_TRY(scan_bins(st));
+    hipLaunchKernelGGL(k_row_scatter, dim3(pb), dim3(256), 0, st, coord, (int)n_, p.L, w, (const int*)pkey,
+                       (const int*)prank, (const int*)hist, dep, flist);
+    LD_LAUNCHED();
+    return LD_OK;
+  }
+  static unsigned quad_blocks(int64_t n_) { return (unsigned)(((4 * n_ + 255) / 256 + 7) / 8 * 8); }
+  // FP64 brick deposit of the sorted rows' weights; writes every node of c
+  int deposit_rows(int64_t n_, T* c) {
+    hipLaunchKernelGGL((k_brick_deposit<T, N, false>), dim3(Brick<N>::NB * Brick<N>::NB * Brick<N>::NB),
+                       dim3(Brick<N>::NT), 0, st, (const double4*)dep, (const int*)hist, (int)n_,
+                       (const unsigned long long*)nullptr, c, dp, (size_t)0);
+    LD_LAUNCHED();
+    return LD_OK;
+  }
+  // Droplet right-hand side of rows in any order; fcp receives the deposit.
+  int prhs_rows(const double* coord, int64_t n_, const T* uf, const T* usf, const T* nf, T* fcp, double* rhs,
+                double* interpm, double* exterpm) {
+    if (n_ > 0 && rows_sorted(ROW_PRHS, n_)) {
+      LD_TRY(sort_rows(coord, n_, nullptr));
+      hipLaunchKernelGGL((k_prhs_sorted<T, N>), dim3(quad_blocks(n_)), dim3(256), 0, st, coord, (int)n_, uf, usf, nf,
+                         dep, (const int*)flist, rhs, interpm, exterpm, dp);
+      LD_LAUNCHED();
+      LD_TRY(deposit_rows(n_, fcp));
+      return rows_end();
+    }
+    LD_TRY(fill<T>(st, fcp, RF, (T)0));
+    if (n_ <= 0) return LD_OK;
+    hipLaunchKernelGGL((k_prhs<T, N>), dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, coord, (int)n_, uf, usf,
+                       nf, (const double*)clip_none, fcp, rhs, interpm, exterpm, dp);
+    LD_LAUNCHED();
+    return LD_OK;
+  }
+  // The sorted path's scratch belongs to the context: a call on another stream
+  // than the last one waits for it (the one-thread-per-row kernels share
+  // nothing).  Not under capture, where the caller orders its own replays.
+  hipEvent_t evR = nullptr;
+  hipStream_t rows_stream = nullptr;
+  bool rows_used = false;
+  int capturing(bool& yes) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    LD_HIP(hipStreamIsCapturing(st, &cs));
+    yes = cs != hipStreamCaptureStatusNone;
+    return LD_OK;
+  }
+  int rows_begin() {
+    if (!rows_used || rows_stream == st) return LD_OK;
+    bool cap_ = false;
+    LD_TRY(capturing(cap_));
+    if (!cap_) LD_HIP(hipStreamWaitEvent(st, evR, 0));
+    return LD_OK;
+  }
+  int rows_end() {
+    bool cap_ = false;
+    LD_TRY(capturing(cap_));
+    if (cap_) return LD_OK;
+    LD_HIP(hipEventRecord(evR, st));
+    rows_stream = st;
+    rows_used = true;
+    return LD_OK;
+  }
   int interp(const double* coord, int64_t n_, const void* f, int nc, double* out) override {
     if (n_ <= 0) return LD_OK;
     LD_TRY(join(st, st2, evB));
+    if (rows_sorted(ROW_INTERP, n_, nc)) {
+      LD_TRY(sort_rows(coord, n_, nullptr));
+      hipLaunchKernelGGL((k_interp_sorted<T, N>), dim3(quad_blocks(n_)), dim3(256), 0, st, (int)n_, (const T*)f, nc,
+                         (const double4*)dep, (const int*)flist, out, dp);
+      LD_LAUNCHED();
+      return rows_end();
+    }
     hipLaunchKernelGGL((k_interp<T, N>), dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, coord, (int)n_,
                        (const T*)f, nc, out, dp);
     LD_LAUNCHED();
@@ -1503,6 +1610,11 @@ struct Engine final : EngineBase {
   }
   int exterp(const double* coord, int64_t n_, const double* w, void* c) override {
     LD_TRY(join(st, st2, evB));
+    if (n_ > 0 && rows_sorted(ROW_EXTERP, n_)) {
+      LD_TRY(sort_rows(coord, n_, w));
+      LD_TRY(deposit_rows(n_, (T*)c));
+      return rows_end();
+    }
     LD_TRY(fill<T>(st, (T*)c, RF, (T)0));
     if (n_ <= 0) return LD_OK;
     hipLaunchKernelGGL((k_exterp<T, N>), dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, coord, (int)n_, w,
@@ -1555,13 +1667,7 @@ struct Engine final : EngineBase {
   int prhs(const double* coord, int64_t n_, const void* uf, const void* usf, const void* nf, void* fcout,
            double* rhs, double* interpm, double* exterpm) override {
     LD_TRY(join(st, st2, evB));
-    LD_TRY(fill<T>(st, (T*)fcout, RF, (T)0));
-    if (n_ <= 0) return LD_OK;
-    hipLaunchKernelGGL((k_prhs<T, N>), dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, coord, (int)n_,
-                       (const T*)uf, (const T*)usf, (const T*)nf, (const double*)clip_none, (T*)fcout, rhs, interpm,
-                       exterpm, dp);
-    LD_LAUNCHED();
-    return LD_OK;
+    return prhs_rows(coord, n_, (const T*)uf, (const T*)usf, (const T*)nf, (T*)fcout, rhs, interpm, exterpm);
   }
 };
 

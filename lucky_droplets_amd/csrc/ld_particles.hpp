@@ -545,7 +545,12 @@ template <int N> struct Brick {
   static_assert(N % S == 0 && (NB * NB * NB) % 8 == 0, "brick grid");
 };
 
-template <typename T, int N>
+//
+// FIX = false (the API's deposits, whose weights may be negative, of any
+// range or not finite): the tile is FP64 and added to in FP64 (ds_add_f64, 27
+// against 15 cycles), every candidate with W != 0 deposits, and the stencil
+// weights are FP64 as the API's are.
+template <typename T, int N, bool FIX = true>
 __global__ void __launch_bounds__(Brick<N>::NT)
 k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0, int np,
                 const unsigned long long* __restrict__ wmax0, T* __restrict__ fc0, DropPhys P, size_t rs) {
@@ -558,7 +563,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   constexpr int TS = Bins<N>::TS;
   constexpr int BS = Bins<N>::BS, B = Bins<N>::B;
   constexpr int NBIN = B * B * B;
-  __shared__ unsigned long long tile[S * S * S];
+  __shared__ std::conditional_t<FIX, unsigned long long, double> tile[S * S * S];
   __shared__ int rb[NR], rn[NR], rl[NR + 1];
   __shared__ int list[CH];
   __shared__ int cnt;
@@ -567,7 +572,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   const int nb = gridDim.x, per = nb / 8;
   const int br = (blockIdx.x % 8) * per + blockIdx.x / 8;
   const int c0x = (br / (NBr * NBr)) * S, c0y = ((br / NBr) % NBr) * S, c0z = (br % NBr) * S;
-  for (int i = tid; i < S * S * S; i += NT) tile[i] = 0ull;
+  for (int i = tid; i < S * S * S; i += NT) tile[i] = 0;
   if (tid == 0) cnt = 0;
   // slot ranges of the window's z-runs
   const int lo = (NBX == B) ? 0 : 1;
@@ -620,7 +625,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   __syncthreads();
   const int total = rl[NR];
   const double dx = P.dx, pi_2dx = P.pi_2dx, inv_dx = P.inv_dx;
-  const double bound = (double)total * __longlong_as_double((long long)*wmax) * P.inv_vol * 0.125;
+  const double bound = FIX ? (double)total * __longlong_as_double((long long)*wmax) * P.inv_vol * 0.125 : 0.0;
   const bool finite = isfinite(bound);
   // FP32 fields: sums below 2^52, so a value converts to its integer by one
   // addition of 2^52 (round to nearest even, as llrint); FP64 fields keep the
@@ -644,7 +649,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
         }
         t = rb[a] + (f - rl[a]);
         const double4 d = dep[t];
-        if (d.w > 0.0) {
+        if (FIX ? d.w > 0.0 : d.w != 0.0) {
           const int rx = ((originOf(d.x, inv_dx) - c0x) % N + N) % N;
           const int ry = ((originOf(d.y, inv_dx) - c0y) % N + N) % N;
           const int rz = ((originOf(d.z, inv_dx) - c0z) % N + N) % N;
@@ -664,7 +669,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
     for (int i = tid; i < n; i += NT) {
       const double4 d = dep[list[i]];
       // stencil weights in the field precision (FP32 fields: FP32 sines and cosines)
-      using GT = std::conditional_t<sizeof(T) == 4, float, double>;
+      using GT = std::conditional_t<FIX && sizeof(T) == 4, float, double>;
       GT wx[4], wy[4], wz[4];
       const int i0 = cosW4F<GT>(d.x, dx, inv_dx, pi_2dx, wx), j0 = cosW4F<GT>(d.y, dx, inv_dx, pi_2dx, wy),
                 k0 = cosW4F<GT>(d.z, dx, inv_dx, pi_2dx, wz);
@@ -688,12 +693,16 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
             const int nz = (rz + cc) % N;
             if (nz >= S) continue;
             const double v = wab * wzd[cc];
+            if constexpr (!FIX) {
+              atomicAdd(&tile[(nx * S + ny) * S + nz], v);
+              continue;
+            }
             unsigned long long q;
             if constexpr (F32)
               q = (unsigned long long)(__double_as_longlong(v + 0x1p52) - __double_as_longlong(0x1p52));
             else
               q = (unsigned long long)llrint(v);
-            atomicAdd(&tile[(nx * S + ny) * S + nz], q);
+            if constexpr (FIX) atomicAdd(&tile[(nx * S + ny) * S + nz], q);
           }
         }
       }
@@ -857,6 +866,157 @@ k_prhs(const double* __restrict__ coord, int np, const T* __restrict__ u, const 
   deposit<T, N>(s, W, P.inv_vol, fc);
   for (int c = 0; c < 7; ++c) { rhs[(size_t)p * 7 + c] = r[c]; interp[(size_t)p * 7 + c] = I[c]; }
   exterp[p] = W;
+}
+
+// ------------------------------------------------------------ sorted API path
+// With enough rows the API's gathers and deposits work on rows sorted by bin
+// (Engine::rows_sorted): k_row_bin counts the rows of each bin, the scans of
+// the step's sort give the bin starts, k_row_scatter writes each row's wrapped
+// position, weight and row number to its slot.  The gather then runs four
+// lanes per row (lane c owns z node c of the stencil), so one load touches 16
+// rows that lie in neighbouring cells, and the deposit takes the bricks.
+// Positions, weights and sums stay FP64.
+template <int N>
+__global__ void __launch_bounds__(256)
+k_row_bin(const double* __restrict__ rows, int np, double L, double inv_dx, int* __restrict__ key,
+          int* __restrict__ rank, int* __restrict__ hist) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= np) return;
+  int b[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) b[c] = cellOf<N>(wrapL(rows[(size_t)p * 7 + c], L), inv_dx) / Bins<N>::BS;
+  const int k = Bins<N>::key(b[0], b[1], b[2]);
+  key[p] = k;
+  rank[p] = atomicAdd(&hist[k], 1);
+}
+static __global__ void __launch_bounds__(256)
+k_row_scatter(const double* __restrict__ rows, int np, double L, const double* __restrict__ w,
+              const int* __restrict__ key, const int* __restrict__ rank, const int* __restrict__ start,
+              double4* __restrict__ dep, int* __restrict__ row) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= np) return;
+  const double* r = rows + (size_t)p * 7;
+  double4 d;
+  d.x = wrapL(r[0], L); d.y = wrapL(r[1], L); d.z = wrapL(r[2], L);
+  d.w = w ? w[p] : 0.0;
+  const int s = start[key[p]] + rank[p];
+  dep[s] = d;
+  row[s] = p;
+}
+
+// One slot's stencil, four lanes per slot: this lane's z node and weight, all
+// x and y nodes.  Lane c takes the sine and cosine of axis c (FP64) and the
+// four lanes share them.
+template <int N> struct QuadStencil {
+  int i0, j0, iz;
+  double wx[4], wy[4], wz;
+  __device__ __forceinline__ QuadStencil(const double4& d, int c, const DropPhys& P) {
+    i0 = originOf(d.x, P.inv_dx); j0 = originOf(d.y, P.inv_dx);
+    const int k0 = originOf(d.z, P.inv_dx);
+    const double x = c == 0 ? d.x : c == 1 ? d.y : d.z;
+    const int o = c == 0 ? i0 : c == 1 ? j0 : k0;
+    double sn, cs;
+    sincos((x - (double)o * P.dx) * P.pi_2dx, &sn, &cs);
+    const double xs = __shfl(sn, 0, 4), xc = __shfl(cs, 0, 4), ys = __shfl(sn, 1, 4), yc = __shfl(cs, 1, 4),
+                 zs = __shfl(sn, 2, 4), zc = __shfl(cs, 2, 4);
+    wx[0] = 0.25 * (1.0 + xc); wx[1] = 0.25 * (1.0 + xs); wx[2] = 0.25 * (1.0 - xc); wx[3] = 0.25 * (1.0 - xs);
+    wy[0] = 0.25 * (1.0 + yc); wy[1] = 0.25 * (1.0 + ys); wy[2] = 0.25 * (1.0 - yc); wy[3] = 0.25 * (1.0 - ys);
+    const double zt = (c & 1) ? zs : zc;
+    wz = 0.25 * (1.0 + ((c & 2) ? -zt : zt));
+    iz = wrapIdx<N>(k0 + c);
+  }
+  // node index of x node a, y node b and this lane's z node (< N^3 <= 2^27)
+  __device__ __forceinline__ uint32_t node(int a, int b) const {
+    return ((uint32_t)wrapIdx<N>(i0 + a) * N + (uint32_t)wrapIdx<N>(j0 + b)) * N + (uint32_t)iz;
+  }
+  // sum over the four lanes of v times this lane's z weight
+  __device__ __forceinline__ double sum(double v) const {
+    v *= wz;
+    v += __shfl_xor(v, 1, 4);
+    v += __shfl_xor(v, 2, 4);
+    return v;
+  }
+};
+// this lane's slot: blocks map XCD-aware (each XCD one contiguous range of slots)
+__device__ __forceinline__ int quadSlot() {
+  const int per = gridDim.x / 8, lb = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  return (lb * (int)blockDim.x + (int)threadIdx.x) >> 2;
+}
+
+// pRHS (particles.py:817-837) on sorted rows: rhs, interpolants and growth
+// rate in row order, W to the slot's deposit record.  Bound by the stencil
+// loads (112 per lane, each one 16-byte (FP32) run per row).
+template <typename T, int N>
+__global__ void __launch_bounds__(256)
+k_prhs_sorted(const double* __restrict__ coord, int np, const T* __restrict__ u, const T* __restrict__ us,
+              const T* __restrict__ n, double4* __restrict__ dep, const int* __restrict__ row0,
+              double* __restrict__ rhs, double* __restrict__ interp, double* __restrict__ exterp, DropPhys P) {
+  constexpr size_t R = (size_t)N * N * N;
+  const int s = quadSlot(), c = threadIdx.x & 3;
+  const bool live = s < np;
+  const double4 d = dep[live ? s : 0];
+  const size_t p = (size_t)row0[live ? s : 0];
+  const QuadStencil<N> q(d, c, P);
+  double I[7];
+#pragma unroll
+  for (int k = 0; k < 7; ++k) I[k] = 0.0;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    T f[4][7];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const uint32_t o = q.node(a, b);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) { f[b][k] = ld32(u + k * R, o); f[b][3 + k] = ld32(us + k * R, o); }
+      f[b][6] = ld32(n, o);
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const double w = q.wx[a] * q.wy[b];
+#pragma unroll
+      for (int k = 0; k < 7; ++k) I[k] += (double)f[b][k] * w;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 7; ++k) I[k] = q.sum(I[k]);
+  if (!live) return;
+  double vp[3], r[7], W;
+  const double* rw = coord + p * 7;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) vp[k] = rw[3 + k];
+  dropletRhs(P, vp, rw[6], I, r, W);
+  // the four lanes write the row's 56 bytes together
+#pragma unroll
+  for (int k = 0; k < 7; ++k)
+    if ((k & 3) == c) { rhs[p * 7 + k] = r[k]; interp[p * 7 + k] = I[k]; }
+  if (c == 0) {
+    exterp[p] = W;
+    dep[s].w = W;
+  }
+}
+
+// interp_cosine (particles.py:435-511) of sorted rows, one component at a time.
+template <typename T, int N>
+__global__ void __launch_bounds__(256)
+k_interp_sorted(int np, const T* __restrict__ f, int ncomp, const double4* __restrict__ dep,
+                const int* __restrict__ row0, double* __restrict__ out, DropPhys P) {
+  constexpr size_t R = (size_t)N * N * N;
+  const int s = quadSlot(), c = threadIdx.x & 3;
+  const bool live = s < np;
+  const double4 d = dep[live ? s : 0];
+  const size_t p = (size_t)row0[live ? s : 0];
+  const QuadStencil<N> q(d, c, P);
+  for (int k = 0; k < ncomp; ++k) {
+    const T* fk = f + (size_t)k * R;
+    T v[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) v[e] = ld32(fk, q.node(e >> 2, e & 3));
+    double t = 0.0;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) t += (double)v[e] * (q.wx[e >> 2] * q.wy[e & 3]);
+    t = q.sum(t);
+    if (live && c == (k & 3)) out[p * ncomp + k] = t;
+  }
 }
 
 // AoS (Np, 7) rows <-> engine SoA state.

@@ -177,7 +177,7 @@ class ForcedDNS:
         kn = self.zeros_real() if kn is None else self._chk(kn, self.rdtype, self.rshape(), "kn")
         fc = self.zeros_real() if fc is None else self._chk(fc, self.rdtype, self.rshape(), "fc")
         coord, npart = self._rows(coord)
-        kp = torch.zeros((npart, 7), dtype=torch.float64, device=self.device)
+        kp = torch.empty((npart, 7), dtype=torch.float64, device=self.device)     # every row is written
         if u_out is not None:
             self._chk(u_out, self.rdtype, self.rshape(3), "u_out")
         if v_out is not None:

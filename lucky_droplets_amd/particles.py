@@ -93,7 +93,7 @@ class MPI_particles:
         ncomp = u.shape[0]
         self.dns._chk(u, self.dns.rdtype, (ncomp,) + (self.N,) * 3, "u")
         coord, npart = self.dns._rows(coord)
-        out = torch.zeros((npart, ncomp), dtype=torch.float64, device=self.dns.device)
+        out = torch.empty((npart, ncomp), dtype=torch.float64, device=self.dns.device)
         self.dns._stream()
         _lib.check(self.dns.lib.ld_interp_cosine(self.dns.ctx, _ptr(coord), npart, _ptr(u), ncomp, _ptr(out)))
         self.interpmat = out
@@ -180,9 +180,9 @@ class MPI_particles:
         dns._chk(us, dns.rdtype, (3,) + (self.N,) * 3, "us")
         dns._chk(c, dns.rdtype, (self.N,) * 3, "c")
         dns._chk(fc, dns.rdtype, (self.N,) * 3, "fc")
-        rhs = torch.zeros((npart, 7), dtype=torch.float64, device=dns.device)
-        interp = torch.zeros((npart, 7), dtype=torch.float64, device=dns.device)
-        ext = torch.zeros((npart,), dtype=torch.float64, device=dns.device)
+        rhs = torch.empty((npart, 7), dtype=torch.float64, device=dns.device)     # every row is written
+        interp = torch.empty((npart, 7), dtype=torch.float64, device=dns.device)
+        ext = torch.empty((npart,), dtype=torch.float64, device=dns.device)
         dns._stream()
         _lib.check(dns.lib.ld_prhs(dns.ctx, _ptr(coord), npart, _ptr(u), _ptr(us), _ptr(c), _ptr(fc), _ptr(rhs),
                                    _ptr(interp), _ptr(ext)))

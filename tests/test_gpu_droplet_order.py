@@ -3,6 +3,12 @@ the result.
 
 * RK4 sorts its rows by bin; the deposit's fixed-point sums do not depend on
   the order, so permuted rows give the same bits, row by row.
+* interp_cosine, exterp_cosine_scalar and pRHS sort their rows by bin when
+  there are enough of them; LD_ROW_SORT_MIN moves that line, so both paths run
+  on the same rows here.  FP64 tolerance: the stencil angle (x - X) pi / (2 dx)
+  carries x's rounding, eps 2 pi / dx pi/2 < 4e-14 at 64^3; 1e-12 of the
+  largest value covers sums of it.  FP32 deposits: the general path rounds each
+  of the up to 100 additions into a node to FP32, 100 x 6e-8.
 """
 import numpy as np
 import pytest
@@ -45,3 +51,69 @@ def test_rk4_row_order_keeps_the_bits(gpu, N, prec, npart, speed):
     assert np.isfinite(out[0][0]).all() and np.isfinite(out[0][2]).all()
     assert np.array_equal(out[0][0][perm], out[1][0])
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
+
+
+def _edge_rows(cfg, npart, seed):
+    """Rows over several boxes (unwrapped), on nodes, on the box faces, at bin and brick edges."""
+    rng = np.random.default_rng(seed)
+    rows = rng.uniform(0, cfg.L, (npart, 7))
+    rows[:, :3] += cfg.L * rng.integers(-3, 4, (npart, 3))
+    dx = cfg.L / cfg.N
+    special = [0.0, cfg.L, -dx, np.nextafter(cfg.L, 0), np.nextafter(0.0, -1), 8 * dx, 16 * dx, 2 * dx, cfg.L - dx]
+    for i, v in enumerate(special[:npart]):
+        rows[i, :3] = np.roll([v, special[(i + 1) % len(special)], 0.3 * cfg.L], i)
+    rows[:, 6] = rng.uniform(0.05, 1.0, npart) ** 1.5 * cfg.factor
+    return rows
+
+
+@pytest.mark.parametrize("N,prec,npart", [(16, "f64", 1), (16, "f32", 8000), (32, "f64", 63), (32, "f32", 4097),
+                                          (64, "f64", 20011), (64, "f32", 20011)])
+def test_sorted_rows_match_general_path(gpu, N, prec, npart, monkeypatch):
+    import torch
+    from lucky_droplets_amd.dns import ForcedDNS
+    cfg = Config(N=N, precision=prec, nu=0.02, n_particles=npart, gravity=True)
+    rng = np.random.default_rng(N + npart)
+    fields = rng.standard_normal((5, N, N, N))
+    dens = rng.standard_normal((N, N, N))         # negative values too: signed growth
+    w = rng.standard_normal(npart) * 10.0 ** rng.uniform(-6, 6, npart)
+    rows = _edge_rows(cfg, npart, 5)
+    got = {}
+    for line in (0, 1 << 40):
+        monkeypatch.setenv("LD_ROW_SORT_MIN", str(line))
+        d = ForcedDNS(cfg)
+        stb = _population(d, cfg, rows)
+        f, n = _t(fields, gpu, d.rdtype), _t(dens, gpu, d.rdtype)
+        out = {"interp": stb.interp_cosine(stb.coord, f).clone()}
+        stb.exterpmat = _t(w, gpu, torch.float64)[:, None]
+        out["deposit"] = stb.exterp_cosine_scalar(stb.coord, torch.full_like(n, 7.0))
+        _, rhs, fc = stb.pRHS(0.0, stb.coord, f[:3].contiguous(), f[2:].contiguous(), n, torch.full_like(n, 7.0), None)
+        out.update(rhs=rhs, fc=fc, I=stb.interpmat, W=stb.exterpmat)
+        # a weight that is not finite reaches its own 64 nodes only
+        w2 = w.copy(); w2[npart // 2] = np.nan
+        stb.exterpmat = _t(w2, gpu, torch.float64)[:, None]
+        out["poison"] = stb.exterp_cosine_scalar(stb.coord, torch.zeros_like(n))
+        got[line] = {k: v.cpu().numpy() for k, v in out.items()}
+        d.close()
+    a, b = got[0], got[1 << 40]
+    for k in a:
+        if k == "poison":
+            assert np.array_equal(np.isnan(a[k]), np.isnan(b[k])) and np.isnan(a[k]).any()
+            continue
+        tol = 1e-12 if prec == "f64" or k not in ("deposit", "fc") else 100 * 6e-8
+        assert np.max(np.abs(a[k].astype(np.float64) - b[k])) <= tol * np.max(np.abs(b[k])), k
+
+
+def test_more_rows_than_the_capacity(gpu):
+    """The sorted path's scratch holds the context's capacity; more rows take the general path."""
+    import torch
+    from lucky_droplets_amd.dns import ForcedDNS
+    cfg = Config(N=32, precision="f64", nu=0.02, n_particles=4096)
+    rows = _edge_rows(cfg, 9000, 6)
+    f = np.random.default_rng(1).standard_normal((1, 32, 32, 32))
+    out = []
+    for cap in (4096, 9000):
+        d = ForcedDNS(cfg, max_particles=cap)
+        stb = _population(d, cfg, rows)
+        out.append(stb.interp_cosine(stb.coord, _t(f, gpu, torch.float64)).cpu().numpy())
+        d.close()
+    assert np.max(np.abs(out[0] - out[1])) <= 1e-12 * np.max(np.abs(out[1]))
