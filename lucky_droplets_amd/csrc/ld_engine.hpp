@@ -1305,20 +1305,22 @@ struct Engine final : EngineBase {
       return LD_ERR_ARG;
     }
     LD_TRY(join(st, st2, evB));
-    hipLaunchKernelGGL((k_shell_partial<T, N>), dim3(NBLK_DIAG), dim3(256), 0, st, (const C<T>*)f, (const C<T>*)nullptr,
+    hipLaunchKernelGGL((k_shell_partial<T, N>), dim3(NBLK_DIAG), dim3(DIAG_NT), 0, st, (const C<T>*)f, (const C<T>*)nullptr,
                        nf, CF, 0, w, norm0(), ws);
     LD_LAUNCHED();
-    hipLaunchKernelGGL((k_shell_final<N>), dim3(1), dim3(256), 0, st, (const double*)ws, NBLK_DIAG, 0, out);
+    hipLaunchKernelGGL((k_shell_final<N>), dim3(Nf), dim3(64), 0, st, (const double*)ws, NBLK_DIAG, out);
     LD_LAUNCHED();
     return LD_OK;
   }
   int flux(const void* ukin, const void* kuin, double* out) override {
     LD_TRY(diag_alloc());
     LD_TRY(join(st, st2, evB));
-    hipLaunchKernelGGL((k_shell_partial<T, N>), dim3(NBLK_DIAG), dim3(256), 0, st, (const C<T>*)ukin,
+    hipLaunchKernelGGL((k_shell_partial<T, N>), dim3(NBLK_DIAG), dim3(DIAG_NT), 0, st, (const C<T>*)ukin,
                        (const C<T>*)kuin, 3, CF, 1, 1.0, norm0(), dpart);
     LD_LAUNCHED();
-    hipLaunchKernelGGL((k_shell_final<N>), dim3(1), dim3(256), 0, st, (const double*)dpart, NBLK_DIAG, 1, out);
+    hipLaunchKernelGGL((k_shell_final<N>), dim3(Nf), dim3(64), 0, st, (const double*)dpart, NBLK_DIAG, out);
+    LD_LAUNCHED();
+    hipLaunchKernelGGL((k_shell_cumulate<N>), dim3(1), dim3(64), 0, st, out);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -1327,10 +1329,10 @@ struct Engine final : EngineBase {
   int dissipation(const void* ukin, double* out) override {
     LD_TRY(diag_alloc());
     LD_TRY(join(st, st2, evB));
-    hipLaunchKernelGGL((k_shell_partial<T, N>), dim3(NBLK_DIAG), dim3(256), 0, st, (const C<T>*)ukin,
+    hipLaunchKernelGGL((k_shell_partial<T, N>), dim3(NBLK_DIAG), dim3(DIAG_NT), 0, st, (const C<T>*)ukin,
                        (const C<T>*)nullptr, 3, CF, 2, p.nu, norm0(), dpart);
     LD_LAUNCHED();
-    hipLaunchKernelGGL((k_shell_final<N>), dim3(1), dim3(256), 0, st, (const double*)dpart, NBLK_DIAG, 0, out);
+    hipLaunchKernelGGL((k_shell_final<N>), dim3(Nf), dim3(64), 0, st, (const double*)dpart, NBLK_DIAG, out);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -1354,7 +1356,7 @@ struct Engine final : EngineBase {
       LD_HIP(hipStreamSynchronize(st));
       return LD_OK;
     }
-    hipLaunchKernelGGL((k_stats_partial<PT>), dim3(NBLK_DIAG), dim3(256), 0, st, (const PT*)(v0 + 3 * cap),
+    hipLaunchKernelGGL((k_stats_partial<PT>), dim3(NBLK_DIAG), dim3(DIAG_NT), 0, st, (const PT*)(v0 + 3 * cap),
                        (size_t)np, dpart);
     LD_LAUNCHED();
     hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(64), 0, st, (const double*)dpart, NBLK_DIAG, out);
@@ -1364,7 +1366,7 @@ struct Engine final : EngineBase {
   int stats(const void* x, int nf, double* out) override {
     LD_TRY(diag_alloc());
     LD_TRY(join(st, st2, evB));
-    hipLaunchKernelGGL((k_stats_partial<T>), dim3(NBLK_DIAG), dim3(256), 0, st, (const T*)x, (size_t)nf * RF, dpart);
+    hipLaunchKernelGGL((k_stats_partial<T>), dim3(NBLK_DIAG), dim3(DIAG_NT), 0, st, (const T*)x, (size_t)nf * RF, dpart);
     LD_LAUNCHED();
     hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(64), 0, st, (const double*)dpart, NBLK_DIAG, out);
     LD_LAUNCHED();

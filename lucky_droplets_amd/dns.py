@@ -287,7 +287,7 @@ class ForcedDNS:
         (forced-dns-sm.py:423, 431), the n spectrum with weight 1 (plot.py:37-38)."""
         nf = 1 if fk.dim() == 3 else fk.shape[0]
         self._chk(fk, self.cdtype, self.cshape(None if fk.dim() == 3 else nf), "fk")
-        out = torch.zeros(self.Nf, dtype=torch.float64, device=self.device)
+        out = torch.empty(self.Nf, dtype=torch.float64, device=self.device)
         self._stream()
         _lib.check(self.lib.ld_spectrum(self.ctx, _ptr(fk), nf, float(weight), _ptr(out)))
         return out
@@ -296,7 +296,7 @@ class ForcedDNS:
         """Pi(k) of save() (forced-dns-sm.py:425-428): full_RHS with visc = forc = 0
         (no droplets), Re(conj(uk) . ku) dealiased, shell-binned, cumulated from high k."""
         ku, _, _, _ = self.full_RHS(0.0, uk, n, None, None, visc=0, forc=0)
-        out = torch.zeros(self.Nf, dtype=torch.float64, device=self.device)
+        out = torch.empty(self.Nf, dtype=torch.float64, device=self.device)
         self._stream()
         _lib.check(self.lib.ld_flux(self.ctx, _ptr(uk), _ptr(ku), _ptr(out)))
         return out
@@ -305,7 +305,7 @@ class ForcedDNS:
         """(sum, min, max, sum of squares) of one or several real fields."""
         nf = 1 if x.dim() == 3 else x.shape[0]
         self._chk(x, self.rdtype, self.rshape(None if x.dim() == 3 else nf), "x")
-        out = torch.zeros(4, dtype=torch.float64, device=self.device)
+        out = torch.empty(4, dtype=torch.float64, device=self.device)
         self._stream()
         _lib.check(self.lib.ld_field_stats(self.ctx, _ptr(x), nf, _ptr(out)))
         return tuple(out.cpu().tolist())
@@ -314,7 +314,7 @@ class ForcedDNS:
         """Dissipation spectrum nu |k|^2 sum_c |u_c|^2 normalize by shell (N/2+1,);
         its sum is the dissipation rate 2 nu sum_k k^2 E(k)."""
         self._chk(uk, self.cdtype, self.cshape(3), "uk")
-        out = torch.zeros(self.Nf, dtype=torch.float64, device=self.device)
+        out = torch.empty(self.Nf, dtype=torch.float64, device=self.device)
         self._stream()
         _lib.check(self.lib.ld_dissipation(self.ctx, _ptr(uk), _ptr(out)))
         return out
@@ -334,7 +334,7 @@ class ForcedDNS:
 
     def droplet_stats(self):
         """(sum, min, max, sum of squares) of the resident droplets' mass m/M0."""
-        out = torch.zeros(4, dtype=torch.float64, device=self.device)
+        out = torch.empty(4, dtype=torch.float64, device=self.device)
         self._stream()
         _lib.check(self.lib.ld_droplet_stats(self.ctx, _ptr(out)))
         return tuple(out.cpu().tolist())
