@@ -34,129 +34,235 @@ k_coll_count(const double* __restrict__ rows, int np, double L, double cell, int
   rank[p] = atomicAdd(&hist[k], 1);
 }
 
+// Droplets in cell order: wrapped position and radius, input row, and (for the
+// statistics) velocity, so the pair search reads 32-byte records that its
+// neighbours read too instead of 56-byte rows through an index.
 static __global__ void __launch_bounds__(256)
-k_coll_scatter(int np, const int* __restrict__ key, const int* __restrict__ rank, const int* __restrict__ start,
-               int* __restrict__ order) {
+k_coll_scatter(const double* __restrict__ rows, const double* __restrict__ rad, int np, double L,
+               const int* __restrict__ key, const int* __restrict__ rank, const int* __restrict__ start,
+               int* __restrict__ order, double4* __restrict__ pos, double4* __restrict__ vel) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < np) order[start[key[p]] + rank[p]] = p;
-}
-
-// Minimum-image separation and the pair test, no contraction into FMA.
-__device__ __forceinline__ bool collideTest(const double* __restrict__ ri, const double* __restrict__ rj, double L,
-                                            double radi, double radj) {
-#pragma clang fp contract(off)
-  double d[3];
-  for (int a = 0; a < 3; ++a) {
-    double t = wrapL(rj[a], L) - wrapL(ri[a], L);
-    t = t - L * rint(t / L);
-    d[a] = t;
+  if (p >= np) return;
+  const int s = start[key[p]] + rank[p];
+  const double* r = rows + (size_t)p * 7;
+  order[s] = p;
+  double4 x;
+  x.x = wrapL(r[0], L); x.y = wrapL(r[1], L); x.z = wrapL(r[2], L); x.w = rad ? rad[p] : 0.0;
+  pos[s] = x;
+  if (vel) {
+    double4 v;
+    v.x = r[3]; v.y = r[4]; v.z = r[5]; v.w = 0.0;
+    vel[s] = v;
   }
-  const double d2 = (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2];
-  const double s = radi + radj;
-  return d2 < s * s;
 }
 
-// One thread per droplet i: every droplet j > i in the 27 neighbouring cells
-// (nc >= 3) or in the single cell (nc == 1).  Pairs are appended as
-// (i << 32 | j) through an atomic counter; the caller sorts them.
-static __global__ void __launch_bounds__(256)
-k_coll_pairs(const double* __restrict__ rows, const double* __restrict__ rad, int np, double L, double cell, int nc,
-             const int* __restrict__ start, const int* __restrict__ order, const int* __restrict__ key,
-             unsigned long long* __restrict__ out, unsigned long long max_pairs,
-             unsigned long long* __restrict__ count) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  const double* xi = rows + (size_t)i * 7;
-  const double ri = rad[i];
-  const int ki = key[i];
-  const int cx = ki / (nc * nc), cy = (ki / nc) % nc, cz = ki % nc;
-  const int span = nc >= 3 ? 1 : 0;
-  const int ncells = nc * nc * nc;
-  for (int ox = -span; ox <= span; ++ox)
-    for (int oy = -span; oy <= span; ++oy)
-      for (int oz = -span; oz <= span; ++oz) {
-        const int c = ((((cx + ox) % nc + nc) % nc) * nc + (((cy + oy) % nc + nc) % nc)) * nc + (((cz + oz) % nc + nc) % nc);
-        const int b = start[c], e = (c + 1 < ncells) ? start[c + 1] : np;
-        for (int t = b; t < e; ++t) {
-          const int j = order[t];
-          if (j <= i) continue;
-          if (collideTest(xi, rows + (size_t)j * 7, L, ri, rad[j])) {
-            const unsigned long long slot = atomicAdd(count, 1ull);
-            if (slot < max_pairs) out[slot] = ((unsigned long long)i << 32) | (unsigned long long)(unsigned)j;
-          }
-        }
-      }
+// Minimum-image separation b - a of wrapped positions.  t / L of a wrapped
+// difference lies in [-1, 1], so rint(t / L) is 1 above L/2, -1 below -L/2
+// and 0 between: t > L/2 makes the quotient round above 1/2 (the distance
+// from L/2 to the next double is more than half the quotient's spacing), and
+// t <= L/2 makes it round to at most 1/2, which rint takes to 0.
+__device__ __forceinline__ double minImage(double a, double b, double L) {
+#pragma clang fp contract(off)
+  const double t = b - a, h = 0.5 * L;
+  return t > h ? t - L : (t < -h ? t + L : t);
+}
+__device__ __forceinline__ double separation(const double4& a, const double4& b, double L, double d[3]) {
+#pragma clang fp contract(off)
+  d[0] = minImage(a.x, b.x, L); d[1] = minImage(a.y, b.y, L); d[2] = minImage(a.z, b.z, L);
+  return (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2];
 }
 
-// Pair statistics within a cutoff (no reference counterpart; the input of the
-// radial distribution function and the kinematic collision kernel).  For every
-// pair i < j with d2 < rmax^2 (minimum image, the pair-test formula above):
-//   dist = sqrt(d2), bin k = min((int)(dist / dr), nbins - 1),
+// Pair search over the cell list, one thread per droplet in cell order.  Each
+// unordered pair is met once: a droplet tests the slots after it in its own
+// cell and every slot of the next z cell and of four of the eight neighbouring
+// (x, y) columns (nc >= 3; one cell holding everything tests the slots after
+// its own).  The cells along z are consecutive, so that is at most ten slot
+// ranges, which a lane walks as one sequence: a wavefront's steps are its
+// longest lane's candidates.  Pairs that pass the test go to a queue in LDS,
+// and the wavefront works them off 64 at a time, so that the pair work (square
+// root and divisions for the statistics) runs with full lanes.
+//
+// STATS = false: pairs with d2 < (r_i + r_j)^2, appended as (i << 32 | j), i < j
+// the input rows, through one atomic per batch; the caller sorts them.
+// STATS = true (no reference counterpart; the input of the radial
+// distribution function and the kinematic collision kernel): for every pair
+// with d2 < rmax^2: dist = sqrt(d2), bin k = min((int)(dist / dr), nbins - 1),
 //   w_r = ((dv_x d_x + dv_y d_y) + dv_z d_z) / dist  (dv = v_j - v_i; 0 if dist == 0),
-//   counts[k] += 1, wsum[k] += |w_r|, wneg[k] += max(-w_r, 0).
-// Per-block LDS histograms, then one global atomic per bin and block; counts
+//   counts[k] += 1, wsum[k] += |w_r|, wneg[k] += max(-w_r, 0),
+// in LDS histograms per block, then one global atomic per bin and block; counts
 // are exact, the FP64 sums depend on the summation order.
-static __global__ void __launch_bounds__(256)
-k_pair_stats(const double* __restrict__ rows, int np, double L, double cell, int nc, const int* __restrict__ start,
-             const int* __restrict__ order, const int* __restrict__ key, double rmax, double dr, int nbins,
-             unsigned long long* __restrict__ counts, double* __restrict__ wsum, double* __restrict__ wneg) {
+//
+// Bound by the candidates' 32-byte loads and FP64 tests.  10^6 droplets, rmax
+// 0.1 (8.4 million pairs): 2590 us when each droplet read all 27 cells' rows
+// through the index with a wrap and divisions per candidate and the pair work
+// ran in the lanes that found a pair; 286 us now.  Collision pairs of the same
+// droplets 522 -> 95 us.
+struct NearArgs {
+  const double4 *pos, *vel;
+  const int *order, *start;
+  int np, nc;
+  double L, cell;
+  unsigned long long *out, max_pairs, *count;                   // pairs
+  double rmax, dr;                                               // statistics
+  int nbins;
+  unsigned long long* counts;
+  double *wsum, *wneg;
+};
+template <bool STATS> struct NearHist { unsigned long long c[512]; double w[512], n[512]; };
+template <> struct NearHist<false> {};
+template <bool STATS>
+__global__ void __launch_bounds__(256) k_near(NearArgs A) {
 #pragma clang fp contract(off)
-  __shared__ unsigned long long hc[512];
-  __shared__ double hw[512], hn[512];
-  for (int k = threadIdx.x; k < nbins; k += blockDim.x) { hc[k] = 0ull; hw[k] = 0.0; hn[k] = 0.0; }
-  __syncthreads();
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < np) {
-    const double* xi = rows + (size_t)i * 7;
-    double pi[3];
-    for (int a = 0; a < 3; ++a) pi[a] = wrapL(xi[a], L);
-    const double r2max = rmax * rmax;
-    const int ki = key[i];
-    const int cx = ki / (nc * nc), cy = (ki / nc) % nc, cz = ki % nc;
-    const int span = nc >= 3 ? 1 : 0;
-    const int ncells = nc * nc * nc;
-    for (int ox = -span; ox <= span; ++ox)
-      for (int oy = -span; oy <= span; ++oy)
-        for (int oz = -span; oz <= span; ++oz) {
-          const int c = ((((cx + ox) % nc + nc) % nc) * nc + (((cy + oy) % nc + nc) % nc)) * nc + (((cz + oz) % nc + nc) % nc);
-          const int b = start[c], e = (c + 1 < ncells) ? start[c + 1] : np;
-          for (int t = b; t < e; ++t) {
-            const int j = order[t];
-            if (j <= i) continue;
-            const double* xj = rows + (size_t)j * 7;
-            double d[3];
-            for (int a = 0; a < 3; ++a) {
-              double u = wrapL(xj[a], L) - pi[a];
-              u = u - L * rint(u / L);
-              d[a] = u;
-            }
-            const double d2 = (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2];
-            if (!(d2 < r2max)) continue;
-            const double dist = sqrt(d2);
-            int k = (int)(dist / dr);
-            k = k < nbins ? k : nbins - 1;
-            double wr = 0.0;
-            if (dist > 0.0) {
-              const double dv0 = xj[3] - xi[3], dv1 = xj[4] - xi[4], dv2 = xj[5] - xi[5];
-              wr = ((dv0 * d[0] + dv1 * d[1]) + dv2 * d[2]) / dist;
-            }
-            atomicAdd(&hc[k], 1ull);
-            atomicAdd(&hw[k], fabs(wr));
-            if (wr < 0.0) atomicAdd(&hn[k], -wr);
-          }
-        }
+  __shared__ NearHist<STATS> H;
+  __shared__ int2 queue[4][128];
+  if constexpr (STATS) {
+    for (int k = threadIdx.x; k < A.nbins; k += 256) { H.c[k] = 0ull; H.w[k] = 0.0; H.n[k] = 0.0; }
+    __syncthreads();
   }
-  __syncthreads();
-  for (int k = threadIdx.x; k < nbins; k += blockDim.x) {
-    if (hc[k]) {
-      atomicAdd(&counts[k], hc[k]);
-      unsafeAtomicAdd(&wsum[k], hw[k]);
-      unsafeAtomicAdd(&wneg[k], hn[k]);
+  const int lane = threadIdx.x & 63;
+  int2* q = queue[threadIdx.x >> 6];
+  const int per = gridDim.x / 8, lb = (blockIdx.x % 8) * per + blockIdx.x / 8;   // XCD-aware: contiguous slots
+  const int nc = A.nc, np = A.np;
+  const uint32_t slot = (uint32_t)lb * 256u + threadIdx.x;
+  bool run = slot < (uint32_t)np;
+  const int s = run ? (int)slot : 0;
+  double4 me = {0.0, 0.0, 0.0, 0.0};
+  int cx = 0, cy = 0, cz = 0, t = 0, e = 0;
+  if (run) {
+    me = A.pos[s];
+    cx = collCell(me.x, A.cell, nc); cy = collCell(me.y, A.cell, nc); cz = collCell(me.z, A.cell, nc);
+    const int own = (cx * nc + cy) * nc + cz, last = (nc >= 3 && cz + 1 < nc) ? own + 1 : own;
+    t = s + 1;
+    e = last + 1 < nc * nc * nc ? A.start[last + 1] : np;
+  }
+  int r = 0;                         // range number: 0 done above, 1 own column's wrapped cell, 2.. columns
+  const double r2max = A.rmax * A.rmax;
+  int qn = 0;
+  auto work = [&](int n) {           // the queue's first n (<= 64) pairs, one per lane
+    int2 ij = {0, 0};
+    if (lane < n) ij = q[lane];
+    if constexpr (STATS) {
+      if (lane < n) {
+        double d[3];
+        const double4 a = A.pos[ij.x], b = A.pos[ij.y], va = A.vel[ij.x], vb = A.vel[ij.y];
+        const double dist = sqrt(separation(a, b, A.L, d));
+        int k = (int)(dist / A.dr);
+        k = k < A.nbins ? k : A.nbins - 1;
+        double wr = 0.0;
+        if (dist > 0.0) {
+          const double dv0 = vb.x - va.x, dv1 = vb.y - va.y, dv2 = vb.z - va.z;
+          wr = ((dv0 * d[0] + dv1 * d[1]) + dv2 * d[2]) / dist;
+        }
+        atomicAdd(&H.c[k], 1ull);
+        atomicAdd(&H.w[k], fabs(wr));
+        if (wr < 0.0) atomicAdd(&H.n[k], -wr);
+      }
+    } else {
+      unsigned long long base = 0;
+      if (lane == 0) base = atomicAdd(A.count, (unsigned long long)n);
+      base = __shfl(base, 0, 64);
+      if (lane < n && base + lane < A.max_pairs) {
+        const int i = A.order[ij.x], j = A.order[ij.y];
+        A.out[base + lane] = ((unsigned long long)(i < j ? i : j) << 32) | (unsigned long long)(unsigned)(i < j ? j : i);
+      }
     }
+  };
+  while (__any(run)) {
+    // the next non-empty range of a lane that has used up its own
+    while (run && t >= e) {
+      if (++r > 9 || nc < 3) { run = false; break; }
+      // r = 1: cell 0 of the own column when the next z cell wraps; then per
+      // column (0,1), (1,-1), (1,0), (1,1) the z-run cz-1..cz+1 as two pieces
+      const int col = r >> 1, piece = r & 1;
+      const int ox = col < 2 ? 0 : 1, oy = col == 0 ? 0 : col == 1 ? 1 : col - 3;
+      int z0, z1;                    // cells [z0, z1) of the column
+      if (col == 0) {
+        if (cz + 1 < nc) continue;
+        z0 = 0; z1 = 1;
+      } else if (piece == 0) {
+        z0 = cz > 0 ? cz - 1 : 0; z1 = cz + 2 < nc ? cz + 2 : nc;
+      } else {
+        if (cz > 0 && cz + 1 < nc) continue;
+        z0 = cz == 0 ? nc - 1 : 0; z1 = z0 + 1;
+      }
+      const int x = cx + ox < nc ? cx + ox : 0, y = cy + oy < 0 ? nc - 1 : (cy + oy < nc ? cy + oy : 0);
+      const int c0 = (x * nc + y) * nc;
+      t = A.start[c0 + z0];
+      e = c0 + z1 < nc * nc * nc ? A.start[c0 + z1] : np;
+    }
+    bool near = false;
+    if (run) {
+      double d[3];
+      const double4 b = A.pos[t];
+      const double d2 = separation(me, b, A.L, d);
+      if constexpr (STATS) near = d2 < r2max;
+      else { const double sr = me.w + b.w; near = d2 < sr * sr; }
+    }
+    const unsigned long long m = __ballot(near);
+    if (m) {
+      if (near) {
+        const int at = qn + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+        q[at] = make_int2(s, t);
+      }
+      qn += __popcll(m);
+      __builtin_amdgcn_wave_barrier();
+      if (qn >= 64) {
+        work(64);
+        __builtin_amdgcn_wave_barrier();
+        qn -= 64;
+        int2 rest = {0, 0};
+        if (lane < qn) rest = q[64 + lane];
+        __builtin_amdgcn_wave_barrier();
+        if (lane < qn) q[lane] = rest;
+        __builtin_amdgcn_wave_barrier();
+      }
+    }
+    ++t;
+  }
+  if (qn) work(qn);
+  if constexpr (STATS) {
+    __syncthreads();
+    for (int k = threadIdx.x; k < A.nbins; k += 256)
+      if (H.c[k]) {
+        atomicAdd(&A.counts[k], H.c[k]);
+        unsafeAtomicAdd(&A.wsum[k], H.w[k]);
+        unsafeAtomicAdd(&A.wneg[k], H.n[k]);
+      }
   }
 }
 
-// One compare-exchange step of a bitonic sort over n = 2^m keys.
+// Bitonic sort of n = 2^m keys (the first cnt are given, the rest count as
+// largest).  k_bitonic_block does every step whose partner lies in the same
+// 2048-key chunk in LDS: with k = 0 it sorts each chunk from unsorted keys,
+// else it finishes the merges of length k.  k_bitonic does one step across
+// chunks.  116 pairs of 10^6 droplets: 28 launches of one step each before,
+// one now, which also writes the pairs (`pairs` set: n <= 2048).
+constexpr int SORT_CHUNK = 2048;
+static __global__ void __launch_bounds__(1024)
+k_bitonic_block(unsigned long long* __restrict__ a, int cnt, int n, int k, int64_t* __restrict__ pairs) {
+  __shared__ unsigned long long sh[SORT_CHUNK];
+  const int base = blockIdx.x * SORT_CHUNK, len = n < SORT_CHUNK ? n : SORT_CHUNK;
+  for (int i = threadIdx.x; i < len; i += 1024) sh[i] = base + i < cnt ? a[base + i] : ~0ull;
+  __syncthreads();
+  for (int kk = k ? k : 2; kk <= (k ? k : len); kk <<= 1)
+    for (int j = kk / 2 < len / 2 ? kk / 2 : len / 2; j > 0; j >>= 1) {
+      for (int p = threadIdx.x; p < len / 2; p += 1024) {
+        const int i = 2 * p - (p & (j - 1));        // the pair's lower key: bit j clear
+        const bool up = ((base + i) & kk) == 0;
+        const unsigned long long x = sh[i], y = sh[i + j];
+        if ((x > y) == up) { sh[i] = y; sh[i + j] = x; }
+      }
+      __syncthreads();
+    }
+  if (pairs) {
+    for (int i = threadIdx.x; i < cnt; i += 1024) {
+      pairs[2 * i] = (int64_t)(sh[i] >> 32);
+      pairs[2 * i + 1] = (int64_t)(sh[i] & 0xffffffffull);
+    }
+  } else {
+    for (int i = threadIdx.x; i < len; i += 1024) a[base + i] = sh[i];
+  }
+}
 static __global__ void __launch_bounds__(256)
 k_bitonic(unsigned long long* __restrict__ a, int n, int j, int k) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;

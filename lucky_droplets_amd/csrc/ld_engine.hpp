@@ -1375,6 +1375,7 @@ struct Engine final : EngineBase {
 
   // ------------------------------------------------------------ collisions
   int *ckey = nullptr, *crank = nullptr, *corder = nullptr, *chist = nullptr, *cbsum = nullptr, *cused = nullptr;
+  double4 *cpos = nullptr, *cvel = nullptr;
   unsigned long long *ckeys = nullptr, *ccount = nullptr;
   int *cnev = nullptr;
   int64_t ccap = 0, ckcap = 0;
@@ -1382,18 +1383,33 @@ struct Engine final : EngineBase {
 
   static int64_t pow2ceil(int64_t x) { int64_t v = 2; while (v < x) v <<= 1; return v; }
 
+  // Workspaces grow by at least half, so what earlier sizes leave behind (until
+  // the context goes) stays below twice the largest.
+  int coll_reserve(int64_t n_) {
+    if (n_ <= ccap) return LD_OK;
+    const int64_t n2 = n_ > ccap + ccap / 2 ? n_ : ccap + ccap / 2;
+    ccap = 0;
+    LD_TRY(alloc(ckey, n2)); LD_TRY(alloc(crank, n2)); LD_TRY(alloc(corder, n2)); LD_TRY(alloc(cused, n2));
+    LD_TRY(alloc(cpos, n2)); LD_TRY(alloc(cvel, n2));
+    ccap = n2;
+    return LD_OK;
+  }
+
   // Cell list of the droplet rows on st: cells of side >= reach (fewer than 3
-  // per side -> one cell, all pairs); bin starts in chist, slots in corder.
-  int build_cells(const double* rows, int64_t n_, double reach, int& nc, double& cell) {
-    nc = (reach > 0.0) ? (int)floor(p.L / reach) : 256;
-    if (nc > 256) nc = 256;
+  // per side -> one cell, all pairs), and no more of them than about one per
+  // droplet (256 per side at most): 10^6 droplets whose pairs reach 1/4000 of
+  // the box took 256^3 cells, whose counts and scans cost more than the few
+  // candidates that 100^3 add.  Cell starts in chist; positions, radii and
+  // (with_vel) velocities in cell order in cpos and cvel, input rows in corder.
+  int build_cells(const double* rows, const double* rad, int64_t n_, double reach, bool with_vel, int& nc,
+                  double& cell) {
+    int most = 3;
+    while (most < 256 && (int64_t)most * most * most < n_) ++most;
+    nc = (reach > 0.0 && p.L / reach < (double)most) ? (int)floor(p.L / reach) : most;
     if (nc < 3) nc = 1;
     cell = p.L / nc;
     const int ncells = nc * nc * nc;
-    if (n_ > ccap) {
-      LD_TRY(alloc(ckey, n_)); LD_TRY(alloc(crank, n_)); LD_TRY(alloc(corder, n_)); LD_TRY(alloc(cused, n_));
-      ccap = n_;
-    }
+    LD_TRY(coll_reserve(n_));
     if (ncells > chist_cap) {
       LD_TRY(alloc(chist, ncells)); LD_TRY(alloc(cbsum, (ncells + 4095) / 4096));
       chist_cap = ncells;
@@ -1410,11 +1426,18 @@ struct Engine final : EngineBase {
     hipLaunchKernelGGL(k_scan_add, dim3((ncells + 255) / 256), dim3(256), 0, st, chist, ncells, (const int*)cbsum,
                        (size_t)0);
     LD_LAUNCHED();
-    hipLaunchKernelGGL(k_coll_scatter, dim3(pb), dim3(256), 0, st, (int)n_, (const int*)ckey, (const int*)crank,
-                       (const int*)chist, corder);
+    hipLaunchKernelGGL(k_coll_scatter, dim3(pb), dim3(256), 0, st, rows, rad, (int)n_, p.L, (const int*)ckey,
+                       (const int*)crank, (const int*)chist, corder, cpos, with_vel ? cvel : (double4*)nullptr);
     LD_LAUNCHED();
     return LD_OK;
   }
+  NearArgs near_args(int64_t n_, int nc, double cell) const {
+    NearArgs a{};
+    a.pos = cpos; a.vel = cvel; a.order = corder; a.start = chist;
+    a.np = (int)n_; a.nc = nc; a.L = p.L; a.cell = cell;
+    return a;
+  }
+  static unsigned near_blocks(int64_t n_) { return (unsigned)(((n_ + 255) / 256 + 7) / 8 * 8); }
 
   int pair_stats(const double* rows, int64_t n_, double rmax, int nbins, int64_t* counts, double* wsum,
                  double* wneg) override {
@@ -1428,10 +1451,11 @@ struct Engine final : EngineBase {
     if (n_ < 2) return LD_OK;
     int nc;
     double cell;
-    LD_TRY(build_cells(rows, n_, rmax, nc, cell));
-    hipLaunchKernelGGL(k_pair_stats, dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, rows, (int)n_, p.L, cell,
-                       nc, (const int*)chist, (const int*)corder, (const int*)ckey, rmax, rmax / nbins, nbins,
-                       (unsigned long long*)counts, wsum, wneg);
+    LD_TRY(build_cells(rows, nullptr, n_, rmax, true, nc, cell));
+    NearArgs a = near_args(n_, nc, cell);
+    a.rmax = rmax; a.dr = rmax / nbins; a.nbins = nbins;
+    a.counts = (unsigned long long*)counts; a.wsum = wsum; a.wneg = wneg;
+    hipLaunchKernelGGL((k_near<true>), dim3(near_blocks(n_)), dim3(256), 0, st, a);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -1445,15 +1469,14 @@ struct Engine final : EngineBase {
     // cells of side >= 2 rmax (the largest pair distance)
     int nc;
     double cell;
-    LD_TRY(build_cells(rows, n_, 2.0 * rmax, nc, cell));
+    LD_TRY(build_cells(rows, rad, n_, 2.0 * rmax, false, nc, cell));
     const int64_t kc = pow2ceil(max_pairs > 2 ? max_pairs : 2);
     if (kc > ckcap) { LD_TRY(alloc(ckeys, kc)); ckcap = kc; }
     if (!ccount) { LD_TRY(alloc(ccount, 1)); LD_TRY(alloc(cnev, 1)); }
-    const unsigned pb = (unsigned)((n_ + 255) / 256);
     LD_TRY(fill<unsigned long long>(st, ccount, 1, 0ull));
-    hipLaunchKernelGGL(k_coll_pairs, dim3(pb), dim3(256), 0, st, rows, rad, (int)n_, p.L, cell, nc,
-                       (const int*)chist, (const int*)corder, (const int*)ckey, ckeys,
-                       (unsigned long long)max_pairs, ccount);
+    NearArgs a = near_args(n_, nc, cell);
+    a.out = ckeys; a.max_pairs = (unsigned long long)max_pairs; a.count = ccount;
+    hipLaunchKernelGGL((k_near<false>), dim3(near_blocks(n_)), dim3(256), 0, st, a);
     LD_LAUNCHED();
     unsigned long long cnt = 0;
     LD_HIP(hipMemcpyAsync(&cnt, ccount, sizeof(cnt), hipMemcpyDeviceToHost, st));
@@ -1465,13 +1488,20 @@ struct Engine final : EngineBase {
     }
     if (cnt == 0) return LD_OK;
     const int n2 = (int)pow2ceil((int64_t)cnt);
-    if ((int64_t)n2 > (int64_t)cnt)
-      LD_TRY(fill<unsigned long long>(st, ckeys + cnt, (size_t)(n2 - (int64_t)cnt), ~0ull));
-    for (int k = 2; k <= n2; k <<= 1)
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        hipLaunchKernelGGL(k_bitonic, dim3((n2 + 255) / 256), dim3(256), 0, st, ckeys, n2, j, k);
+    const bool one = n2 <= SORT_CHUNK;
+    const unsigned chunks = one ? 1u : (unsigned)(n2 / SORT_CHUNK);
+    hipLaunchKernelGGL(k_bitonic_block, dim3(chunks), dim3(1024), 0, st, ckeys, (int)cnt, n2, 0,
+                       one ? pairs : (int64_t*)nullptr);
+    LD_LAUNCHED();
+    if (one) return LD_OK;
+    for (int64_t k = 2 * SORT_CHUNK; k <= n2; k <<= 1) {
+      for (int64_t j = k >> 1; j >= SORT_CHUNK; j >>= 1) {
+        hipLaunchKernelGGL(k_bitonic, dim3((n2 + 255) / 256), dim3(256), 0, st, ckeys, n2, (int)j, (int)k);
         LD_LAUNCHED();
       }
+      hipLaunchKernelGGL(k_bitonic_block, dim3(chunks), dim3(1024), 0, st, ckeys, n2, n2, (int)k, (int64_t*)nullptr);
+      LD_LAUNCHED();
+    }
     hipLaunchKernelGGL(k_pairs_out, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st,
                        (const unsigned long long*)ckeys, (int)cnt, pairs);
     LD_LAUNCHED();
@@ -1482,10 +1512,7 @@ struct Engine final : EngineBase {
                int64_t* nevents) override {
     *nevents = 0;
     if (npairs <= 0) return LD_OK;
-    if (n_ > ccap) {
-      LD_TRY(alloc(ckey, n_)); LD_TRY(alloc(crank, n_)); LD_TRY(alloc(corder, n_)); LD_TRY(alloc(cused, n_));
-      ccap = n_;
-    }
+    LD_TRY(coll_reserve(n_));
     if (!ccount) { LD_TRY(alloc(ccount, 1)); LD_TRY(alloc(cnev, 1)); }
     LD_TRY(join(st, st2, evB));
     LD_TRY(fill<int>(st, cused, (size_t)n_, 0));

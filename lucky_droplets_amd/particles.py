@@ -137,15 +137,12 @@ class MPI_particles:
         (Sundaram & Collins 1997).  Returns a dict of numpy arrays."""
         dns = self.dns
         coord, npart = dns._rows(self.coord)
-        counts = torch.empty((nbins,), dtype=torch.int64, device=dns.device)
-        wsum = torch.empty((nbins,), dtype=torch.float64, device=dns.device)
-        wneg = torch.empty((nbins,), dtype=torch.float64, device=dns.device)
+        buf = torch.empty((3, int(nbins)), dtype=torch.float64, device=dns.device)   # counts (int64), wsum, wneg
         dns._stream()
-        _lib.check(dns.lib.ld_pair_stats(dns.ctx, _ptr(coord), npart, float(rmax), int(nbins), _ptr(counts),
-                                         _ptr(wsum), _ptr(wneg)))
-        c = counts.cpu().numpy()
-        ws = wsum.cpu().numpy()
-        wn = wneg.cpu().numpy()
+        _lib.check(dns.lib.ld_pair_stats(dns.ctx, _ptr(coord), npart, float(rmax), int(nbins), _ptr(buf[0]),
+                                         _ptr(buf[1]), _ptr(buf[2])))
+        h = buf.cpu().numpy()
+        c, ws, wn = h[0].view(np.int64), h[1], h[2]
         edges = np.arange(nbins + 1) * (rmax / nbins)
         centre = 0.5 * (edges[1:] + edges[:-1])
         shell = 4.0 / 3.0 * math.pi * (edges[1:] ** 3 - edges[:-1] ** 3)
