@@ -11,7 +11,6 @@ using namespace ld::cnn;
 // blocks of the loss kernel (one FP64 partial sum each)
 #define LD_CNN_MSE_BLOCKS 2048
 using ld::set_error;
-
 struct ld_cnn {
   int N = 0, L = 0, cin = 0, cout = 0;
   int ch[LD_CNN_MAX_LAYERS + 1] = {};     // padded channels at each layer boundary
@@ -25,7 +24,7 @@ struct ld_cnn {
   bf16* Wt[LD_CNN_MAX_LAYERS] = {};
   bf16* act[LD_CNN_MAX_LAYERS] = {};        // act[l]: input of layer l
   bf16* dz[2] = {nullptr, nullptr};
-  float* yp = nullptr;                      // FP32 output [node][ch[L]]
+  float* yp = nullptr;                      // FP32 output rows [node][cout] of a gradient evaluation
   float* part = nullptr;
   double* mpart = nullptr;
   int nblk_w = 0, chunk = 0;
@@ -68,27 +67,24 @@ namespace {
 // gfx950 double-rate form: NT node tiles of 16 per wavefront (a z-line
 // segment of 16 NT nodes), persistent blocks of WPB wavefronts.
 template <int CI, int CO, bool FLIP, bool RELU, bool MASK>
-int conv2(ld_cnn* c, const bf16* X, const bf16* W, const float* b, const bf16* mask, bf16* Yb, float* Yf,
-          bf16* Yblk) {
+int conv2(ld_cnn* c, const bf16* X, const bf16* W, const float* b, const bf16* mask, const ConvOut& O) {
   const int N = c->N;
-  // 4 node tiles per wavefront and 8 wavefronts per block (sharing one LDS
-  // copy of the weights): measured at 128^3, channels 3-32-32-32-3, forward
-  // 0.76 -> 0.67 ms against 8 tiles and 4 wavefronts (2 tiles: 0.75 ms;
-  // 8 tiles with 8 wavefronts: 0.74 ms)
+  // 4 node tiles per wavefront and 8 wavefronts per block, which share one LDS
+  // copy of the weights; persistent blocks, two per CU at a time: 1024 of them
+  // (128^3, 32 -> 32 channels, inference: 153 us with 256, 129 with 512, 122
+  // with 1024), 512 for the data gradient (208 / 179 / 185)
   constexpr int WPB = 8;
   const int NT = N >= 64 ? 4 : N / 16;
   const int nseg = (int)(c->nodes / (16 * NT));
   int G = (nseg + WPB - 1) / WPB;
-  if (G > 2048) G = 2048;
+  if (G > (MASK ? 512 : 1024)) G = MASK ? 512 : 1024;
   const dim3 g((unsigned)G), t(64 * WPB);
 #define LD_NT_CASE(K)                                                                                            \
   if (NT == K) {                                                                                                 \
     if constexpr (CI == 32)                                                                                      \
-      hipLaunchKernelGGL((k_conv3<CO, FLIP, RELU, MASK, K, WPB>), g, t, 0, c->st, X, W, b, mask, Yb, Yf, N, nseg,  \
-                         Yblk);                                                                                  \
+      hipLaunchKernelGGL((k_conv3<CO, FLIP, RELU, MASK, K, WPB>), g, t, 0, c->st, X, W, b, mask, O, N, nseg);     \
     else                                                                                                         \
-      hipLaunchKernelGGL((k_conv2<CI, CO, FLIP, RELU, MASK, K, WPB>), g, t, 0, c->st, X, W, b, mask, Yb, Yf, N,    \
-                         nseg, Yblk);                                                                            \
+      hipLaunchKernelGGL((k_conv2<CI, CO, FLIP, RELU, MASK, K, WPB>), g, t, 0, c->st, X, W, b, mask, O, N, nseg); \
     LAUNCHED();                                                                                                  \
     return LD_OK;                                                                                                \
   }
@@ -98,21 +94,24 @@ int conv2(ld_cnn* c, const bf16* X, const bf16* W, const float* b, const bf16* m
   return LD_ERR_ARG;
 }
 
-// Yblk (N >= 16 only; may be null): a second copy of Yb in the node-blocked
-// layout the weight gradient reads.
+// Yf: FP32 rows of cout channels; Yblk (N >= 16 only): a second copy of Yb in
+// the node-blocked layout the weight gradient reads.  Each output may be null.
 template <bool FLIP, bool RELU, bool MASK>
 int conv(ld_cnn* c, int CI, int CO, const bf16* X, const bf16* W, const float* b, const bf16* mask, bf16* Yb,
-         float* Yf, bf16* Yblk = nullptr) {
+         float* Yf, int cout, bf16* Yblk = nullptr) {
   if (c->N >= 16) {
-    if (CI == 16 && CO == 16) return conv2<16, 16, FLIP, RELU, MASK>(c, X, W, b, mask, Yb, Yf, Yblk);
-    if (CI == 16 && CO == 32) return conv2<16, 32, FLIP, RELU, MASK>(c, X, W, b, mask, Yb, Yf, Yblk);
-    if (CI == 32 && CO == 16) return conv2<32, 16, FLIP, RELU, MASK>(c, X, W, b, mask, Yb, Yf, Yblk);
-    if (CI == 32 && CO == 32) return conv2<32, 32, FLIP, RELU, MASK>(c, X, W, b, mask, Yb, Yf, Yblk);
+    ConvOut O;
+    O.Yb = Yb; O.Yf = Yf; O.cout = cout; O.Yblk = Yblk;
+    O.vec = cout % 4 == 0 && (reinterpret_cast<uintptr_t>(Yf) & 15) == 0;
+    if (CI == 16 && CO == 16) return conv2<16, 16, FLIP, RELU, MASK>(c, X, W, b, mask, O);
+    if (CI == 16 && CO == 32) return conv2<16, 32, FLIP, RELU, MASK>(c, X, W, b, mask, O);
+    if (CI == 32 && CO == 16) return conv2<32, 16, FLIP, RELU, MASK>(c, X, W, b, mask, O);
+    if (CI == 32 && CO == 32) return conv2<32, 32, FLIP, RELU, MASK>(c, X, W, b, mask, O);
   }
   const dim3 g((unsigned)(c->nodes / 64)), t(256);
 #define LD_CONV_CASE(A, B)                                                                                    \
   if (CI == A && CO == B) {                                                                                   \
-    hipLaunchKernelGGL((k_conv<A, B, FLIP, RELU, MASK>), g, t, 0, c->st, X, W, b, mask, Yb, Yf, c->N);      \
+    hipLaunchKernelGGL((k_conv<A, B, FLIP, RELU, MASK>), g, t, 0, c->st, X, W, b, mask, Yb, Yf, cout, c->N); \
     LAUNCHED();                                                                                               \
     return LD_OK;                                                                                             \
   }
@@ -122,21 +121,11 @@ int conv(ld_cnn* c, int CI, int CO, const bf16* X, const bf16* W, const float* b
   return LD_ERR_ARG;
 }
 
-template <int C> int cmajor(ld_cnn* c, const bf16* A, bf16* AT) {
-  const size_t n = c->nodes / 8 * (C / 8);
-  hipLaunchKernelGGL((k_cblock<C>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->st, A, AT, c->nodes);
-  LAUNCHED();
-  return LD_OK;
-}
-
 // Weight and bias gradients of one layer into c->part (per-block partials);
-// returns the number of partial blocks in *nblk.  XB / dZB: node-blocked
-// copies of X / dZ when a producing kernel already wrote them (N >= 16), else
-// null and they are made here.
+// returns the number of partial blocks in *nblk.  XB / dZB: the node-blocked
+// copies of X / dZ that the producing kernels wrote (N >= 16).
 int wgrad(ld_cnn* c, int CI, int CO, const bf16* X, const bf16* dZ, const bf16* XB, const bf16* dZB, int* nblk) {
   if (c->N >= 16) {
-    if (!XB) { CK(CI == 16 ? cmajor<16>(c, X, c->xt) : cmajor<32>(c, X, c->xt)); XB = c->xt; }
-    if (!dZB) { CK(CO == 16 ? cmajor<16>(c, dZ, c->dzt) : cmajor<32>(c, dZ, c->dzt)); dZB = c->dzt; }
     // one neighbour line per wavefront (three measured slower: 396 -> 411 us at 128^3, 32 -> 32)
     constexpr int LPW = 1;
     const dim3 g((unsigned)c->nblk_w2), t(64 * 9 / LPW);
@@ -177,22 +166,21 @@ int pack_weights(ld_cnn* c) {
 }
 
 // Forward pass from the FP32 input rows x[node][cin]; keeps every layer's
-// input for the backward pass; FP32 output in c->yp.  for_grad: the hidden
-// layers also write node-blocked copies of their outputs (c->actB, N >= 16)
-// for the weight gradient.
-int forward(ld_cnn* c, const float* x, bool for_grad) {
+// input for the backward pass; FP32 output rows [node][cout] in y.  for_grad:
+// the input and the hidden layers' outputs are also written node-blocked
+// (c->xt, c->actB, N >= 16) for the weight gradient.
+int forward(ld_cnn* c, const float* x, float* y, bool for_grad) {
   if (!c->packed) CK(pack_weights(c));
-  const size_t gp = (c->nodes + 255) / 256;
-  hipLaunchKernelGGL(k_pack_input, dim3((unsigned)(gp < (1u << 20) ? gp : (1u << 20))), dim3(256), 0, c->st, x, c->cin,
-                     c->ch[0], c->nodes, c->act[0]);
+  hipLaunchKernelGGL(k_pack_input, dim3((unsigned)((c->nodes + EN - 1) / EN)), dim3(256), 0, c->st, x, c->cin, c->ch[0],
+                     c->nodes, c->N, c->act[0], for_grad ? c->xt : (bf16*)nullptr);
   LAUNCHED();
   for (int l = 0; l < c->L; ++l) {
     const float* b = c->params + c->off[l] + 27LL * c->ch[l + 1] * c->ch[l];
     if (l + 1 < c->L)
-      CK((conv<false, true, false>(c, c->ch[l], c->ch[l + 1], c->act[l], c->Wb[l], b, nullptr, c->act[l + 1], nullptr,
+      CK((conv<false, true, false>(c, c->ch[l], c->ch[l + 1], c->act[l], c->Wb[l], b, nullptr, c->act[l + 1], nullptr, 0,
                                    for_grad ? c->actB[l + 1] : nullptr)));
     else
-      CK((conv<false, false, false>(c, c->ch[l], c->ch[l + 1], c->act[l], c->Wb[l], b, nullptr, nullptr, c->yp)));
+      CK((conv<false, false, false>(c, c->ch[l], c->ch[l + 1], c->act[l], c->Wb[l], b, nullptr, nullptr, y, c->cout)));
   }
   return LD_OK;
 }
@@ -202,14 +190,13 @@ int forward(ld_cnn* c, const float* x, bool for_grad) {
 int backward(ld_cnn* c, const float* target, double* loss) {
   const int nb = LD_CNN_MSE_BLOCKS;
   hipLaunchKernelGGL(k_mse, dim3(nb), dim3(256), 0, c->st, (const float*)c->yp, target, c->cout, c->ch[c->L], c->nodes,
-                     c->dz[0], c->mpart);
+                     c->N, c->dz[0], c->dzt, c->mpart);
   LAUNCHED();
-  int cur = 0;
-  bool dzb = false;        // c->dzt holds the node-blocked copy of dz[cur]
+  int cur = 0;             // c->dzt holds the node-blocked copy of dz[cur]
   for (int l = c->L - 1; l >= 0; --l) {
     const int CI = c->ch[l], CO = c->ch[l + 1];
     int nblk = 0;
-    CK(wgrad(c, CI, CO, c->act[l], c->dz[cur], l > 0 ? c->actB[l] : nullptr, dzb ? c->dzt : nullptr, &nblk));
+    CK(wgrad(c, CI, CO, c->act[l], c->dz[cur], l > 0 ? c->actB[l] : c->xt, c->dzt, &nblk));
     const int n = 27 * CO * CI + CO;
     hipLaunchKernelGGL(k_reduce_parts, dim3((n + 255) / 256), dim3(256), 0, c->st, (const float*)c->part, nblk, n,
                        c->grads + c->off[l]);
@@ -217,9 +204,8 @@ int backward(ld_cnn* c, const float* target, double* loss) {
     if (l > 0) {
       // data gradient through the convolution (transposed weights, mirrored taps)
       // and the ReLU of layer l - 1 (whose output is act[l])
-      CK((conv<true, false, true>(c, CO, CI, c->dz[cur], c->Wt[l], nullptr, c->act[l], c->dz[cur ^ 1], nullptr,
-                                  c->N >= 16 ? c->dzt : nullptr)));
-      dzb = c->N >= 16;
+      CK((conv<true, false, true>(c, CO, CI, c->dz[cur], c->Wt[l], nullptr, c->act[l], c->dz[cur ^ 1], nullptr, 0,
+                                  c->dzt)));
       cur ^= 1;
     }
   }
@@ -290,7 +276,7 @@ int ld_cnn_create(const ld_cnn_params* p, ld_cnn** out) {
   }
   if (rc == LD_OK) rc = c->alloc(c->dz[0], c->nodes * 32);
   if (rc == LD_OK) rc = c->alloc(c->dz[1], c->nodes * 32);
-  if (rc == LD_OK) rc = c->alloc(c->yp, c->nodes * c->ch[c->L]);
+  if (rc == LD_OK) rc = c->alloc(c->yp, c->nodes * c->cout);
   if (rc == LD_OK) rc = c->alloc(c->part, (size_t)(c->nblk_w > c->nblk_w2 ? c->nblk_w : c->nblk_w2) * maxlayer);
   if (rc == LD_OK && c->N >= 16) rc = c->alloc(c->xt, c->nodes * 32);
   if (rc == LD_OK && c->N >= 16) rc = c->alloc(c->dzt, c->nodes * 32);
@@ -342,16 +328,12 @@ int ld_cnn_get_params(ld_cnn* c, float* params) {
 
 int ld_cnn_forward(ld_cnn* c, const float* x, float* y) {
   if (!c || !x || !y) { set_error("null argument"); return LD_ERR_ARG; }
-  CK(forward(c, x, false));
-  hipLaunchKernelGGL(k_unpack_output, dim3(1024), dim3(256), 0, c->st, (const float*)c->yp, c->ch[c->L], c->cout,
-                     c->nodes, y);
-  LAUNCHED();
-  return LD_OK;
+  return forward(c, x, y, false);
 }
 
 int ld_cnn_grad(ld_cnn* c, const float* x, const float* target, float* grads, double* loss) {
   if (!c || !x || !target) { set_error("null argument"); return LD_ERR_ARG; }
-  CK(forward(c, x, true));
+  CK(forward(c, x, c->yp, true));
   CK(backward(c, target, loss));
   if (grads) HK(hipMemcpyAsync(grads, c->grads, c->nparams * sizeof(float), hipMemcpyDeviceToDevice, c->st));
   return LD_OK;
@@ -360,7 +342,7 @@ int ld_cnn_grad(ld_cnn* c, const float* x, const float* target, float* grads, do
 int ld_cnn_train_step(ld_cnn* c, const float* x, const float* target, float lr, float beta1, float beta2, float eps,
                       double* loss) {
   if (!c || !x || !target) { set_error("null argument"); return LD_ERR_ARG; }
-  CK(forward(c, x, true));
+  CK(forward(c, x, c->yp, true));
   CK(backward(c, target, loss));
   c->adam_t += 1;
   hipLaunchKernelGGL(k_adam, dim3((unsigned)((c->nparams + 255) / 256)), dim3(256), 0, c->st, c->params,

@@ -2,10 +2,19 @@
 // run with hand-written bf16 MFMA kernels (FP32 accumulation).  No
 // counterpart in the reference.
 //
-// Layout: activations channels-last, A[node][C] in bf16, node = (x N + y) N + z,
-// C a multiple of 16; weights per layer W[tap][co][ci] (and the transposed
-// copy Wt[tap][ci][co] for the data gradient), tap = (dx+1) 9 + (dy+1) 3 +
-// (dz+1) for offsets in {-1, 0, 1}; periodic neighbours.
+// Layouts of the bf16 activations, C a multiple of 16:
+//   N < 16: channels-last, A[node][C], node = (x N + y) N + z;
+//   N >= 16: per z-line, segments of 16 NT nodes (NT = min(4, N / 16)), in each
+//   C/8 planes of 8 channels, in each the nodes z = NT l + t ordered [t][l]
+//   (tiled_at()).  Tile t of a segment is then 16 consecutive 16-byte cells per
+//   channel plane, which the 16 lanes of an MFMA operand row read as 256
+//   consecutive bytes: channels-last rows put neighbouring lanes 64 bytes
+//   apart, and the cache lines a load then touched bounded the convolutions
+//   (32 -> 32 channels at 128^3, inference: 192 us, 603 TFLOP/s; 122 us, 950
+//   TFLOP/s now, against 1200 TFLOP/s that the instruction reaches by itself).
+// Weights per layer W[tap][co][ci] (and the transposed copy Wt[tap][ci][co] for
+// the data gradient), tap = (dx+1) 9 + (dy+1) 3 + (dz+1) for offsets in
+// {-1, 0, 1}; periodic neighbours.
 //
 // A 3x3x3 convolution is an implicit GEMM: M = nodes, K = 27 taps x CI,
 // N = CO.  One wavefront computes 16 nodes x CO outputs with
@@ -34,6 +43,12 @@ __device__ __forceinline__ bf16 f2b(float f) {
 }
 __device__ __forceinline__ float b2f(bf16 b) { return __uint_as_float((uint32_t)b << 16); }
 
+// element offset of (z, channel c) in a tiled line of C channels
+template <int NT> __device__ __forceinline__ int tiled_at(int z, int c, int C) {
+  const int seg = z / (16 * NT), r = z % (16 * NT);
+  return ((seg * (C / 8) + c / 8) * (16 * NT) + (r % NT) * 16 + r / NT) * 8 + c % 8;
+}
+
 __device__ __forceinline__ int nbr(int node, int tap, int N, bool flip) {
   int dx = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dz = tap % 3 - 1;
   if (flip) { dx = -dx; dy = -dy; dz = -dz; }
@@ -44,12 +59,12 @@ __device__ __forceinline__ int nbr(int node, int tap, int N, bool flip) {
 // out[node][co] = bias[co] + sum_{tap, ci} X[nbr(node, tap)][ci] W[tap][co][ci]
 // FLIP: neighbours at -offset (the data gradient, with Wt);
 // RELU: max(., 0); MASK: times (mask[node][co] > 0) (ReLU derivative of the
-// layer below); Yb / Yf: bf16 / FP32 outputs (either may be null).
+// layer below); Yb: bf16 output, Yf: FP32 rows of cout channels (either may be null).
 // 256 threads = 4 wavefronts x 16 nodes; N^3 must be a multiple of 64.
 template <int CI, int CO, bool FLIP, bool RELU, bool MASK>
 __global__ void __launch_bounds__(256)
 k_conv(const bf16* __restrict__ X, const bf16* __restrict__ W, const float* __restrict__ bias,
-       const bf16* __restrict__ mask, bf16* __restrict__ Yb, float* __restrict__ Yf, int N) {
+       const bf16* __restrict__ mask, bf16* __restrict__ Yb, float* __restrict__ Yf, int cout, int N) {
   static_assert(CI % 16 == 0 && CO % 16 == 0, "channels: multiples of 16");
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int node0 = blockIdx.x * 64 + wv * 16;
@@ -81,7 +96,7 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ W, const float* __re
       if (RELU) v = v > 0.f ? v : 0.f;
       if (MASK) v = b2f(mask[o]) > 0.f ? v : 0.f;
       if (Yb) Yb[o] = f2b(v);
-      if (Yf) Yf[o] = v;
+      if (Yf && co < cout) Yf[(size_t)(node0 + kq + i) * cout + co] = v;
     }
   }
 }
@@ -90,91 +105,195 @@ k_conv(const bf16* __restrict__ X, const bf16* __restrict__ W, const float* __re
 // __builtin_amdgcn_mfma_f32_16x16x32_bf16, oriented M = output channels,
 // N = nodes, K = (tap, input channel) pairs in steps of 32:
 //   A (16x32): lane l holds W[tap][co0 + l % 16][ci0 + i]       (8 bf16, 16 B)
-//   B (32x16): lane l holds X[nbr(node0 + l % 16, tap)][ci0 + i] (8 bf16, 16 B)
-//   D (16x16): lane l holds Y[node0 + l % 16][co0 + 4 (l / 16) + i], i < 4
+//   B (32x16): lane l holds X[nbr(node(l % 16), tap)][ci0 + i]   (8 bf16, 16 B)
+//   D (16x16): lane l holds Y[node(l % 16)][co0 + 4 (l / 16) + i], i < 4
 // with (tap, ci0) = divmod(32 ks + 8 (l / 16), CI) for K-step ks (CI = 16: a
 // step covers two taps; the 28th tap of the last step has zero weights).
 // The layer's weights are staged in LDS once per block; a wavefront computes
-// NT tiles of 16 consecutive nodes along z (one z-line segment) for all CO,
-// so each weight fragment feeds NT instructions and each input fragment CO/16.
-// Blocks loop over segments (persistent grid), XCD-aware: each XCD takes a
-// contiguous run of blocks, so neighbouring lines share its L2.
-// Needs N >= 16 * NT and N a multiple of 16 * NT.
+// a z-line segment of 16 NT nodes for all CO as NT tiles of 16 nodes, so each
+// weight fragment feeds NT instructions and each input fragment CO/16.
+//
+// Tile t holds the nodes z0 + NT n + t (n = lane % 16), not 16 consecutive
+// ones: the z neighbour of a node then lies in the next or previous tile of
+// the same lane, and only one tile per direction needs a lane shift (64
+// instructions per neighbour line with consecutive nodes, 16 now); and a
+// lane's NT nodes are consecutive, so the node-blocked copy needs no transpose
+// through LDS.  Inputs and outputs are in the tiled layout.
+// Blocks loop over segments (persistent grid: two blocks fill a CU's LDS),
+// XCD-aware: each XCD takes a contiguous run of blocks, so neighbouring lines
+// share its L2.  The K order of a sum (taps, then channels) is part of the
+// result: the hidden layers round it to bf16.
+// Needs N a multiple of 16 * NT.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// Writes a wavefront's 16-node x 16-channel output tile (lane l: node n0 +
-// l % 16, channels c0 + 4 (l / 16) + i, i < 4, in v) to the node-blocked
-// channel-major layout of k_cblock through 512 bytes of LDS owned by the
-// wavefront: 32 runs of 8 nodes x 1 channel, one 16-byte store each.  n0 is a
-// multiple of 16.  The LDS writes and reads are issued by one wavefront, whose
-// LDS operations complete in order.
-template <int CO>
-__device__ __forceinline__ void store_blocked(bf16* __restrict__ Yblk, bf16* sT, size_t n0, int c0, const uint32_t pk[2]) {
-  const int lane = threadIdx.x & 63, n16 = lane & 15, q = lane >> 4;
-  sT[(4 * q + 0) * 16 + n16] = (bf16)(pk[0] & 0xffff);
-  sT[(4 * q + 1) * 16 + n16] = (bf16)(pk[0] >> 16);
-  sT[(4 * q + 2) * 16 + n16] = (bf16)(pk[1] & 0xffff);
-  sT[(4 * q + 3) * 16 + n16] = (bf16)(pk[1] >> 16);
-  __builtin_amdgcn_wave_barrier();
-  if (lane < 32) {
-    const int cl = lane >> 1, half = lane & 1;
-    const uint4 v = *reinterpret_cast<const uint4*>(sT + cl * 16 + half * 8);
-    *reinterpret_cast<uint4*>(Yblk + (((n0 >> 3) + half) * CO + c0 + cl) * 8) = v;
-  }
-  __builtin_amdgcn_wave_barrier();
+template <unsigned CTRL>
+__device__ __forceinline__ uint32_t dpp_u(uint32_t old, uint32_t src) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, CTRL, 0xf, 0xf, false);
+}
+// lanes of a 16-lane row take the next lane's fragment; lane 15 takes its own of `edge`
+__device__ __forceinline__ uint4 shift_up(const uint4& a, const uint4& edge) {
+  return make_uint4(dpp_u<0x101>(edge.x, a.x), dpp_u<0x101>(edge.y, a.y), dpp_u<0x101>(edge.z, a.z),
+                    dpp_u<0x101>(edge.w, a.w));
+}
+// the previous lane's fragment; lane 0 takes its own of `edge`
+__device__ __forceinline__ uint4 shift_down(const uint4& a, const uint4& edge) {
+  return make_uint4(dpp_u<0x111>(edge.x, a.x), dpp_u<0x111>(edge.y, a.y), dpp_u<0x111>(edge.z, a.z),
+                    dpp_u<0x111>(edge.w, a.w));
 }
 
+// Where a convolution's results go; each may be null.
+struct ConvOut {
+  bf16* Yb;            // tiled
+  float* Yf;           // FP32 rows of cout channels
+  int cout, vec;       // vec: 16-byte stores into the rows (cout % 4 == 0, Yf aligned)
+  bf16* Yblk;          // node-blocked channel-major copy (blocked_at()): runs of 8 nodes x 1 channel
+};
+__device__ __forceinline__ size_t blocked_at(size_t node, int c, int C) { return ((node >> 3) * C + c) * 8 + (node & 7); }
+
+// Bias, ReLU / mask and stores of a segment's accumulators: tile t's lane node
+// z0 + NT n16 + t of z-line `line`, channels 16 m + 4 q + i.  With NT = 4 a lane
+// holds half a run of each of its channels of the blocked copy; neighbouring
+// lanes exchange two channels each and store whole runs.
+template <int CO, bool RELU, bool MASK, int NT>
+__device__ __forceinline__ void conv_out(const f32x4 (&acc)[NT][CO / 16], const float4 (&bv)[CO / 16], int N, int line,
+                                         int z0, const bf16* __restrict__ mask, const ConvOut& O) {
+  const int lane = threadIdx.x & 63, n16 = lane & 15, q = lane >> 4;
+  const size_t node0 = (size_t)line * N + z0 + NT * n16;
+  const size_t cell0 = (size_t)line * N * CO + z0 * CO;       // the segment's cells
+#pragma unroll
+  for (int m = 0; m < CO / 16; ++m) {
+    const int co = m * 16 + 4 * q;
+    const size_t tb = cell0 + ((2 * m + (q >> 1)) * (16 * NT) + n16) * 8 + 4 * (q & 1);
+    uint32_t pk[NT][2];                // channels (0, 1) and (2, 3) of each node
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const size_t o = tb + t * 128;
+      const float b4[4] = {bv[m].x, bv[m].y, bv[m].z, bv[m].w};
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[i] = acc[t][m][i] + b4[i];
+        if (RELU) v[i] = v[i] > 0.f ? v[i] : 0.f;
+      }
+      if (MASK) {
+        const uint2 mk = *reinterpret_cast<const uint2*>(mask + o);
+        const bf16 mb[4] = {(bf16)(mk.x & 0xffff), (bf16)(mk.x >> 16), (bf16)(mk.y & 0xffff), (bf16)(mk.y >> 16)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = b2f(mb[i]) > 0.f ? v[i] : 0.f;
+      }
+      if (O.Yf) {
+        float* row = O.Yf + (node0 + t) * O.cout + co;
+        if (O.vec) {
+          if (co < O.cout) *reinterpret_cast<float4*>(row) = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (co + i < O.cout) row[i] = v[i];
+        }
+      }
+      pk[t][0] = (uint32_t)f2b(v[0]) | ((uint32_t)f2b(v[1]) << 16);
+      pk[t][1] = (uint32_t)f2b(v[2]) | ((uint32_t)f2b(v[3]) << 16);
+      if (O.Yb) *reinterpret_cast<uint2*>(O.Yb + o) = make_uint2(pk[t][0], pk[t][1]);
+    }
+    if (!O.Yblk) continue;
+    if constexpr (NT == 4) {
+      // c[i]: nodes 0..3 of channel i
+      uint2 c[4];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        c[2 * h] = make_uint2((pk[0][h] & 0xffffu) | (pk[1][h] << 16), (pk[2][h] & 0xffffu) | (pk[3][h] << 16));
+        c[2 * h + 1] = make_uint2((pk[0][h] >> 16) | (pk[1][h] & 0xffff0000u), (pk[2][h] >> 16) | (pk[3][h] & 0xffff0000u));
+      }
+      const bool odd = n16 & 1;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {    // even lanes store channels 0, 1; odd lanes 2, 3
+        const uint2 mine = odd ? c[2 + e] : c[e], theirs = odd ? c[e] : c[2 + e];
+        const uint2 got = make_uint2(dpp_u<0xb1>(0u, theirs.x), dpp_u<0xb1>(0u, theirs.y));   // quad_perm 1,0,3,2
+        const uint4 run = odd ? make_uint4(got.x, got.y, mine.x, mine.y) : make_uint4(mine.x, mine.y, got.x, got.y);
+        *reinterpret_cast<uint4*>(O.Yblk + ((node0 >> 3) * CO + co + (odd ? 2 : 0) + e) * 8) = run;
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          O.Yblk[blocked_at(node0 + t, co + i, CO)] = (bf16)(pk[t][i >> 1] >> (16 * (i & 1)));
+    }
+  }
+}
+template <int CO> __device__ __forceinline__ void load_bias(const float* __restrict__ bias, float4 (&bv)[CO / 16]) {
+  const int q = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int m = 0; m < CO / 16; ++m)
+    bv[m] = bias ? *reinterpret_cast<const float4*>(bias + m * 16 + 4 * q) : make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
+// CI = 16: every K-step covers two taps, lanes q < 2 the even one and q >= 2
+// the odd one.  The K-steps are unrolled, so a lane's tap offsets are selects
+// between constants and the tiles' addresses differ by constants (only the
+// first and last tile can reach past the lane's nodes).
 template <int CI, int CO, bool FLIP, bool RELU, bool MASK, int NT, int WPB>
 __global__ void __launch_bounds__(64 * WPB)
 k_conv2(const bf16* __restrict__ X, const bf16* __restrict__ W, const float* __restrict__ bias,
-        const bf16* __restrict__ mask, bf16* __restrict__ Yb, float* __restrict__ Yf, int N, int nseg,
-        bf16* __restrict__ Yblk) {
-  static_assert(CI % 16 == 0 && CO % 16 == 0, "channels: multiples of 16");
+        const bf16* __restrict__ mask, ConvOut O, int N, int nseg) {
+  static_assert(CI == 16 && CO % 16 == 0, "16 input channels");
   constexpr int MT = CO / 16;
   constexpr int KS = (27 * CI + 31) / 32;
   constexpr int WN = 27 * CO * CI;
   __shared__ __attribute__((aligned(16))) bf16 sW[WN];
-  __shared__ __attribute__((aligned(16))) bf16 sT[WPB][256];   // per-wavefront tile for the blocked copy
   for (int e = threadIdx.x; e < WN / 8; e += 64 * WPB)
     reinterpret_cast<uint4*>(sW)[e] = reinterpret_cast<const uint4*>(W)[e];
   __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = lane & 15, q = lane >> 4;
+  const bool hi = q >= 2;
+  const int ci0 = 8 * (q & 1);
   const int G = gridDim.x;
   const int lb = (G % 8 == 0) ? (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8 : blockIdx.x;
   const int spl = N / (16 * NT);                  // segments per z-line
   const int msk = N - 1;
+  float4 bv[MT];
+  load_bias<CO>(bias, bv);
   for (int seg = lb * WPB + wv; seg < nseg; seg += G * WPB) {
     const int line = seg / spl, z0 = (seg % spl) * 16 * NT;
     const int x = line / N, y = line & msk;
+    // element offsets inside a line: tile 0 of the lane's nodes (tile t 128 t
+    // further), the node before tile 0's and the one after tile NT - 1's
+    const int zl = z0 + NT * n16;
+    const int own = tiled_at<NT>(zl, ci0, CI), prev = tiled_at<NT>((zl - 1) & msk, ci0, CI),
+              next = tiled_at<NT>((zl + NT) & msk, ci0, CI);
     f32x4 acc[NT][MT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
+#pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const int k = 32 * ks + 8 * q;
-      const int tap0 = k / CI, ci0 = k % CI;
-      const bool valid = tap0 < 27;
-      const int tap = valid ? tap0 : 26;
-      int dx = tap / 9 - 1, dy = (tap / 3) % 3 - 1, dz = tap % 3 - 1;
-      if (FLIP) { dx = -dx; dy = -dy; dz = -dz; }
+      constexpr int S = FLIP ? -1 : 1;
+      const int tA = 2 * ks, tB = 2 * ks + 1 < 27 ? 2 * ks + 1 : 26;
+      const bool valid = 2 * ks + 1 < 27 || !hi;
+      const size_t rA = ((size_t)((x + S * (tA / 9 - 1)) & msk) * N + ((y + S * ((tA / 3) % 3 - 1)) & msk)) * N;
+      const size_t rB = ((size_t)((x + S * (tB / 9 - 1)) & msk) * N + ((y + S * ((tB / 3) % 3 - 1)) & msk)) * N;
+      const int dA = S * (tA % 3 - 1), dB = S * (tB % 3 - 1);      // z offsets of the two taps
+      const bf16* row = X + (hi ? rB : rA) * CI;
+      const bf16* mid = row + own + (hi ? dB : dA) * 128;
       bf16x8 wf[MT], xf[NT];
       // opaque to the compiler, so the weight fragments are re-read from LDS
       // per segment instead of being hoisted into registers for all K-steps
-      int wofs = (tap * CO + n16) * CI + ci0;
+      int wofs = ((hi ? tB : tA) * CO + n16) * CI + ci0;
       asm volatile("" : "+v"(wofs));
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         const uint4 v = *reinterpret_cast<const uint4*>(sW + wofs + m * 16 * CI);
         wf[m] = valid ? __builtin_bit_cast(bf16x8, v) : bf16x8{};
       }
-      const size_t row = ((size_t)((x + dx) & msk) * N + ((y + dy) & msk)) * N;
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
-        const int zz = (z0 + 16 * t + n16 + dz) & msk;
-        const uint4 v = *reinterpret_cast<const uint4*>(X + (row + zz) * CI + ci0);
+        // only the first and last tile can reach past the lane's nodes
+        auto far = [&](int d) { return t + d < 0 || t + d >= NT; };
+        auto at = [&](int d) { return t + d < 0 ? prev : t + d >= NT ? next : own + (t + d) * 128; };
+        const bf16* src = far(dA) || far(dB) ? row + (hi ? at(dB) : at(dA)) : mid + t * 128;
+        const uint4 v = *reinterpret_cast<const uint4*>(src);
         xf[t] = valid ? __builtin_bit_cast(bf16x8, v) : bf16x8{};
       }
 #pragma unroll
@@ -182,102 +301,59 @@ k_conv2(const bf16* __restrict__ X, const bf16* __restrict__ W, const float* __r
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[m], xf[t], acc[t][m], 0, 0, 0);
     }
-    const size_t nbase = (size_t)line * N + z0 + n16;
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const int co = m * 16 + 4 * q;
-        const size_t o = (nbase + 16 * t) * CO + co;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          v[i] = acc[t][m][i] + (bias ? bias[co + i] : 0.f);
-          if (RELU) v[i] = v[i] > 0.f ? v[i] : 0.f;
-        }
-        if (MASK) {
-          const uint2 mk = *reinterpret_cast<const uint2*>(mask + o);
-          const bf16 mb[4] = {(bf16)(mk.x & 0xffff), (bf16)(mk.x >> 16), (bf16)(mk.y & 0xffff), (bf16)(mk.y >> 16)};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = b2f(mb[i]) > 0.f ? v[i] : 0.f;
-        }
-        uint32_t pk[2];
-        pk[0] = (uint32_t)f2b(v[0]) | ((uint32_t)f2b(v[1]) << 16);
-        pk[1] = (uint32_t)f2b(v[2]) | ((uint32_t)f2b(v[3]) << 16);
-        if (Yb) *reinterpret_cast<uint2*>(Yb + o) = make_uint2(pk[0], pk[1]);
-        if (Yf) *reinterpret_cast<float4*>(Yf + o) = make_float4(v[0], v[1], v[2], v[3]);
-        if (Yblk) store_blocked<CO>(Yblk, sT[wv], nbase - n16 + 16 * t, m * 16, pk);
-      }
+    conv_out<CO, RELU, MASK, NT>(acc, bv, N, line, z0, mask, O);
   }
 }
 
-// CI = 32 form of k_conv2 that reuses input fragments across the dz taps: per
-// neighbour line (dx, dy) a wavefront loads its NT tiles once (plus the node
-// before and after the segment) and forms the dz = +1 and -1 operands by
-// shifting lanes within each 16-lane row (DPP row_shl:1 / row_shr:1, with the
-// row's end lane filled from the neighbouring tile by row_shr:15 / row_shl:15),
-// so one 16-byte load feeds 3 MT instructions instead of MT.
-template <unsigned CTRL>
-__device__ __forceinline__ uint32_t dpp_u(uint32_t old, uint32_t src) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, CTRL, 0xf, 0xf, false);
-}
-// lanes of a 16-lane row take the fragment of the next node (dz = +1): lane i
-// <- lane i + 1 of `a`, lane 15 <- lane 0 of `next`
-__device__ __forceinline__ uint4 shift_up(const uint4& a, const uint4& next) {
-  uint4 r;
-  r.x = dpp_u<0x101>(dpp_u<0x11f>(0u, next.x), a.x);
-  r.y = dpp_u<0x101>(dpp_u<0x11f>(0u, next.y), a.y);
-  r.z = dpp_u<0x101>(dpp_u<0x11f>(0u, next.z), a.z);
-  r.w = dpp_u<0x101>(dpp_u<0x11f>(0u, next.w), a.w);
-  return r;
-}
-// dz = -1: lane i <- lane i - 1 of `a`, lane 0 <- lane 15 of `prev`
-__device__ __forceinline__ uint4 shift_down(const uint4& a, const uint4& prev) {
-  uint4 r;
-  r.x = dpp_u<0x111>(dpp_u<0x10f>(0u, prev.x), a.x);
-  r.y = dpp_u<0x111>(dpp_u<0x10f>(0u, prev.y), a.y);
-  r.z = dpp_u<0x111>(dpp_u<0x10f>(0u, prev.z), a.z);
-  r.w = dpp_u<0x111>(dpp_u<0x10f>(0u, prev.w), a.w);
-  return r;
-}
-
+// CI = 32: the input fragments of a neighbour line (dx, dy) serve its three dz
+// taps: a wavefront loads its NT tiles once plus the node before and after the
+// segment (one load: lane 0 the one before, lane 15 the one after).  The next
+// line's loads are issued before this line's products.
 template <int CO, bool FLIP, bool RELU, bool MASK, int NT, int WPB>
 __global__ void __launch_bounds__(64 * WPB)
 k_conv3(const bf16* __restrict__ X, const bf16* __restrict__ W, const float* __restrict__ bias,
-        const bf16* __restrict__ mask, bf16* __restrict__ Yb, float* __restrict__ Yf, int N, int nseg,
-        bf16* __restrict__ Yblk) {
+        const bf16* __restrict__ mask, ConvOut O, int N, int nseg) {
   constexpr int CI = 32, MT = CO / 16;
   constexpr int WN = 27 * CO * CI;
   __shared__ __attribute__((aligned(16))) bf16 sW[WN];
-  __shared__ __attribute__((aligned(16))) bf16 sT[WPB][256];   // per-wavefront tile for the blocked copy
   for (int e = threadIdx.x; e < WN / 8; e += 64 * WPB)
     reinterpret_cast<uint4*>(sW)[e] = reinterpret_cast<const uint4*>(W)[e];
   __syncthreads();
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n16 = lane & 15, q = lane >> 4, ci0 = 8 * q;
   const int G = gridDim.x;
   const int lb = (G % 8 == 0) ? (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8 : blockIdx.x;
   const int spl = N / (16 * NT);
   const int msk = N - 1;
+  float4 bv[MT];
+  load_bias<CO>(bias, bv);
   for (int seg = lb * WPB + wv; seg < nseg; seg += G * WPB) {
     const int line = seg / spl, z0 = (seg % spl) * 16 * NT;
     const int x = line / N, y = line & msk;
+    const int zl = z0 + NT * n16;
+    // element offsets inside a line: the lane's first node; the node before or
+    // after the segment for the end lanes
+    const int own = tiled_at<NT>(zl, ci0, CI);         // tile t 128 t further
+    const int end = n16 == 0 ? tiled_at<NT>((z0 - 1) & msk, ci0, CI)
+                             : n16 == 15 ? tiled_at<NT>((z0 + 16 * NT) & msk, ci0, CI) : own;
     f32x4 acc[NT][MT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
       for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
+    uint4 xc[NT], edge;
+    auto fetch = [&](int dxy, uint4 (&f)[NT], uint4& e) {
+      const bf16* row = X + ((size_t)((x + dxy / 3 - 1) & msk) * N + ((y + dxy % 3 - 1) & msk)) * N * CI;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) f[t] = *reinterpret_cast<const uint4*>(row + own + t * 128);
+      e = *reinterpret_cast<const uint4*>(row + end);
+    };
+    fetch(0, xc, edge);
+#pragma unroll
     for (int dxy = 0; dxy < 9; ++dxy) {
       const int ndx = dxy / 3 - 1, ndy = dxy % 3 - 1;     // neighbour line offset
-      const size_t row = ((size_t)((x + ndx) & msk) * N + ((y + ndy) & msk)) * N;
-      uint4 xc[NT];
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        xc[t] = *reinterpret_cast<const uint4*>(X + (row + ((z0 + 16 * t + n16) & msk)) * CI + ci0);
-      uint4 blo = make_uint4(0u, 0u, 0u, 0u), bhi = make_uint4(0u, 0u, 0u, 0u);
-      if (n16 == 15) blo = *reinterpret_cast<const uint4*>(X + (row + ((z0 - 1) & msk)) * CI + ci0);
-      if (n16 == 0) bhi = *reinterpret_cast<const uint4*>(X + (row + ((z0 + 16 * NT) & msk)) * CI + ci0);
+      uint4 xn[NT], en;
+      if (dxy < 8) fetch(dxy + 1, xn, en);
 #pragma unroll
       for (int ndz = -1; ndz <= 1; ++ndz) {
         // weight tap of this neighbour offset (mirrored for the data gradient)
@@ -291,42 +367,22 @@ k_conv3(const bf16* __restrict__ X, const bf16* __restrict__ W, const float* __r
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           uint4 v;
-          if (ndz == 0) v = xc[t];
-          else if (ndz > 0) v = shift_up(xc[t], t + 1 < NT ? xc[t + 1] : bhi);
-          else v = shift_down(xc[t], t > 0 ? xc[t - 1] : blo);
+          if (t + ndz < 0) v = shift_down(xc[NT - 1], edge);
+          else if (t + ndz >= NT) v = shift_up(xc[0], edge);
+          else v = xc[t + ndz];
           const bf16x8 xf = __builtin_bit_cast(bf16x8, v);
 #pragma unroll
           for (int m = 0; m < MT; ++m)
             acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[m], xf, acc[t][m], 0, 0, 0);
         }
       }
-    }
-    const size_t nbase = (size_t)line * N + z0 + n16;
+      if (dxy < 8) {
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        const int co = m * 16 + 4 * q;
-        const size_t o = (nbase + 16 * t) * CO + co;
-        float v[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          v[i] = acc[t][m][i] + (bias ? bias[co + i] : 0.f);
-          if (RELU) v[i] = v[i] > 0.f ? v[i] : 0.f;
-        }
-        if (MASK) {
-          const uint2 mk = *reinterpret_cast<const uint2*>(mask + o);
-          const bf16 mb[4] = {(bf16)(mk.x & 0xffff), (bf16)(mk.x >> 16), (bf16)(mk.y & 0xffff), (bf16)(mk.y >> 16)};
-#pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = b2f(mb[i]) > 0.f ? v[i] : 0.f;
-        }
-        uint32_t pk[2];
-        pk[0] = (uint32_t)f2b(v[0]) | ((uint32_t)f2b(v[1]) << 16);
-        pk[1] = (uint32_t)f2b(v[2]) | ((uint32_t)f2b(v[3]) << 16);
-        if (Yb) *reinterpret_cast<uint2*>(Yb + o) = make_uint2(pk[0], pk[1]);
-        if (Yf) *reinterpret_cast<float4*>(Yf + o) = make_float4(v[0], v[1], v[2], v[3]);
-        if (Yblk) store_blocked<CO>(Yblk, sT[wv], nbase - n16 + 16 * t, m * 16, pk);
+        for (int t = 0; t < NT; ++t) xc[t] = xn[t];
+        edge = en;
       }
+    }
+    conv_out<CO, RELU, MASK, NT>(acc, bv, N, line, z0, mask, O);
   }
 }
 
@@ -404,40 +460,8 @@ k_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ, float* __restri
   if (threadIdx.x < CO) out[27 * CO * CI + threadIdx.x] = db;
 }
 
-// Channels-last A[node][C] -> node-blocked channel-major AB (bf16): entry
-// (node, c) at ((node / 8) C + c) 8 + node % 8, i.e. for each group of 8
-// nodes, C runs of 8 consecutive nodes (16 bytes each).  One thread per group
-// and 8 channels: eight 16-byte loads, an 8 x 8 transpose in registers,
-// eight 16-byte stores.
-template <int C>
-__global__ void __launch_bounds__(256)
-k_cblock(const bf16* __restrict__ A, bf16* __restrict__ AB, size_t nodes) {
-  constexpr int CG = C / 8;
-  const size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  if (e >= nodes / 8 * CG) return;
-  const size_t g = e / CG;
-  const int c8 = (int)(e % CG) * 8;
-  uint32_t r[8][4];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint4 v = *reinterpret_cast<const uint4*>(A + (g * 8 + i) * C + c8);
-    r[i][0] = v.x; r[i][1] = v.y; r[i][2] = v.z; r[i][3] = v.w;
-  }
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    uint32_t o[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t a = (r[2 * k][j / 2] >> (16 * (j & 1))) & 0xffffu;
-      const uint32_t b = (r[2 * k + 1][j / 2] >> (16 * (j & 1))) & 0xffffu;
-      o[k] = a | (b << 16);
-    }
-    *reinterpret_cast<uint4*>(AB + (g * C + c8 + j) * 8) = make_uint4(o[0], o[1], o[2], o[3]);
-  }
-}
-
 // Weight and bias gradients from node-blocked channel-major operands
-// (k_cblock layout) on the 16x16x32 bf16 MFMA (M = output channels,
+// (blocked_at()) on the 16x16x32 bf16 MFMA (M = output channels,
 // N = input channels, K = nodes):
 //   A (16x32): lane l holds dZ[node k0 + 8 (l / 16) + i][co0 + l % 16]  (one 16-byte run)
 //   B (32x16): lane l holds X[nbr(node k0 + 8 (l / 16) + i, tap)][ci0 + l % 16]
@@ -577,23 +601,57 @@ k_reduce_parts(const float* __restrict__ part, int nblk, int n, float* __restric
   out[i] = s;
 }
 
-// x[node][cin] FP32 -> A[node][CP] bf16 (channels cin..CP-1 zero).
-// One node per thread and step, 16-byte stores (CP is 16 or 32).
-static __global__ void k_pack_input(const float* __restrict__ x, int cin, int CP, size_t nodes, bf16* __restrict__ A) {
-  for (size_t node = blockIdx.x * (size_t)blockDim.x + threadIdx.x; node < nodes;
-       node += (size_t)gridDim.x * blockDim.x) {
-    for (int c8 = 0; c8 < CP; c8 += 8) {
-      uint32_t w[4];
+// Rows of bf16 values of EN nodes staged in LDS (sh[node][c], c < cn real
+// channels) -> an activation of CP channels (the others zero) in the layout of
+// N (channels-last for N < 16, else tiled), and with AB its node-blocked copy;
+// 16-byte stores.  Nodes node0 .. node0 + n - 1 (n a multiple of 8).
+constexpr int EN = 256;
+__device__ __forceinline__ void emit_rows(const bf16* sh, int cn, int CP, size_t node0, int n, int N,
+                                          bf16* __restrict__ A, bf16* __restrict__ AB) {
+  const int G = CP / 8;
+  for (int e = threadIdx.x; e < n * G; e += blockDim.x) {
+    const int k = e % n, g = e / n;                       // node fastest
+    uint32_t w[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int c = c8 + 2 * i;
-        const uint32_t lo = c < cin ? f2b(x[node * cin + c]) : 0u;
-        const uint32_t hi = c + 1 < cin ? f2b(x[node * cin + c + 1]) : 0u;
-        w[i] = lo | (hi << 16);
-      }
-      *reinterpret_cast<uint4*>(A + node * CP + c8) = make_uint4(w[0], w[1], w[2], w[3]);
+    for (int i = 0; i < 4; ++i) {
+      const int c = 8 * g + 2 * i;
+      const uint32_t lo = c < cn ? sh[k * cn + c] : 0u, hi = c + 1 < cn ? sh[k * cn + c + 1] : 0u;
+      w[i] = lo | (hi << 16);
     }
+    const size_t node = node0 + k;
+    size_t o;
+    if (N < 16) {
+      o = node * CP + 8 * g;
+    } else {
+      const int z = (int)(node & (N - 1));
+      o = (node - z) * CP + (N >= 64 ? tiled_at<4>(z, 8 * g, CP) : N == 32 ? tiled_at<2>(z, 8 * g, CP)
+                                                                     : tiled_at<1>(z, 8 * g, CP));
+    }
+    *reinterpret_cast<uint4*>(A + o) = make_uint4(w[0], w[1], w[2], w[3]);
   }
+  if (!AB) return;
+  for (int e = threadIdx.x; e < n / 8 * CP; e += blockDim.x) {
+    const int c = e % CP, g = e / CP;                     // channel fastest
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t lo = c < cn ? sh[(8 * g + 2 * i) * cn + c] : 0u, hi = c < cn ? sh[(8 * g + 2 * i + 1) * cn + c] : 0u;
+      w[i] = lo | (hi << 16);
+    }
+    *reinterpret_cast<uint4*>(AB + ((node0 / 8 + g) * CP + c) * 8) = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
+// Input rows x[node][cin] FP32 -> bf16 activation of CP channels (and blocked copy).
+static __global__ void __launch_bounds__(256)
+k_pack_input(const float* __restrict__ x, int cin, int CP, size_t nodes, int N, bf16* __restrict__ A,
+             bf16* __restrict__ AB) {
+  __shared__ bf16 sh[EN * 32];
+  const size_t node0 = (size_t)blockIdx.x * EN;
+  const int n = nodes - node0 < EN ? (int)(nodes - node0) : EN;
+  for (int e = threadIdx.x; e < n * cin; e += 256) sh[e] = f2b(x[node0 * cin + e]);
+  __syncthreads();
+  emit_rows(sh, cin, CP, node0, n, N, A, AB);
 }
 
 // Master FP32 weights w[tap][co][ci] -> bf16 W[tap][co][ci] and Wt[tap][ci][co].
@@ -609,32 +667,25 @@ static __global__ void k_pack_weights(const float* __restrict__ w, int CI, int C
 }
 
 // Mean squared error over nodes x cout: dY[node][co] = 2 (y - t) / (nodes cout)
-// for co < cout (0 for padding channels), per-block partial sums of (y - t)^2.
+// for co < cout (0 for padding channels) as an activation and its blocked copy,
+// per-block sums of (y - t)^2.  y and t are rows of cout channels.
 static __global__ void __launch_bounds__(256)
-k_mse(const float* __restrict__ y, const float* __restrict__ t, int cout, int CP, size_t nodes,
-      bf16* __restrict__ dY, double* __restrict__ part) {
+k_mse(const float* __restrict__ y, const float* __restrict__ t, int cout, int CP, size_t nodes, int N,
+      bf16* __restrict__ dY, bf16* __restrict__ dYB, double* __restrict__ part) {
+  __shared__ bf16 rows[EN * 32];
   __shared__ double sh[256];
   double s = 0.0;
   const double scale = 2.0 / ((double)nodes * cout);
-  // one node per thread and step, 16-byte stores of dY (CP is 16 or 32)
-  for (size_t node = blockIdx.x * (size_t)blockDim.x + threadIdx.x; node < nodes;
-       node += (size_t)gridDim.x * blockDim.x) {
-    for (int c8 = 0; c8 < CP; c8 += 8) {
-      uint32_t w[4];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int c = c8 + i;
-        float g = 0.f;
-        if (c < cout) {
-          const double d = (double)y[node * CP + c] - (double)t[node * cout + c];
-          s += d * d;
-          g = (float)(scale * d);
-        }
-        const uint32_t b = f2b(g);
-        if (i & 1) w[i / 2] |= b << 16; else w[i / 2] = b;
-      }
-      *reinterpret_cast<uint4*>(dY + node * CP + c8) = make_uint4(w[0], w[1], w[2], w[3]);
+  for (size_t node0 = (size_t)blockIdx.x * EN; node0 < nodes; node0 += (size_t)gridDim.x * EN) {
+    const int n = nodes - node0 < EN ? (int)(nodes - node0) : EN;
+    for (int e = threadIdx.x; e < n * cout; e += 256) {
+      const double d = (double)y[node0 * cout + e] - (double)t[node0 * cout + e];
+      s += d * d;
+      rows[e] = f2b((float)(scale * d));
     }
+    __syncthreads();
+    emit_rows(rows, cout, CP, node0, n, N, dY, dYB);
+    __syncthreads();
   }
   sh[threadIdx.x] = s;
   __syncthreads();
@@ -657,12 +708,6 @@ static __global__ void k_adam(float* __restrict__ w, const float* __restrict__ g
   v[i] = vi;
   const float mh = mi / (1.f - powf(b1, (float)t)), vh = vi / (1.f - powf(b2, (float)t));
   w[i] -= lr * mh / (sqrtf(vh) + eps);
-}
-
-// Output rows [node][CP] FP32 -> [node][cout].
-static __global__ void k_unpack_output(const float* __restrict__ yp, int CP, int cout, size_t nodes, float* __restrict__ y) {
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < nodes * cout; e += (size_t)gridDim.x * blockDim.x)
-    y[e] = yp[(e / cout) * CP + e % cout];
 }
 
 }  // namespace cnn
