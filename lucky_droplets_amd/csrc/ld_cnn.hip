@@ -28,7 +28,8 @@ struct ld_cnn {
   float* part = nullptr;
   double* mpart = nullptr;
   int nblk_w = 0, chunk = 0;
-  int nblk_w2 = 0, chunk2 = 0;              // k_wgrad2 blocks and nodes per block (N >= 16)
+  int nblk_w2 = 0, chunk2 = 0;              // k_wgrad2 / k_wgrad3 blocks (N >= 16), nodes per k_wgrad2 block
+  int units = 0, ysplit = 1;                // k_wgrad3: units of work, y-splits per x and z chunk
   bf16 *xt = nullptr, *dzt = nullptr;       // node-blocked channel-major copies for the weight gradient
   bf16* actB[LD_CNN_MAX_LAYERS] = {};       // node-blocked copies of the hidden activations (N >= 16)
   int adam_t = 0;
@@ -126,12 +127,14 @@ int conv(ld_cnn* c, int CI, int CO, const bf16* X, const bf16* W, const float* b
 // copies of X / dZ that the producing kernels wrote (N >= 16).
 int wgrad(ld_cnn* c, int CI, int CO, const bf16* X, const bf16* dZ, const bf16* XB, const bf16* dZB, int* nblk) {
   if (c->N >= 16) {
-    // one neighbour line per wavefront (three measured slower: 396 -> 411 us at 128^3, 32 -> 32)
-    constexpr int LPW = 1;
-    const dim3 g((unsigned)c->nblk_w2), t(64 * 9 / LPW);
 #define LD_WG2_CASE(A, B)                                                                                  \
     if (CI == A && CO == B) {                                                                              \
-      hipLaunchKernelGGL((k_wgrad2<A, B, LPW>), g, t, 0, c->st, XB, dZB, c->part, c->N, c->chunk2);          \
+      if (c->N >= 32)                                                                                      \
+        hipLaunchKernelGGL((k_wgrad3<A, B>), dim3((unsigned)c->nblk_w2), dim3(768), 0, c->st, XB, dZB, c->part, \
+                           c->N, c->units, c->ysplit);                                                     \
+      else                                                                                                 \
+        hipLaunchKernelGGL((k_wgrad2<A, B>), dim3((unsigned)c->nblk_w2), dim3(576), 0, c->st, XB, dZB, c->part, \
+                           c->N, c->chunk2);                                                               \
       LAUNCHED();                                                                                          \
       *nblk = c->nblk_w2;                                                                                  \
       return LD_OK;                                                                                        \
@@ -198,7 +201,7 @@ int backward(ld_cnn* c, const float* target, double* loss) {
     int nblk = 0;
     CK(wgrad(c, CI, CO, c->act[l], c->dz[cur], l > 0 ? c->actB[l] : c->xt, c->dzt, &nblk));
     const int n = 27 * CO * CI + CO;
-    hipLaunchKernelGGL(k_reduce_parts, dim3((n + 255) / 256), dim3(256), 0, c->st, (const float*)c->part, nblk, n,
+    hipLaunchKernelGGL(k_reduce_parts, dim3((n + 31) / 32), dim3(256), 0, c->st, (const float*)c->part, nblk, n,
                        c->grads + c->off[l]);
     LAUNCHED();
     if (l > 0) {
@@ -256,10 +259,19 @@ int ld_cnn_create(const ld_cnn_params* p, ld_cnn** out) {
   c->chunk = 64;
   while (c->nodes / c->chunk > 256) c->chunk *= 2;
   c->nblk_w = (int)(c->nodes / c->chunk);
-  // k_wgrad2: at most 512 blocks, each over a multiple of 32 nodes
-  c->chunk2 = 32;
-  while (c->nodes / c->chunk2 > 512) c->chunk2 *= 2;
-  c->nblk_w2 = (int)(c->nodes / c->chunk2);
+  if (c->N >= 32) {
+    // units of (x, 32-node z chunk, N / ysplit y-lines), at most 256 blocks (one
+    // per CU); small grids are split in y, down to 16 lines
+    const int base = c->N * (c->N / 32);
+    while (base * c->ysplit < 256 && c->N / (2 * c->ysplit) >= 16) c->ysplit *= 2;
+    c->units = base * c->ysplit;
+    c->nblk_w2 = c->units < 256 ? c->units : 256;
+  } else {
+    // k_wgrad2 (N = 16): 64 blocks of 64 nodes (32 -> 32 channels 8.1 us; 32
+    // blocks 8.9, 128 blocks 10.6)
+    c->chunk2 = 64;
+    c->nblk_w2 = (int)(c->nodes / c->chunk2);
+  }
   int64_t maxlayer = 0;
   for (int l = 0; l < c->L; ++l) {
     const int64_t n = 27LL * c->ch[l] * c->ch[l + 1] + c->ch[l + 1];

@@ -461,8 +461,8 @@ k_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ, float* __restri
 }
 
 // Weight and bias gradients from node-blocked channel-major operands
-// (blocked_at()) on the 16x16x32 bf16 MFMA (M = output channels,
-// N = input channels, K = nodes):
+// (blocked_at()) on the 16x16x32 bf16 MFMA (M = output channels, N = input
+// channels, K = nodes):
 //   A (16x32): lane l holds dZ[node k0 + 8 (l / 16) + i][co0 + l % 16]  (one 16-byte run)
 //   B (32x16): lane l holds X[nbr(node k0 + 8 (l / 16) + i, tap)][ci0 + l % 16]
 // so the 16 lanes of a row read 256 consecutive bytes.
@@ -470,22 +470,159 @@ k_wgrad(const bf16* __restrict__ X, const bf16* __restrict__ dZ, float* __restri
 // tap (dx, dy, dz) are eight consecutive z on the neighbour line, shifted by
 // dz: the lane loads the aligned 16 bytes at z plus one dword on each side
 // (periodic in z) and forms the dz = -1 and +1 operands with v_alignbyte.
-// Neighbour line l = 3 (dx + 1) + (dy + 1) carries taps 3 l .. 3 l + 2; a
-// wavefront owns LPW consecutive lines.  Block b sums nodes
-// [b chunk, (b + 1) chunk) in K-steps of 32 and writes its partial
-//   part[b][(tap CO + co) CI + ci],  part[b][27 CO CI + co] (bias, wavefront 0).
-// LPW neighbour lines per wavefront (9 / LPW wavefronts per block): LPW = 3
-// gives wavefront w the lines (w - 1, -1..1), so the dZ fragments are read by
-// three wavefronts instead of nine and each feeds 9 taps.
-template <int CI, int CO, int LPW>
-__global__ void __launch_bounds__(64 * 9 / LPW)
+struct XRun {
+  uint4 c;
+  uint32_t pv, nv;           // the dwords before and after the run
+  // the line's runs of this lane's channel: own at o, before at op, after at on
+  // (byte offsets; a uniform line pointer plus 32-bit lane offsets)
+  __device__ __forceinline__ void load(const bf16* __restrict__ line, uint32_t o, uint32_t op, uint32_t on) {
+    const char* l = reinterpret_cast<const char*>(line);
+    c = *reinterpret_cast<const uint4*>(l + o);
+    pv = *reinterpret_cast<const uint32_t*>(l + op + 12);
+    nv = *reinterpret_cast<const uint32_t*>(l + on);
+  }
+  __device__ __forceinline__ void taps(bf16x8 f[3]) const {      // dz = -1, 0, 1
+    const uint32_t s1 = __builtin_amdgcn_alignbyte(c.y, c.x, 2), s2 = __builtin_amdgcn_alignbyte(c.z, c.y, 2),
+                   s3 = __builtin_amdgcn_alignbyte(c.w, c.z, 2);
+    f[0] = __builtin_bit_cast(bf16x8, make_uint4(__builtin_amdgcn_alignbyte(c.x, pv, 2), s1, s2, s3));
+    f[1] = __builtin_bit_cast(bf16x8, c);
+    f[2] = __builtin_bit_cast(bf16x8, make_uint4(s1, s2, s3, __builtin_amdgcn_alignbyte(nv, c.w, 2)));
+  }
+};
+
+// N >= 32.  A unit of work is a run of y-lines of one x and one 32-node z chunk;
+// wavefront (dx, t) of a block owns the nine taps of one dx and 16 input
+// channels, and walks the unit's X lines in y: each X run it loads meets the
+// dZ runs of the three lines around it, which it keeps in registers (one new
+// dZ line per step), so a step's loads (one X run, CO/16 dZ runs, the next
+// step's issued before this step's products) feed 9 CO/16 instructions.  One
+// neighbour line per wavefront, nine wavefronts reading the same dZ, fed 3 per
+// X run and was bound by the loads.  Twelve wavefronts fill a CU (three per
+// SIMD): two (32 input channels) or four shares of the unit's lines, which add
+// up through LDS.
+// Blocks take consecutive units and write one partial each:
+//   part[b][(tap CO + co) CI + ci],  part[b][27 CO CI + co] (bias: products
+// with a run of ones).  128^3: 32 -> 32 channels 315 -> 119 us (980 TFLOP/s),
+// 32 -> 16 213 -> 97, 16 -> 32 204 -> 70.  Blocks of six wavefronts took 189 us
+// (SIMDs unevenly filled), a scheduling barrier after the loads 180 (spills).
+template <int CI, int CO>
+__global__ void __launch_bounds__(768, 3)
+k_wgrad3(const bf16* __restrict__ XB, const bf16* __restrict__ dZB, float* __restrict__ part, int N, int units,
+         int ysplit) {
+  constexpr int MT = CO / 16, TI = CI / 16, H = 4 / TI;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n16 = lane & 15, q = lane >> 4, msk = N - 1, G8 = N >> 3;
+  const int role = w % (3 * TI), h = w / (3 * TI);       // taps and channels; share of the unit's lines
+  const int dxi = role % 3, t = role / 3;
+  const bool bias = role == 1;
+  f32x4 acc[9][MT], db[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    db[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 9; ++d) acc[d][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
+  const int G = gridDim.x, per = (units + G - 1) / G;
+  const int lb = (G % 8 == 0) ? (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int zcs = N / 32, len = N / ysplit / H;
+  const size_t xs = (size_t)N * CI, zs = (size_t)N * CO;            // elements per line
+  for (int u = lb * per; u < units && u < (lb + 1) * per; ++u) {
+    const int zc = u % zcs, ys = (u / zcs) % ysplit, x = u / zcs / ysplit;
+    const int y0 = (ys * H + h) * len;
+    const int g = zc * 4 + q;
+    const int ci = t * 16 + n16;
+    const uint32_t xo = (uint32_t)(g * CI + ci) * 16, xp = (uint32_t)((g ? g - 1 : G8 - 1) * CI + ci) * 16,
+                   xn = (uint32_t)((g + 1 < G8 ? g + 1 : 0) * CI + ci) * 16, zo = (uint32_t)(g * CO + n16) * 16;
+    const bf16* xb = XB + (size_t)((x + dxi - 1) & msk) * N * xs;
+    const bf16* zb = dZB + (size_t)x * N * zs;
+    auto loadz = [&](int y, uint4 (&d)[MT]) {
+      const char* line = reinterpret_cast<const char*>(zb + (size_t)(uint32_t)(y & msk) * zs);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) d[m] = *reinterpret_cast<const uint4*>(line + zo + m * 256);
+    };
+    // four steps per turn: dZ lines y - 1 .. y + 2 rotate through d[0..3], X lines
+    // y and y + 1 through xr[0..1], without register moves (len is a multiple of 4)
+    uint4 d[4][MT];
+    XRun xr[2];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) loadz(y0 - 1 + k, d[k]);
+    xr[0].load(xb + (size_t)y0 * xs, xo, xp, xn);
+#pragma unroll 1
+    for (int s4 = 0; s4 < len; s4 += 4) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int y = y0 + s4 + k;
+        loadz(y + 2, d[(k + 3) & 3]);
+        xr[(k + 1) & 1].load(xb + (size_t)(uint32_t)((y + 1) & msk) * xs, xo, xp, xn);
+        bf16x8 f[3];
+        xr[k & 1].taps(f);
+        // X line y is the neighbour dy = 1, 0, -1 of dZ lines y - 1, y, y + 1
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+#pragma unroll
+          for (int dz = 0; dz < 3; ++dz)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+              const int a = 3 * (2 - e) + dz;
+              acc[a][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, d[(k + e) & 3][m]), f[dz],
+                                                                  acc[a][m], 0, 0, 0);
+            }
+        if (bias) {
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            db[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, d[(k + 1) & 3][m]), ones, db[m], 0, 0, 0);
+        }
+      }
+    }
+  }
+  // the shares add up in order, CO/16 parts of the accumulators at a time
+  __shared__ f32x4 sum[3 * TI][10][64];
+#pragma unroll
+  for (int k = 1; k < H; ++k)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      __syncthreads();
+      if (h == k) {
+        sum[role][9][lane] = db[m];
+#pragma unroll
+        for (int d = 0; d < 9; ++d) sum[role][d][lane] = acc[d][m];
+      }
+      __syncthreads();
+      if (h == 0) {
+        db[m] += sum[role][9][lane];
+#pragma unroll
+        for (int d = 0; d < 9; ++d) acc[d][m] += sum[role][d][lane];
+      }
+    }
+  if (h) return;
+  float* out = part + (size_t)blockIdx.x * (27 * CO * CI + CO);
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+#pragma unroll
+    for (int d = 0; d < 9; ++d)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        out[((size_t)(dxi * 9 + d) * CO + m * 16 + 4 * q + i) * CI + t * 16 + n16] = acc[d][m][i];
+    if (bias && n16 == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) out[27 * CO * CI + m * 16 + 4 * q + i] = db[m][i];
+    }
+  }
+}
+
+// N = 16: a K-step of 32 nodes covers two z-lines.  Wavefront w owns neighbour
+// line (dx, dy) = (w / 3 - 1, w % 3 - 1) and its three taps; block b sums nodes
+// [b chunk, (b + 1) chunk) and writes its partial as above.
+template <int CI, int CO>
+__global__ void __launch_bounds__(576)
 k_wgrad2(const bf16* __restrict__ XB, const bf16* __restrict__ dZB, float* __restrict__ part, int N, int chunk) {
   constexpr int MT = CO / 16, NT = CI / 16;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int n16 = lane & 15, q = lane >> 4, msk = N - 1;
-  f32x4 acc[3 * LPW][MT][NT];
+  const int n16 = lane & 15, q = lane >> 4, msk = N - 1, G = N >> 3;
+  f32x4 acc[3][MT][NT];
 #pragma unroll
-  for (int d = 0; d < 3 * LPW; ++d)
+  for (int d = 0; d < 3; ++d)
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -493,13 +630,13 @@ k_wgrad2(const bf16* __restrict__ XB, const bf16* __restrict__ dZB, float* __res
   float db[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) db[m] = 0.f;
-  // one K-step: the lane's 8 nodes start at z = zq on line (x, y) (8-node
-  // group gq of the dZ copy); A from dZ, B from the neighbour lines' X copy
-  auto kstep = [&](size_t gq, int zq, int x, int y) {
+  for (int ks = 0; ks < chunk / 32; ++ks) {
+    const size_t node = (size_t)blockIdx.x * chunk + 32 * ks + 8 * q, line = node / N;
+    const int g = (int)(node & msk) >> 3, x = (int)(line / N), y = (int)(line & msk);
     bf16x8 a[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-      const uint4 v = *reinterpret_cast<const uint4*>(dZB + (gq * CO + m * 16 + n16) * 8);
+      const uint4 v = *reinterpret_cast<const uint4*>(dZB + ((node >> 3) * CO + m * 16 + n16) * 8);
       a[m] = __builtin_bit_cast(bf16x8, v);
       if (w == 0) {
         const uint32_t u[4] = {v.x, v.y, v.z, v.w};
@@ -507,70 +644,32 @@ k_wgrad2(const bf16* __restrict__ XB, const bf16* __restrict__ dZB, float* __res
         for (int i = 0; i < 4; ++i) db[m] += b2f((bf16)(u[i] & 0xffff)) + b2f((bf16)(u[i] >> 16));
       }
     }
-    const int G = N >> 3;                          // 8-node groups per z-line
+    const bf16* nl = XB + ((size_t)((x + w / 3 - 1) & msk) * N + ((y + w % 3 - 1) & msk)) * N * CI;
 #pragma unroll
-    for (int li = 0; li < LPW; ++li) {
-      const int wl = w * LPW + li;                 // neighbour line index 0..8
-      const int dx = wl / 3 - 1, dy = wl % 3 - 1;
-      const size_t gb = ((size_t)((x + dx) & msk) * N + ((y + dy) & msk)) * G;   // its first group
-      const size_t cg = gb + (zq >> 3);
-      const size_t pg = zq ? cg - 1 : gb + G - 1;                                // periodic in z
-      const size_t ng = zq + 8 < N ? cg + 1 : gb;
+    for (int t = 0; t < NT; ++t) {
+      const int ci = t * 16 + n16;
+      XRun r;
+      r.load(nl, (uint32_t)(g * CI + ci) * 16, (uint32_t)((g ? g - 1 : G - 1) * CI + ci) * 16,
+             (uint32_t)((g + 1 < G ? g + 1 : 0) * CI + ci) * 16);
+      bf16x8 f[3];
+      r.taps(f);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int ci = t * 16 + n16;
-        const uint4 c = *reinterpret_cast<const uint4*>(XB + (cg * CI + ci) * 8);
-        const uint32_t pv = *reinterpret_cast<const uint32_t*>(XB + (pg * CI + ci) * 8 + 6);
-        const uint32_t nv = *reinterpret_cast<const uint32_t*>(XB + (ng * CI + ci) * 8);
-        const uint32_t s1 = __builtin_amdgcn_alignbyte(c.y, c.x, 2), s2 = __builtin_amdgcn_alignbyte(c.z, c.y, 2),
-                       s3 = __builtin_amdgcn_alignbyte(c.w, c.z, 2);
-        const bf16x8 fm = __builtin_bit_cast(bf16x8, make_uint4(__builtin_amdgcn_alignbyte(c.x, pv, 2), s1, s2, s3));
-        const bf16x8 f0 = __builtin_bit_cast(bf16x8, c);
-        const bf16x8 fp = __builtin_bit_cast(bf16x8, make_uint4(s1, s2, s3, __builtin_amdgcn_alignbyte(nv, c.w, 2)));
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-          acc[3 * li][m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], fm, acc[3 * li][m][t], 0, 0, 0);
-          acc[3 * li + 1][m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], f0, acc[3 * li + 1][m][t], 0, 0, 0);
-          acc[3 * li + 2][m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], fp, acc[3 * li + 2][m][t], 0, 0, 0);
-        }
-      }
-    }
-  };
-  const size_t kb = (size_t)blockIdx.x * chunk;
-  if (N >= 32) {
-    // the chunk is whole z-lines: line coordinates once per line, K-steps
-    // along z with plain increments
-    const int lines = chunk / N;
-    const size_t l0 = kb / N;
-    for (int li0 = 0; li0 < lines; ++li0) {
-      const size_t line = l0 + li0;
-      const int x = (int)(line / N), y = (int)(line & msk);
-      const size_t gl = line * (size_t)(N >> 3);
-#pragma unroll 2
-      for (int z0 = 0; z0 < N; z0 += 32) {
-        const int zq = z0 + 8 * q;
-        kstep(gl + (zq >> 3), zq, x, y);
-      }
-    }
-  } else {
-    for (int ks = 0; ks < chunk / 32; ++ks) {
-      const size_t nq = kb + 32 * ks + 8 * q;
-      const size_t line = nq / N;
-      kstep(nq >> 3, (int)(nq & msk), (int)(line / N), (int)(line & msk));
+        for (int d = 0; d < 3; ++d)
+          acc[d][m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], f[d], acc[d][m][t], 0, 0, 0);
     }
   }
   float* out = part + (size_t)blockIdx.x * (27 * CO * CI + CO);
 #pragma unroll
-  for (int d = 0; d < 3 * LPW; ++d) {
-    const int tap = 3 * (w * LPW) + d;
+  for (int d = 0; d < 3; ++d)
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          out[((size_t)tap * CO + m * 16 + 4 * q + i) * CI + t * 16 + n16] = acc[d][m][t][i];
-  }
+          out[((size_t)(3 * w + d) * CO + m * 16 + 4 * q + i) * CI + t * 16 + n16] = acc[d][m][t][i];
   if (w == 0) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
@@ -582,23 +681,35 @@ k_wgrad2(const bf16* __restrict__ XB, const bf16* __restrict__ dZB, float* __res
   }
 }
 
-// out[i] = sum over blocks of part[b][i] (fixed order), i < n.
+// out[i] = sum over blocks of part[b][i], i < n, in a fixed order: thread group
+// k of a block's 8 sums the partials b = k (mod 8), loads in batches of 8 ahead
+// of their additions, and the eight sums are added in order.  The four layers
+// of 3-32-32-32-3 at 128^3: 75 us over 512 partials with one thread per entry,
+// 34 us like this, 23 us over k_wgrad3's 256.
 static __global__ void __launch_bounds__(256)
 k_reduce_parts(const float* __restrict__ part, int nblk, int n, float* __restrict__ out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  // loads in batches of 16 ahead of their (ordered) additions
+  __shared__ float sh[8][32];
+  const int e = threadIdx.x & 31, k = threadIdx.x >> 5;
+  const int i = blockIdx.x * 32 + e;
   float s = 0.f;
-  int b = 0;
-  for (; b + 16 <= nblk; b += 16) {
-    float v[16];
+  if (i < n) {
+    int b = k;
+    for (; b + 56 < nblk; b += 64) {
+      float v[8];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = part[(size_t)(b + u) * n + i];
+      for (int u = 0; u < 8; ++u) v[u] = part[(size_t)(b + 8 * u) * n + i];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) s += v[u];
+      for (int u = 0; u < 8; ++u) s += v[u];
+    }
+    for (; b < nblk; b += 8) s += part[(size_t)b * n + i];
   }
-  for (; b < nblk; ++b) s += part[(size_t)b * n + i];
-  out[i] = s;
+  sh[k][e] = s;
+  __syncthreads();
+  if (k == 0 && i < n) {
+#pragma unroll
+    for (int u = 1; u < 8; ++u) s += sh[u][e];
+    out[i] = s;
+  }
 }
 
 // Rows of bf16 values of EN nodes staged in LDS (sh[node][c], c < cn real
