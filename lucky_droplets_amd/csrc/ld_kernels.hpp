@@ -378,12 +378,14 @@ template <int NT, int NQ> struct Quads {
 template <typename T> __device__ __forceinline__ V4<T> scale4(const V4<T>& a, T s) {
   V4<T> r; r.x = a.x * s; r.y = a.y * s; r.z = a.z * s; r.w = a.w * s; return r;
 }
-// Plain c2r along z of F fields, times `scale` (last pass of irfft_mpi,
-// forced-dns-sm.py:212).
+// Plain c2r along z of the fields of a call (blockIdx.z), times `scale` (last
+// pass of irfft_mpi, forced-dns-sm.py:212).
 template <typename T, int N, int P, int F>
 struct OpZInv {
   const C<T>* in; T* out; size_t fin, fout; T scale;
-  __device__ OpZInv shifted(size_t rs) const { OpZInv o = *this; o.in = rsel1(in, rs); o.out = rsel1(out, rs); return o; }
+  __device__ OpZInv shifted(size_t) const {
+    OpZInv o = *this; o.in = in + blockIdx.z * fin; o.out = out + blockIdx.z * fout; return o;
+  }
   __device__ const C<T>* specIn(int f) const { return in + f * fin; }
   __device__ C<T>* specOut(int) const { return nullptr; }
   __device__ void physical(const ZTile<T, N, P>& t, int line0) const {
@@ -397,10 +399,16 @@ struct OpZInv {
   }
 };
 // Plain r2c along z of F fields (first pass of rfft_mpi, forced-dns-sm.py:202).
-template <typename T, int N, int P, int F>
+// CALL: blockIdx.z is the field of a call, not the realization.
+template <typename T, int N, int P, int F, bool CALL = false>
 struct OpZFwd {
   const T* in; C<T>* out; size_t fin, fout;
-  __device__ OpZFwd shifted(size_t rs) const { OpZFwd o = *this; o.in = rsel1(in, rs); o.out = rsel1(out, rs); return o; }
+  __device__ OpZFwd shifted(size_t rs) const {
+    OpZFwd o = *this;
+    if constexpr (CALL) { o.in = in + blockIdx.z * fin; o.out = out + blockIdx.z * fout; }
+    else { o.in = rsel1(in, rs); o.out = rsel1(out, rs); }
+    return o;
+  }
   __device__ const C<T>* specIn(int) const { return nullptr; }
   __device__ C<T>* specOut(int f) const { return out + f * fout; }
   __device__ void physical(const ZTile<T, N, P>& t, int line0) const {
