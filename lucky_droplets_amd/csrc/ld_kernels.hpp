@@ -699,8 +699,15 @@ k_x_uw3(const C<T>* __restrict__ uk0, C<T>* __restrict__ out0, size_t fs, const 
   const bool wr = live;
   C<T> u[N2], w[N2];
   if (live) {
+    // of a live line only the modes inside the mask radius are nonzero (44 % of
+    // the live lines' entries at kcut = N/3): the others are not read (256^3
+    // FP32: 105 -> 89 us)
 #pragma unroll
-    for (int r = 0; r < N2; ++r) u[r] = ld32(uk + f * fs, (uint32_t)(q + posOut<N>(n1, r) * js));
+    for (int r = 0; r < N2; ++r) {
+      const int ix = posOut<N>(n1, r), kx = kwave(ix, N);
+      u[r] = kcut >= N / 2 || kx * kx + kyi * kyi + kzi * kzi <= kcut * (kcut + 1)
+                 ? ld32(uk + f * fs, (uint32_t)(q + ix * js)) : mkc<T>((T)0, (T)0);
+    }
   } else {
 #pragma unroll
     for (int r = 0; r < N2; ++r) u[r] = mkc<T>((T)0, (T)0);
@@ -808,6 +815,13 @@ k_x_rhs3(RhsArgs<T> A0, const C<T>* __restrict__ tw, size_t rs) {
     if (idle) break;
     const int ix = posOut<N>(n1, r);
     const Mode<T> md = mode<T, N>(ix, iy, iz);
+    // band: a mode outside the mask has u_hat = 0 at every stage, so its RK
+    // update is the zero already in place and its v_hat is zero (256^3 FP32,
+    // 56 % of the live lines' modes: 172 -> 123 us)
+    if (A.band && md.mask == (T)0) {
+      L0[ix] = mkc<T>((T)0, (T)0); L1[ix] = mkc<T>((T)0, (T)0); L2[ix] = mkc<T>((T)0, (T)0);
+      continue;
+    }
     const uint32_t o = (uint32_t)(q + ix * js);
     const C<T> us0 = ld32(US0, o), us1 = ld32(US1, o), us2 = ld32(US2, o);
     // forcing (forced-dns-sm.py:262-275)
