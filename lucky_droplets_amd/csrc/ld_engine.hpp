@@ -348,6 +348,7 @@ struct Engine final : EngineBase {
     if (const char* e = getenv("LD_SERIAL")) serial = atoi(e) != 0;
     if (const char* e = getenv("LD_YSPLIT")) ysplit = atoi(e) != 0;
     if (const char* e = getenv("LD_LATE_DENSITY")) late_density = atoi(e) != 0;
+    if (const char* e = getenv("LD_ROW_TILE_MIN")) tile_rows_min = atoll(e);   // measurement, tests
     if (const char* e = getenv("LD_ROW_SORT_MIN")) api_sort_min = atoll(e);   // measurement, tests
     if (const char* e = getenv("LD_TRUNCATE")) kc = atoi(e) != 0 ? N / 3 : N / 2;
     if (const char* e = getenv("LD_PSTAGE_LDS")) {
@@ -1561,8 +1562,24 @@ struct Engine final : EngineBase {
     hipLaunchKernelGGL((k_row_bin<N>), dim3(pb), dim3(256), 0, st, coord, (int)n_, p.L, dp.inv_dx, pkey, prank, hist);
     LD_LAUNCHED();
     LD_TRY(scan_bins(st));
-    hipLaunchKernelGGL(k_row_scatter, dim3(pb), dim3(256), 0, st, coord, (int)n_, p.L, w, (const int*)pkey,
-                       (const int*)prank, (const int*)hist, dep, flist);
+    hipLaunchKernelGGL((k_row_scatter<N>), dim3(pb), dim3(256), 0, st, coord, (int)n_, p.L, dp.inv_dx, w,
+                       (const int*)pkey, (const int*)prank, (const int*)hist, dep, flist);
+    LD_LAUNCHED();
+    return LD_OK;
+  }
+  static constexpr int NTILE = GatherTile<N, 0>::NTILE;
+  // Tile gather from this many rows (us per call, tiles / four lanes per row):
+  // pRHS from 48 rows per tile (256^3 FP32: 281 / 284 at 24, 359 / 561 at 96;
+  // FP64 489 / 500 at 48; 128^3 FP64 96 / 96 at 48, 106 / 162 at 200), interp
+  // from 96 (256^3 FP64, 7 components: 469 / 477 at 96, FP32 286 / 371); below
+  // 512 tiles (up to 64^3) the blocks are too few and the two are equal: never.
+  int64_t tile_rows_min = -1;        // >= 0: the line for every call (LD_ROW_TILE_MIN)
+  bool rows_tiled(int64_t n_, int per) const {
+    return tile_rows_min >= 0 ? n_ >= tile_rows_min : NTILE >= 512 && n_ >= per * (int64_t)NTILE;
+  }
+  int tile_gather_rows(const GatherFields<T>& g, int64_t n_, const int* rowmap, double* out) {
+    hipLaunchKernelGGL((k_tile_gather<T, double, N, 0, 256>), dim3(NTILE * g.n), dim3(256), 0, st, g, (const double4*)dep,
+                       (const int*)hist, (int)n_, (int)cap, rowmap, out, dp, (size_t)0);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -1580,8 +1597,15 @@ struct Engine final : EngineBase {
                 double* interpm, double* exterpm) {
     if (n_ > 0 && rows_sorted(ROW_PRHS, n_)) {
       LD_TRY(sort_rows(coord, n_, nullptr));
-      hipLaunchKernelGGL((k_prhs_sorted<T, N>), dim3(quad_blocks(n_)), dim3(256), 0, st, coord, (int)n_, uf, usf, nf,
-                         dep, (const int*)flist, rhs, interpm, exterpm, dp);
+      if (rows_tiled(n_, 48)) {
+        GatherFields<T> g{uf, usf, nf, 3, 3, 7, nullptr};
+        LD_TRY(tile_gather_rows(g, n_, nullptr, rows_b));
+        hipLaunchKernelGGL(k_prhs_finish, dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, coord, (int)n_, (int)cap,
+                           (const double*)rows_b, dep, (const int*)flist, rhs, interpm, exterpm, dp);
+      } else {
+        hipLaunchKernelGGL((k_prhs_sorted<T, N>), dim3(quad_blocks(n_)), dim3(256), 0, st, coord, (int)n_, uf, usf, nf,
+                           dep, (const int*)flist, rhs, interpm, exterpm, dp);
+      }
       LD_LAUNCHED();
       LD_TRY(deposit_rows(n_, fcp));
       return rows_end();
@@ -1626,9 +1650,14 @@ struct Engine final : EngineBase {
     LD_TRY(join(st, st2, evB));
     if (rows_sorted(ROW_INTERP, n_, nc)) {
       LD_TRY(sort_rows(coord, n_, nullptr));
-      hipLaunchKernelGGL((k_interp_sorted<T, N>), dim3(quad_blocks(n_)), dim3(256), 0, st, (int)n_, (const T*)f, nc,
-                         (const double4*)dep, (const int*)flist, out, dp);
-      LD_LAUNCHED();
+      if (rows_tiled(n_, 96) && nc <= 64) {
+        GatherFields<T> g{(const T*)f, nullptr, nullptr, nc, 0, nc, nullptr};
+        LD_TRY(tile_gather_rows(g, n_, flist, out));
+      } else {
+        hipLaunchKernelGGL((k_interp_sorted<T, N>), dim3(quad_blocks(n_)), dim3(256), 0, st, (int)n_, (const T*)f, nc,
+                           (const double4*)dep, (const int*)flist, out, dp);
+        LD_LAUNCHED();
+      }
       return rows_end();
     }
     hipLaunchKernelGGL((k_interp<T, N>), dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, coord, (int)n_,

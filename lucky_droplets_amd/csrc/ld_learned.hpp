@@ -198,9 +198,9 @@ k_frozen_rk4(double* __restrict__ rows, int np, const V4<T>* __restrict__ g, dou
       }
       const int i0 = originOf(xw[0], P.inv_dx), j0 = originOf(xw[1], P.inv_dx), k0 = originOf(xw[2], P.inv_dx);
       GT xsn, xcs, ysn, ycs, zsn, zcs;
-      sincosGT((xw[0] - (double)i0 * P.dx) * P.pi_2dx, xsn, xcs);
-      sincosGT((xw[1] - (double)j0 * P.dx) * P.pi_2dx, ysn, ycs);
-      sincosGT((xw[2] - (double)k0 * P.dx) * P.pi_2dx, zsn, zcs);
+      sincosStencil<GT>(xw[0], i0, P.dx, P.inv_dx, P.pi_2dx, xsn, xcs);
+      sincosStencil<GT>(xw[1], j0, P.dx, P.inv_dx, P.pi_2dx, ysn, ycs);
+      sincosStencil<GT>(xw[2], k0, P.dx, P.inv_dx, P.pi_2dx, zsn, zcs);
       const GT wy[4] = {q * ((GT)1 + ycs), q * ((GT)1 + ysn), q * ((GT)1 - ycs), q * ((GT)1 - ysn)};
       const GT wz = q * ((GT)1 + ((c & 2) ? (GT)-1 : (GT)1) * ((c & 1) ? zsn : zcs));
       const uint32_t iz = (uint32_t)wrapIdx<N>(k0 + c);

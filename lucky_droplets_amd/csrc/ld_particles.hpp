@@ -49,6 +49,15 @@ template <typename G> __device__ __forceinline__ void sincosGT(double th, G& s, 
   }
 }
 
+// sin and cos of the stencil angle (x - i0 dx) pi / (2 dx), which lies in
+// [pi/2, pi).  FP64: as sincospi of the angle over pi (no reduction of large
+// arguments, whose code costs registers and scratch memory).
+template <typename G>
+__device__ __forceinline__ void sincosStencil(double x, int i0, double dx, double inv_dx, double pi_2dx, G& s, G& c) {
+  if constexpr (sizeof(G) == 4) sincosGT<G>((x - (double)i0 * dx) * pi_2dx, s, c);
+  else sincospi((x - (double)i0 * dx) * (0.5 * inv_dx), &s, &c);
+}
+
 // cosW4 with the sines and cosines taken in precision G (the angle in FP64).
 template <typename G>
 __device__ __forceinline__ int cosW4G(double x, double dx, double pi_2dx, G w[4]) {
@@ -100,7 +109,7 @@ template <typename G>
 __device__ __forceinline__ int cosW4F(double x, double dx, double inv_dx, double pi_2dx, G w[4]) {
   const int i0 = originOf(x, inv_dx);
   G sn, cs;
-  sincosGT<G>((x - (double)i0 * dx) * pi_2dx, sn, cs);
+  sincosStencil<G>(x, i0, dx, inv_dx, pi_2dx, sn, cs);
   const G q = (G)0.25;
   w[0] = q * ((G)1 + cs);
   w[1] = q * ((G)1 + sn);
@@ -265,6 +274,18 @@ template <int N> struct Bins {
     for (int i = 0; i < 8; ++i) r |= ((v >> i) & 1) << (2 * i);
     return r;
   }
+  // every second bit of v, packed (the inverse of spread2)
+  static __device__ __forceinline__ int pack2(int v) {
+    int r = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r |= ((v >> (2 * i)) & 1) << i;
+    return r;
+  }
+  // first cell of tile number `tile` (key / TS^3)
+  static __device__ __forceinline__ void tileCell(int tile, int& cx, int& cy, int& cz) {
+    const int col = tile / NTt;
+    cx = pack2(col >> 1) * TC; cy = pack2(col) * TC; cz = (tile % NTt) * TC;
+  }
   // key of bin (bx, by, bz): tile columns along z, the columns in Morton order
   // of (tile x, tile y); x-major inside the tile
   static __device__ __forceinline__ int key(int bx, int by, int bz) {
@@ -366,9 +387,9 @@ k_particles_stage(PStage<T, PT> A0) {
   // the angles are formed in FP64; their sines and cosines are taken in the
   // weight precision GT (the FP32 form rounds the angle in [pi/2, pi) to FP32)
   GT xsn, xcs, ysn, ycs, zsn, zcs;
-  sincosGT((xw - (double)i0 * dx) * pi_2dx, xsn, xcs);
-  sincosGT((yw - (double)j0 * dx) * pi_2dx, ysn, ycs);
-  sincosGT((zw - (double)k0 * dx) * pi_2dx, zsn, zcs);
+  sincosStencil<GT>(xw, i0, dx, inv_dx, pi_2dx, xsn, xcs);
+  sincosStencil<GT>(yw, j0, dx, inv_dx, pi_2dx, ysn, ycs);
+  sincosStencil<GT>(zw, k0, dx, inv_dx, pi_2dx, zsn, zcs);
   const GT q = (GT)0.25;
   const GT wy[4] = {q * ((GT)1 + ycs), q * ((GT)1 + ysn), q * ((GT)1 - ycs), q * ((GT)1 - ysn)};
   int iy[4];
@@ -808,6 +829,128 @@ k_fallback_fold(const double4* __restrict__ dep0, const int* __restrict__ flist0
   }
 }
 
+// ------------------------------------------------------------ tile gather
+// Gather of several planar fields at bin-sorted slots, one field of one bin
+// tile per workgroup: the field's nodes that the stencils of the tile's S^3
+// cells reach, and W cells of motion since the sort on every side, are staged
+// in LDS and one thread per slot sums its 64 nodes from there.
+//
+// A gather straight from global memory reads a 128-byte line of L2 for every
+// 16 (planar FP32) or 64 bytes (node records) of a stencil row, which bounds
+// it; a tile of a field is 35 KB (FP32, W = 0) for all of the tile's slots.
+// One field per workgroup, not all of them in turn: blocks run field by field
+// over groups of 64 neighbouring tiles, so that neighbours read a field's halo
+// while it is in their L2 (seven fields per block: 357 us for 10^6 rows at
+// 256^3 FP32, the same with 256, 384 and 512 threads; 221 us like this, against
+// 737 us for four lanes per row on planar fields, k_prhs_sorted).
+template <typename T> struct GatherFields {
+  const T *a, *b, *c;          // fields 0 .. na - 1 of a, na .. na + nb - 1 of b (N^3 apart), then c
+  int na, nb, n;               // n fields in all
+  const double* clip;          // c is taken as the stage density nStage(c, clip) (null: as it is)
+  __device__ __forceinline__ const T* field(int k, size_t R) const {
+    return k < na ? a + k * R : k < na + nb ? b + (k - na) * R : c;
+  }
+};
+template <int N, int W> struct GatherTile {
+  static constexpr int S = Bins<N>::TC;
+  static constexpr int RX = S + 3 + 2 * W;                       // nodes per side in x and y
+  static constexpr int QZ = S / 4 + 2, PZ = 4 * QZ;              // along z: aligned quads from 4 nodes before
+  static constexpr int NQ = RX * RX * QZ;
+  static constexpr int TSB = Bins<N>::TS * Bins<N>::TS * Bins<N>::TS, NTILE = Bins<N>::NB / TSB;
+  static constexpr int XT = NTILE / 8, GS = XT < 64 ? XT : 64;   // tiles per XCD and per group
+  static_assert(W <= 2 && RX <= N && PZ <= N && NTILE % 8 == 0 && XT % GS == 0, "gather tile");
+};
+// G: precision of the weights and sums.  rowmap null: out[k cap + slot]; else
+// out[rowmap[slot] n + k].
+template <typename T, typename G, int N, int W, int NT>
+__global__ void __launch_bounds__(NT)
+k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep0, const int* __restrict__ start0, int np, int cap,
+              const int* __restrict__ rowmap, G* __restrict__ out0, DropPhys P, size_t rs) {
+  using GT = GatherTile<N, W>;
+  constexpr int S = GT::S, RX = GT::RX, QZ = GT::QZ, PZ = GT::PZ, NQ = GT::NQ, IT = (NQ + NT - 1) / NT;
+  constexpr size_t R = (size_t)N * N * N;
+  __shared__ __attribute__((aligned(32))) T lds[4 * NQ];
+  const int* __restrict__ start = rsel1(start0, rs);
+  const int j = blockIdx.x / 8, r = j % (GT::GS * F.n);
+  const int tile = (blockIdx.x % 8) * GT::XT + j / (GT::GS * F.n) * GT::GS + r % GT::GS, k = r / GT::GS;
+  const int s0 = start[tile * GT::TSB], s1 = tile + 1 < GT::NTILE ? start[(tile + 1) * GT::TSB] : np;
+  if (s0 == s1) return;
+  const double4* __restrict__ dep = rsel1(dep0, rs);
+  G* __restrict__ out = rsel1(out0, rs);
+  int cx, cy, cz;
+  Bins<N>::tileCell(tile, cx, cy, cz);
+  const T* __restrict__ f = rsel1(F.field(k, R), rs);
+  const bool dens = F.clip && k == F.na + F.nb;
+  const double* __restrict__ clip = dens ? rsel1(F.clip, rs) : nullptr;
+  {
+    V4<T> q[IT];
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int e0 = (int)threadIdx.x + it * NT, e = (NQ % NT == 0 || e0 < NQ) ? e0 : 0;
+      const int z4 = e % QZ, row = e / QZ;
+      const uint32_t x = (uint32_t)(cx - 1 - W + row / RX) & (N - 1), y = (uint32_t)(cy - 1 - W + row % RX) & (N - 1),
+                     z = (uint32_t)(cz - 4 + 4 * z4) & (N - 1);
+      q[it] = ld32(reinterpret_cast<const V4<T>*>(f), ((x * N + y) * N + z) / 4);
+    }
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int e = (int)threadIdx.x + it * NT;
+      if (NQ % NT == 0 || e < NQ) {
+        if (dens) {
+          q[it].x = nStage<T>(q[it].x, clip); q[it].y = nStage<T>(q[it].y, clip);
+          q[it].z = nStage<T>(q[it].z, clip); q[it].w = nStage<T>(q[it].w, clip);
+        }
+        *reinterpret_cast<V4<T>*>(lds + 4 * e) = q[it];
+      }
+    }
+  }
+  __syncthreads();
+  for (int s = s0 + (int)threadIdx.x; s < s1; s += NT) {
+    const double4 d = dep[s];
+    const int i0 = originOf(d.x, P.inv_dx), j0 = originOf(d.y, P.inv_dx), k0 = originOf(d.z, P.inv_dx);
+    G xs, xc, ys, yc, zs, zc;
+    sincosStencil<G>(d.x, i0, P.dx, P.inv_dx, P.pi_2dx, xs, xc);
+    sincosStencil<G>(d.y, j0, P.dx, P.inv_dx, P.pi_2dx, ys, yc);
+    sincosStencil<G>(d.z, k0, P.dx, P.inv_dx, P.pi_2dx, zs, zc);
+    const G qr = (G)0.25, one = (G)1;
+    const G wx[4] = {qr * (one + xc), qr * (one + xs), qr * (one - xc), qr * (one - xs)};
+    const G wy[4] = {qr * (one + yc), qr * (one + ys), qr * (one - yc), qr * (one - ys)};
+    const G wz[4] = {qr * (one + zc), qr * (one + zs), qr * (one - zc), qr * (one - zs)};
+    const int lx = (i0 - cx + 1 + W) & (N - 1), ly = (j0 - cy + 1 + W) & (N - 1), lz = (k0 - cz + 4) & (N - 1);
+    G sum = (G)0;
+    if (lx <= S - 1 + 2 * W && ly <= S - 1 + 2 * W && lz + 3 < PZ) {
+      const T* o = lds + (lx * RX + ly) * PZ + lz;
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        // the plane's 16 values are read ahead of their sum
+        T v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = o[(a * RX + (e >> 2)) * PZ + (e & 3)];
+        G sa = (G)0;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+          sa += wy[b] * ((G)v[4 * b] * wz[0] + (G)v[4 * b + 1] * wz[1] + (G)v[4 * b + 2] * wz[2] + (G)v[4 * b + 3] * wz[3]);
+        sum += wx[a] * sa;
+      }
+    } else {
+      // moved out of the tile's window since the sort: from global memory
+#pragma unroll 1
+      for (int e = 0; e < 64; ++e) {
+        const int a = e >> 4, b = (e >> 2) & 3, c = e & 3;
+        const uint32_t o = ((uint32_t)wrapIdx<N>(i0 + a) * N + (uint32_t)wrapIdx<N>(j0 + b)) * N + (uint32_t)wrapIdx<N>(k0 + c);
+        T v = ld32(f, o);
+        if (dens) v = nStage<T>(v, clip);
+        const G wa = qr * (one + ((a & 2) ? -one : one) * ((a & 1) ? xs : xc));
+        const G wb = qr * (one + ((b & 2) ? -one : one) * ((b & 1) ? ys : yc));
+        const G wc = qr * (one + ((c & 2) ? -one : one) * ((c & 1) ? zs : zc));
+        sum += (G)v * (wa * wb * wc);
+      }
+    }
+    if (rowmap) out[(size_t)rowmap[s] * F.n + k] = sum;
+    else out[(size_t)k * cap + s] = sum;
+  }
+}
+
 // ------------------------------------------------------------ API kernels
 // interp_cosine (particles.py:435-511) of NC fields at rows of coord (Np, 7).
 template <typename T, int N>
@@ -876,6 +1019,11 @@ k_prhs(const double* __restrict__ coord, int np, const T* __restrict__ u, const 
 // lanes per row (lane c owns z node c of the stencil), so one load touches 16
 // rows that lie in neighbouring cells, and the deposit takes the bricks.
 // Positions, weights and sums stay FP64.
+// wrapped coordinate whose cell is below N (a position that rounds to L is 0)
+template <int N> __device__ __forceinline__ double wrapRow(double x, double L, double inv_dx) {
+  const double r = wrapL(x, L);
+  return r * inv_dx < (double)N ? r : 0.0;
+}
 template <int N>
 __global__ void __launch_bounds__(256)
 k_row_bin(const double* __restrict__ rows, int np, double L, double inv_dx, int* __restrict__ key,
@@ -884,20 +1032,21 @@ k_row_bin(const double* __restrict__ rows, int np, double L, double inv_dx, int*
   if (p >= np) return;
   int b[3];
 #pragma unroll
-  for (int c = 0; c < 3; ++c) b[c] = cellOf<N>(wrapL(rows[(size_t)p * 7 + c], L), inv_dx) / Bins<N>::BS;
+  for (int c = 0; c < 3; ++c) b[c] = cellOf<N>(wrapRow<N>(rows[(size_t)p * 7 + c], L, inv_dx), inv_dx) / Bins<N>::BS;
   const int k = Bins<N>::key(b[0], b[1], b[2]);
   key[p] = k;
   rank[p] = atomicAdd(&hist[k], 1);
 }
-static __global__ void __launch_bounds__(256)
-k_row_scatter(const double* __restrict__ rows, int np, double L, const double* __restrict__ w,
+template <int N>
+__global__ void __launch_bounds__(256)
+k_row_scatter(const double* __restrict__ rows, int np, double L, double inv_dx, const double* __restrict__ w,
               const int* __restrict__ key, const int* __restrict__ rank, const int* __restrict__ start,
               double4* __restrict__ dep, int* __restrict__ row) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= np) return;
   const double* r = rows + (size_t)p * 7;
   double4 d;
-  d.x = wrapL(r[0], L); d.y = wrapL(r[1], L); d.z = wrapL(r[2], L);
+  d.x = wrapRow<N>(r[0], L, inv_dx); d.y = wrapRow<N>(r[1], L, inv_dx); d.z = wrapRow<N>(r[2], L, inv_dx);
   d.w = w ? w[p] : 0.0;
   const int s = start[key[p]] + rank[p];
   dep[s] = d;
@@ -916,7 +1065,7 @@ template <int N> struct QuadStencil {
     const double x = c == 0 ? d.x : c == 1 ? d.y : d.z;
     const int o = c == 0 ? i0 : c == 1 ? j0 : k0;
     double sn, cs;
-    sincos((x - (double)o * P.dx) * P.pi_2dx, &sn, &cs);
+    sincosStencil<double>(x, o, P.dx, P.inv_dx, P.pi_2dx, sn, cs);
     const double xs = __shfl(sn, 0, 4), xc = __shfl(cs, 0, 4), ys = __shfl(sn, 1, 4), yc = __shfl(cs, 1, 4),
                  zs = __shfl(sn, 2, 4), zc = __shfl(cs, 2, 4);
     wx[0] = 0.25 * (1.0 + xc); wx[1] = 0.25 * (1.0 + xs); wx[2] = 0.25 * (1.0 - xc); wx[3] = 0.25 * (1.0 - xs);
@@ -993,6 +1142,29 @@ k_prhs_sorted(const double* __restrict__ coord, int np, const T* __restrict__ u,
     exterp[p] = W;
     dep[s].w = W;
   }
+}
+
+// The droplet side of pRHS on sorted rows whose interpolants k_tile_gather left
+// in I[k cap + slot].  Bound by the scattered rows (10^6: 110 us; moving them
+// through LDS with neighbouring lanes took the same).
+static __global__ void __launch_bounds__(256)
+k_prhs_finish(const double* __restrict__ coord, int np, int cap, const double* __restrict__ I0,
+              double4* __restrict__ dep, const int* __restrict__ row0, double* __restrict__ rhs,
+              double* __restrict__ interp, double* __restrict__ exterp, DropPhys P) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= np) return;
+  const size_t p = (size_t)row0[s];
+  const double* rw = coord + p * 7;
+  double I[7], vp[3], r[7], W;
+#pragma unroll
+  for (int k = 0; k < 7; ++k) I[k] = I0[(size_t)k * cap + s];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) vp[k] = rw[3 + k];
+  dropletRhs(P, vp, rw[6], I, r, W);
+#pragma unroll
+  for (int k = 0; k < 7; ++k) { rhs[p * 7 + k] = r[k]; interp[p * 7 + k] = I[k]; }
+  exterp[p] = W;
+  dep[s].w = W;
 }
 
 // interp_cosine (particles.py:435-511) of sorted rows, one component at a time.

@@ -103,6 +103,35 @@ def test_sorted_rows_match_general_path(gpu, N, prec, npart, monkeypatch):
         assert np.max(np.abs(a[k].astype(np.float64) - b[k])) <= tol * np.max(np.abs(b[k])), k
 
 
+@pytest.mark.parametrize("N,prec,npart", [(16, "f64", 300), (32, "f32", 1), (32, "f64", 4097), (64, "f32", 20011),
+                                          (128, "f32", 30011)])
+def test_tile_gather_matches_four_lane_gather(gpu, N, prec, npart, monkeypatch):
+    """LD_ROW_TILE_MIN moves the line between the two gathers of sorted rows (same weights and sums in another
+    order: FP64 tolerance as above); a cluster fills one tile with more rows than a block has threads."""
+    import torch
+    from lucky_droplets_amd.dns import ForcedDNS
+    monkeypatch.setenv("LD_ROW_SORT_MIN", "0")
+    cfg = Config(N=N, precision=prec, nu=0.02, n_particles=npart, gravity=True)
+    rows = _edge_rows(cfg, npart, 9)
+    k = npart // 3
+    rows[:k, :3] = np.random.default_rng(2).uniform(0, 5 * cfg.dx, (k, 3))
+    fields = np.random.default_rng(N).standard_normal((7, N, N, N))
+    got = {}
+    for line in (0, 1 << 40):
+        monkeypatch.setenv("LD_ROW_TILE_MIN", str(line))
+        d = ForcedDNS(cfg)
+        stb = _population(d, cfg, rows)
+        f = _t(fields, gpu, d.rdtype)
+        out = {"interp": stb.interp_cosine(stb.coord, f).clone()}
+        _, rhs, _ = stb.pRHS(0.0, stb.coord, f[:3], f[3:6], f[6], torch.empty_like(f[0]), None)
+        out.update(rhs=rhs, I=stb.interpmat, W=stb.exterpmat)
+        got[line] = {n: v.cpu().numpy() for n, v in out.items()}
+        d.close()
+    for n in got[0]:
+        a, b = got[0][n], got[1 << 40][n]
+        assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b)), n
+
+
 def test_more_rows_than_the_capacity(gpu):
     """The sorted path's scratch holds the context's capacity; more rows take the general path."""
     import torch
