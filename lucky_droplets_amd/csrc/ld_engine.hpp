@@ -45,10 +45,13 @@ template <> struct PrecTraits<double> { static constexpr int M = 8; using PT = d
 
 // z-pass tile height P for F fields: <= 256 threads and <= 64 KB LDS (one
 // field: <= 512 threads and <= 72 KB, measured at 256^3 FP32: 64 lines instead
-// of 32 took 5.82 -> 5.79 ms per step), >= 2.
+// of 32 took 5.82 -> 5.79 ms per step), >= 2.  One field on small grids: 64
+// threads up to 64^3 and 128 at 128^3, so that 32 to 512 blocks run instead of
+// 4 to 128, each with a short reduction (ten steps at 64^3 FP64 5.05 -> 4.85
+// ms, 4 at 128^3 FP32 4.14 -> 4.05 ms).
 template <typename T, int N, int F> constexpr int zTileP() {
   constexpr int N1 = Plan<N>::N1, Nf = N / 2 + 1;
-  constexpr int TMAX = F == 1 ? 512 : 256;
+  constexpr int TMAX = F > 1 ? 256 : N <= 64 ? 64 : N == 128 ? 128 : 512;
   constexpr long LMAX = F == 1 ? 73728 : 65536;
   int P = 2;
   for (;;) {
@@ -151,13 +154,13 @@ struct Engine final : EngineBase {
   int *flist = nullptr, *fcount = nullptr;
   unsigned long long* fx = nullptr;  // fixed-point scratch field of the fallback deposit (zero between steps)
   unsigned long long* wmaxp = nullptr;   // largest W of a droplet stage (fixed-point deposit bound)
-  bool sort_enabled = true;
   // y and z passes of a chain run slab by slab (x-planes) so the y<->z
   // intermediate of one slab stays in the Infinity Cache; 1 = whole field.
   int nslab = 1;
-  bool sorted_ok = false;            // bin starts (hist) describe the current slots
   static constexpr int NB = Bins<N>::NB;
   static constexpr int NBS = (NB + 4095) / 4096;
+  static constexpr int NBRICK = Brick<N>::NB * Brick<N>::NB * Brick<N>::NB;
+  static constexpr int FB_BLOCKS = 32;   // extra blocks of a stage's brick launch: fallback slots
   DropPhys dp;
   // kernel timing (ld_profile): event pairs around launches of one kernel class
   int prof_id = -1;
@@ -531,11 +534,12 @@ struct Engine final : EngineBase {
     LD_LAUNCHED();
     return LD_OK;
   }
-  int clip_sums(hipStream_t s, const T* x, double* clip) {
+  // counters: also clear the droplet stage's counters (before a step's first stage)
+  int clip_sums(hipStream_t s, const T* x, double* clip, bool counters = false) {
     hipLaunchKernelGGL((k_sum2<T>), dim3(NBLK_SUM, 1, B), dim3(256), 0, s, x, RF, partials, rs);
     LD_LAUNCHED();
     hipLaunchKernelGGL(k_clip_final, dim3(1, 1, B), dim3(256), 0, s, (const double*)partials, NBLK_SUM,
-                       1.0 / ((double)N * N * N), clip, rs);
+                       1.0 / ((double)N * N * N), clip, rs, counters && np > 0 ? fcount : (int*)nullptr, wmaxp);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -720,11 +724,14 @@ struct Engine final : EngineBase {
   // wn[0..4); kn_hat x-inverse in wn[0]; y-inverse.
   // (leaves kn_hat y-inverse-transformed in wn[0] when kz == nullptr; with
   // kz the z pass runs per slab too)
-  template <class OpKn> int density_rhs(hipStream_t s, const T* fcin, const OpKn* kz) {
+  // fold: fc is a droplet stage's deposit, whose fallback sums fx are added
+  template <class OpKn> int density_rhs(hipStream_t s, const T* fcin, const OpKn* kz, bool fold = false) {
     OpZFwd<T, N, P1, 1> of{fcin, wn + 3 * CF, RF, CF};
+    OpZFwdFc<T, N, P1> off{fcin, wn + 3 * CF, fx, fcount, wmaxp, dp.inv_vol};
     const int nx = N / nslab;
     for (int x0 = 0; x0 < N; x0 += nx) {
-      LD_TRY((zrun<P1, 0, 1>(s, of, -2, x0, nx, kc)));
+      if (fold) LD_TRY((zrun<P1, 0, 1>(s, off, -2, x0, nx, kc)));
+      else LD_TRY((zrun<P1, 0, 1>(s, of, -2, x0, nx, kc)));
       LD_TRY((pass<1, -1>(s, wn, wn, 4, (T)1, x0, nx, kc, sphere())));
     }
     LD_TRY(prof_mark(LD_K_XKN, s));
@@ -782,15 +789,12 @@ struct Engine final : EngineBase {
     const double wh = (s == 0 || s == 3) ? h / 6.0 : h / 3.0;
     const double anext = a_coef[s + 1] * h;
     LD_TRY(join(st2, st, evA));
-    if (!sorted_ok || np == 0) LD_TRY(fill<T>(st2, fc, RF, (T)0));
+    if (np == 0) LD_TRY(fill<T>(st2, fc, RF, (T)0));
     if (np > 0) {
-      LD_TRY(fill<int>(st2, fcount, 1, 0));
-      LD_TRY(fill<unsigned long long>(st2, wmaxp, 1, 0ull));
       PStage<T, PT> ps;
       ps.np = (int)np; ps.cap = (int)cap; ps.stage = s;
       ps.x0 = x0; ps.v0 = v0; ps.sx = sx; ps.sv = sv; ps.kx = kxp; ps.kv = kvp;
       ps.gu = gup; ps.gv = gup; ps.dep = dep; ps.flist = flist; ps.fcount = fcount;
-      ps.all_fallback = sorted_ok ? 0 : 1;
       ps.wmax = wmaxp;
       ps.ah = a_coef[s] * h; ps.wh = wh; ps.P = dp; ps.rs = rs;
       // 4 lanes per droplet; block count a multiple of 8 for the XCD mapping
@@ -805,18 +809,9 @@ struct Engine final : EngineBase {
       LD_LAUNCHED();
       LD_TRY(prof_mark(LD_K_DROPLETS, st2));
       LD_TRY(prof_mark(LD_K_DEPOSIT, st2));
-      if (sorted_ok) {
-        hipLaunchKernelGGL((k_brick_deposit<T, N>), dim3(Brick<N>::NB * Brick<N>::NB * Brick<N>::NB, 1, B),
-                           dim3(Brick<N>::NT), 0, st2, (const double4*)dep, (const int*)hist, (int)np,
-                           (const unsigned long long*)wmaxp, fc, dp, rs);
-        LD_LAUNCHED();
-      }
-      const unsigned fb = sorted_ok ? 64u : (unsigned)((np + 255) / 256);
-      hipLaunchKernelGGL((k_fallback_accum<T, N>), dim3(fb, 1, B), dim3(256), 0, st2, (const double4*)dep,
-                         (const int*)flist, (const int*)fcount, (const unsigned long long*)wmaxp, fx, dp, rs);
-      LD_LAUNCHED();
-      hipLaunchKernelGGL((k_fallback_fold<T, N>), dim3(fb, 1, B), dim3(256), 0, st2, (const double4*)dep,
-                         (const int*)flist, (const int*)fcount, (const unsigned long long*)wmaxp, fx, fc, dp, rs);
+      hipLaunchKernelGGL((k_brick_deposit<T, N>), dim3(NBRICK + FB_BLOCKS, 1, B), dim3(Brick<N>::NT), 0, st2,
+                         (const double4*)dep, (const int*)hist, (int)np, (const unsigned long long*)wmaxp, fc, dp, rs,
+                         (const int*)flist, (const int*)fcount, fx);
       LD_LAUNCHED();
       LD_TRY(prof_mark(LD_K_DEPOSIT, st2));
     }
@@ -825,9 +820,10 @@ struct Engine final : EngineBase {
     ok.n0 = n_state; ok.nacc = nacc; ok.nnext = (s < 3) ? n_stage : nullptr;
     ok.wacc = (T)wh; ok.anext = (T)anext; ok.acc_init = (s == 0);
     ok.sum_target = (s < 3) ? 0 : 1; ok.partials = partials2;
-    LD_TRY(density_rhs(st2, fc, &ok));
+    LD_TRY(density_rhs(st2, fc, &ok, np > 0));
     hipLaunchKernelGGL(k_clip_final, dim3(1, 1, B), dim3(256), 0, st2, (const double*)partials2, NBLK_Z1,
-                       1.0 / ((double)N * N * N), (s < 3) ? clip_stage : clip_end, rs);
+                       1.0 / ((double)N * N * N), (s < 3) ? clip_stage : clip_end, rs,
+                       np > 0 ? fcount : (int*)nullptr, wmaxp);
     LD_LAUNCHED();
     LD_HIP(hipEventRecord(evB, st2));
     if (serial) LD_TRY(join(st, st2, evB));
@@ -836,7 +832,7 @@ struct Engine final : EngineBase {
 
   // Stage-1 clip_zero(n) sums (forced-dns-sm.py:341) on the density stream.
   int begin_rk4() {
-    LD_TRY(clip_sums(st2, n_state, clip_stage));
+    LD_TRY(clip_sums(st2, n_state, clip_stage, true));
     LD_HIP(hipEventRecord(evB, st2));
     if (serial) LD_TRY(join(st, st2, evB));
     return LD_OK;
@@ -875,7 +871,6 @@ struct Engine final : EngineBase {
   // ------------------------------------------------------------ state
   // Droplet rows of every realization: coord holds B blocks of n_ rows.
   int set_rows(const double* coord, int64_t n_) {
-    sorted_ok = false;
     if (n_ > cap) { set_error("%lld droplets exceed the context capacity %lld", (long long)n_, (long long)cap); return LD_ERR_CAPACITY; }
     np = n_;
     if (np > 0) {
@@ -952,8 +947,7 @@ struct Engine final : EngineBase {
   // Counting sort of the droplet slots by spatial bin of the base position
   // (on the density stream, which owns the droplet state during a step).
   int sort_droplets(hipStream_t s) {
-    sorted_ok = false;
-    if (np < 1 || !sort_enabled) return LD_OK;
+    if (np < 1) return LD_OK;
     const unsigned pb = (unsigned)((np + 255) / 256);
     LD_TRY(fill<int>(s, hist, NB, 0));
     hipLaunchKernelGGL((k_bin_count<N>), dim3(pb, 1, B), dim3(256), 0, s, (const double*)x0, (int)np, (int)cap, p.L,
@@ -971,6 +965,7 @@ struct Engine final : EngineBase {
   int scan_bins(hipStream_t s) {
     hipLaunchKernelGGL(k_scan_local, dim3(NBS, 1, B), dim3(1024), 0, s, hist, NB, bsum, rs);
     LD_LAUNCHED();
+    if (NBS == 1) return LD_OK;          // one block scanned them all
     hipLaunchKernelGGL(k_scan_bsums, dim3(1, 1, B), dim3(1024), 0, s, bsum, NBS, rs);
     LD_LAUNCHED();
     hipLaunchKernelGGL(k_scan_add, dim3((NB + 255) / 256, 1, B), dim3(256), 0, s, hist, NB, (const int*)bsum, rs);
@@ -982,10 +977,9 @@ struct Engine final : EngineBase {
     std::swap(x0, x0b);
     std::swap(v0, v0b);
     std::swap(rid, rid2);
-    sorted_ok = true;
     parity ^= 1;
   }
-  bool sorts() const { return np >= 1 && sort_enabled; }
+  bool sorts() const { return np >= 1; }
 
   // ------------------------------------------------------------ HIP graphs
   // With graphs on, one step (sort, four stages, epilogue on both streams) is
@@ -1586,9 +1580,9 @@ struct Engine final : EngineBase {
   static unsigned quad_blocks(int64_t n_) { return (unsigned)(((4 * n_ + 255) / 256 + 7) / 8 * 8); }
   // FP64 brick deposit of the sorted rows' weights; writes every node of c
   int deposit_rows(int64_t n_, T* c) {
-    hipLaunchKernelGGL((k_brick_deposit<T, N, false>), dim3(Brick<N>::NB * Brick<N>::NB * Brick<N>::NB),
-                       dim3(Brick<N>::NT), 0, st, (const double4*)dep, (const int*)hist, (int)n_,
-                       (const unsigned long long*)nullptr, c, dp, (size_t)0);
+    hipLaunchKernelGGL((k_brick_deposit<T, N, false>), dim3(NBRICK), dim3(Brick<N>::NT), 0, st, (const double4*)dep,
+                       (const int*)hist, (int)n_, (const unsigned long long*)nullptr, c, dp, (size_t)0,
+                       (const int*)nullptr, (const int*)nullptr, (unsigned long long*)nullptr);
     LD_LAUNCHED();
     return LD_OK;
   }

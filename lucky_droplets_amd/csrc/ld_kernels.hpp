@@ -425,6 +425,64 @@ struct OpZFwd {
   }
 };
 
+// Scale of the fallback deposit's 64-bit fixed point: 2^e with slots x Wmax /
+// dx^3 / 8 x 2^e < 2^62, from the launch's largest W (bits of a double).
+struct FallbackScale {
+  double scale, unit;
+  bool finite;
+  __device__ __forceinline__ FallbackScale(int nf, unsigned long long wmax_bits, double inv_vol) {
+    const double bound = (double)nf * __longlong_as_double((long long)wmax_bits) * inv_vol * 0.125;
+    finite = isfinite(bound);
+    const int e = (bound > 0.0 && finite) ? 61 - ilogb(bound) : 0;
+    scale = ldexp(1.0, e);
+    unit = ldexp(1.0, -e);
+  }
+};
+
+// r2c along z of the deposit field fc, with the fallback deposit's fixed-point
+// sums fx added where there are any (*fcount > 0) and cleared.  A NaN or
+// negative growth somewhere (the bound of the scale is not finite) makes the
+// field NaN.
+template <typename T, int N, int P>
+struct OpZFwdFc {
+  const T* in; C<T>* out; unsigned long long* fx; const int* fcount; const unsigned long long* wmax; double inv_vol;
+  __device__ OpZFwdFc shifted(size_t rs) const {
+    OpZFwdFc o = *this;
+    o.in = rsel1(in, rs); o.out = rsel1(out, rs); o.fx = rsel1(fx, rs); o.fcount = rsel1(fcount, rs);
+    o.wmax = rsel1(wmax, rs);
+    return o;
+  }
+  __device__ const C<T>* specIn(int) const { return nullptr; }
+  __device__ C<T>* specOut(int) const { return out; }
+  __device__ void physical(const ZTile<T, N, P>& t, int line0) const {
+    using Q = Quads<ZThreads<N, P, 0, 1>::v, P * N / 4>;
+    const int nf = *fcount;
+#pragma unroll
+    for (int it = 0; it < Q::IT; ++it) {
+      if (Q::ok(it)) {
+        const int e4 = 4 * Q::e(it), p = e4 / N, j = e4 % N;
+        t.re4(0, p, j) = *reinterpret_cast<const V4<T>*>(in + (size_t)(line0 + p) * N + j);
+      }
+    }
+    if (nf == 0) return;
+    const FallbackScale sc(nf, *wmax, inv_vol);
+#pragma unroll 1
+    for (int it = 0; it < Q::IT; ++it) {
+      if (!Q::ok(it)) break;
+      const int e4 = 4 * Q::e(it), p = e4 / N, j = e4 % N;
+      unsigned long long* f = fx + (size_t)(line0 + p) * N + j;
+      V4<T>& v = t.re4(0, p, j);
+      T* x[4] = {&v.x, &v.y, &v.z, &v.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (!sc.finite) { *x[k] = (T)NAN; continue; }
+        const unsigned long long q = f[k];
+        if (q) { *x[k] = *x[k] + (T)((double)q * sc.unit); f[k] = 0ull; }
+      }
+    }
+  }
+};
+
 // Droplet gather records.  Per node two 16-byte records, {u_x, u_y, u_z, 0}
 // and {v_x, v_y, v_z, n_stage}, laid out in z-quads: the four u records of
 // nodes z = 4q .. 4q+3 of an (x, y) line (64 bytes), then their four v records,
@@ -1123,9 +1181,12 @@ k_sum2(const T* __restrict__ x0, size_t n, double* __restrict__ partials0, size_
   if (threadIdx.x == 0) partials[2 * blockIdx.x + 1] = c;
 }
 
-// Final clip_zero means: clip = {sum/N^3, sum+/N^3, 1}.
+// Final clip_zero means: clip = {sum/N^3, sum+/N^3, 1}.  It is the last kernel
+// of a stage's density chain and also clears the next stage's counters
+// (fcount, wmax; may be null).
 static __global__ void __launch_bounds__(256)
-k_clip_final(const double* __restrict__ partials0, int nblk, double inv_n3, double* __restrict__ clip0, size_t rs) {
+k_clip_final(const double* __restrict__ partials0, int nblk, double inv_n3, double* __restrict__ clip0, size_t rs,
+             int* fcount0, unsigned long long* wmax0) {
   const double* __restrict__ partials = rsel1(partials0, rs);
   double* __restrict__ clip = rsel1(clip0, rs);
   constexpr int NT = 256;
@@ -1135,7 +1196,10 @@ k_clip_final(const double* __restrict__ partials0, int nblk, double inv_n3, doub
   const double a = blockSum<NT>(s0, sh);
   __syncthreads();
   const double b = blockSum<NT>(s1, sh);
-  if (threadIdx.x == 0) { clip[0] = a * inv_n3; clip[1] = b * inv_n3; clip[2] = 1.0; }
+  if (threadIdx.x == 0) {
+    clip[0] = a * inv_n3; clip[1] = b * inv_n3; clip[2] = 1.0;
+    if (fcount0) { *rsel1(fcount0, rs) = 0; *rsel1(wmax0, rs) = 0ull; }
+  }
 }
 
 // out = clip_zero(x) with x clipped in place when clip_x (forced-dns-sm.py:282-285).

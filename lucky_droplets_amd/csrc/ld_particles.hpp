@@ -304,8 +304,7 @@ template <typename T, typename PT> struct PStage {
   const V4<T>* gu; const V4<T>* gv;   // gather records {u, 0} (recU) and {v, n_stage} (recV); one array
   double4* dep;                // out: wrapped stage position and W per slot (brick deposit input)
   int* flist; int* fcount;     // out: slots whose stage bin moved > 1 bin since the sort
-  int all_fallback;            // 1: slots are not bin-sorted, every slot takes the fallback deposit
-  unsigned long long* wmax;    // out: largest W > 0 of the launch (bits of a positive double); zeroed before
+  unsigned long long* wmax;    // out: largest W > 0 of the launch (bits of a positive double); zero before
   double ah, wh;               // a_s * h, w_s * h
   DropPhys P;
   size_t rs;                   // realization stride in bytes (batched launches)
@@ -370,7 +369,6 @@ k_particles_stage(PStage<T, PT> A0) {
   // +-1-bin window around their sorted bin go to the fallback list.
   bool far = false;
   if (live && c == 0) {
-    far = A.all_fallback != 0;
     const double xb[3] = {xw, yw, zw};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -529,6 +527,48 @@ k_particles_stage(PStage<T, PT> A0) {
   }
 }
 
+// ------------------------------------------------------------ fallback deposit
+// Fallback deposit of the slots that moved more than one bin since the sort, by
+// extra blocks of the brick launch (one launch instead of three: on small grids
+// the density chain is a sequence of launches of a few microseconds each: with
+// the counters' two fills gone as well, ten steps at 64^3 FP64 went from 4.85
+// to 4.40 ms; at 256^3 and above the step is unchanged).
+// Deterministic like the bricks: each slot's 64 node values are added as 64-bit
+// fixed-point integers to the scratch field fx (zero between stages; integer
+// sums do not depend on the order of the additions), with the scale 2^e of the
+// largest value any node can reach (slots x Wmax / dx^3 / 8); the z pass that
+// reads the deposit adds fx to it and clears it (OpZFwdFc).
+template <typename T, int N>
+__device__ __forceinline__ void fallbackAccum(const double4* __restrict__ dep, const int* __restrict__ flist, int nf,
+                                              unsigned long long wmax_bits, unsigned long long* fx, const DropPhys& P,
+                                              int first, int stride) {
+  const FallbackScale sc(nf, wmax_bits, P.inv_vol);
+  if (!sc.finite) return;
+  using GT = std::conditional_t<sizeof(T) == 4, float, double>;
+  for (int f = first; f < nf; f += stride) {
+    const double4 d = dep[flist[f]];
+    const double w = -d.w;                       // fallback slots carry -W
+    if (!(w > 0.0)) continue;
+    GT wx[4], wy[4], wz[4];
+    const int i0 = cosW4F<GT>(d.x, P.dx, P.inv_dx, P.pi_2dx, wx), j0 = cosW4F<GT>(d.y, P.dx, P.inv_dx, P.pi_2dx, wy),
+              k0 = cosW4F<GT>(d.z, P.dx, P.inv_dx, P.pi_2dx, wz);
+    const double W = w * P.inv_vol * sc.scale;
+#pragma unroll 1
+    for (int a = 0; a < 4; ++a) {
+      const double wa = W * (double)wx[a];
+      const size_t plane = (size_t)wrapIdx<N>(i0 + a) * N;
+#pragma unroll 1
+      for (int b = 0; b < 4; ++b) {
+        const double wab = wa * (double)wy[b];
+        const size_t row = (plane + wrapIdx<N>(j0 + b)) * N;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          atomicAdd(&fx[row + wrapIdx<N>(k0 + c)], (unsigned long long)llrint(wab * (double)wz[c]));
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------ brick deposit
 // Deposit of W with the cosine kernel / dx^3 (particles.py:23-35, 529-575),
 // organised by output: one workgroup per brick of S^3 grid nodes accumulates
@@ -574,11 +614,22 @@ template <int N> struct Brick {
 template <typename T, int N, bool FIX = true>
 __global__ void __launch_bounds__(Brick<N>::NT)
 k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0, int np,
-                const unsigned long long* __restrict__ wmax0, T* __restrict__ fc0, DropPhys P, size_t rs) {
+                const unsigned long long* __restrict__ wmax0, T* __restrict__ fc0, DropPhys P, size_t rs,
+                const int* __restrict__ flist0, const int* __restrict__ fcount0, unsigned long long* fx0) {
   const double4* __restrict__ dep = rsel1(dep0, rs);
   const int* __restrict__ start = rsel1(start0, rs);
   const unsigned long long* __restrict__ wmax = rsel1(wmax0, rs);
   T* __restrict__ fc = rsel1(fc0, rs);
+  constexpr int NBRICK = Brick<N>::NB * Brick<N>::NB * Brick<N>::NB;
+  if constexpr (FIX) {
+    if (blockIdx.x >= NBRICK) {          // the extra blocks: fallback slots
+      const int nf = *rsel1(fcount0, rs), b = (int)blockIdx.x - NBRICK;
+      if (nf)
+        fallbackAccum<T, N>(dep, rsel1(flist0, rs), nf, *wmax, rsel1(fx0, rs), P, b * Brick<N>::NT + (int)threadIdx.x,
+                            ((int)gridDim.x - NBRICK) * Brick<N>::NT);
+      return;
+    }
+  }
   using Bk = Brick<N>;
   constexpr int S = Bk::S, NBr = Bk::NB, NBX = Bk::NBX, NR = Bk::NR, NT = Bk::NT, NZS = Bk::NZS, CH = Bk::CH;
   constexpr int TS = Bins<N>::TS;
@@ -590,7 +641,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   __shared__ int cnt;
   const int tid = threadIdx.x, lane = tid & 63;
   // XCD-aware: each of the 8 XCDs takes a contiguous run of bricks
-  const int nb = gridDim.x, per = nb / 8;
+  constexpr int per = NBRICK / 8;
   const int br = (blockIdx.x % 8) * per + blockIdx.x / 8;
   const int c0x = (br / (NBr * NBr)) * S, c0y = ((br / NBr) % NBr) * S, c0z = (br % NBr) * S;
   for (int i = tid; i < S * S * S; i += NT) tile[i] = 0;
@@ -735,97 +786,6 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   for (int i = tid; i < S * S * S; i += NT) {
     const int nx = i / (S * S), ny = (i / S) % S, nz = i % S;
     fc[((size_t)(c0x + nx) * N + (c0y + ny)) * N + (c0z + nz)] = finite ? (T)((double)tile[i] * unit) : (T)NAN;
-  }
-}
-
-// Fallback deposit of the slots that moved more than one bin since the sort
-// (or of every slot when the slots are not sorted); runs after
-// k_brick_deposit.  Deterministic like the bricks: k_fallback_accum adds each
-// slot's 64 node values as 64-bit fixed-point integers into the scratch field
-// fx (zero between steps; integer sums do not depend on the order of the
-// additions), with the scale 2^e of the largest value any node can reach
-// (slots x Wmax / dx^3 / 8); k_fallback_fold then moves each touched node's
-// sum into fc and clears it (the first slot to exchange a node takes its whole
-// sum; the others find zero).
-struct FallbackScale {
-  double scale, unit;
-  bool finite;
-  __device__ FallbackScale(int nf, unsigned long long wmax_bits, double inv_vol) {
-    const double bound = (double)nf * __longlong_as_double((long long)wmax_bits) * inv_vol * 0.125;
-    finite = isfinite(bound);
-    const int e = (bound > 0.0 && finite) ? 61 - ilogb(bound) : 0;
-    scale = ldexp(1.0, e);
-    unit = ldexp(1.0, -e);
-  }
-};
-
-template <typename T, int N>
-__global__ void __launch_bounds__(256)
-k_fallback_accum(const double4* __restrict__ dep0, const int* __restrict__ flist0, const int* __restrict__ fcount0,
-                 const unsigned long long* __restrict__ wmax0, unsigned long long* fx0, DropPhys P, size_t rs) {
-  const double4* __restrict__ dep = rsel1(dep0, rs);
-  const int* __restrict__ flist = rsel1(flist0, rs);
-  unsigned long long* fx = rsel1(fx0, rs);
-  const int nf = *rsel1(fcount0, rs);
-  if (nf == 0) return;
-  const FallbackScale sc(nf, *rsel1(wmax0, rs), P.inv_vol);
-  if (!sc.finite) return;
-  using GT = std::conditional_t<sizeof(T) == 4, float, double>;
-  for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < nf; f += gridDim.x * blockDim.x) {
-    const double4 d = dep[flist[f]];
-    const double w = -d.w;                       // fallback slots carry -W
-    if (!(w > 0.0)) continue;
-    GT wx[4], wy[4], wz[4];
-    const int i0 = cosW4F<GT>(d.x, P.dx, P.inv_dx, P.pi_2dx, wx), j0 = cosW4F<GT>(d.y, P.dx, P.inv_dx, P.pi_2dx, wy),
-              k0 = cosW4F<GT>(d.z, P.dx, P.inv_dx, P.pi_2dx, wz);
-    const double W = w * P.inv_vol * sc.scale;
-#pragma unroll 1
-    for (int a = 0; a < 4; ++a) {
-      const double wa = W * (double)wx[a];
-      const size_t plane = (size_t)wrapIdx<N>(i0 + a) * N;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const double wab = wa * (double)wy[b];
-        const size_t row = (plane + wrapIdx<N>(j0 + b)) * N;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          atomicAdd(&fx[row + wrapIdx<N>(k0 + c)], (unsigned long long)llrint(wab * (double)wz[c]));
-      }
-    }
-  }
-}
-
-template <typename T, int N>
-__global__ void __launch_bounds__(256)
-k_fallback_fold(const double4* __restrict__ dep0, const int* __restrict__ flist0, const int* __restrict__ fcount0,
-                const unsigned long long* __restrict__ wmax0, unsigned long long* fx0, T* fc0, DropPhys P, size_t rs) {
-  const double4* __restrict__ dep = rsel1(dep0, rs);
-  const int* __restrict__ flist = rsel1(flist0, rs);
-  unsigned long long* fx = rsel1(fx0, rs);
-  T* fc = rsel1(fc0, rs);
-  const int nf = *rsel1(fcount0, rs);
-  if (nf == 0) return;
-  const FallbackScale sc(nf, *rsel1(wmax0, rs), P.inv_vol);
-  for (int f = blockIdx.x * blockDim.x + threadIdx.x; f < nf; f += gridDim.x * blockDim.x) {
-    const double4 d = dep[flist[f]];
-    const int i0 = originOf(d.x, P.inv_dx), j0 = originOf(d.y, P.inv_dx), k0 = originOf(d.z, P.inv_dx);
-    // a NaN or negative growth somewhere: NaN at every node the slot reaches
-    const bool poison = !sc.finite;
-#pragma unroll 1
-    for (int a = 0; a < 4; ++a) {
-      const size_t plane = (size_t)wrapIdx<N>(i0 + a) * N;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const size_t row = (plane + wrapIdx<N>(j0 + b)) * N;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const size_t o = row + wrapIdx<N>(k0 + c);
-          if (poison) { fc[o] = (T)NAN; continue; }
-          const unsigned long long v = atomicExch(&fx[o], 0ull);
-          if (v) fc[o] = fc[o] + (T)((double)v * sc.unit);
-        }
-      }
-    }
   }
 }
 
