@@ -75,8 +75,6 @@ struct Engine final : EngineBase {
   static constexpr int NBLK_X = N * Nf / M;         // blocks of an x pass
   static constexpr int M3 = XM3<T, N, M>::v;         // lines per block of a field-parallel x pass
   static constexpr int NBLK_X3 = N * Nf / M3;
-  static constexpr int M4 = XM4<T, N, M>::v;         // lines per block of the four-field x pass
-  static constexpr int NBLK_X4 = N * Nf / M4;
   // the autotuner's alternatives: half the z-tile height (>= 2) and half the
   // x-pass lines per block (>= 2); a block's lines do not change any line's
   // arithmetic, so every choice gives the same bits
@@ -86,7 +84,7 @@ struct Engine final : EngineBase {
     return F * (P / 2) * N1 <= 512 && (long)F * (P / 2) * 2 * Nf * (long)sizeof(C<T>) <= 65536 && P <= N * N;
   }
   static constexpr int P6D = zfits(2 * P6, 6) ? 2 * P6 : P6, P3D = zfits(2 * P3, 3) ? 2 * P3 : P3;
-  static constexpr int M3H = M3 / 2 >= 2 ? M3 / 2 : M3, M4H = M4 / 2 >= 2 ? M4 / 2 : M4;
+  static constexpr int M3H = M3 / 2 >= 2 ? M3 / 2 : M3;
   // launch-geometry choices: 0 = default, 1 = the alternative above (2 = the
   // doubled z tile, z passes only), for the
   // u x omega z pass, the v z pass, the u/omega x pass, the RHS x pass and the
@@ -242,7 +240,7 @@ struct Engine final : EngineBase {
     LD_TRY(fill<C<T>>(st, uk, 3 * CF, C<T>{}));
     LD_TRY(fill<C<T>>(st, acc, 3 * CF, C<T>{}));
     LD_TRY(fill<T>(st, n_state, RF, (T)0));
-    const bool alt[5] = {P6H != P6, P3H != P3, M3H != M3, M3H != M3, M4H != M4};
+    const bool alt[5] = {P6H != P6, P3H != P3, true, M3H != M3, true};
     const bool dbl[5] = {P6D != P6, P3D != P3, false, false, false};
     RhsArgs<T> ra;
     ra.nl = w6; ra.us = us; ra.ubase = uk; ra.acc = acc; ra.usnext = us; ra.ku = nullptr;
@@ -312,7 +310,7 @@ struct Engine final : EngineBase {
     return rc;
   }
   int tuning_all(int32_t* choice, double* us_out) override {
-    const int32_t sizes[5][3] = {{P6, P6H, P6D}, {P3, P3H, P3D}, {M3, M3H, M3}, {M3, M3H, M3}, {M4, M4H, M4}};
+    const int32_t sizes[5][3] = {{P6, P6H, P6D}, {P3, P3H, P3D}, {M, MH, M}, {M3, M3H, M3}, {M, MH, M}};
     if (choice) {
       choice[0] = my;
       for (int k = 0; k < 5; ++k) choice[1 + k] = sizes[k][vsel[k]];
@@ -644,10 +642,10 @@ struct Engine final : EngineBase {
   int nonlinear_x(hipStream_t s, const C<T>* usp, int kcu = N / 2) {
     LD_TRY(prof_mark(LD_K_XUW, s));
     if (vsel[2])
-      hipLaunchKernelGGL((k_x_uw3<T, N, M3H>), dim3(N * Nf / M3H, 1, B), dim3(3 * M3H * N1), 0, s, usp, w6, CF,
+      hipLaunchKernelGGL((k_x_uw<T, N, MH>), dim3(6 * (N * Nf / MH), 1, B), dim3(MH * N1), 0, s, usp, w6, CF,
                          (const C<T>*)tw, inv(), rs, kcu);
     else
-      hipLaunchKernelGGL((k_x_uw3<T, N, M3>), dim3(NBLK_X3, 1, B), dim3(3 * M3 * N1), 0, s, usp, w6, CF,
+      hipLaunchKernelGGL((k_x_uw<T, N, M>), dim3(6 * NBLK_X, 1, B), dim3(M * N1), 0, s, usp, w6, CF,
                          (const C<T>*)tw, inv(), rs, kcu);
     LD_LAUNCHED();
     LD_TRY(prof_mark(LD_K_XUW, s));
@@ -701,13 +699,33 @@ struct Engine final : EngineBase {
     }
     return LD_OK;
   }
+  // forward y pass of the density source, in the launch shape of the y passes
+  int ykn(hipStream_t s, int x0, int nx) {
+    const int lw = (kc < N / 2 ? kc : N / 2) + 1, nl = nx * lw;
+    auto launch = [&](auto mc, auto qc) {
+      constexpr int m = decltype(mc)::value, Q = decltype(qc)::value;
+      hipLaunchKernelGGL((k_y_kn<T, N, m, Q>), dim3((nl + m - 1) / m, 2, B), dim3(m * Plan<N, Q>::N1), 0, s, wn, CF,
+                         (const C<T>*)tw, x0 * lw, rs, lw, (x0 + nx) * lw, sphere());
+    };
+    auto lines = [&](auto qc) {
+      if (my == MH) launch(std::integral_constant<int, MH>{}, qc);
+      else if (my == M2) launch(std::integral_constant<int, M2>{}, qc);
+      else launch(std::integral_constant<int, M>{}, qc);
+    };
+    LD_TRY(prof_mark(LD_K_YPASS, s));
+    if (ysplit) lines(std::integral_constant<int, NQ>{});
+    else lines(std::integral_constant<int, 0>{});
+    LD_TRY(prof_mark(LD_K_YPASS, s));
+    LD_LAUNCHED();
+    return LD_OK;
+  }
   int xkn(hipStream_t s) {
     if (vsel[4])
-      hipLaunchKernelGGL((k_x_kn4<T, N, M4H>), dim3(N * Nf / M4H, 1, B), dim3(4 * M4H * N1), 0, s, wn, CF,
-                         (const C<T>*)tw, inv(), rs, kc);
-    else
-      hipLaunchKernelGGL((k_x_kn4<T, N, M4>), dim3(NBLK_X4, 1, B), dim3(4 * M4 * N1), 0, s, wn, CF, (const C<T>*)tw,
+      hipLaunchKernelGGL((k_x_kn<T, N, MH>), dim3(N * Nf / MH, 1, B), dim3(MH * N1), 0, s, wn, CF, (const C<T>*)tw,
                          inv(), rs, kc);
+    else
+      hipLaunchKernelGGL((k_x_kn<T, N, M>), dim3(NBLK_X, 1, B), dim3(M * N1), 0, s, wn, CF, (const C<T>*)tw, inv(),
+                         rs, kc);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -721,7 +739,7 @@ struct Engine final : EngineBase {
     return LD_OK;
   }
   // Density chain on stream s: fc -> z-forward into wn[3]; y-forward of
-  // wn[0..4); kn_hat x-inverse in wn[0]; y-inverse.
+  // wn[0..4) to wn[0..2) (k_y_kn); kn_hat x-inverse in wn[0]; y-inverse.
   // (leaves kn_hat y-inverse-transformed in wn[0] when kz == nullptr; with
   // kz the z pass runs per slab too)
   // fold: fc is a droplet stage's deposit, whose fallback sums fx are added
@@ -732,7 +750,7 @@ struct Engine final : EngineBase {
     for (int x0 = 0; x0 < N; x0 += nx) {
       if (fold) LD_TRY((zrun<P1, 0, 1>(s, off, -2, x0, nx, kc)));
       else LD_TRY((zrun<P1, 0, 1>(s, of, -2, x0, nx, kc)));
-      LD_TRY((pass<1, -1>(s, wn, wn, 4, (T)1, x0, nx, kc, sphere())));
+      LD_TRY(ykn(s, x0, nx));
     }
     LD_TRY(prof_mark(LD_K_XKN, s));
     LD_TRY(xkn(s));

@@ -178,6 +178,65 @@ k_pass(const C<T>* in, C<T>* out, size_t fstride, const C<T>* __restrict__ tw, T
   }
 }
 
+// Forward y pass of the density source, in place in the four z-transformed
+// fields w = {nv_x, nv_y, nv_z, fc} (lines and masks as in k_pass, forward):
+// the source -i k.(nv) - fc takes its ky and kz parts here, where ky and kz are
+// the line's own indices, so two fields leave the pass instead of four,
+//   w[0] = Y(nv_x),  w[1] = Y(-i kz nv_z - fc) - i ky Y(nv_y),
+// with three transforms instead of four.  blockIdx.y = 0 forms w[1] (the
+// longer blocks first), blockIdx.y = 1 transforms nv_x.
+template <typename T, int N, int M, int Q = 0>
+__global__ void __launch_bounds__((M * Plan<N, Q>::N1))
+k_y_kn(C<T>* w0, size_t fs, const C<T>* __restrict__ tw, int qoff, size_t rs, int lw, int qend, int r2) {
+  constexpr int N1 = Plan<N, Q>::N1, N2 = Plan<N, Q>::N2, js = JS<N, 1>::v;
+  __shared__ C<T> lds[M * (N + 1)];
+  const int m = threadIdx.x % M, n1 = threadIdx.x / M;
+  const int nbx = gridDim.x;
+  const int bx = (nbx % 8 == 0) ? (blockIdx.x % 8) * (nbx / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int qc = qoff + bx * M + m, kzi = qc % lw;
+  const int q = lw != N / 2 + 1 ? (qc / lw) * (N / 2 + 1) + kzi : qc;
+  const bool live = qc < qend;
+  C<T>* w = rsel1(w0, rs);
+  const uint32_t lb = (uint32_t)lineBase<N, 1>(q);
+  C<T>* L = lds + m * (N + 1);
+  C<T> a[N2];
+  auto load = [&](int f, int n2) {
+    return live ? ld32((const C<T>*)(w + f * fs), lb + (uint32_t)(posIn<N, Q>(n1, n2) * js)) : mkc<T>((T)0, (T)0);
+  };
+  auto keep = [&](int iy) {
+    const int ky = kwave(iy, N);
+    return live && (r2 < 0 || ky * ky + kzi * kzi <= r2);
+  };
+  if (blockIdx.y) {
+#pragma unroll
+    for (int n2 = 0; n2 < N2; ++n2) a[n2] = load(0, n2);
+    lineFwd<T, N, Q>(a, L, n1, true, tw);
+#pragma unroll
+    for (int r = 0; r < N2; ++r) {
+      const int iy = posOut<N, Q>(n1, r);
+      if (keep(iy)) st32(w, lb + (uint32_t)(iy * js), a[r]);
+    }
+    return;
+  }
+  const T kz = (T)kzi;
+  C<T> b[N2];
+#pragma unroll
+  for (int n2 = 0; n2 < N2; ++n2) {
+    const C<T> z = load(2, n2), c = load(3, n2);
+    a[n2] = mkc<T>(kz * z.y - c.x, -(kz * z.x) - c.y);
+  }
+#pragma unroll
+  for (int n2 = 0; n2 < N2; ++n2) b[n2] = load(1, n2);
+  lineFwd<T, N, Q>(a, L, n1, true, tw);
+  lineFwd<T, N, Q>(b, L, n1, true, tw);
+#pragma unroll
+  for (int r = 0; r < N2; ++r) {
+    const int iy = posOut<N, Q>(n1, r);
+    const T ky = (T)kwave(iy, N);
+    if (keep(iy)) st32(w + fs, lb + (uint32_t)(iy * js), mkc<T>(a[r].x + ky * b[r].y, a[r].y - ky * b[r].x));
+  }
+}
+
 // ============================================================= z-pass machinery
 // A block owns P consecutive (x,y) lines of several fields.  Real lines are
 // paired two-for-one into complex lines: lines (f, 2c) and (f, 2c+1) share one
@@ -730,77 +789,77 @@ template <typename T, int N, int M0> struct XM3 {
 };
 
 // Velocity and vorticity (forced-dns-sm.py:291-297): x-inverse of u_hat and of
-// i k x u_hat, 6 output fields (u_x, u_y, u_z, w_x, w_y, w_z).  Group f
-// inverse-transforms u_f and w_f.
+// i k x u_hat, 6 output fields (u_x, u_y, u_z, w_x, w_y, w_z), one field of M
+// lines per block: a block holds one field's lines, so several are in flight on
+// a CU in different phases of load, transform and store.  The six blocks of a
+// line group run one after the other on one XCD, where the rows of u_hat that
+// they share are in its L2.
 template <typename T, int N, int M>
-__global__ void __launch_bounds__(3 * M * Plan<N>::N1)
-k_x_uw3(const C<T>* __restrict__ uk0, C<T>* __restrict__ out0, size_t fs, const C<T>* __restrict__ tw, T scale,
-        size_t rs, int kcut) {
+__global__ void __launch_bounds__(M * Plan<N>::N1)
+k_x_uw(const C<T>* __restrict__ uk0, C<T>* __restrict__ out0, size_t fs, const C<T>* __restrict__ tw, T scale,
+       size_t rs, int kcut) {
   const C<T>* __restrict__ uk = rsel1(uk0, rs);
   C<T>* __restrict__ out = rsel1(out0, rs);
-  constexpr int N1 = Plan<N>::N1, N2 = Plan<N>::N2, Nf = N / 2 + 1, js = N * Nf, G = M * N1;
-  __shared__ C<T> lds[3 * M * (N + 1)];
-  if (!xBlockLive<N, M>(xPairBlock() * M, kcut)) return;   // zero lines, nothing stored
-  const int f = threadIdx.x / G, loc = threadIdx.x % G;
-  const int m = loc % M, n1 = loc / M;
-  const Twiddles<T, N> wt(n1, tw);         // line-FFT twiddles of n1, both directions
-  const int q = xPairBlock() * M + m;
-  const T ky = (T)kwave(q / Nf, N), kz = (T)(q % Nf);
-  C<T>* L[3] = {lds + m * (N + 1), lds + (M + m) * (N + 1), lds + (2 * M + m) * (N + 1)};
-  C<T>* Lf = lds + (f * M + m) * (N + 1);
+  constexpr int N1 = Plan<N>::N1, N2 = Plan<N>::N2, Nf = N / 2 + 1, js = N * Nf, NBL = N * Nf / M;
+  __shared__ C<T> lds[M * (N + 1)];
+  int lb, f;
+  if constexpr (NBL % 8 == 0) {
+    const int k = blockIdx.x / 8;
+    f = k % 6; lb = (k / 6) * 8 + blockIdx.x % 8;
+  } else {
+    f = blockIdx.x % 6; lb = blockIdx.x / 6;
+  }
+  if (!xBlockLive<N, M>(lb * M, kcut)) return;   // zero lines, nothing stored
+  const int m = threadIdx.x % M, n1 = threadIdx.x / M;
+  const Twiddles<T, N> wt(n1, tw);         // line-FFT twiddles of n1
+  const int q = lb * M + m;
   // kcut < N/2: u_hat has no mode outside the mask, so a line with
   // ky^2 + kz^2 > kcut (kcut + 1) is zero: it is not read, and its zero
   // outputs are not written (the y pass skips those entries, the z pass takes
-  // kz > kcut as zero without reading it)
+  // kz > kcut as zero without reading it).  Of a live line only the modes
+  // inside the mask radius are read (44 % of the live lines' entries at
+  // kcut = N/3; 256^3 FP32: 105 -> 89 us).
   const int kyi = kwave(q / Nf, N), kzi = q % Nf;
   const bool live = kcut >= N / 2 || kyi * kyi + kzi * kzi <= kcut * (kcut + 1);
-  const bool wr = live;
-  C<T> u[N2], w[N2];
-  if (live) {
-    // of a live line only the modes inside the mask radius are nonzero (44 % of
-    // the live lines' entries at kcut = N/3): the others are not read (256^3
-    // FP32: 105 -> 89 us)
+  auto inside = [&](int ix) {
+    const int kx = kwave(ix, N);
+    return live && (kcut >= N / 2 || kx * kx + kyi * kyi + kzi * kzi <= kcut * (kcut + 1));
+  };
+  const C<T> zero = mkc<T>((T)0, (T)0);
+  C<T> a[N2];
+  if (f < 3) {
+    // vorticity component f = i (k_b u_c - k_c u_b), (f, b, c) cyclic (forced-dns-sm.py:294-296)
+    const int b = f == 2 ? 0 : f + 1, c = f == 0 ? 2 : f - 1;
+    const C<T>* ub = uk + b * fs;
+    const C<T>* uc = uk + c * fs;
+    const T ky = (T)kyi, kz = (T)kzi;
+    C<T> x[N2];
 #pragma unroll
     for (int r = 0; r < N2; ++r) {
-      const int ix = posOut<N>(n1, r), kx = kwave(ix, N);
-      u[r] = kcut >= N / 2 || kx * kx + kyi * kyi + kzi * kzi <= kcut * (kcut + 1)
-                 ? ld32(uk + f * fs, (uint32_t)(q + ix * js)) : mkc<T>((T)0, (T)0);
+      const int ix = posOut<N>(n1, r);
+      const bool in = inside(ix);
+      a[r] = in ? ld32(ub, (uint32_t)(q + ix * js)) : zero;
+      x[r] = in ? ld32(uc, (uint32_t)(q + ix * js)) : zero;
+    }
+#pragma unroll
+    for (int r = 0; r < N2; ++r) {
+      const T kx = (T)kwave(posOut<N>(n1, r), N);
+      const T kb = b == 0 ? kx : b == 1 ? ky : kz, kc = c == 0 ? kx : c == 1 ? ky : kz;
+      a[r] = cmuli<T>(mkc<T>(kb * x[r].x - kc * a[r].x, kb * x[r].y - kc * a[r].y));
     }
   } else {
+    const C<T>* u = uk + (f - 3) * fs;
 #pragma unroll
-    for (int r = 0; r < N2; ++r) u[r] = mkc<T>((T)0, (T)0);
-  }
-#pragma unroll
-  for (int r = 0; r < N2; ++r) Lf[posOut<N>(n1, r)] = u[r];
-  __syncthreads();
-  // vorticity component f = i (k x u)_f  (forced-dns-sm.py:294-296)
-#pragma unroll
-  for (int r = 0; r < N2; ++r) {
-    const int ix = posOut<N>(n1, r);
-    const T kx = (T)kwave(ix, N);
-    if (f == 0) {
-      const C<T> u1 = L[1][ix], u2 = L[2][ix];
-      w[r] = cmuli<T>(mkc<T>(ky * u2.x - kz * u1.x, ky * u2.y - kz * u1.y));
-    } else if (f == 1) {
-      const C<T> u0 = L[0][ix], u2 = L[2][ix];
-      w[r] = cmuli<T>(mkc<T>(kz * u0.x - kx * u2.x, kz * u0.y - kx * u2.y));
-    } else {
-      const C<T> u0 = L[0][ix], u1 = L[1][ix];
-      w[r] = cmuli<T>(mkc<T>(kx * u1.x - ky * u0.x, kx * u1.y - ky * u0.y));
+    for (int r = 0; r < N2; ++r) {
+      const int ix = posOut<N>(n1, r);
+      a[r] = inside(ix) ? ld32(u, (uint32_t)(q + ix * js)) : zero;
     }
   }
-  // (lineInv synchronises before it reuses the regions)
-  lineInvT<T, N, 0>(w, Lf, n1, true, wt);
-  C<T>* Ow = out + (3 + f) * fs;
-  if (wr) {
+  lineInvT<T, N, 0>(a, lds + m * (N + 1), n1, true, wt);
+  C<T>* O = out + (f < 3 ? 3 + f : f - 3) * fs;
+  if (live) {
 #pragma unroll
-    for (int n2 = 0; n2 < N2; ++n2) st32(Ow, (uint32_t)(q + posIn<N>(n1, n2) * js), cscale<T>(w[n2], scale));
-  }
-  lineInvT<T, N, 0>(u, Lf, n1, true, wt);
-  C<T>* Ou = out + f * fs;
-  if (wr) {
-#pragma unroll
-    for (int n2 = 0; n2 < N2; ++n2) st32(Ou, (uint32_t)(q + posIn<N>(n1, n2) * js), cscale<T>(u[n2], scale));
+    for (int n2 = 0; n2 < N2; ++n2) st32(O, (uint32_t)(q + posIn<N>(n1, n2) * js), cscale<T>(a[n2], scale));
   }
 }
 
@@ -1019,70 +1078,46 @@ k_epi_proj(const C<T>* acc0, C<T>* uk0, size_t fs, double* maxpart0, size_t rs, 
 
 // Density RHS in spectral space (forced-dns-sm.py:325-330):
 //   kn_hat = (-i k.(nv)_hat*mask - fc_hat*mask) * mask, then x-inverse.
-// In: 4 fields (nv_x, nv_y, nv_z, fc) forward-transformed along z and y;
-// out: field 0 (x-inverse of kn_hat).
-// Four field groups (4 * M * N1 threads) forward-transform one input each;
-// the pointwise stage runs on the LDS spectra (modes r = g, g+4, ... of each
-// thread's line) and group 0 inverse-transforms the result.  Lines per block
-// keep the four LDS regions <= 132 KB.
-template <typename T, int N, int M0> struct XM4 {
-  static constexpr int v = (4L * M0 * (N + 1) * (long)sizeof(C<T>) <= 135168L) ? M0 : M0 / 2;
-};
+// In: the two fields of k_y_kn, A = nv_x and B = -i (ky nv_y + kz nv_z) - fc,
+// forward-transformed along z and y, so that kn_hat = (B - i kx A) mask; out:
+// field 0 (x-inverse of kn_hat).  One thread group transforms B, A and the
+// result in turn and keeps both spectra in registers.
 template <typename T, int N, int M>
-__global__ void __launch_bounds__(4 * M * Plan<N>::N1)
-k_x_kn4(C<T>* w0, size_t fs, const C<T>* __restrict__ tw, T scale, size_t rs, int kcut) {
+__global__ void __launch_bounds__(M * Plan<N>::N1)
+k_x_kn(C<T>* w0, size_t fs, const C<T>* __restrict__ tw, T scale, size_t rs, int kcut) {
   C<T>* w = rsel1(w0, rs);
-  constexpr int N1 = Plan<N>::N1, N2 = Plan<N>::N2, Nf = N / 2 + 1, js = N * Nf, G = M * N1;
-  __shared__ C<T> lds[4 * M * (N + 1)];
+  constexpr int N1 = Plan<N>::N1, N2 = Plan<N>::N2, Nf = N / 2 + 1, js = N * Nf;
+  __shared__ C<T> lds[M * (N + 1)];
   if (!xBlockLive<N, M>(xPairBlock() * M, kcut)) return;   // zero lines, nothing stored
-  const int g = threadIdx.x / G, loc = threadIdx.x % G;
-  const int m = loc % M, n1 = loc / M;
+  const int m = threadIdx.x % M, n1 = threadIdx.x / M;
   const Twiddles<T, N> wt(n1, tw);         // line-FFT twiddles of n1, both directions
   const int q = xPairBlock() * M + m;
   const int iy = q / Nf, iz = q % Nf;
-  C<T>* L0 = lds + m * (N + 1);
-  C<T>* L1 = lds + (M + m) * (N + 1);
-  C<T>* L2 = lds + (2 * M + m) * (N + 1);
-  C<T>* L3 = lds + (3 * M + m) * (N + 1);
-  C<T>* Lg = lds + (g * M + m) * (N + 1);
+  C<T>* L = lds + m * (N + 1);
   // kcut < N/2: kn_hat is masked, so lines with ky^2 + kz^2 > kcut (kcut + 1)
   // read no input (the previous y pass wrote none there) and give zero, which
   // is not written (the y pass skips those entries, the z pass takes kz > kcut
   // as zero without reading it)
   const int kyl = kwave(iy, N);
   const bool live = kcut >= N / 2 || kyl * kyl + iz * iz <= kcut * (kcut + 1);
-  C<T> a[N2];
-  const C<T>* W = w + g * fs;
+  C<T> a[N2], b[N2];
+#pragma unroll
+  for (int n2 = 0; n2 < N2; ++n2) {
+    const uint32_t o = (uint32_t)(q + posIn<N>(n1, n2) * js);
+    b[n2] = live ? ld32((const C<T>*)(w + fs), o) : mkc<T>((T)0, (T)0);
+    a[n2] = live ? ld32((const C<T>*)w, o) : mkc<T>((T)0, (T)0);
+  }
+  lineFwdT<T, N, 0>(b, L, n1, true, wt);
+  lineFwdT<T, N, 0>(a, L, n1, true, wt);
+#pragma unroll
+  for (int r = 0; r < N2; ++r) {
+    const Mode<T> md = mode<T, N>(posOut<N>(n1, r), iy, iz);
+    b[r] = cscale<T>(mkc<T>(b[r].x + md.kx * a[r].y, b[r].y - md.kx * a[r].x), md.mask);
+  }
+  lineInvT<T, N, 0>(b, L, n1, true, wt);
   if (live) {
 #pragma unroll
-    for (int n2 = 0; n2 < N2; ++n2) a[n2] = ld32(W, (uint32_t)(q + posIn<N>(n1, n2) * js));
-  } else {
-#pragma unroll
-    for (int n2 = 0; n2 < N2; ++n2) a[n2] = mkc<T>((T)0, (T)0);
-  }
-  lineFwdT<T, N, 0>(a, Lg, n1, true, wt);
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < N2; ++r) Lg[posOut<N>(n1, r)] = a[r];
-  __syncthreads();
-  for (int r = g; r < N2; r += 4) {
-    const int ix = posOut<N>(n1, r);
-    const Mode<T> md = mode<T, N>(ix, iy, iz);
-    C<T> acc = cscale<T>(cscale<T>(L0[ix], md.mask), md.kx);
-    acc = cadd<T>(acc, cscale<T>(cscale<T>(L1[ix], md.mask), md.ky));
-    acc = cadd<T>(acc, cscale<T>(cscale<T>(L2[ix], md.mask), md.kz));
-    const C<T> mi = mkc<T>(acc.y, -acc.x);   // -i * (k . nv)
-    L0[ix] = cscale<T>(csub<T>(mi, cscale<T>(L3[ix], md.mask)), md.mask);
-  }
-  __syncthreads();
-  if (g == 0) {
-#pragma unroll
-    for (int r = 0; r < N2; ++r) a[r] = L0[posOut<N>(n1, r)];
-  }
-  lineInvT<T, N, 0>(a, L0, n1, g == 0, wt);
-  if (g == 0 && live) {
-#pragma unroll
-    for (int n2 = 0; n2 < N2; ++n2) st32(w, (uint32_t)(q + posIn<N>(n1, n2) * js), cscale<T>(a[n2], scale));
+    for (int n2 = 0; n2 < N2; ++n2) st32(w, (uint32_t)(q + posIn<N>(n1, n2) * js), cscale<T>(b[n2], scale));
   }
 }
 
