@@ -99,7 +99,12 @@ struct Engine final : EngineBase {
   C<T>* tw = nullptr;
   hipStream_t st2 = nullptr;        // density/droplet stream (created here)
   bool serial = false;              // no overlap of the flow and density chains
-  unsigned pstage_lds = 0;          // dynamic LDS bytes per block of the droplet stage kernel
+  // Dynamic LDS bytes per block of the droplet stage kernel: four blocks per CU
+  // instead of six, which keeps the droplets in flight per XCD (whose stencils
+  // share its L2) fewer.  Four steps at 256^3 FP32 with 10^6 droplets 22.55 ->
+  // 22.38 ms, two at 512^3 103.0 -> 102.1 ms, the 64 x 64^3 ensemble 45.9 ->
+  // 44.4 ms, 128^3 FP64 6.05 -> 6.00 ms.
+  unsigned pstage_lds = 38000;
   // queue a stage's density chain after the next flow x pass (measured at 256^3:
   // 8.18 vs 8.31 ms/step; the 64^3 ensemble is faster in the plain order)
   bool late_density = N >= 128;
@@ -415,7 +420,7 @@ struct Engine final : EngineBase {
       arena(rid, cap); arena(rid2, cap); arena(pkey, cap); arena(prank, cap);
       arena(hist, NB); arena(bsum, NBS);
       arena(x0b, 3 * cap); arena(v0b, 4 * cap);
-      arena(dep, cap); arena(flist, cap); arena(fcount, 1); arena(wmaxp, 1); arena(fx, RF);
+      arena(dep, cap); arena(flist, cap); arena(fcount, 1); arena(wmaxp, WSLOTS * 16); arena(fx, RF);
     }
     LD_TRY(arena_commit());
     LD_TRY(alloc(shells, 8));
@@ -815,15 +820,19 @@ struct Engine final : EngineBase {
       ps.gu = gup; ps.gv = gup; ps.dep = dep; ps.flist = flist; ps.fcount = fcount;
       ps.wmax = wmaxp;
       ps.ah = a_coef[s] * h; ps.wh = wh; ps.P = dp; ps.rs = rs;
-      // 4 lanes per droplet; block count a multiple of 8 for the XCD mapping
-      const unsigned nb = (unsigned)(((4 * np + 255) / 256 + 7) / 8 * 8);
       LD_TRY(prof_mark(LD_K_DROPLETS, st2));
-      // pstage_lds: dynamic LDS reserved per block, which caps the blocks per CU
-      // (and so the droplets in flight per XCD, whose stencils share its L2)
-      if (B == 1)
-        hipLaunchKernelGGL((k_particles_stage<T, PT, N, false>), dim3(nb), dim3(256), pstage_lds, st2, ps);
-      else
-        hipLaunchKernelGGL((k_particles_stage<T, PT, N, true>), dim3(nb, 1, B), dim3(256), pstage_lds, st2, ps);
+      auto stage = [&](auto bat, auto lanes) {
+        constexpr int NL = decltype(lanes)::value;
+        // block count a multiple of 8 for the XCD mapping
+        const unsigned nb = (unsigned)(((NL * np + 255) / 256 + 7) / 8 * 8);
+        hipLaunchKernelGGL((k_particles_stage<T, PT, N, decltype(bat)::value, NL>), dim3(nb, 1, B), dim3(256),
+                           pstage_lds, st2, ps);
+      };
+      using L4 = std::integral_constant<int, 4>;
+      using L8 = std::integral_constant<int, 8>;
+      const bool sparse = 6 * np < (int64_t)RF;       // lanes per droplet: see the kernel
+      if (B == 1) { if (sparse) stage(std::false_type{}, L8{}); else stage(std::false_type{}, L4{}); }
+      else { if (sparse) stage(std::true_type{}, L8{}); else stage(std::true_type{}, L4{}); }
       LD_LAUNCHED();
       LD_TRY(prof_mark(LD_K_DROPLETS, st2));
       LD_TRY(prof_mark(LD_K_DEPOSIT, st2));

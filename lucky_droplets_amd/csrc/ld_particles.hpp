@@ -213,41 +213,59 @@ struct DropPhys {
   double invL, inv_dx, inv_factor;
 };
 
-// Droplet RHS at one stage coordinate (particles.py:823-835).  xw: wrapped
-// position, vp: velocity, m: mass/M0.  I: the 7 interpolated components
-// [u, v, n].  Returns rhs[7] and W (= mdot / M0).
-__device__ __forceinline__ void dropletRhs(const DropPhys& P, const double vp[3], double m, const double I[7],
-                                           double rhs[7], double& W) {
+// Growth rate W (= mdot / M0) and St tau_eta of a droplet at one stage
+// coordinate (particles.py:823-828).  vp: velocity, m: mass/M0.  I: the 7
+// interpolated components [u, v, n].
+__device__ __forceinline__ double dropletGrowth(const DropPhys& P, const double vp[3], double m, const double I[7],
+                                                double& W) {
   const double st = pow(m / P.factor, 2.0 / 3.0);                          // :823
   const double d0 = vp[0] - I[3], d1 = vp[1] - I[4], d2 = vp[2] - I[5];
   const double nrm = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
   const double q = 1.0 + sqrt(P.st_s / st);
   W = P.growth * (q * q) * I[6] * nrm;                                      // :828
+  return st * P.tau_eta;
+}
+// Droplet RHS at one stage coordinate (particles.py:823-835): rhs[7] and W.
+__device__ __forceinline__ void dropletRhs(const DropPhys& P, const double vp[3], double m, const double I[7],
+                                           double rhs[7], double& W) {
+  const double den = dropletGrowth(P, vp, m, I, W);
   rhs[0] = vp[0]; rhs[1] = vp[1]; rhs[2] = vp[2];                           // :831
-  const double den = st * P.tau_eta;
   rhs[3] = (I[0] - vp[0]) / den;                                            // :832
   rhs[4] = (I[1] - vp[1]) / den;
   rhs[5] = (I[2] - vp[2]) / den - P.g;                                      // :834
   rhs[6] = W;                                                               // :835
 }
 
-// The same RHS in single precision for the FP32 form (velocities and masses
-// are FP32 there); St from exp2(2/3 log2(m / factor)), divisions by one
-// reciprocal.
-__device__ __forceinline__ void dropletRhsF(const DropPhys& P, const float vp[3], float m, const float I[7],
-                                            float rhs[7], float& W) {
+// The growth rate in single precision for the FP32 form (velocities and masses
+// are FP32 there); St from exp2(2/3 log2(m / factor)).
+__device__ __forceinline__ float dropletGrowth(const DropPhys& P, const float vp[3], float m, const float I[7],
+                                               float& W) {
   const float st = exp2f((2.0f / 3.0f) * log2f(m * (float)P.inv_factor));   // :823
   const float d0 = vp[0] - I[3], d1 = vp[1] - I[4], d2 = vp[2] - I[5];
   const float nrm = sqrtf(d0 * d0 + d1 * d1 + d2 * d2);
   const float q = 1.0f + sqrtf((float)P.st_s / st);
   W = (float)P.growth * (q * q) * I[6] * nrm;                                // :828
-  rhs[0] = vp[0]; rhs[1] = vp[1]; rhs[2] = vp[2];                           // :831
-  const float rden = 1.0f / (st * (float)P.tau_eta);
-  rhs[3] = (I[0] - vp[0]) * rden;                                           // :832
-  rhs[4] = (I[1] - vp[1]) * rden;
-  rhs[5] = (I[2] - vp[2]) * rden - (float)P.g;                              // :834
-  rhs[6] = W;                                                               // :835
+  return st * (float)P.tau_eta;
 }
+// x / den (FP32: by the reciprocal), less g
+__device__ __forceinline__ double dragTerm(double x, double den, double g) { return x / den - g; }
+__device__ __forceinline__ float dragTerm(float x, float den, float g) { return x * (1.0f / den) - g; }
+
+// ------------------------------------------------------------ lane quads
+// v of the lane L of the caller's quad of lanes (all four active), and of the
+// lane whose number in the quad differs in the bits X: DPP moves, no LDS.
+template <int CTRL, typename G> __device__ __forceinline__ G dppMove(G v) {
+  if constexpr (sizeof(G) == 4) {
+    return __builtin_bit_cast(G, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+  } else {
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(G, ((long long)hi << 32) | (unsigned int)lo);
+  }
+}
+template <int L, typename G> __device__ __forceinline__ G quadLane(G v) { return dppMove<L * 0x55>(v); }
+template <int X, typename G> __device__ __forceinline__ G quadXor(G v) { return dppMove<X == 1 ? 0xB1 : 0x4E>(v); }
 
 // ------------------------------------------------------------ spatial sort
 // Droplets are reordered by spatial bin once per step (counting sort), so
@@ -304,7 +322,7 @@ template <typename T, typename PT> struct PStage {
   const V4<T>* gu; const V4<T>* gv;   // gather records {u, 0} (recU) and {v, n_stage} (recV); one array
   double4* dep;                // out: wrapped stage position and W per slot (brick deposit input)
   int* flist; int* fcount;     // out: slots whose stage bin moved > 1 bin since the sort
-  unsigned long long* wmax;    // out: largest W > 0 of the launch (bits of a positive double); zero before
+  unsigned long long* wmax;    // out: largest W > 0 of the launch (bits of positive doubles, WSLOTS slots); zero before
   double ah, wh;               // a_s * h, w_s * h
   DropPhys P;
   size_t rs;                   // realization stride in bytes (batched launches)
@@ -322,13 +340,26 @@ template <typename T, typename PT> struct PStage {
 // [u, v, n] (:826), growth rate and deposit (:828-829), RHS (:831-835) and
 // sump accumulation (forced-dns-sm.py:342-358).
 //
-// Four lanes per droplet: lane c owns z-node c of the 4x4x4 stencil, so one
-// wavefront load or atomic touches 16 droplets x 4 consecutive z cells (one
-// 16-byte segment per droplet).  Partial sums are combined across the four
-// lanes with xor shuffles.
+// NL = 4 or 8 lanes per droplet.  Lane c of a quad owns z-node c of the 4x4x4
+// stencil, so a load touches one 64-byte run of each droplet; with 8 lanes the
+// first quad takes the u records and the second the v records, which lie on the
+// same 128-byte lines, so a line is asked for once instead of twice, by half as
+// many droplets at a time.  Around the gather the lanes of a quad split the
+// droplet's components instead of repeating each other: lane c forms axis c's
+// wrap, cell and sincos (lane 3 repeats z) and loads, updates and stores
+// component c of the position and of (velocity, mass); what all need moves by
+// DPP.  Every choice gives the same bits.
+// Measured per launch (one lane forming everything, one slot for the largest W
+// -> 4 lanes -> 8 lanes): 10^6 droplets at 256^3 FP32 288 -> 300 -> 278 us (8
+// lanes, four blocks per CU: 267); 10^7 at 512^3 FP32 2470 -> 2562 -> 2358
+// (2262); 10^5 in each of 64 times 64^3 FP32 895 -> 871 -> 929 (4 lanes, four
+// blocks: 834); 10^5 at 64^3 FP32 26.2 -> 15.0 -> 17.7; 123457 at 128^3 FP64
+// 79.5 -> 83.7 -> 72.7.  Sparse droplets (each of the 28 lines of a stencil
+// serves few of them) are bound by the lines asked of L2, dense ones by
+// instructions: 8 lanes below one droplet in 6 cells, 4 above.
 // BAT: batched launch (blockIdx.z = realization); the single-realization
 // instantiation skips the pointer offsets and their registers.
-template <typename T, typename PT, int N, bool BAT>
+template <typename T, typename PT, int N, bool BAT, int NL>
 __global__ void __launch_bounds__(256)
 k_particles_stage(PStage<T, PT> A0) {
   const PStage<T, PT> A = BAT ? A0.shifted() : A0;
@@ -337,8 +368,9 @@ k_particles_stage(PStage<T, PT> A0) {
   // sees one region of the fields.
   const int nb = gridDim.x, per = nb / 8;
   const int lb = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  const int gt = lb * blockDim.x + threadIdx.x;
-  const int p = gt >> 2, c = gt & 3;
+  static_assert(NL == 4 || NL == 8, "one or two quads per droplet");
+  const int p = lb * (256 / NL) + threadIdx.x / NL, c = threadIdx.x & 3;
+  const bool hi = NL == 8 && (threadIdx.x & 4);         // second quad: v records
   const bool live = p < A.np;
   const int pp = live ? p : 0;
   constexpr size_t R = (size_t)N * N * N;
@@ -348,17 +380,12 @@ k_particles_stage(PStage<T, PT> A0) {
   // branches (stage 0 takes k = 0 and the sump inputs from the RK base).
   const bool s0 = A.stage == 0;
   const double ah = s0 ? 0.0 : A.ah;
-  double x0v[3], xs[3], kxv[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int k = 0; k < 3; ++k) x0v[k] = A.x0[k * cap + pp];
-  if (!s0) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) kxv[k] = (double)A.kx[k * cap + pp];
-  }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) xs[k] = x0v[k] + ah * kxv[k];
+  const int ax = c < 3 ? c : 2;
+  const double x0c = A.x0[ax * cap + pp];
+  double kxc = 0.0;
+  if (!s0) kxc = (double)A.kx[ax * cap + pp];
   const double L = A.P.L, dx = A.P.dx, pi_2dx = A.P.pi_2dx, invL = A.P.invL, inv_dx = A.P.inv_dx;
-  const double xw = wrapFast(xs[0], L, invL), yw = wrapFast(xs[1], L, invL), zw = wrapFast(xs[2], L, invL);
+  const double xw = wrapFast(x0c + ah * kxc, L, invL);
   // one sincos per axis (cosW4); node i0 + a has weight (1 +- {cos, sin})/4.
   // The angles and the sincos are FP64; the weights and the gather sums are
   // kept in the field precision GT (FP32 fields: FP32 sums of 64 terms).
@@ -367,27 +394,28 @@ k_particles_stage(PStage<T, PT> A0) {
   // gather so the wrapped position holds no registers across it: the wrapped
   // stage position now, W after the RHS.  Slots whose stage bin left the
   // +-1-bin window around their sorted bin go to the fallback list.
-  bool far = false;
-  if (live && c == 0) {
-    const double xb[3] = {xw, yw, zw};
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      // bins exactly as k_bin_count forms them
-      const int cs = cellOf<N>(xb[k], inv_dx), c0 = cellOf<N>(wrapFast(x0v[k], L, invL), inv_dx);
-      const int d = ((cs / Bins<N>::BS - c0 / Bins<N>::BS) % Bins<N>::B + Bins<N>::B) % Bins<N>::B;
-      far = far || (d > 1 && d < Bins<N>::B - 1);
-    }
-    double* dp = reinterpret_cast<double*>(A.dep + p);
-    dp[0] = xw; dp[1] = yw; dp[2] = zw;
-    if (far) A.flist[atomicAdd(A.fcount, 1)] = p;
+  bool far;
+  {
+    // bins exactly as k_bin_count forms them
+    const int cs = cellOf<N>(xw, inv_dx), c0 = cellOf<N>(wrapFast(x0c, L, invL), inv_dx);
+    const int d = ((cs / Bins<N>::BS - c0 / Bins<N>::BS) % Bins<N>::B + Bins<N>::B) % Bins<N>::B;
+    int f = d > 1 && d < Bins<N>::B - 1;
+    f |= quadXor<1>(f);
+    f |= quadXor<2>(f);
+    far = f != 0;
   }
-  const int i0 = originOf(xw, inv_dx), j0 = originOf(yw, inv_dx), k0 = originOf(zw, inv_dx);
+  if (live) {
+    if (c < 3 && !hi) reinterpret_cast<double*>(A.dep + p)[c] = xw;
+    if (far && c == 0 && !hi) A.flist[atomicAdd(A.fcount, 1)] = p;
+  }
+  const int o0 = originOf(xw, inv_dx);
   // the angles are formed in FP64; their sines and cosines are taken in the
   // weight precision GT (the FP32 form rounds the angle in [pi/2, pi) to FP32)
-  GT xsn, xcs, ysn, ycs, zsn, zcs;
-  sincosStencil<GT>(xw, i0, dx, inv_dx, pi_2dx, xsn, xcs);
-  sincosStencil<GT>(yw, j0, dx, inv_dx, pi_2dx, ysn, ycs);
-  sincosStencil<GT>(zw, k0, dx, inv_dx, pi_2dx, zsn, zcs);
+  GT snc, csc;
+  sincosStencil<GT>(xw, o0, dx, inv_dx, pi_2dx, snc, csc);
+  const int i0 = quadLane<0>(o0), j0 = quadLane<1>(o0), k0 = quadLane<2>(o0);
+  const GT xsn = quadLane<0>(snc), xcs = quadLane<0>(csc), ysn = quadLane<1>(snc), ycs = quadLane<1>(csc),
+           zsn = quadLane<2>(snc), zcs = quadLane<2>(csc);
   const GT q = (GT)0.25;
   const GT wy[4] = {q * ((GT)1 + ycs), q * ((GT)1 + ysn), q * ((GT)1 - ycs), q * ((GT)1 - ysn)};
   int iy[4];
@@ -403,127 +431,149 @@ k_particles_stage(PStage<T, PT> A0) {
   const PT* kvp = s0 ? A.v0 : A.kv;
   const double* sxp = s0 ? A.x0 : A.sx;
   const PT* svp = s0 ? A.v0 : A.sv;
-  PT v0v[4], kvv[4], prv[4];
-  double prx[3];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) { v0v[k] = A.v0[k * cap + pp]; kvv[k] = kvp[k * cap + pp]; prv[k] = svp[k * cap + pp]; }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) prx[k] = sxp[k * cap + pp];
+  const PT v0c = A.v0[c * cap + pp], kvc = kvp[c * cap + pp], prv = svp[c * cap + pp];
+  const double prx = sxp[ax * cap + pp];
   // gather: this lane's z node, all (x, y) nodes; two 16-byte records per node
-  GT Ig[7];
+  PT I[7];
+  if constexpr (NL == 8) {
+    // this quad's record of each node, all 16 loads ahead of the sums
+    GT Ig[4] = {(GT)0, (GT)0, (GT)0, (GT)0};
+    if (live) {
+      V4<T> U[16];
 #pragma unroll
-  for (int k = 0; k < 7; ++k) Ig[k] = (GT)0;
-  // FP32 fields: all 32 record loads are written ahead of the sums, so the
-  // compiler keeps about a dozen in flight per lane (at 5 waves per SIMD);
-  // this measured faster than a plane-by-plane loop at 8 waves per SIMD.
-  // FP64 records are twice the size; they keep the loop.
-  if (sizeof(T) == 4 && live) {
-    V4<T> U[16], V[16];
+      for (int a = 0; a < 4; ++a) {
+        const uint32_t plane = (uint32_t)wrapIdx<N>(i0 + a) * N;
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const uint32_t plane = (uint32_t)wrapIdx<N>(i0 + a) * N;
+        for (int b = 0; b < 4; ++b)
+          U[a * 4 + b] = ldRec<T, N>(A.gu, recU((plane + (uint32_t)iy[b]) * N + (uint32_t)iz) | (hi ? 4u : 0u));
+      }
 #pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const uint32_t o = (plane + (uint32_t)iy[b]) * N + (uint32_t)iz;
-        U[a * 4 + b] = ldRec<T, N>(A.gu, recU(o));
-        V[a * 4 + b] = ldRec<T, N>(A.gv, recV(o));
+      for (int a = 0; a < 4; ++a) {
+        const GT wx = (GT)0.25 * ((GT)1 + ((a & 2) ? (GT)-1 : (GT)1) * ((a & 1) ? gxs : gxc));
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const GT w = wy[b] * wx;
+          const V4<T>& u = U[a * 4 + b];
+          Ig[0] += (GT)u.x * w;
+          Ig[1] += (GT)u.y * w;
+          Ig[2] += (GT)u.z * w;
+          Ig[3] += (GT)u.w * w;
+        }
       }
     }
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const GT wx = (GT)0.25 * ((GT)1 + ((a & 2) ? (GT)-1 : (GT)1) * ((a & 1) ? gxs : gxc));
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const GT w = wy[b] * wx;
-        const V4<T>& u = U[a * 4 + b];
-        const V4<T>& v = V[a * 4 + b];
-        Ig[0] += (GT)u.x * w;
-        Ig[1] += (GT)u.y * w;
-        Ig[2] += (GT)u.z * w;
-        Ig[3] += (GT)v.x * w;
-        Ig[4] += (GT)v.y * w;
-        Ig[5] += (GT)v.z * w;
-        Ig[6] += (GT)v.w * w;
-      }
+    for (int k = 0; k < 4; ++k) {
+      GT v = Ig[k] * wz;
+      v += quadXor<1>(v);
+      v += quadXor<2>(v);
+      const GT o = dppMove<0x141>(v);          // the other quad's sum (mirrored half row)
+      if (k < 3) I[k] = (PT)(hi ? o : v);
+      I[3 + k] = (PT)(hi ? v : o);
     }
-  } else if (live) {
-#pragma unroll 1
-    for (int a = 0; a < 4; ++a) {
-      const GT wx = (GT)0.25 * ((GT)1 + ((a & 2) ? (GT)-1 : (GT)1) * ((a & 1) ? gxs : gxc));
-      const uint32_t plane = (uint32_t)wrapIdx<N>(i0 + a) * N;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const uint32_t o = (plane + (uint32_t)iy[b]) * N + (uint32_t)iz;   // < N^3 <= 2^27
-        const GT w = wy[b] * wx;
-        const V4<T> U = ldRec<T, N>(A.gu, recU(o));
-        const V4<T> V = ldRec<T, N>(A.gv, recV(o));
-        Ig[0] += (GT)U.x * w;
-        Ig[1] += (GT)U.y * w;
-        Ig[2] += (GT)U.z * w;
-        Ig[3] += (GT)V.x * w;
-        Ig[4] += (GT)V.y * w;
-        Ig[5] += (GT)V.z * w;
-        Ig[6] += (GT)V.w * w;
-      }
-    }
-  }
-  double I[7];
-#pragma unroll
-  for (int k = 0; k < 7; ++k) {
-    GT v = Ig[k] * wz;
-    v += __shfl_xor(v, 1, 64);
-    v += __shfl_xor(v, 2, 64);
-    I[k] = (double)v;
-  }
-  double rhs[7], W = 0.0;
-  if constexpr (sizeof(PT) == 4) {
-    float vpf[3], If[7], rf[7], Wf = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) vpf[k] = v0v[k] + (PT)ah * kvv[k];
-    const float mf = v0v[3] + (PT)ah * kvv[3];
-#pragma unroll
-    for (int k = 0; k < 7; ++k) If[k] = (float)I[k];
-    if (live) dropletRhsF(A.P, vpf, mf, If, rf, Wf);
-#pragma unroll
-    for (int k = 0; k < 7; ++k) rhs[k] = (double)rf[k];
-    W = (double)Wf;
   } else {
-    double vp[3], m;
+    GT Ig[7];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) vp[k] = (double)(PT)(v0v[k] + (PT)ah * kvv[k]);
-    m = (double)(PT)(v0v[3] + (PT)ah * kvv[3]);
-    if (live) dropletRhs(A.P, vp, m, I, rhs, W);
+    for (int k = 0; k < 7; ++k) Ig[k] = (GT)0;
+    // FP32 fields: all 32 record loads are written ahead of the sums, so the
+    // compiler keeps about a dozen in flight per lane (at 5 waves per SIMD);
+    // this measured faster than a plane-by-plane loop at 8 waves per SIMD.
+    // FP64 records are twice the size; they keep the loop.
+    if (sizeof(T) == 4 && live) {
+      V4<T> U[16], V[16];
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const uint32_t plane = (uint32_t)wrapIdx<N>(i0 + a) * N;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const uint32_t o = (plane + (uint32_t)iy[b]) * N + (uint32_t)iz;
+          U[a * 4 + b] = ldRec<T, N>(A.gu, recU(o));
+          V[a * 4 + b] = ldRec<T, N>(A.gv, recV(o));
+        }
+      }
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const GT wx = (GT)0.25 * ((GT)1 + ((a & 2) ? (GT)-1 : (GT)1) * ((a & 1) ? gxs : gxc));
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const GT w = wy[b] * wx;
+          const V4<T>& u = U[a * 4 + b];
+          const V4<T>& v = V[a * 4 + b];
+          Ig[0] += (GT)u.x * w;
+          Ig[1] += (GT)u.y * w;
+          Ig[2] += (GT)u.z * w;
+          Ig[3] += (GT)v.x * w;
+          Ig[4] += (GT)v.y * w;
+          Ig[5] += (GT)v.z * w;
+          Ig[6] += (GT)v.w * w;
+        }
+      }
+    } else if (live) {
+#pragma unroll 1
+      for (int a = 0; a < 4; ++a) {
+        const GT wx = (GT)0.25 * ((GT)1 + ((a & 2) ? (GT)-1 : (GT)1) * ((a & 1) ? gxs : gxc));
+        const uint32_t plane = (uint32_t)wrapIdx<N>(i0 + a) * N;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const uint32_t o = (plane + (uint32_t)iy[b]) * N + (uint32_t)iz;   // < N^3 <= 2^27
+          const GT w = wy[b] * wx;
+          const V4<T> U = ldRec<T, N>(A.gu, recU(o));
+          const V4<T> V = ldRec<T, N>(A.gv, recV(o));
+          Ig[0] += (GT)U.x * w;
+          Ig[1] += (GT)U.y * w;
+          Ig[2] += (GT)U.z * w;
+          Ig[3] += (GT)V.x * w;
+          Ig[4] += (GT)V.y * w;
+          Ig[5] += (GT)V.z * w;
+          Ig[6] += (GT)V.w * w;
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+      GT v = Ig[k] * wz;
+      v += quadXor<1>(v);
+      v += quadXor<2>(v);
+      I[k] = (PT)v;
+    }
   }
+  // lane c's velocity component or, c == 3, the mass, and the droplet's four
+  const PT vc = v0c + (PT)ah * kvc;
+  const PT vp[3] = {quadLane<0>(vc), quadLane<1>(vc), quadLane<2>(vc)};
+  PT W = (PT)0;
+  const PT den = dropletGrowth(A.P, vp, quadLane<3>(vc), I, W);
+  const PT Ic = c == 0 ? I[0] : c == 1 ? I[1] : I[2];
+  const PT drag = dragTerm(Ic - vc, den, c == 2 ? (PT)A.P.g : (PT)0);      // :832-834
+  const PT rc = c < 3 ? drag : W;                                          // :835
   // largest growth rate of the launch: the bound of the deposits' fixed-point
   // scale.  A NaN or negative W (not a growth) makes it infinite, so the
   // deposit writes NaN everywhere, as the reference's would spread it.
   {
-    __shared__ double wm[4];
-    double v = !live ? 0.0 : (W > 0.0 ? W : (W == 0.0 ? 0.0 : INFINITY));
+    __shared__ PT wm[4];
+    PT v = !live ? (PT)0 : (W > (PT)0 ? W : (W == (PT)0 ? (PT)0 : (PT)INFINITY));
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
+    for (int off = 32; off > NL / 2; off >>= 1) {      // a droplet's lanes hold one W
+      const PT o = __shfl_xor(v, off, 64);
+      v = o > v ? o : v;
+    }
     if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
-      const double b = fmax(fmax(wm[0], wm[1]), fmax(wm[2], wm[3]));
-      if (b > 0.0) atomicMax(A.wmax, (unsigned long long)__double_as_longlong(b));
+      const PT a = wm[0] > wm[1] ? wm[0] : wm[1], b = wm[2] > wm[3] ? wm[2] : wm[3], m = a > b ? a : b;
+      if (m > (PT)0) atomicMax(A.wmax + wslot(blockIdx.x), (unsigned long long)__double_as_longlong((double)m));
     }
   }
-  if (!live || c != 0) return;
-  // a fallback slot stores -W so the brick pass (which takes W > 0) skips it
-  reinterpret_cast<double*>(A.dep + p)[3] = far ? -W : W;
+  if (!live || hi) return;
   // sump (forced-dns-sm.py:337, 342-358); the last stage writes the new state
   double* dxp = A.stage == 3 ? A.x0 : A.sx;
   PT* dvp = A.stage == 3 ? A.v0 : A.sv;
-#pragma unroll
-  for (int k = 0; k < 3; ++k) dxp[k * cap + p] = prx[k] + A.wh * rhs[k];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) dvp[k * cap + p] = prv[k] + (PT)A.wh * (PT)rhs[3 + k];
-  if (A.stage < 3) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) A.kx[k * cap + p] = (PT)rhs[k];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) A.kv[k * cap + p] = (PT)rhs[3 + k];
+  dvp[c * cap + p] = prv + (PT)A.wh * rc;
+  if (A.stage < 3) A.kv[c * cap + p] = rc;
+  if (c < 3) {
+    dxp[c * cap + p] = prx + A.wh * (double)vc;                            // :831
+    if (A.stage < 3) A.kx[c * cap + p] = vc;
+  } else {
+    // a fallback slot stores -W so the brick pass (which takes W > 0) skips it
+    reinterpret_cast<double*>(A.dep + p)[3] = far ? -(double)W : (double)W;
   }
 }
 
@@ -625,7 +675,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
     if (blockIdx.x >= NBRICK) {          // the extra blocks: fallback slots
       const int nf = *rsel1(fcount0, rs), b = (int)blockIdx.x - NBRICK;
       if (nf)
-        fallbackAccum<T, N>(dep, rsel1(flist0, rs), nf, *wmax, rsel1(fx0, rs), P, b * Brick<N>::NT + (int)threadIdx.x,
+        fallbackAccum<T, N>(dep, rsel1(flist0, rs), nf, maxOfSlots(wmax), rsel1(fx0, rs), P, b * Brick<N>::NT + (int)threadIdx.x,
                             ((int)gridDim.x - NBRICK) * Brick<N>::NT);
       return;
     }
@@ -639,6 +689,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   __shared__ int rb[NR], rn[NR], rl[NR + 1];
   __shared__ int list[CH];
   __shared__ int cnt;
+  __shared__ unsigned long long wtop;
   const int tid = threadIdx.x, lane = tid & 63;
   // XCD-aware: each of the 8 XCDs takes a contiguous run of bricks
   constexpr int per = NBRICK / 8;
@@ -646,6 +697,15 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   const int c0x = (br / (NBr * NBr)) * S, c0y = ((br / NBr) % NBr) * S, c0z = (br % NBr) * S;
   for (int i = tid; i < S * S * S; i += NT) tile[i] = 0;
   if (tid == 0) cnt = 0;
+  if (FIX && tid < WSLOTS) {
+    unsigned long long v = wmax[wslot(tid)];
+#pragma unroll
+    for (int off = WSLOTS / 2; off > 0; off >>= 1) {
+      const unsigned long long o = __shfl_xor(v, off, 64);
+      v = o > v ? o : v;
+    }
+    if (tid == 0) wtop = v;
+  }
   // slot ranges of the window's z-runs
   const int lo = (NBX == B) ? 0 : 1;
   const int blx = ((c0x - 2 + N) % N) / BS - lo, bly = ((c0y - 2 + N) % N) / BS - lo;
@@ -697,7 +757,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   __syncthreads();
   const int total = rl[NR];
   const double dx = P.dx, pi_2dx = P.pi_2dx, inv_dx = P.inv_dx;
-  const double bound = FIX ? (double)total * __longlong_as_double((long long)*wmax) * P.inv_vol * 0.125 : 0.0;
+  const double bound = FIX ? (double)total * __longlong_as_double((long long)wtop) * P.inv_vol * 0.125 : 0.0;
   const bool finite = isfinite(bound);
   // FP32 fields: sums below 2^52, so a value converts to its integer by one
   // addition of 2^52 (round to nearest even, as llrint); FP64 fields keep the
