@@ -249,6 +249,9 @@ struct ZTile {
   static constexpr int REG = 2 * Nf;
   C<T>* lds;
   __device__ __forceinline__ C<T>* region(int r) const { return lds + r * REG; }
+  // node j of lines 2c and 2c + 1 of field f, for the operations that declare
+  // `pairs`: their real lines are kept as the transforms hold them
+  __device__ __forceinline__ C<T>& pair(int f, int c, int j) const { return region(f * (P / 2) + c)[j]; }
   __device__ __forceinline__ T& re(int f, int p, int j) const {
     T* Rr = (T*)region(f * (P / 2) + p / 2);
     return Rr[(p & 1) * N + j];
@@ -266,7 +269,7 @@ struct ZTile {
 // spectral lines into the tile; leaves real lines in the tile.  Imaginary
 // parts of the kz = 0 and kz = N/2 modes are ignored, as a c2r transform does.
 // w: this thread's twiddles (n1 = threadIdx.x % N1).
-template <typename T, int N, int P, int FIN>
+template <typename T, int N, int P, int FIN, bool PAIR>
 __device__ __forceinline__ void zInverse(const ZTile<T, N, P>& tile, const Twiddles<T, N>& w) {
   constexpr int N1 = Plan<N>::N1, N2 = Plan<N>::N2, Nf = N / 2 + 1;
   const int r = threadIdx.x / N1, n1 = threadIdx.x % N1;
@@ -296,8 +299,12 @@ __device__ __forceinline__ void zInverse(const ZTile<T, N, P>& tile, const Twidd
 #pragma unroll
     for (int n2 = 0; n2 < N2; ++n2) {
       const int j = posIn<N>(n1, n2);
-      Rr[j] = a[n2].x;
-      Rr[N + j] = a[n2].y;
+      if constexpr (PAIR) {
+        reg[j] = a[n2];
+      } else {
+        Rr[j] = a[n2].x;
+        Rr[N + j] = a[n2].y;
+      }
     }
   }
   __syncthreads();
@@ -305,8 +312,8 @@ __device__ __forceinline__ void zInverse(const ZTile<T, N, P>& tile, const Twidd
 
 // Forward z transform (r2c, unnormalised) of FOUT real fields in the tile;
 // leaves each pair's complex spectrum Z (natural order, N entries) in its
-// region.  Split with zSplit().  w as for zInverse.
-template <typename T, int N, int P, int FOUT>
+// region (k_z splits it into the two lines).  w as for zInverse.
+template <typename T, int N, int P, int FOUT, bool PAIR>
 __device__ __forceinline__ void zForward(const ZTile<T, N, P>& tile, const Twiddles<T, N>& w) {
   constexpr int N1 = Plan<N>::N1, N2 = Plan<N>::N2;
   const int r = threadIdx.x / N1, n1 = threadIdx.x % N1;
@@ -318,7 +325,8 @@ __device__ __forceinline__ void zForward(const ZTile<T, N, P>& tile, const Twidd
 #pragma unroll
     for (int n2 = 0; n2 < N2; ++n2) {
       const int j = posIn<N>(n1, n2);
-      a[n2] = mkc<T>(Rr[j], Rr[N + j]);
+      if constexpr (PAIR) a[n2] = reg[j];
+      else a[n2] = mkc<T>(Rr[j], Rr[N + j]);
     }
   }
   lineFwdT<T, N, 0>(a, reg, n1, active, w);
@@ -341,6 +349,13 @@ __device__ __forceinline__ C<T> zSplit(const ZTile<T, N, P>& tile, int f, int p,
   return mkc<T>((T)0.5 * (zk.y - zm.y), (T)-0.5 * (zk.x - zm.x));
 }
 
+// The real lines of an operation that declares `pairs` lie in LDS as pairs
+// (line 2c, line 2c + 1) per node: 8-byte FP32 accesses, half as many as with
+// the two lines one after the other, which the one-field operations keep for
+// their 16-byte runs of one line.
+template <class Op, class = void> constexpr bool opPairs = false;
+template <class Op> constexpr bool opPairs<Op, std::void_t<decltype(Op::pairs)>> = Op::pairs;
+
 template <int FIN, int FOUT> struct ZMax { static constexpr int v = FIN > FOUT ? FIN : FOUT; };
 template <int N, int P, int FIN, int FOUT> struct ZThreads {
   static constexpr int v = ZMax<FIN, FOUT>::v * P / 2 * Plan<N>::N1;
@@ -358,8 +373,8 @@ template <typename T> struct alignas(2 * sizeof(C<T>)) C2 { C<T> a, b; };
 // line0 * Nf is even (P and the line offset are even), so every pair is
 // aligned.  Input entries with kz > kcin are zero by the caller's contract
 // (dealiasing truncation: no earlier pass writes them): they are set in LDS,
-// not loaded.  Output pairs whose two entries both have kz > kcout are not
-// written (no later pass reads them).
+// not loaded.  Output entries with kz > kcout are not written (no later pass
+// reads them), but for one at the end of an entry pair.
 template <typename T, int N, int P, int FIN, int FOUT, class Op>
 __global__ void __launch_bounds__((ZThreads<N, P, FIN, FOUT>::v))
 k_z(Op op0, const C<T>* __restrict__ tw, int lineoff, size_t rs, int kcin, int kcout) {
@@ -373,7 +388,6 @@ k_z(Op op0, const C<T>* __restrict__ tw, int lineoff, size_t rs, int kcin, int k
   ZTile<T, N, P> tile{lds};
   const int line0 = lineoff + blockIdx.x * P;
   const size_t g0 = (size_t)line0 * Nf;
-  const int nt = blockDim.x;
   // the thread's line-FFT twiddles (the same n1 in both directions), loaded
   // first so that their latency overlaps the tile loads
   const Twiddles<T, N> w((int)threadIdx.x % Plan<N>::N1, tw);
@@ -383,41 +397,74 @@ k_z(Op op0, const C<T>* __restrict__ tw, int lineoff, size_t rs, int kcin, int k
     // unconditional (a branch around one would wait for it), a pair that is
     // not needed (both kz > kcin, or past the end) reads the block's first
     // pair of the field instead, which other lanes load anyway.
-    constexpr int NT = ZThreads<N, P, FIN, FOUT>::v, NPR = FIN * (NE / 2), IT = (NPR + NT - 1) / NT;
+    // Field, pair and kz of pair e follow from those of pair e - NT by addition
+    // (with the pairs and quotients below, OpZCross 1824 -> 1571 and OpZVel 2073
+    // -> 1701 vector instructions per thread at 256^3 FP32; 211 -> 206 and 164 ->
+    // 163 us there, 24.1 -> 21.9 us for OpZVel at 128^3, 11.9 -> 10.6 at 64^3 FP64).
+    constexpr int NT = ZThreads<N, P, FIN, FOUT>::v, NPF = NE / 2, NPR = FIN * NPF, IT = (NPR + NT - 1) / NT;
     C2<T> x[IT];
+    bool za[IT], zb[IT];                  // the entry is inside kcin
+    int f = (int)threadIdx.x / NPF, v = (int)threadIdx.x % NPF, z = (2 * (int)threadIdx.x) % Nf;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int e0 = (int)threadIdx.x + it * NT;
-      const int e = (NPR % NT == 0 || e0 < NPR) ? e0 : 0;
-      const int f = e / (NE / 2), v = e % (NE / 2);
-      const bool need = (2 * v) % Nf <= kcin || (2 * v + 1) % Nf <= kcin;
-      x[it] = reinterpret_cast<const C2<T>*>(op.specIn(f) + g0)[need ? v : 0];
+      const bool in = (it + 1) * NT <= NPR || (int)threadIdx.x + it * NT < NPR;
+      za[it] = z <= kcin;
+      zb[it] = (z + 1 == Nf ? 0 : z + 1) <= kcin;
+      x[it] = reinterpret_cast<const C2<T>*>(op.specIn(in ? f : 0) + g0)[in && (za[it] || zb[it]) ? v : 0];
+      f += NT / NPF; v += NT % NPF;
+      if (v >= NPF) { v -= NPF; ++f; }
+      z += (2 * NT) % Nf;
+      if (z >= Nf) z -= Nf;
     }
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
       const int e = (int)threadIdx.x + it * NT;
-      if (NPR % NT == 0 || e < NPR) {
-        const int v = e % (NE / 2);
-        if ((2 * v) % Nf > kcin) x[it].a = mkc<T>((T)0, (T)0);
-        if ((2 * v + 1) % Nf > kcin) x[it].b = mkc<T>((T)0, (T)0);
+      if ((it + 1) * NT <= NPR || e < NPR) {
+        if (!za[it]) x[it].a = mkc<T>((T)0, (T)0);
+        if (!zb[it]) x[it].b = mkc<T>((T)0, (T)0);
         lds2[e] = x[it];
       }
     }
     __syncthreads();
-    zInverse<T, N, P, FIN>(tile, w);
+    zInverse<T, N, P, FIN, opPairs<Op>>(tile, w);
   }
   op.physical(tile, line0);
   __syncthreads();
   if constexpr (FOUT > 0) {
-    zForward<T, N, P, FOUT>(tile, w);
-    for (int e = threadIdx.x; e < FOUT * (NE / 2); e += nt) {
-      const int f = e / (NE / 2), q = 2 * (e % (NE / 2));
-      const int za = q % Nf, zb = (q + 1) % Nf;
-      if (za > kcout && zb > kcout) continue;
-      C2<T> v;
-      v.a = zSplit<T, N, P>(tile, f, q / Nf, za);
-      v.b = zSplit<T, N, P>(tile, f, (q + 1) / Nf, zb);
-      reinterpret_cast<C2<T>*>(op.specOut(f) + g0)[q / 2] = v;
+    zForward<T, N, P, FOUT, opPairs<Op>>(tile, w);
+    constexpr int NT = ZThreads<N, P, FIN, FOUT>::v;
+    if constexpr (N >= 128) {
+      // both lines of a pair need the same two entries Z[k], Z[N - k]: a thread
+      // takes entry k of pair r and stores both lines (entries in order over the
+      // block's pairs; the next one follows by addition).  At 128^3 FP32 OpZVel
+      // 23.5 -> 21.9 us, OpZFwdFc 7.8 -> 7.0 us; on 33 entry lines the 8-byte
+      // stores cost more than the arithmetic saved (64 times 64^3: OpZVel 189 ->
+      // 193 us), so shorter lines move entry pairs in one 16-byte store.
+      constexpr int NR = FOUT * (P / 2);
+      const int kmax = kcout < N / 2 ? kcout : N / 2;
+      int r = (int)threadIdx.x / Nf, k = (int)threadIdx.x % Nf;
+      while (r < NR) {
+        if (k <= kmax) {
+          const C<T>* Z = tile.region(r);
+          const C<T> zk = Z[k];
+          const C<T> zm = cconj<T>(Z[(N - k) & (N - 1)]);
+          C<T>* o = op.specOut(r / (P / 2)) + g0 + (uint32_t)((r % (P / 2)) * (2 * Nf) + k);
+          o[0] = mkc<T>((T)0.5 * (zk.x + zm.x), (T)0.5 * (zk.y + zm.y));
+          o[Nf] = mkc<T>((T)0.5 * (zk.y - zm.y), (T)-0.5 * (zk.x - zm.x));   // -i/2 (zk - zm)
+        }
+        r += NT / Nf; k += NT % Nf;
+        if (k >= Nf) { k -= Nf; ++r; }
+      }
+    } else {
+      for (int e = threadIdx.x; e < FOUT * (NE / 2); e += NT) {
+        const int f = e / (NE / 2), q = 2 * (e % (NE / 2));
+        const int za = q % Nf, zb = (q + 1) % Nf;
+        if (za > kcout && zb > kcout) continue;
+        C2<T> v;
+        v.a = zSplit<T, N, P>(tile, f, q / Nf, za);
+        v.b = zSplit<T, N, P>(tile, f, (q + 1) / Nf, zb);
+        reinterpret_cast<C2<T>*>(op.specOut(f) + g0)[q / 2] = v;
+      }
     }
   }
 }
@@ -580,6 +627,7 @@ __device__ __forceinline__ V4<T> ldRec(const V4<T>* base, uint32_t idx) {
 // 3 fields written over inputs 0..2.
 template <typename T, int N, int P>
 struct OpZCross {
+  static constexpr bool pairs = true;
   C<T>* w; size_t fs; T* u; V4<T>* gu; T scale;   // u planar (may be null) and/or gather records (may be null)
   __device__ OpZCross shifted(size_t rs) const {
     OpZCross o = *this; o.w = rsel1(w, rs); o.u = rsel(u, rs); o.gu = rsel(gu, rs); return o;
@@ -588,21 +636,28 @@ struct OpZCross {
   __device__ C<T>* specOut(int f) const { return w + f * fs; }
   __device__ void physical(const ZTile<T, N, P>& t, int line0) const {
     constexpr size_t R = (size_t)N * N * N;
-    // one element per thread and step, so consecutive lanes write
+    // one node of two lines per thread and step, so consecutive lanes write
     // consecutive 16-byte records
-    using Q = Quads<ZThreads<N, P, 6, 3>::v, P * N>;
+    using Q = Quads<ZThreads<N, P, 6, 3>::v, P / 2 * N>;
 #pragma unroll
     for (int it = 0; it < Q::IT; ++it) {
       if (!Q::ok(it)) break;
-      const int e = Q::e(it), p = e / N, j = e % N;
-      const T ux = t.re(0, p, j) * scale, uy = t.re(1, p, j) * scale, uz = t.re(2, p, j) * scale;
-      const T wx = t.re(3, p, j) * scale, wy = t.re(4, p, j) * scale, wz = t.re(5, p, j) * scale;
-      const size_t o = (size_t)(line0 + p) * N + j;
-      if (u) { u[o] = ux; u[R + o] = uy; u[2 * R + o] = uz; }
-      if (gu) { V4<T> q; q.x = ux; q.y = uy; q.z = uz; q.w = (T)0; gu[recU((uint32_t)o)] = q; }
-      t.re(0, p, j) = wz * uy - wy * uz;
-      t.re(1, p, j) = wx * uz - wz * ux;
-      t.re(2, p, j) = wy * ux - wx * uy;
+      const int e = Q::e(it), c = e / N, j = e % N;
+      C<T> q[6];
+#pragma unroll
+      for (int f = 0; f < 6; ++f) q[f] = cscale<T>(t.pair(f, c, j), scale);
+      const size_t o = (size_t)(line0 + 2 * c) * N + j;
+      if (u) {
+#pragma unroll
+        for (int f = 0; f < 3; ++f) { u[f * R + o] = q[f].x; u[f * R + o + N] = q[f].y; }
+      }
+      if (gu) {
+        gu[recU((uint32_t)o)] = V4<T>{q[0].x, q[1].x, q[2].x, (T)0};
+        gu[recU((uint32_t)o + N)] = V4<T>{q[0].y, q[1].y, q[2].y, (T)0};
+      }
+      t.pair(0, c, j) = mkc<T>(q[5].x * q[1].x - q[4].x * q[2].x, q[5].y * q[1].y - q[4].y * q[2].y);
+      t.pair(1, c, j) = mkc<T>(q[3].x * q[2].x - q[5].x * q[0].x, q[3].y * q[2].y - q[5].y * q[0].y);
+      t.pair(2, c, j) = mkc<T>(q[4].x * q[0].x - q[3].x * q[1].x, q[4].y * q[0].y - q[3].y * q[1].y);
     }
   }
 };
@@ -619,11 +674,31 @@ __device__ __forceinline__ T nStage(T x, const double* __restrict__ clip) {
   }
   return x;
 }
+// nStage for many nodes: in FP32 the quotient oldmean / newmean is formed once
+// per thread (the product stays in FP64 until it is rounded) instead of a
+// division per node.
+template <typename T> struct NStage {
+  const double* __restrict__ clip;
+  bool on;
+  double ratio;
+  __device__ __forceinline__ explicit NStage(const double* __restrict__ c) : clip(c), on(c[2] != 0.0), ratio(1.0) {
+    if (sizeof(T) == 4 && on) ratio = c[0] / c[1];
+  }
+  __device__ __forceinline__ T operator()(T x) const {
+    if constexpr (sizeof(T) == 4) {
+      const T y = (T)((x > (T)0 ? (double)x : 0.0) * ratio);
+      return on ? y : x;
+    } else {
+      return nStage<T>(x, clip);
+    }
+  }
+};
 
 // Slow-manifold velocity v to physical space (forced-dns-sm.py:319-321, last
 // pass), v stored, then n*v transformed along z (:326-329, first pass).
 template <typename T, int N, int P>
 struct OpZVel {
+  static constexpr bool pairs = true;
   const C<T>* w; C<T>* wout; size_t fs; T* v; V4<T>* gv; const T* n; const double* clip; T scale; T tpsg;
   __device__ OpZVel shifted(size_t rs) const {
     OpZVel o = *this;
@@ -635,28 +710,38 @@ struct OpZVel {
   __device__ C<T>* specOut(int f) const { return wout + f * fs; }
   __device__ void physical(const ZTile<T, N, P>& t, int line0) const {
     constexpr size_t R = (size_t)N * N * N;
-    // one element per thread and step (consecutive lanes write consecutive
-    // 16-byte records); all loads of n are issued before the first use
-    using Q = Quads<ZThreads<N, P, 3, 3>::v, P * N>;
-    T nq[Q::IT];
+    // one node of two lines per thread and step (consecutive lanes write
+    // consecutive 16-byte records); all loads of n are issued before the first use
+    using Q = Quads<ZThreads<N, P, 3, 3>::v, P / 2 * N>;
+    T nq[Q::IT][2];
+    const NStage<T> stage(clip);
 #pragma unroll
     for (int it = 0; it < Q::IT; ++it) {
       if (!Q::ok(it)) break;
-      nq[it] = n[(size_t)line0 * N + Q::e(it)];
+      const size_t o = (size_t)(line0 + 2 * (Q::e(it) / N)) * N + Q::e(it) % N;
+      nq[it][0] = n[o];
+      nq[it][1] = n[o + N];
     }
 #pragma unroll
     for (int it = 0; it < Q::IT; ++it) {
       if (!Q::ok(it)) break;
-      const int e = Q::e(it), p = e / N, j = e % N;
-      const size_t o = (size_t)(line0 + p) * N + j;
-      const T vx = t.re(0, p, j) * scale, vy = t.re(1, p, j) * scale;
-      const T vz = t.re(2, p, j) * scale - tpsg;
-      const T nn = nStage<T>(nq[it], clip);
-      if (v) { v[o] = vx; v[R + o] = vy; v[2 * R + o] = vz; }
-      if (gv) { V4<T> q; q.x = vx; q.y = vy; q.z = vz; q.w = nn; gv[recV((uint32_t)o)] = q; }
-      t.re(0, p, j) = nn * vx;
-      t.re(1, p, j) = nn * vy;
-      t.re(2, p, j) = nn * vz;
+      const int e = Q::e(it), c = e / N, j = e % N;
+      const size_t o = (size_t)(line0 + 2 * c) * N + j;
+      const C<T> vx = cscale<T>(t.pair(0, c, j), scale), vy = cscale<T>(t.pair(1, c, j), scale);
+      C<T> vz = cscale<T>(t.pair(2, c, j), scale);
+      vz = mkc<T>(vz.x - tpsg, vz.y - tpsg);
+      const T na = stage(nq[it][0]), nb = stage(nq[it][1]);
+      if (v) {
+        v[o] = vx.x; v[R + o] = vy.x; v[2 * R + o] = vz.x;
+        v[o + N] = vx.y; v[R + o + N] = vy.y; v[2 * R + o + N] = vz.y;
+      }
+      if (gv) {
+        gv[recV((uint32_t)o)] = V4<T>{vx.x, vy.x, vz.x, na};
+        gv[recV((uint32_t)o + N)] = V4<T>{vx.y, vy.y, vz.y, nb};
+      }
+      t.pair(0, c, j) = mkc<T>(na * vx.x, nb * vx.y);
+      t.pair(1, c, j) = mkc<T>(na * vy.x, nb * vy.y);
+      t.pair(2, c, j) = mkc<T>(na * vz.x, nb * vz.y);
     }
   }
 };
