@@ -283,7 +283,7 @@ struct Engine final : EngineBase {
     const bool wide_ok = (N / nslab) % M2 == 0 && M2 * N1 <= 1024;
     for (int c = 0; c < 3; ++c) {
       if (c == 2 && !wide_ok) { tune_us[2] = 0.0; continue; }
-      my = cand[c];
+      my = myi = cand[c];
       std::vector<float> t;
       for (int r = 0; r < 6; ++r) {
         LD_HIP(hipEventRecord(e0, st));
@@ -300,7 +300,7 @@ struct Engine final : EngineBase {
     int best = 0;
     for (int c = 1; c < 3; ++c)
       if (tune_us[c] > 0.0 && tune_us[c] < tune_us[best]) best = c;
-    my = cand[best];
+    my = myi = cand[best];
     // the other line split at the chosen lines, timed for the record only
     {
       const int keep = ysplit;
@@ -470,6 +470,10 @@ struct Engine final : EngineBase {
   // change the arithmetic.
   static constexpr int MH = M / 2, M2 = 2 * M;
   int my = M;
+  // lines of the inverse passes: 2M at 256^3 FP32 and above (256^3 58.6 -> 55.8
+  // us per pass, four steps 22.40 -> 22.21 ms; 512^3 518 -> 503 us; but 128^3
+  // 10.3 -> 12.1 us, FP64 15.75 -> 16.25 us, and the forward passes are no faster)
+  int myi = sizeof(T) == 4 && N >= 256 ? M2 : M;
   // ysplit = 1 (LD_YSPLIT=1): y passes split each line N = (N1/2) (2 N2)
   // instead of N1 N2.  Another factorisation rounds differently, so this is
   // a measurement switch, not an autotuner choice (the autotuner only chooses
@@ -485,6 +489,7 @@ struct Engine final : EngineBase {
     const int qoff = AXIS == 1 ? x0 * lw : 0, qend = AXIS == 1 ? (x0 + nx) * lw : 0;
     const int nl = nx * lw;
     LD_TRY(prof_mark(kid, s));
+    const int my = DIR < 0 ? this->my : myi == M2 && (N / nslab) % M2 ? M : myi;
     if (AXIS == 1 && ysplit) {
       if (my == MH)
         hipLaunchKernelGGL((k_pass<T, N, MH, AXIS, DIR, NQ>), dim3((nl + MH - 1) / MH, nf, B), dim3(MH * NQ), 0, s,
