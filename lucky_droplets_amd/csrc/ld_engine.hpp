@@ -906,35 +906,38 @@ struct Engine final : EngineBase {
     if (n_ > cap) { set_error("%lld droplets exceed the context capacity %lld", (long long)n_, (long long)cap); return LD_ERR_CAPACITY; }
     np = n_;
     if (np > 0) {
-      for (int b = 0; b < B; ++b) {
-        hipLaunchKernelGGL((k_rows_to_soa<PT>), dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st,
-                           coord + (size_t)b * np * 7, (int)np, (int)cap, at(x0, b), at(v0, b));
-        LD_LAUNCHED();
-        hipLaunchKernelGGL(k_iota64, dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st, at(rid, b), (int)np);
-        LD_LAUNCHED();
-      }
+      hipLaunchKernelGGL((k_rows_to_soa<PT>), dim3((unsigned)((np + 255) / 256), 1, B), dim3(256), 0, st, coord, (int)np,
+                         (int)cap, x0, v0, rid, rs);
+      LD_LAUNCHED();
     }
     return LD_OK;
   }
   int get_rows(double* coord) {
     if (np > 0) {
-      for (int b = 0; b < B; ++b) {
-        hipLaunchKernelGGL((k_soa_to_rows<PT>), dim3((unsigned)((np + 255) / 256)), dim3(256), 0, st,
-                           (const double*)at(x0, b), (const PT*)at(v0, b), (const int64_t*)at(rid, b), (int)np,
-                           (int)cap, coord + (size_t)b * np * 7);
-        LD_LAUNCHED();
-      }
+      hipLaunchKernelGGL((k_soa_to_rows<PT>), dim3((unsigned)((np + 255) / 256), 1, B), dim3(256), 0, st,
+                         (const double*)x0, (const PT*)v0, (const int64_t*)rid, (int)np, (int)cap, coord, rs);
+      LD_LAUNCHED();
     }
+    return LD_OK;
+  }
+  // Copy `bytes` of every realization, ss and ds bytes apart (all multiples of
+  // 16: field arrays are 32-byte aligned, the realizations' slabs 256-byte).
+  int copy_fields(void* dst, size_t ds, const void* src, size_t ss, size_t bytes) {
+    if (B == 1) {
+      LD_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, st));
+      return LD_OK;
+    }
+    const size_t n = bytes / sizeof(uint4), nb = (n + 255) / 256;
+    hipLaunchKernelGGL(k_copy_fields, dim3(nb < 1024 ? (unsigned)nb : 1024u, 1, B), dim3(256), 0, st,
+                       (const char*)src, ss, (char*)dst, ds, n);
+    LD_LAUNCHED();
     return LD_OK;
   }
   // uk, n and coord hold B realizations back to back.
   int state_set(const void* ukin, const void* nin, const double* coord, int64_t n_) override {
     LD_TRY(join(st, st2, evB));
-    for (int b = 0; b < B; ++b) {
-      LD_HIP(hipMemcpyAsync(at(uk, b), (const C<T>*)ukin + (size_t)b * 3 * CF, 3 * CF * sizeof(C<T>),
-                            hipMemcpyDeviceToDevice, st));
-      LD_HIP(hipMemcpyAsync(at(n_state, b), (const T*)nin + (size_t)b * RF, RF * sizeof(T), hipMemcpyDeviceToDevice, st));
-    }
+    LD_TRY(copy_fields(uk, rs, ukin, 3 * CF * sizeof(C<T>), 3 * CF * sizeof(C<T>)));
+    LD_TRY(copy_fields(n_state, rs, nin, RF * sizeof(T), RF * sizeof(T)));
     LD_TRY(check_band());
     return set_rows(coord, n_);
   }
@@ -945,11 +948,9 @@ struct Engine final : EngineBase {
     if (kc >= N / 2) return LD_OK;
     hipLaunchKernelGGL((k_fill<int>), dim3(1), dim3(256), 0, st, bandflag, (size_t)1, 0, (size_t)0);
     LD_LAUNCHED();
-    for (int b = 0; b < B; ++b) {
-      hipLaunchKernelGGL((k_band_check<T, N>), dim3(1024), dim3(256), 0, st, (const C<T>*)at(uk, b),
-                         (size_t)3 * CF, sphere(), bandflag);
-      LD_LAUNCHED();
-    }
+    hipLaunchKernelGGL((k_band_check<T, N>), dim3(1024, 1, B), dim3(256), 0, st, (const C<T>*)uk, (size_t)3 * CF,
+                       sphere(), bandflag, rs);
+    LD_LAUNCHED();
     int h = 1;
     LD_HIP(hipMemcpyAsync(&h, bandflag, sizeof(int), hipMemcpyDeviceToHost, st));
     LD_HIP(hipStreamSynchronize(st));
@@ -965,13 +966,8 @@ struct Engine final : EngineBase {
   }
   int state_get(void* ukout, void* nout, double* coord) override {
     LD_TRY(join(st, st2, evB));
-    for (int b = 0; b < B; ++b) {
-      if (ukout)
-        LD_HIP(hipMemcpyAsync((C<T>*)ukout + (size_t)b * 3 * CF, at(uk, b), 3 * CF * sizeof(C<T>),
-                              hipMemcpyDeviceToDevice, st));
-      if (nout)
-        LD_HIP(hipMemcpyAsync((T*)nout + (size_t)b * RF, at(n_state, b), RF * sizeof(T), hipMemcpyDeviceToDevice, st));
-    }
+    if (ukout) LD_TRY(copy_fields(ukout, 3 * CF * sizeof(C<T>), uk, rs, 3 * CF * sizeof(C<T>)));
+    if (nout) LD_TRY(copy_fields(nout, RF * sizeof(T), n_state, rs, RF * sizeof(T)));
     if (coord) LD_TRY(get_rows(coord));
     return LD_OK;
   }

@@ -966,7 +966,8 @@ k_x_uw(const C<T>* __restrict__ uk0, C<T>* __restrict__ out0, size_t fs, const C
 // = kc (kc + 1) those are the modes outside the dealiasing mask, and a state
 // without them keeps none through the RK4 stages and the step epilogue.
 template <typename T, int N>
-__global__ void __launch_bounds__(256) k_band_check(const C<T>* __restrict__ u, size_t n, int r2, int* flag) {
+__global__ void __launch_bounds__(256) k_band_check(const C<T>* __restrict__ u0, size_t n, int r2, int* flag, size_t rs) {
+  const C<T>* __restrict__ u = rsel1(u0, rs);
   constexpr int Nf = N / 2 + 1;
   bool any = false;
   for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n; e += (size_t)gridDim.x * 256) {
