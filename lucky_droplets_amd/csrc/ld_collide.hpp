@@ -237,15 +237,19 @@ __global__ void __launch_bounds__(256) k_near(NearArgs A) {
 // else it finishes the merges of length k.  k_bitonic does one step across
 // chunks.  116 pairs of 10^6 droplets: 28 launches of one step each before,
 // one now, which also writes the pairs (`pairs` set: n <= 2048).
+// Key numbers and merge lengths are 64-bit: 2^29 + 1 pairs (33000 droplets that
+// all overlap) already sort 2^30 keys, whose last doubling of an int overflows.
 constexpr int SORT_CHUNK = 2048;
 static __global__ void __launch_bounds__(1024)
-k_bitonic_block(unsigned long long* __restrict__ a, int cnt, int n, int k, int64_t* __restrict__ pairs) {
+k_bitonic_block(unsigned long long* __restrict__ a, int64_t cnt, int64_t n, int64_t k, int64_t* __restrict__ pairs) {
   __shared__ unsigned long long sh[SORT_CHUNK];
-  const int base = blockIdx.x * SORT_CHUNK, len = n < SORT_CHUNK ? n : SORT_CHUNK;
+  const int64_t base = (int64_t)blockIdx.x * SORT_CHUNK;
+  const int len = n < SORT_CHUNK ? (int)n : SORT_CHUNK;
   for (int i = threadIdx.x; i < len; i += 1024) sh[i] = base + i < cnt ? a[base + i] : ~0ull;
   __syncthreads();
-  for (int kk = k ? k : 2; kk <= (k ? k : len); kk <<= 1)
-    for (int j = kk / 2 < len / 2 ? kk / 2 : len / 2; j > 0; j >>= 1) {
+  // the steps of merges of length kk from partner distance j down
+  auto merge = [&](int64_t kk, int j) {
+    for (; j > 0; j >>= 1) {
       for (int p = threadIdx.x; p < len / 2; p += 1024) {
         const int i = 2 * p - (p & (j - 1));        // the pair's lower key: bit j clear
         const bool up = ((base + i) & kk) == 0;
@@ -254,6 +258,10 @@ k_bitonic_block(unsigned long long* __restrict__ a, int cnt, int n, int k, int64
       }
       __syncthreads();
     }
+  };
+  if (k) merge(k, len / 2);
+  else
+    for (int kk = 2; kk <= len; kk <<= 1) merge(kk, kk / 2);
   if (pairs) {
     for (int i = threadIdx.x; i < cnt; i += 1024) {
       pairs[2 * i] = (int64_t)(sh[i] >> 32);
@@ -264,10 +272,10 @@ k_bitonic_block(unsigned long long* __restrict__ a, int cnt, int n, int k, int64
   }
 }
 static __global__ void __launch_bounds__(256)
-k_bitonic(unsigned long long* __restrict__ a, int n, int j, int k) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+k_bitonic(unsigned long long* __restrict__ a, int64_t n, int64_t j, int64_t k) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= n) return;
-  const int ixj = i ^ j;
+  const int64_t ixj = i ^ j;
   if (ixj > i) {
     const bool up = (i & k) == 0;
     const unsigned long long x = a[i], y = a[ixj];
@@ -275,8 +283,9 @@ k_bitonic(unsigned long long* __restrict__ a, int n, int j, int k) {
   }
 }
 
-static __global__ void k_pairs_out(const unsigned long long* __restrict__ keys, int n, int64_t* __restrict__ pairs) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+static __global__ void __launch_bounds__(256)
+k_pairs_out(const unsigned long long* __restrict__ keys, int64_t n, int64_t* __restrict__ pairs) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (t >= n) return;
   pairs[2 * t] = (int64_t)(keys[t] >> 32);
   pairs[2 * t + 1] = (int64_t)(keys[t] & 0xffffffffull);

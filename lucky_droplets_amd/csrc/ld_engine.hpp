@@ -1509,23 +1509,23 @@ struct Engine final : EngineBase {
       return LD_ERR_CAPACITY;
     }
     if (cnt == 0) return LD_OK;
-    const int n2 = (int)pow2ceil((int64_t)cnt);
+    const int64_t n2 = pow2ceil((int64_t)cnt);
     const bool one = n2 <= SORT_CHUNK;
     const unsigned chunks = one ? 1u : (unsigned)(n2 / SORT_CHUNK);
-    hipLaunchKernelGGL(k_bitonic_block, dim3(chunks), dim3(1024), 0, st, ckeys, (int)cnt, n2, 0,
+    hipLaunchKernelGGL(k_bitonic_block, dim3(chunks), dim3(1024), 0, st, ckeys, (int64_t)cnt, n2, (int64_t)0,
                        one ? pairs : (int64_t*)nullptr);
     LD_LAUNCHED();
     if (one) return LD_OK;
     for (int64_t k = 2 * SORT_CHUNK; k <= n2; k <<= 1) {
       for (int64_t j = k >> 1; j >= SORT_CHUNK; j >>= 1) {
-        hipLaunchKernelGGL(k_bitonic, dim3((n2 + 255) / 256), dim3(256), 0, st, ckeys, n2, (int)j, (int)k);
+        hipLaunchKernelGGL(k_bitonic, dim3((unsigned)((n2 + 255) / 256)), dim3(256), 0, st, ckeys, n2, j, k);
         LD_LAUNCHED();
       }
-      hipLaunchKernelGGL(k_bitonic_block, dim3(chunks), dim3(1024), 0, st, ckeys, n2, n2, (int)k, (int64_t*)nullptr);
+      hipLaunchKernelGGL(k_bitonic_block, dim3(chunks), dim3(1024), 0, st, ckeys, n2, n2, k, (int64_t*)nullptr);
       LD_LAUNCHED();
     }
     hipLaunchKernelGGL(k_pairs_out, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, st,
-                       (const unsigned long long*)ckeys, (int)cnt, pairs);
+                       (const unsigned long long*)ckeys, (int64_t)cnt, pairs);
     LD_LAUNCHED();
     return LD_OK;
   }
