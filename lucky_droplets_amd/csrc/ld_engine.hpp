@@ -1568,14 +1568,21 @@ struct Engine final : EngineBase {
   //    200000: the bricks write every node).
   enum RowOp { ROW_PRHS, ROW_INTERP, ROW_EXTERP };
   int64_t api_sort_min = -1;         // >= 0: the line for every call (LD_ROW_SORT_MIN)
-  bool rows_sorted(RowOp op, int64_t n_, int nc = 1) const {
-    if (n_ > cap || n_ > 2 * (int64_t)RF) return false;
+  bool rows_rule(RowOp op, int64_t n_, int nc) const {
+    if (n_ < 1 || n_ > cap || n_ > 2 * (int64_t)RF) return false;
     if (api_sort_min >= 0) return n_ >= api_sort_min;
     const bool small = 7 * RF * sizeof(T) <= (size_t)4 << 20;
     if (op == ROW_PRHS) return !small || n_ >= 12288;
     if (small) return false;
     if (op == ROW_INTERP) return (nc >= 4 && n_ >= 1024) || n_ * nc >= 131072;
     return n_ >= 16384 && n_ >= (int64_t)(RF / 2048);
+  }
+  int rows_sorted(RowOp op, int64_t n_, int nc, bool& yes) {
+    bool cap_ = false;
+    yes = rows_rule(op, n_, nc);
+    if (yes) LD_TRY(capturing(cap_));
+    yes = yes && !cap_;
+    return LD_OK;
   }
   int sort_rows(const double* coord, int64_t n_, const double* w) {
     LD_TRY(rows_begin());
@@ -1617,7 +1624,9 @@ struct Engine final : EngineBase {
   // Droplet right-hand side of rows in any order; fcp receives the deposit.
   int prhs_rows(const double* coord, int64_t n_, const T* uf, const T* usf, const T* nf, T* fcp, double* rhs,
                 double* interpm, double* exterpm) {
-    if (n_ > 0 && rows_sorted(ROW_PRHS, n_)) {
+    bool sorted = false;
+    LD_TRY(rows_sorted(ROW_PRHS, n_, 7, sorted));
+    if (sorted) {
       LD_TRY(sort_rows(coord, n_, nullptr));
       if (rows_tiled(n_, 48)) {
         GatherFields<T> g{uf, usf, nf, 3, 3, 7, nullptr};
@@ -1639,38 +1648,34 @@ struct Engine final : EngineBase {
     LD_LAUNCHED();
     return LD_OK;
   }
-  // The sorted path's scratch belongs to the context: a call on another stream
-  // than the last one waits for it (the one-thread-per-row kernels share
-  // nothing).  Not under capture, where the caller orders its own replays.
+  // The sorted path's scratch belongs to the context (the one-thread-per-row
+  // kernels share nothing): a call that uses it waits for the last one that
+  // did, whatever their streams (nothing to wait for on the same stream), and
+  // so does a step.  A stream under capture takes the one-thread-per-row
+  // kernels: nothing here could order its replays with other users of the scratch.
   hipEvent_t evR = nullptr;
-  hipStream_t rows_stream = nullptr;
   bool rows_used = false;
   int capturing(bool& yes) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    LD_HIP(hipStreamIsCapturing(st, &cs));
+    if (st) LD_HIP(hipStreamIsCapturing(st, &cs));       // the default stream cannot be captured
     yes = cs != hipStreamCaptureStatusNone;
     return LD_OK;
   }
   int rows_begin() {
-    if (!rows_used || rows_stream == st) return LD_OK;
-    bool cap_ = false;
-    LD_TRY(capturing(cap_));
-    if (!cap_) LD_HIP(hipStreamWaitEvent(st, evR, 0));
+    if (rows_used) LD_HIP(hipStreamWaitEvent(st, evR, 0));
     return LD_OK;
   }
   int rows_end() {
-    bool cap_ = false;
-    LD_TRY(capturing(cap_));
-    if (cap_) return LD_OK;
     LD_HIP(hipEventRecord(evR, st));
-    rows_stream = st;
     rows_used = true;
     return LD_OK;
   }
   int interp(const double* coord, int64_t n_, const void* f, int nc, double* out) override {
     if (n_ <= 0) return LD_OK;
     LD_TRY(join(st, st2, evB));
-    if (rows_sorted(ROW_INTERP, n_, nc)) {
+    bool sorted = false;
+    LD_TRY(rows_sorted(ROW_INTERP, n_, nc, sorted));
+    if (sorted) {
       LD_TRY(sort_rows(coord, n_, nullptr));
       if (rows_tiled(n_, 96) && nc <= 64) {
         GatherFields<T> g{(const T*)f, nullptr, nullptr, nc, 0, nc, nullptr};
@@ -1689,7 +1694,9 @@ struct Engine final : EngineBase {
   }
   int exterp(const double* coord, int64_t n_, const double* w, void* c) override {
     LD_TRY(join(st, st2, evB));
-    if (n_ > 0 && rows_sorted(ROW_EXTERP, n_)) {
+    bool sorted = false;
+    LD_TRY(rows_sorted(ROW_EXTERP, n_, 1, sorted));
+    if (sorted) {
       LD_TRY(sort_rows(coord, n_, w));
       LD_TRY(deposit_rows(n_, (T*)c));
       return rows_end();
