@@ -812,7 +812,8 @@ struct Engine final : EngineBase {
     // v, nv need the previous density chain done (n_s, clip, wn and v free)
     return velocity(st, nullptr, gup, ns, clip_stage, evB);
   }
-  int stage_d(int s, double h) {
+  // wide: the deposit's sums keep a 2^62 range in FP32 contexts too (RK4 on a caller's rows)
+  int stage_d(int s, double h, bool wide) {
     V4<T>* gup = grec[s & 1];
     const double wh = (s == 0 || s == 3) ? h / 6.0 : h / 3.0;
     const double anext = a_coef[s + 1] * h;
@@ -841,9 +842,13 @@ struct Engine final : EngineBase {
       LD_LAUNCHED();
       LD_TRY(prof_mark(LD_K_DROPLETS, st2));
       LD_TRY(prof_mark(LD_K_DEPOSIT, st2));
-      hipLaunchKernelGGL((k_brick_deposit<T, N>), dim3(NBRICK + FB_BLOCKS, 1, B), dim3(Brick<N>::NT), 0, st2,
-                         (const double4*)dep, (const int*)hist, (int)np, (const unsigned long long*)wmaxp, fc, dp, rs,
-                         (const int*)flist, (const int*)fcount, fx);
+      auto bricks = [&](auto mode) {
+        hipLaunchKernelGGL((k_brick_deposit<T, N, decltype(mode)::value>), dim3(NBRICK + FB_BLOCKS, 1, B),
+                           dim3(Brick<N>::NT), 0, st2, (const double4*)dep, (const int*)hist, (int)np,
+                           (const unsigned long long*)wmaxp, fc, dp, rs, (const int*)flist, (const int*)fcount, fx);
+      };
+      if (wide && sizeof(T) == 4) bricks(std::integral_constant<int, sizeof(T) == 4 ? DEP_WIDE : DEP_STEP>{});
+      else bricks(std::integral_constant<int, DEP_STEP>{});
       LD_LAUNCHED();
       LD_TRY(prof_mark(LD_K_DEPOSIT, st2));
     }
@@ -871,15 +876,15 @@ struct Engine final : EngineBase {
   }
 
   // RK4 over the context state: acc <- uknew, nacc <- nnew, droplet base <- sump.
-  int rk4_stages(double h) {
+  int rk4_stages(double h, bool wide = false) {
     LD_TRY(begin_rk4());
     for (int s = 0; s < 4; ++s) {
       LD_TRY(stage_a(s));
-      if (late_density && s > 0) LD_TRY(stage_d(s - 1, h));
+      if (late_density && s > 0) LD_TRY(stage_d(s - 1, h, wide));
       LD_TRY(stage_b(s, h));
-      if (!late_density) LD_TRY(stage_d(s, h));
+      if (!late_density) LD_TRY(stage_d(s, h, wide));
     }
-    if (late_density) LD_TRY(stage_d(3, h));
+    if (late_density) LD_TRY(stage_d(3, h, wide));
     return LD_OK;
   }
 
@@ -1126,7 +1131,7 @@ struct Engine final : EngineBase {
     // global integer atomics for every row (one RK4 at 128^3 FP32 with 123457
     // rows: 4.19 -> 1.18 ms; at 32^3 FP64 with 100 rows 0.70 -> 0.56 ms)
     LD_TRY(sort_droplets(st2));
-    LD_TRY(rk4_stages(h));
+    LD_TRY(rk4_stages(h, true));
     LD_TRY(join(st, st2, evB));
     LD_HIP(hipMemcpyAsync(uknew, acc, 3 * CF * sizeof(C<T>), hipMemcpyDeviceToDevice, st));
     LD_HIP(hipMemcpyAsync(nnew, nacc, RF * sizeof(T), hipMemcpyDeviceToDevice, st));
@@ -1615,7 +1620,7 @@ struct Engine final : EngineBase {
   static unsigned quad_blocks(int64_t n_) { return (unsigned)(((4 * n_ + 255) / 256 + 7) / 8 * 8); }
   // FP64 brick deposit of the sorted rows' weights; writes every node of c
   int deposit_rows(int64_t n_, T* c) {
-    hipLaunchKernelGGL((k_brick_deposit<T, N, false>), dim3(NBRICK), dim3(Brick<N>::NT), 0, st, (const double4*)dep,
+    hipLaunchKernelGGL((k_brick_deposit<T, N, DEP_ROWS>), dim3(NBRICK), dim3(Brick<N>::NT), 0, st, (const double4*)dep,
                        (const int*)hist, (int)n_, (const unsigned long long*)nullptr, c, dp, (size_t)0,
                        (const int*)nullptr, (const int*)nullptr, (unsigned long long*)nullptr);
     LD_LAUNCHED();

@@ -657,11 +657,14 @@ template <int N> struct Brick {
 };
 
 //
-// FIX = false (the API's deposits, whose weights may be negative, of any
-// range or not finite): the tile is FP64 and added to in FP64 (ds_add_f64, 27
-// against 15 cycles), every candidate with W != 0 deposits, and the stencil
-// weights are FP64 as the API's are.
-template <typename T, int N, bool FIX = true>
+// MODE: DEP_STEP sums growth rates in 64-bit fixed point; DEP_WIDE (RK4 on a
+// caller's rows) the same with a 2^62 range in FP32 contexts too, as that call's
+// fallback deposit has it.  DEP_ROWS (the API's deposits, whose weights may be
+// negative, of any range or not finite): the tile is FP64 and added to in FP64
+// (ds_add_f64, 27 against 15 cycles), every candidate with W != 0 deposits, and
+// the stencil weights are FP64 as the API's are.
+enum { DEP_STEP, DEP_WIDE, DEP_ROWS };
+template <typename T, int N, int MODE = DEP_STEP>
 __global__ void __launch_bounds__(Brick<N>::NT)
 k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0, int np,
                 const unsigned long long* __restrict__ wmax0, T* __restrict__ fc0, DropPhys P, size_t rs,
@@ -670,6 +673,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   const int* __restrict__ start = rsel1(start0, rs);
   const unsigned long long* __restrict__ wmax = rsel1(wmax0, rs);
   T* __restrict__ fc = rsel1(fc0, rs);
+  constexpr bool FIX = MODE != DEP_ROWS;
   constexpr int NBRICK = Brick<N>::NB * Brick<N>::NB * Brick<N>::NB;
   if constexpr (FIX) {
     if (blockIdx.x >= NBRICK) {          // the extra blocks: fallback slots
@@ -759,10 +763,10 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   const double dx = P.dx, pi_2dx = P.pi_2dx, inv_dx = P.inv_dx;
   const double bound = FIX ? (double)total * __longlong_as_double((long long)wtop) * P.inv_vol * 0.125 : 0.0;
   const bool finite = isfinite(bound);
-  // FP32 fields: sums below 2^52, so a value converts to its integer by one
-  // addition of 2^52 (round to nearest even, as llrint); FP64 fields keep the
-  // 2^62 range and llrint
-  constexpr bool F32 = sizeof(T) == 4;
+  // FP32 steps: sums below 2^52, so a value converts to its integer by one
+  // addition of 2^52 (round to nearest even, as llrint); FP64 fields and
+  // DEP_WIDE keep the 2^62 range and llrint
+  constexpr bool F32 = sizeof(T) == 4 && MODE == DEP_STEP;
   constexpr int EMAX = F32 ? 51 : 61;
   const int e = (bound > 0.0 && finite) ? EMAX - ilogb(bound) : 0;
   const double scale = ldexp(1.0, e), unit = ldexp(1.0, -e);
