@@ -34,6 +34,25 @@ k_coll_count(const double* __restrict__ rows, int np, double L, double cell, int
   rank[p] = atomicAdd(&hist[k], 1);
 }
 
+// *same += the pairs of droplets that share a cell, sum of c (c - 1) / 2 over the
+// counts: 16384 cells and one atomic (some 12 ns at one address) per block.
+static __global__ void __launch_bounds__(256)
+k_coll_same(const int* __restrict__ count, int ncells, unsigned long long* __restrict__ same) {
+  __shared__ unsigned long long sh[4];
+  unsigned long long s = 0;
+#pragma unroll 16
+  for (int k = 0; k < 64; ++k) {
+    const int i = (blockIdx.x * 64 + k) * 256 + threadIdx.x;
+    const unsigned long long c = i < ncells ? (unsigned long long)count[i] : 0ull;
+    s += c ? c * (c - 1) / 2 : 0ull;
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(same, sh[0] + sh[1] + sh[2] + sh[3]);
+}
+
 // Droplets in cell order: wrapped position and radius, input row, and (for the
 // statistics) velocity, so the pair search reads 32-byte records that its
 // neighbours read too instead of 56-byte rows through an index.
@@ -107,6 +126,8 @@ struct NearArgs {
   int nbins;
   unsigned long long* counts;
   double *wsum, *wneg;
+  const unsigned long long* same;      // set: nothing is done when *same > many (the caller searches finer cells)
+  unsigned long long many;
 };
 template <bool STATS> struct NearHist { unsigned long long c[512]; double w[512], n[512]; };
 template <> struct NearHist<false> {};
@@ -115,6 +136,7 @@ __global__ void __launch_bounds__(256) k_near(NearArgs A) {
 #pragma clang fp contract(off)
   __shared__ NearHist<STATS> H;
   __shared__ int2 queue[4][128];
+  if (A.same && *A.same > A.many) return;
   if constexpr (STATS) {
     for (int k = threadIdx.x; k < A.nbins; k += 256) { H.c[k] = 0ull; H.w[k] = 0.0; H.n[k] = 0.0; }
     __syncthreads();
