@@ -1407,7 +1407,7 @@ struct Engine final : EngineBase {
   unsigned long long *ckeys = nullptr, *ccount = nullptr;   // ccount: pairs found, pairs of droplets in one cell
   unsigned long long* hcount = nullptr;                      // pinned host copy
   int *cnev = nullptr;
-  int64_t ccap = 0, ckcap = 0;
+  int64_t ccap = 0, cvcap = 0, ckcap = 0;
   int chist_cap = 0;
 
   int coll_counters() {
@@ -1423,15 +1423,33 @@ struct Engine final : EngineBase {
   }
   static int64_t pow2ceil(int64_t x) { int64_t v = 2; while (v < x) v <<= 1; return v; }
 
-  // Workspaces grow by at least half, so what earlier sizes leave behind (until
-  // the context goes) stays below twice the largest.
+  // Workspaces grow at least twofold, so what earlier sizes leave behind (until
+  // the context goes: a captured call may still use it) is less than what the
+  // last one takes, and that less than twice what is needed.
   int coll_reserve(int64_t n_) {
     if (n_ <= ccap) return LD_OK;
-    const int64_t n2 = n_ > ccap + ccap / 2 ? n_ : ccap + ccap / 2;
+    const int64_t n2 = n_ > 2 * ccap ? n_ : 2 * ccap;
     ccap = 0;
     LD_TRY(alloc(ckey, n2)); LD_TRY(alloc(crank, n2)); LD_TRY(alloc(corder, n2)); LD_TRY(alloc(cused, n2));
-    LD_TRY(alloc(cpos, n2)); LD_TRY(alloc(cvel, n2));
+    LD_TRY(alloc(cpos, n2));
     ccap = n2;
+    return LD_OK;
+  }
+  int coll_reserve_vel(int64_t n_) {            // the statistics' velocities
+    if (n_ <= cvcap) return LD_OK;
+    const int64_t n2 = n_ > 2 * cvcap ? n_ : 2 * cvcap;
+    cvcap = 0;
+    LD_TRY(alloc(cvel, n2));
+    cvcap = n2;
+    return LD_OK;
+  }
+  int coll_reserve_cells(int ncells) {          // at most 256^3
+    if (ncells <= chist_cap) return LD_OK;
+    int n2 = ncells > 2 * chist_cap ? ncells : 2 * chist_cap;
+    if (n2 > 256 * 256 * 256) n2 = 256 * 256 * 256;
+    chist_cap = 0;
+    LD_TRY(alloc(chist, n2)); LD_TRY(alloc(cbsum, (n2 + 4095) / 4096));
+    chist_cap = n2;
     return LD_OK;
   }
 
@@ -1462,10 +1480,8 @@ struct Engine final : EngineBase {
     const double cell = p.L / nc;
     const int ncells = nc * nc * nc;
     LD_TRY(coll_reserve(n_));
-    if (ncells > chist_cap) {
-      LD_TRY(alloc(chist, ncells)); LD_TRY(alloc(cbsum, (ncells + 4095) / 4096));
-      chist_cap = ncells;
-    }
+    if (with_vel) LD_TRY(coll_reserve_vel(n_));
+    LD_TRY(coll_reserve_cells(ncells));
     const unsigned pb = (unsigned)((n_ + 255) / 256);
     LD_TRY(fill<int>(st, chist, ncells, 0));
     hipLaunchKernelGGL(k_coll_count, dim3(pb), dim3(256), 0, st, rows, (int)n_, p.L, cell, nc, ckey, crank, chist);
