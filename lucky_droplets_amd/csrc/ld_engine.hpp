@@ -1667,7 +1667,7 @@ struct Engine final : EngineBase {
     LD_LAUNCHED();
     return LD_OK;
   }
-  static constexpr int NTILE = GatherTile<N, 0>::NTILE;
+  static constexpr int NTILE = GatherTile<N>::NTILE;
   // Tile gather from this many rows (us per call, tiles / four lanes per row):
   // pRHS from 48 rows per tile (256^3 FP32: 281 / 284 at 24, 359 / 561 at 96;
   // FP64 489 / 500 at 48; 128^3 FP64 96 / 96 at 48, 106 / 162 at 200), interp
@@ -1678,8 +1678,8 @@ struct Engine final : EngineBase {
     return tile_rows_min >= 0 ? n_ >= tile_rows_min : NTILE >= 512 && n_ >= per * (int64_t)NTILE;
   }
   int tile_gather_rows(const GatherFields<T>& g, int64_t n_, const int* rowmap, double* out) {
-    hipLaunchKernelGGL((k_tile_gather<T, double, N, 0, 256>), dim3(NTILE * g.n), dim3(256), 0, st, g, (const double4*)dep,
-                       (const int*)hist, (int)n_, (int)cap, rowmap, out, dp, (size_t)0);
+    hipLaunchKernelGGL((k_tile_gather<T, N>), dim3(NTILE * g.n), dim3(GatherTile<N>::NT), 0, st, g, (const double4*)dep,
+                       (const int*)hist, (int)n_, (int)cap, rowmap, out, dp);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -1700,7 +1700,7 @@ struct Engine final : EngineBase {
     if (sorted) {
       LD_TRY(sort_rows(coord, n_, nullptr));
       if (rows_tiled(n_, 48)) {
-        GatherFields<T> g{uf, usf, nf, 3, 3, 7, nullptr};
+        GatherFields<T> g{uf, usf, nf, 3, 3, 7};
         LD_TRY(tile_gather_rows(g, n_, nullptr, rows_b));
         hipLaunchKernelGGL(k_prhs_finish, dim3((unsigned)((n_ + 255) / 256)), dim3(256), 0, st, coord, (int)n_, (int)cap,
                            (const double*)rows_b, dep, (const int*)flist, rhs, interpm, exterpm, dp);
@@ -1749,7 +1749,7 @@ struct Engine final : EngineBase {
     if (sorted) {
       LD_TRY(sort_rows(coord, n_, nullptr));
       if (rows_tiled(n_, 96) && nc <= 64) {
-        GatherFields<T> g{(const T*)f, nullptr, nullptr, nc, 0, nc, nullptr};
+        GatherFields<T> g{(const T*)f, nullptr, nullptr, nc, 0, nc};
         LD_TRY(tile_gather_rows(g, n_, flist, out));
       } else {
         hipLaunchKernelGGL((k_interp_sorted<T, N>), dim3(quad_blocks(n_)), dim3(256), 0, st, (int)n_, (const T*)f, nc,

@@ -4,7 +4,9 @@
 //
 // Engine state is structure-of-arrays: positions in FP64 (pos[c*cap + p],
 // unwrapped, as the reference accumulates them), velocity and mass in PT
-// (vm[c*cap + p], c = vx, vy, vz, m/M0).  One thread per droplet.
+// (vm[c*cap + p], c = vx, vy, vz, m/M0).  The step's stage kernel takes 4 or 8
+// lanes per droplet, the gathers of sorted rows four lanes or one thread per
+// row, the rest one thread per row.
 #pragma once
 #include "ld_kernels.hpp"
 #include <type_traits>
@@ -58,20 +60,6 @@ __device__ __forceinline__ void sincosStencil(double x, int i0, double dx, doubl
   else sincospi((x - (double)i0 * dx) * (0.5 * inv_dx), &s, &c);
 }
 
-// cosW4 with the sines and cosines taken in precision G (the angle in FP64).
-template <typename G>
-__device__ __forceinline__ int cosW4G(double x, double dx, double pi_2dx, G w[4]) {
-  const int i0 = (int)floor(x / dx) - 1;
-  G sn, cs;
-  sincosGT<G>((x - (double)i0 * dx) * pi_2dx, sn, cs);
-  const G q = (G)0.25;
-  w[0] = q * ((G)1 + cs);
-  w[1] = q * ((G)1 + sn);
-  w[2] = q * ((G)1 - cs);
-  w[3] = q * ((G)1 - sn);
-  return i0;
-}
-
 // Periodic wrap of one coordinate, x mod L with numpy's sign convention
 // (particles.py:269 `x[:, :d] %= L`).
 __device__ __forceinline__ double wrapL(double x, double L) {
@@ -104,7 +92,8 @@ template <int N> __device__ __forceinline__ int cellOf(double xw, double inv_dx)
 // stencil origin i0 = floor(x / dx) - 1 (nodes i0 .. i0 + 3)
 __device__ __forceinline__ int originOf(double x, double inv_dx) { return (int)floor(x * inv_dx) - 1; }
 
-// cosW4G with the origin from originOf.
+// cosW4 with the origin from originOf, the sines and cosines taken in precision G
+// (the angle in FP64).
 template <typename G>
 __device__ __forceinline__ int cosW4F(double x, double dx, double inv_dx, double pi_2dx, G w[4]) {
   const int i0 = originOf(x, inv_dx);
@@ -856,119 +845,96 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
 // ------------------------------------------------------------ tile gather
 // Gather of several planar fields at bin-sorted slots, one field of one bin
 // tile per workgroup: the field's nodes that the stencils of the tile's S^3
-// cells reach, and W cells of motion since the sort on every side, are staged
-// in LDS and one thread per slot sums its 64 nodes from there.
+// cells reach are staged in LDS and one thread per slot sums its 64 nodes from
+// there.
 //
 // A gather straight from global memory reads a 128-byte line of L2 for every
 // 16 (planar FP32) or 64 bytes (node records) of a stencil row, which bounds
-// it; a tile of a field is 35 KB (FP32, W = 0) for all of the tile's slots.
-// One field per workgroup, not all of them in turn: blocks run field by field
-// over groups of 64 neighbouring tiles, so that neighbours read a field's halo
-// while it is in their L2 (seven fields per block: 357 us for 10^6 rows at
-// 256^3 FP32, the same with 256, 384 and 512 threads; 221 us like this, against
-// 737 us for four lanes per row on planar fields, k_prhs_sorted).
+// it; a tile of a field is 35 KB (FP32) for all of the tile's slots.  One field
+// per workgroup, not all of them in turn: blocks run field by field over groups
+// of 64 neighbouring tiles, so that neighbours read a field's halo while it is
+// in their L2 (seven fields per block: 357 us for 10^6 rows at 256^3 FP32, the
+// same with 256, 384 and 512 threads; 222 us like this, against 737 us for four
+// lanes per row on planar fields, k_prhs_sorted).
 template <typename T> struct GatherFields {
   const T *a, *b, *c;          // fields 0 .. na - 1 of a, na .. na + nb - 1 of b (N^3 apart), then c
   int na, nb, n;               // n fields in all
-  const double* clip;          // c is taken as the stage density nStage(c, clip) (null: as it is)
   __device__ __forceinline__ const T* field(int k, size_t R) const {
     return k < na ? a + k * R : k < na + nb ? b + (k - na) * R : c;
   }
 };
-template <int N, int W> struct GatherTile {
+template <int N> struct GatherTile {
   static constexpr int S = Bins<N>::TC;
-  static constexpr int RX = S + 3 + 2 * W;                       // nodes per side in x and y
+  static constexpr int RX = S + 3;                               // nodes per side in x and y
   static constexpr int QZ = S / 4 + 2, PZ = 4 * QZ;              // along z: aligned quads from 4 nodes before
   static constexpr int NQ = RX * RX * QZ;
   static constexpr int TSB = Bins<N>::TS * Bins<N>::TS * Bins<N>::TS, NTILE = Bins<N>::NB / TSB;
   static constexpr int XT = NTILE / 8, GS = XT < 64 ? XT : 64;   // tiles per XCD and per group
-  static_assert(W <= 2 && RX <= N && PZ <= N && NTILE % 8 == 0 && XT % GS == 0, "gather tile");
+  static constexpr int NT = 256;
+  static_assert(RX <= N && PZ <= N && NTILE % 8 == 0 && XT % GS == 0, "gather tile");
 };
-// G: precision of the weights and sums.  rowmap null: out[k cap + slot]; else
-// out[rowmap[slot] n + k].
-template <typename T, typename G, int N, int W, int NT>
-__global__ void __launch_bounds__(NT)
-k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep0, const int* __restrict__ start0, int np, int cap,
-              const int* __restrict__ rowmap, G* __restrict__ out0, DropPhys P, size_t rs) {
-  using GT = GatherTile<N, W>;
-  constexpr int S = GT::S, RX = GT::RX, QZ = GT::QZ, PZ = GT::PZ, NQ = GT::NQ, IT = (NQ + NT - 1) / NT;
+// FP64 weights and sums.  rowmap null: out[k cap + slot]; else out[rowmap[slot] n + k].
+template <typename T, int N>
+__global__ void __launch_bounds__(GatherTile<N>::NT)
+k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep, const int* __restrict__ start, int np, int cap,
+              const int* __restrict__ rowmap, double* __restrict__ out, DropPhys P) {
+  using GT = GatherTile<N>;
+  constexpr int RX = GT::RX, QZ = GT::QZ, PZ = GT::PZ, NQ = GT::NQ, NT = GT::NT, IT = (NQ + NT - 1) / NT;
   constexpr size_t R = (size_t)N * N * N;
   __shared__ __attribute__((aligned(32))) T lds[4 * NQ];
-  const int* __restrict__ start = rsel1(start0, rs);
   const int j = blockIdx.x / 8, r = j % (GT::GS * F.n);
   const int tile = (blockIdx.x % 8) * GT::XT + j / (GT::GS * F.n) * GT::GS + r % GT::GS, k = r / GT::GS;
   const int s0 = start[tile * GT::TSB], s1 = tile + 1 < GT::NTILE ? start[(tile + 1) * GT::TSB] : np;
   if (s0 == s1) return;
-  const double4* __restrict__ dep = rsel1(dep0, rs);
-  G* __restrict__ out = rsel1(out0, rs);
   int cx, cy, cz;
   Bins<N>::tileCell(tile, cx, cy, cz);
-  const T* __restrict__ f = rsel1(F.field(k, R), rs);
-  const bool dens = F.clip && k == F.na + F.nb;
-  const double* __restrict__ clip = dens ? rsel1(F.clip, rs) : nullptr;
+  const T* __restrict__ f = F.field(k, R);
   {
     V4<T> q[IT];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int e0 = (int)threadIdx.x + it * NT, e = (NQ % NT == 0 || e0 < NQ) ? e0 : 0;
+      const int e0 = (int)threadIdx.x + it * NT, e = ((it + 1) * NT <= NQ || e0 < NQ) ? e0 : 0;
       const int z4 = e % QZ, row = e / QZ;
-      const uint32_t x = (uint32_t)(cx - 1 - W + row / RX) & (N - 1), y = (uint32_t)(cy - 1 - W + row % RX) & (N - 1),
+      const uint32_t x = (uint32_t)(cx - 1 + row / RX) & (N - 1), y = (uint32_t)(cy - 1 + row % RX) & (N - 1),
                      z = (uint32_t)(cz - 4 + 4 * z4) & (N - 1);
       q[it] = ld32(reinterpret_cast<const V4<T>*>(f), ((x * N + y) * N + z) / 4);
     }
+    // the writes wait for one load each, in order (mixed with the loads by the
+    // scheduler, 237 instead of 222 us for 10^6 rows at 256^3 FP32)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
       const int e = (int)threadIdx.x + it * NT;
-      if (NQ % NT == 0 || e < NQ) {
-        if (dens) {
-          q[it].x = nStage<T>(q[it].x, clip); q[it].y = nStage<T>(q[it].y, clip);
-          q[it].z = nStage<T>(q[it].z, clip); q[it].w = nStage<T>(q[it].w, clip);
-        }
-        *reinterpret_cast<V4<T>*>(lds + 4 * e) = q[it];
-      }
+      if ((it + 1) * NT <= NQ || e < NQ) *reinterpret_cast<V4<T>*>(lds + 4 * e) = q[it];
     }
   }
   __syncthreads();
   for (int s = s0 + (int)threadIdx.x; s < s1; s += NT) {
     const double4 d = dep[s];
     const int i0 = originOf(d.x, P.inv_dx), j0 = originOf(d.y, P.inv_dx), k0 = originOf(d.z, P.inv_dx);
-    G xs, xc, ys, yc, zs, zc;
-    sincosStencil<G>(d.x, i0, P.dx, P.inv_dx, P.pi_2dx, xs, xc);
-    sincosStencil<G>(d.y, j0, P.dx, P.inv_dx, P.pi_2dx, ys, yc);
-    sincosStencil<G>(d.z, k0, P.dx, P.inv_dx, P.pi_2dx, zs, zc);
-    const G qr = (G)0.25, one = (G)1;
-    const G wx[4] = {qr * (one + xc), qr * (one + xs), qr * (one - xc), qr * (one - xs)};
-    const G wy[4] = {qr * (one + yc), qr * (one + ys), qr * (one - yc), qr * (one - ys)};
-    const G wz[4] = {qr * (one + zc), qr * (one + zs), qr * (one - zc), qr * (one - zs)};
-    const int lx = (i0 - cx + 1 + W) & (N - 1), ly = (j0 - cy + 1 + W) & (N - 1), lz = (k0 - cz + 4) & (N - 1);
-    G sum = (G)0;
-    if (lx <= S - 1 + 2 * W && ly <= S - 1 + 2 * W && lz + 3 < PZ) {
-      const T* o = lds + (lx * RX + ly) * PZ + lz;
+    double xs, xc, ys, yc, zs, zc;
+    sincosStencil<double>(d.x, i0, P.dx, P.inv_dx, P.pi_2dx, xs, xc);
+    sincosStencil<double>(d.y, j0, P.dx, P.inv_dx, P.pi_2dx, ys, yc);
+    sincosStencil<double>(d.z, k0, P.dx, P.inv_dx, P.pi_2dx, zs, zc);
+    const double wx[4] = {0.25 * (1.0 + xc), 0.25 * (1.0 + xs), 0.25 * (1.0 - xc), 0.25 * (1.0 - xs)};
+    const double wy[4] = {0.25 * (1.0 + yc), 0.25 * (1.0 + ys), 0.25 * (1.0 - yc), 0.25 * (1.0 - ys)};
+    const double wz[4] = {0.25 * (1.0 + zc), 0.25 * (1.0 + zs), 0.25 * (1.0 - zc), 0.25 * (1.0 - zs)};
+    // the slot's cell is one of the tile's (k_row_bin takes it from the same
+    // wrapped position), so its stencil starts at 0 .. S - 1 of the staged nodes
+    const T* o = lds + ((i0 - cx + 1) * RX + (j0 - cy + 1)) * PZ + (k0 - cz + 4);
+    double sum = 0.0;
 #pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        // the plane's 16 values are read ahead of their sum
-        T v[16];
+    for (int a = 0; a < 4; ++a) {
+      // the plane's 16 values are read ahead of their sum
+      T v[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = o[(a * RX + (e >> 2)) * PZ + (e & 3)];
-        G sa = (G)0;
+      for (int e = 0; e < 16; ++e) v[e] = o[(a * RX + (e >> 2)) * PZ + (e & 3)];
+      double sa = 0.0;
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-          sa += wy[b] * ((G)v[4 * b] * wz[0] + (G)v[4 * b + 1] * wz[1] + (G)v[4 * b + 2] * wz[2] + (G)v[4 * b + 3] * wz[3]);
-        sum += wx[a] * sa;
-      }
-    } else {
-      // moved out of the tile's window since the sort: from global memory
-#pragma unroll 1
-      for (int e = 0; e < 64; ++e) {
-        const int a = e >> 4, b = (e >> 2) & 3, c = e & 3;
-        const uint32_t o = ((uint32_t)wrapIdx<N>(i0 + a) * N + (uint32_t)wrapIdx<N>(j0 + b)) * N + (uint32_t)wrapIdx<N>(k0 + c);
-        T v = ld32(f, o);
-        if (dens) v = nStage<T>(v, clip);
-        const G wa = qr * (one + ((a & 2) ? -one : one) * ((a & 1) ? xs : xc));
-        const G wb = qr * (one + ((b & 2) ? -one : one) * ((b & 1) ? ys : yc));
-        const G wc = qr * (one + ((c & 2) ? -one : one) * ((c & 1) ? zs : zc));
-        sum += (G)v * (wa * wb * wc);
-      }
+      for (int b = 0; b < 4; ++b)
+        sa += wy[b] * ((double)v[4 * b] * wz[0] + (double)v[4 * b + 1] * wz[1] + (double)v[4 * b + 2] * wz[2] +
+                       (double)v[4 * b + 3] * wz[3]);
+      sum += wx[a] * sa;
     }
     if (rowmap) out[(size_t)rowmap[s] * F.n + k] = sum;
     else out[(size_t)k * cap + s] = sum;
@@ -1256,12 +1222,6 @@ k_copy_fields(const char* __restrict__ src, size_t ss, char* __restrict__ dst, s
   for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += gridDim.x * (size_t)256) b[i] = a[i];
 }
 
-// Stage coordinate rows X + a*kp (forced-dns-sm.py:347) for the API path.
-static __global__ void k_axpy_rows(const double* __restrict__ x, const double* __restrict__ k, double a, int n, double* out) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = x[i] + a * k[i];
-}
-
 template <int N>
 __global__ void __launch_bounds__(256)
 k_bin_count(const double* __restrict__ pos0, int np, int cap, double L, double invL, double inv_dx, int* __restrict__ key0,
@@ -1393,11 +1353,6 @@ k_bin_scatter(int np, int cap, const int* __restrict__ key0, const int* __restri
 #pragma unroll
   for (int c = 0; c < 4; ++c) vm2[c * cap + d] = vm[c * cap + p];
   id2[d] = id[p];
-}
-
-template <typename X>
-__global__ void k_copy(const X* __restrict__ a, X* __restrict__ b, size_t n) {
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) b[i] = a[i];
 }
 
 }  // namespace ld
