@@ -856,6 +856,15 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
 // in their L2 (seven fields per block: 357 us for 10^6 rows at 256^3 FP32, the
 // same with 256, 384 and 512 threads; 222 us like this, against 737 us for four
 // lanes per row on planar fields, k_prhs_sorted).
+//
+// A tile's block takes its first PART slots at most.  Slots crowd where droplets
+// cluster (10^6 rows in a box of side L/20: 3.7 ms for seven fields when one
+// block per field took a tile's slots).  The others are taken by a second
+// launch (CROWD) with one block per aligned run of PART slots, which takes those
+// of the run that lie beyond the first PART of their tile: they are of one tile,
+// that of the run's first slot, because a tile that starts inside the run has no
+// such slots in it.  (In one launch with the tiles' blocks, the kernel's code
+// took 237 us instead of 222.)
 template <typename T> struct GatherFields {
   const T *a, *b, *c;          // fields 0 .. na - 1 of a, na .. na + nb - 1 of b (N^3 apart), then c
   int na, nb, n;               // n fields in all
@@ -870,31 +879,24 @@ template <int N> struct GatherTile {
   static constexpr int NQ = RX * RX * QZ;
   static constexpr int TSB = Bins<N>::TS * Bins<N>::TS * Bins<N>::TS, NTILE = Bins<N>::NB / TSB;
   static constexpr int XT = NTILE / 8, GS = XT < 64 ? XT : 64;   // tiles per XCD and per group
-  static constexpr int NT = 256;
+  static constexpr int NT = 256, PART = 1024;
+  static constexpr int IT = (NQ + NT - 1) / NT;                  // staged quads per thread (the last ones are padding)
   static_assert(RX <= N && PZ <= N && NTILE % 8 == 0 && XT % GS == 0, "gather tile");
 };
-// FP64 weights and sums.  rowmap null: out[k cap + slot]; else out[rowmap[slot] n + k].
+// Field f, number k of n, at the slots [s0, s1) of the tile with first cell
+// (cx, cy, cz); FP64 weights and sums.  rowmap null: out[k cap + slot]; else
+// out[rowmap[slot] n + k].
 template <typename T, int N>
-__global__ void __launch_bounds__(GatherTile<N>::NT)
-k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep, const int* __restrict__ start, int np, int cap,
-              const int* __restrict__ rowmap, double* __restrict__ out, DropPhys P) {
+__device__ __forceinline__ void gatherTile(T* lds, const T* __restrict__ f, int k, int n, int cx, int cy, int cz, int s0,
+                                           int s1, const double4* __restrict__ dep, int cap,
+                                           const int* __restrict__ rowmap, double* __restrict__ out, const DropPhys& P) {
   using GT = GatherTile<N>;
-  constexpr int RX = GT::RX, QZ = GT::QZ, PZ = GT::PZ, NQ = GT::NQ, NT = GT::NT, IT = (NQ + NT - 1) / NT;
-  constexpr size_t R = (size_t)N * N * N;
-  __shared__ __attribute__((aligned(32))) T lds[4 * NQ];
-  const int j = blockIdx.x / 8, r = j % (GT::GS * F.n);
-  const int tile = (blockIdx.x % 8) * GT::XT + j / (GT::GS * F.n) * GT::GS + r % GT::GS, k = r / GT::GS;
-  const int s0 = start[tile * GT::TSB], s1 = tile + 1 < GT::NTILE ? start[(tile + 1) * GT::TSB] : np;
-  if (s0 == s1) return;
-  int cx, cy, cz;
-  Bins<N>::tileCell(tile, cx, cy, cz);
-  const T* __restrict__ f = F.field(k, R);
+  constexpr int RX = GT::RX, QZ = GT::QZ, PZ = GT::PZ, NT = GT::NT, IT = GT::IT;
   {
     V4<T> q[IT];
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
-      const int e0 = (int)threadIdx.x + it * NT, e = ((it + 1) * NT <= NQ || e0 < NQ) ? e0 : 0;
-      const int z4 = e % QZ, row = e / QZ;
+      const int e = (int)threadIdx.x + it * NT, z4 = e % QZ, row = e / QZ;
       const uint32_t x = (uint32_t)(cx - 1 + row / RX) & (N - 1), y = (uint32_t)(cy - 1 + row % RX) & (N - 1),
                      z = (uint32_t)(cz - 4 + 4 * z4) & (N - 1);
       q[it] = ld32(reinterpret_cast<const V4<T>*>(f), ((x * N + y) * N + z) / 4);
@@ -903,10 +905,7 @@ k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep, const int* __r
     // scheduler, 237 instead of 222 us for 10^6 rows at 256^3 FP32)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int it = 0; it < IT; ++it) {
-      const int e = (int)threadIdx.x + it * NT;
-      if ((it + 1) * NT <= NQ || e < NQ) *reinterpret_cast<V4<T>*>(lds + 4 * e) = q[it];
-    }
+    for (int it = 0; it < IT; ++it) *reinterpret_cast<V4<T>*>(lds + 4 * ((int)threadIdx.x + it * NT)) = q[it];
   }
   __syncthreads();
   for (int s = s0 + (int)threadIdx.x; s < s1; s += NT) {
@@ -936,8 +935,40 @@ k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep, const int* __r
                        (double)v[4 * b + 3] * wz[3]);
       sum += wx[a] * sa;
     }
-    if (rowmap) out[(size_t)rowmap[s] * F.n + k] = sum;
+    if (rowmap) out[(size_t)rowmap[s] * n + k] = sum;
     else out[(size_t)k * cap + s] = sum;
+  }
+}
+template <typename T, int N, bool CROWD>
+__global__ void __launch_bounds__(GatherTile<N>::NT)
+k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep, const int* __restrict__ start, int np, int cap,
+              const int* __restrict__ rowmap, double* __restrict__ out, DropPhys P) {
+  using GT = GatherTile<N>;
+  constexpr int PART = GT::PART;
+  constexpr size_t R = (size_t)N * N * N;
+  __shared__ __attribute__((aligned(32))) T lds[4 * GT::IT * GT::NT];
+  int cx, cy, cz;
+  auto end = [&](int tile) { return tile + 1 < GT::NTILE ? start[(tile + 1) * GT::TSB] : np; };
+  if constexpr (!CROWD) {
+    const int j = blockIdx.x / 8, r = j % (GT::GS * F.n);
+    const int tile = (blockIdx.x % 8) * GT::XT + j / (GT::GS * F.n) * GT::GS + r % GT::GS, k = r / GT::GS;
+    const int s0 = start[tile * GT::TSB], s1 = end(tile);
+    if (s0 == s1) return;
+    Bins<N>::tileCell(tile, cx, cy, cz);
+    gatherTile<T, N>(lds, F.field(k, R), k, F.n, cx, cy, cz, s0, s1 - s0 < PART ? s1 : s0 + PART, dep, cap, rowmap, out, P);
+  } else {
+    const int run = ((int)blockIdx.x + 1) * PART;
+    const double4 d = dep[run];
+    const int tile = Bins<N>::key(cellOf<N>(d.x, P.inv_dx) / Bins<N>::BS, cellOf<N>(d.y, P.inv_dx) / Bins<N>::BS,
+                                  cellOf<N>(d.z, P.inv_dx) / Bins<N>::BS) / GT::TSB;
+    const int first = start[tile * GT::TSB] + PART, last = end(tile);
+    const int s0 = first > run ? first : run, s1 = last < run + PART ? last : run + PART;
+    if (s0 >= s1) return;
+    Bins<N>::tileCell(tile, cx, cy, cz);
+    for (int k = 0; k < F.n; ++k) {
+      if (k) __syncthreads();            // the sums of the field before
+      gatherTile<T, N>(lds, F.field(k, R), k, F.n, cx, cy, cz, s0, s1, dep, cap, rowmap, out, P);
+    }
   }
 }
 

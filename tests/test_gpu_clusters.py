@@ -103,3 +103,44 @@ def test_captured_pair_statistics(gpu):
         torch.cuda.synchronize()
         assert np.array_equal(buf[0].cpu().numpy().view(np.int64), want)
     d.close()
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("counts", [(0, 1, 1024, 1025, 3000, 2047, 5, 4096), (9000, 0, 0, 0, 0, 0, 0, 0), (1,) * 7 + (7000,)])
+def test_tiles_of_more_rows_than_a_block_takes(gpu, prec, counts, monkeypatch):
+    """Rows per tile around the 1024 that a tile's block takes, against the gather by four lanes per row (the same
+    weights and 64 products in another order: 1e-12 of the largest value)."""
+    import torch
+    from lucky_droplets_amd.dns import ForcedDNS
+    monkeypatch.setenv("LD_ROW_SORT_MIN", "0")
+    N = 32
+    rng = np.random.default_rng(sum(counts))
+    h = np.pi                                            # a tile's side: 16 of the 32 cells
+    rows = np.concatenate([np.concatenate([rng.uniform(0, h, (c, 3)) + h * np.array([t >> 2, t >> 1 & 1, t & 1]),
+                                           rng.uniform(0.1, 1.0, (c, 4))], 1) for t, c in enumerate(counts)])
+    rows = rows[rng.permutation(len(rows))]
+    fields = torch.from_numpy(rng.standard_normal((7, N, N, N))).to(gpu)
+    got = []
+    for line in (0, 1 << 40):
+        monkeypatch.setenv("LD_ROW_TILE_MIN", str(line))
+        d, stb = _population(N, prec, rows)
+        f = fields.to(d.rdtype)
+        out = [stb.interp_cosine(stb.coord, f).clone(), stb.interp_cosine(stb.coord, f[:1]).clone()]
+        out.append(stb.pRHS(0.0, stb.coord, f[:3], f[3:6], f[6], torch.empty_like(f[0]), None)[1])
+        out.append(stb.interpmat)
+        got.append([x.cpu().numpy() for x in out])
+        d.close()
+    for a, b in zip(*got):
+        assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b))
+
+
+def test_gather_of_a_cluster_is_not_serial(gpu):
+    """10^6 rows at 128^3, uniform and in 1/20 of the box side."""
+    import torch
+    n, ms = 1_000_000, {}
+    for side in (1.0, 0.05):
+        d, stb = _population(128, "f32", _rows(n, side))
+        f = torch.randn((7, 128, 128, 128), device=gpu)
+        ms[side] = _ms(lambda: stb.interp_cosine(stb.coord, f))
+        d.close()
+    assert ms[0.05] < 5 * ms[1.0], ms
