@@ -155,7 +155,10 @@ struct Engine final : EngineBase {
   PT* v0b = nullptr;
   double4* dep = nullptr;            // per-slot stage position and W for the brick deposit
   int *flist = nullptr, *fcount = nullptr;
-  unsigned long long* fx = nullptr;  // fixed-point scratch field of the fallback deposit (zero between steps)
+  // scratch field, zero between calls: fixed-point sums of the fallback deposit, FP64 sums of the rows' crowded bricks
+  unsigned long long* fx = nullptr;
+  int *crowd_count = nullptr, *crowd_done = nullptr;
+  CrowdShare* crowd_list = nullptr;
   unsigned long long* wmaxp = nullptr;   // largest W of a droplet stage (fixed-point deposit bound)
   // y and z passes of a chain run slab by slab (x-planes) so the y<->z
   // intermediate of one slab stays in the Infinity Cache; 1 = whole field.
@@ -422,6 +425,7 @@ struct Engine final : EngineBase {
       arena(hist, NB); arena(bsum, NBS);
       arena(x0b, 3 * cap); arena(v0b, 4 * cap);
       arena(dep, cap); arena(flist, cap); arena(fcount, 1); arena(wmaxp, WSLOTS * 16); arena(fx, RF);
+      arena(crowd_count, 1); arena(crowd_done, NBRICK); arena(crowd_list, cap / 512 + 1);
     }
     LD_TRY(arena_commit());
     LD_TRY(alloc(shells, 8));
@@ -846,7 +850,8 @@ struct Engine final : EngineBase {
       auto bricks = [&](auto mode) {
         hipLaunchKernelGGL((k_brick_deposit<T, N, decltype(mode)::value>), dim3(NBRICK + FB_BLOCKS, 1, B),
                            dim3(Brick<N>::NT), 0, st2, (const double4*)dep, (const int*)hist, (int)np,
-                           (const unsigned long long*)wmaxp, fc, dp, rs, (const int*)flist, (const int*)fcount, fx);
+                           (const unsigned long long*)wmaxp, fc, dp, rs, (const int*)flist, (const int*)fcount, fx,
+                           Crowd{});
       };
       if (wide && sizeof(T) == 4) bricks(std::integral_constant<int, sizeof(T) == 4 ? DEP_WIDE : DEP_STEP>{});
       else bricks(std::integral_constant<int, DEP_STEP>{});
@@ -1663,7 +1668,7 @@ struct Engine final : EngineBase {
     LD_LAUNCHED();
     LD_TRY(scan_bins(st));
     hipLaunchKernelGGL((k_row_scatter<N>), dim3(pb), dim3(256), 0, st, coord, (int)n_, p.L, dp.inv_dx, w,
-                       (const int*)pkey, (const int*)prank, (const int*)hist, dep, flist);
+                       (const int*)pkey, (const int*)prank, (const int*)hist, dep, flist, crowd_count);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -1691,9 +1696,15 @@ struct Engine final : EngineBase {
   static unsigned quad_blocks(int64_t n_) { return (unsigned)(((4 * n_ + 255) / 256 + 7) / 8 * 8); }
   // FP64 brick deposit of the sorted rows' weights; writes every node of c
   int deposit_rows(int64_t n_, T* c) {
+    const Crowd crowd{crowd_count, crowd_done, crowd_list, reinterpret_cast<double*>(fx)};
     hipLaunchKernelGGL((k_brick_deposit<T, N, DEP_ROWS>), dim3(NBRICK), dim3(Brick<N>::NT), 0, st, (const double4*)dep,
                        (const int*)hist, (int)n_, (const unsigned long long*)nullptr, c, dp, (size_t)0,
-                       (const int*)nullptr, (const int*)nullptr, (unsigned long long*)nullptr);
+                       (const int*)nullptr, (const int*)nullptr, (unsigned long long*)nullptr, crowd);
+    LD_LAUNCHED();
+    if (n_ <= Brick<N>::CROWD) return LD_OK;
+    const unsigned nb = n_ / 512 < 512 ? (unsigned)(n_ / 512) : 512u;
+    hipLaunchKernelGGL((k_brick_crowd<T, N>), dim3(nb), dim3(Brick<N>::NT), 0, st, (const double4*)dep,
+                       (const int*)hist, (int)n_, c, dp, crowd);
     LD_LAUNCHED();
     return LD_OK;
   }

@@ -642,6 +642,7 @@ template <int N> struct Brick {
   static constexpr int NZS = (NBX + Bins<N>::TS - 1) / Bins<N>::TS + 1;
   static constexpr int NR = NZS * NBX * NBX;         // slot ranges
   static constexpr int CH = 2 * NT;                  // candidates tested per round (LDS fits 4 blocks per CU)
+  static constexpr int CROWD = 8 * CH, PARTS = 64;   // DEP_ROWS: candidates that one block takes, most shares
   static_assert(N % S == 0 && (NB * NB * NB) % 8 == 0, "brick grid");
 };
 
@@ -652,27 +653,26 @@ template <int N> struct Brick {
 // negative, of any range or not finite): the tile is FP64 and added to in FP64
 // (ds_add_f64, 27 against 15 cycles), every candidate with W != 0 deposits, and
 // the stencil weights are FP64 as the API's are.
-enum { DEP_STEP, DEP_WIDE, DEP_ROWS };
-template <typename T, int N, int MODE = DEP_STEP>
-__global__ void __launch_bounds__(Brick<N>::NT)
-k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0, int np,
-                const unsigned long long* __restrict__ wmax0, T* __restrict__ fc0, DropPhys P, size_t rs,
-                const int* __restrict__ flist0, const int* __restrict__ fcount0, unsigned long long* fx0) {
-  const double4* __restrict__ dep = rsel1(dep0, rs);
-  const int* __restrict__ start = rsel1(start0, rs);
-  const unsigned long long* __restrict__ wmax = rsel1(wmax0, rs);
-  T* __restrict__ fc = rsel1(fc0, rs);
-  constexpr bool FIX = MODE != DEP_ROWS;
-  constexpr int NBRICK = Brick<N>::NB * Brick<N>::NB * Brick<N>::NB;
-  if constexpr (FIX) {
-    if (blockIdx.x >= NBRICK) {          // the extra blocks: fallback slots
-      const int nf = *rsel1(fcount0, rs), b = (int)blockIdx.x - NBRICK;
-      if (nf)
-        fallbackAccum<T, N>(dep, rsel1(flist0, rs), nf, maxOfSlots(wmax), rsel1(fx0, rs), P, b * Brick<N>::NT + (int)threadIdx.x,
-                            ((int)gridDim.x - NBRICK) * Brick<N>::NT);
-      return;
-    }
-  }
+//
+// DEP_ROWS, more than CROWD candidates in a brick (rows that cluster: 10^6 in a
+// box of side L/20 took 21 ms when a brick's workgroup took them all): the
+// brick's block only lists up to PARTS shares of them, and a second launch of
+// persistent blocks (k_brick_crowd, DEP_SHARE) takes the shares, adds each one's
+// tile to the FP64 scratch field `sums` (zero between calls), and the block that
+// adds a brick's last share rounds the sums into fc and clears them.
+enum { DEP_STEP, DEP_WIDE, DEP_ROWS, DEP_SHARE };
+struct CrowdShare { int brick, part, parts, pad; };
+struct Crowd {
+  int* count;                  // shares listed (zero before the DEP_ROWS launch)
+  int* done;                   // shares added, per brick
+  CrowdShare* list;            // at most np / 512 of them: a slot is a candidate of at most 8 bricks
+  double* sums;
+};
+template <typename T, int N, int MODE>
+__device__ __forceinline__ void brickDeposit(const double4* __restrict__ dep, const int* __restrict__ start, int np,
+                                             const unsigned long long* __restrict__ wmax, T* __restrict__ fc,
+                                             const DropPhys& P, const CrowdShare& it, const Crowd& crowd) {
+  constexpr bool FIX = MODE == DEP_STEP || MODE == DEP_WIDE;
   using Bk = Brick<N>;
   constexpr int S = Bk::S, NBr = Bk::NB, NBX = Bk::NBX, NR = Bk::NR, NT = Bk::NT, NZS = Bk::NZS, CH = Bk::CH;
   constexpr int TS = Bins<N>::TS;
@@ -684,9 +684,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   __shared__ int cnt;
   __shared__ unsigned long long wtop;
   const int tid = threadIdx.x, lane = tid & 63;
-  // XCD-aware: each of the 8 XCDs takes a contiguous run of bricks
-  constexpr int per = NBRICK / 8;
-  const int br = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  const int br = it.brick;
   const int c0x = (br / (NBr * NBr)) * S, c0y = ((br / NBr) % NBr) * S, c0z = (br % NBr) * S;
   for (int i = tid; i < S * S * S; i += NT) tile[i] = 0;
   if (tid == 0) cnt = 0;
@@ -748,7 +746,21 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
     if (tid == 63) rl[NR] = inc;
   }
   __syncthreads();
-  const int total = rl[NR];
+  const int all = rl[NR];
+  if constexpr (MODE == DEP_ROWS) {
+    if (all > Bk::CROWD) {
+      int parts = (all + Bk::CROWD - 1) / Bk::CROWD;
+      parts = parts < Bk::PARTS ? parts : Bk::PARTS;
+      if (tid == 0) { cnt = atomicAdd(crowd.count, parts); crowd.done[br] = 0; }
+      __syncthreads();
+      if (tid < parts) crowd.list[cnt + tid] = CrowdShare{br, tid, parts, 0};
+      return;
+    }
+  }
+  // the candidates [first, total): all of them, or the share
+  const int share = MODE == DEP_SHARE ? (all + it.parts - 1) / it.parts : all;
+  const int first = MODE == DEP_SHARE ? it.part * share : 0;
+  const int total = MODE == DEP_SHARE && first + share < all ? first + share : all;
   const double dx = P.dx, pi_2dx = P.pi_2dx, inv_dx = P.inv_dx;
   const double bound = FIX ? (double)total * __longlong_as_double((long long)wtop) * P.inv_vol * 0.125 : 0.0;
   const bool finite = isfinite(bound);
@@ -759,7 +771,7 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
   constexpr int EMAX = F32 ? 51 : 61;
   const int e = (bound > 0.0 && finite) ? EMAX - ilogb(bound) : 0;
   const double scale = ldexp(1.0, e), unit = ldexp(1.0, -e);
-  for (int base = 0; base < total && finite; base += CH) {
+  for (int base = first; base < total && finite; base += CH) {
     // test and compact: growing candidates whose stencil meets the brick
 #pragma unroll 1
     for (int k = 0; k < CH / NT; ++k) {
@@ -836,9 +848,61 @@ k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0
     if (tid == 0) cnt = 0;
     __syncthreads();
   }
-  for (int i = tid; i < S * S * S; i += NT) {
+  auto node = [&](int i) {
     const int nx = i / (S * S), ny = (i / S) % S, nz = i % S;
-    fc[((size_t)(c0x + nx) * N + (c0y + ny)) * N + (c0z + nz)] = finite ? (T)((double)tile[i] * unit) : (T)NAN;
+    return ((size_t)(c0x + nx) * N + (c0y + ny)) * N + (c0z + nz);
+  };
+  if constexpr (MODE != DEP_SHARE) {
+    for (int i = tid; i < S * S * S; i += NT) fc[node(i)] = finite ? (T)((double)tile[i] * unit) : (T)NAN;
+  } else {
+    for (int i = tid; i < S * S * S; i += NT)
+      if (tile[i] != 0.0) unsafeAtomicAdd(crowd.sums + node(i), tile[i]);
+    __threadfence();                     // this share's additions before its count
+    __syncthreads();
+    if (tid == 0) cnt = atomicAdd(crowd.done + br, 1);
+    __syncthreads();
+    if (cnt == it.parts - 1) {
+      __threadfence();                   // all counts before the loads
+      for (int i = tid; i < S * S * S; i += NT) {
+        double* v = crowd.sums + node(i);
+        fc[node(i)] = (T)__hip_atomic_load(v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *v = 0.0;
+      }
+    }
+  }
+}
+
+template <typename T, int N, int MODE = DEP_STEP>
+__global__ void __launch_bounds__(Brick<N>::NT)
+k_brick_deposit(const double4* __restrict__ dep0, const int* __restrict__ start0, int np,
+                const unsigned long long* __restrict__ wmax0, T* __restrict__ fc0, DropPhys P, size_t rs,
+                const int* __restrict__ flist0, const int* __restrict__ fcount0, unsigned long long* fx0, Crowd crowd) {
+  const double4* __restrict__ dep = rsel1(dep0, rs);
+  const unsigned long long* __restrict__ wmax = rsel1(wmax0, rs);
+  constexpr int NBRICK = Brick<N>::NB * Brick<N>::NB * Brick<N>::NB;
+  if constexpr (MODE != DEP_ROWS) {
+    if (blockIdx.x >= NBRICK) {          // the extra blocks: fallback slots
+      const int nf = *rsel1(fcount0, rs), b = (int)blockIdx.x - NBRICK;
+      if (nf)
+        fallbackAccum<T, N>(dep, rsel1(flist0, rs), nf, maxOfSlots(wmax), rsel1(fx0, rs), P, b * Brick<N>::NT + (int)threadIdx.x,
+                            ((int)gridDim.x - NBRICK) * Brick<N>::NT);
+      return;
+    }
+  }
+  // XCD-aware: each of the 8 XCDs takes a contiguous run of bricks
+  constexpr int per = NBRICK / 8;
+  const int br = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  brickDeposit<T, N, MODE>(dep, rsel1(start0, rs), np, wmax, rsel1(fc0, rs), P, CrowdShare{br, 0, 1, 0}, crowd);
+}
+template <typename T, int N>
+__global__ void __launch_bounds__(Brick<N>::NT)
+k_brick_crowd(const double4* __restrict__ dep, const int* __restrict__ start, int np, T* __restrict__ fc, DropPhys P,
+              Crowd crowd) {
+  const int n = *crowd.count;
+  for (int i = blockIdx.x; i < n; i += gridDim.x) {
+    const CrowdShare it = crowd.list[i];
+    brickDeposit<T, N, DEP_SHARE>(dep, start, np, nullptr, fc, P, it, crowd);
+    __syncthreads();                     // the shared arrays of the next share
   }
 }
 
@@ -1062,8 +1126,9 @@ template <int N>
 __global__ void __launch_bounds__(256)
 k_row_scatter(const double* __restrict__ rows, int np, double L, double inv_dx, const double* __restrict__ w,
               const int* __restrict__ key, const int* __restrict__ rank, const int* __restrict__ start,
-              double4* __restrict__ dep, int* __restrict__ row) {
+              double4* __restrict__ dep, int* __restrict__ row, int* __restrict__ crowd_count) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p == 0) *crowd_count = 0;          // of the deposit that follows
   if (p >= np) return;
   const double* r = rows + (size_t)p * 7;
   double4 d;
