@@ -1683,13 +1683,9 @@ struct Engine final : EngineBase {
     return tile_rows_min >= 0 ? n_ >= tile_rows_min : NTILE >= 512 && n_ >= per * (int64_t)NTILE;
   }
   int tile_gather_rows(const GatherFields<T>& g, int64_t n_, const int* rowmap, double* out) {
-    hipLaunchKernelGGL((k_tile_gather<T, N, false>), dim3(NTILE * g.n), dim3(GatherTile<N>::NT), 0, st, g,
-                       (const double4*)dep, (const int*)hist, (int)n_, (int)cap, rowmap, out, dp);
-    LD_LAUNCHED();
     const unsigned runs = (unsigned)((n_ - 1) / GatherTile<N>::PART);      // aligned runs of slots after the first
-    if (!runs) return LD_OK;
-    hipLaunchKernelGGL((k_tile_gather<T, N, true>), dim3(runs), dim3(GatherTile<N>::NT), 0, st, g, (const double4*)dep,
-                       (const int*)hist, (int)n_, (int)cap, rowmap, out, dp);
+    hipLaunchKernelGGL((k_tile_gather<T, N>), dim3(NTILE * g.n + runs), dim3(GatherTile<N>::NT), 0, st, g,
+                       (const double4*)dep, (const int*)hist, (int)n_, (int)cap, rowmap, out, dp);
     LD_LAUNCHED();
     return LD_OK;
   }

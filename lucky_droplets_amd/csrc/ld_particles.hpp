@@ -923,12 +923,11 @@ k_brick_crowd(const double4* __restrict__ dep, const int* __restrict__ start, in
 //
 // A tile's block takes its first PART slots at most.  Slots crowd where droplets
 // cluster (10^6 rows in a box of side L/20: 3.7 ms for seven fields when one
-// block per field took a tile's slots).  The others are taken by a second
-// launch (CROWD) with one block per aligned run of PART slots, which takes those
-// of the run that lie beyond the first PART of their tile: they are of one tile,
-// that of the run's first slot, because a tile that starts inside the run has no
-// such slots in it.  (In one launch with the tiles' blocks, the kernel's code
-// took 237 us instead of 222.)
+// block per field took a tile's slots).  So behind the tiles' blocks there is one
+// per aligned run of PART slots, which takes those of the run that lie beyond
+// the first PART of their tile, all fields: they are of one tile, that of the
+// run's first slot, because a tile that starts inside the run has no such slots
+// in it.
 template <typename T> struct GatherFields {
   const T *a, *b, *c;          // fields 0 .. na - 1 of a, na .. na + nb - 1 of b (N^3 apart), then c
   int na, nb, n;               // n fields in all
@@ -1003,7 +1002,7 @@ __device__ __forceinline__ void gatherTile(T* lds, const T* __restrict__ f, int 
     else out[(size_t)k * cap + s] = sum;
   }
 }
-template <typename T, int N, bool CROWD>
+template <typename T, int N>
 __global__ void __launch_bounds__(GatherTile<N>::NT)
 k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep, const int* __restrict__ start, int np, int cap,
               const int* __restrict__ rowmap, double* __restrict__ out, DropPhys P) {
@@ -1013,26 +1012,28 @@ k_tile_gather(GatherFields<T> F, const double4* __restrict__ dep, const int* __r
   __shared__ __attribute__((aligned(32))) T lds[4 * GT::IT * GT::NT];
   int cx, cy, cz;
   auto end = [&](int tile) { return tile + 1 < GT::NTILE ? start[(tile + 1) * GT::TSB] : np; };
-  if constexpr (!CROWD) {
+  const int extra = (int)blockIdx.x - GT::NTILE * F.n;
+  if (extra < 0) {
     const int j = blockIdx.x / 8, r = j % (GT::GS * F.n);
     const int tile = (blockIdx.x % 8) * GT::XT + j / (GT::GS * F.n) * GT::GS + r % GT::GS, k = r / GT::GS;
     const int s0 = start[tile * GT::TSB], s1 = end(tile);
     if (s0 == s1) return;
     Bins<N>::tileCell(tile, cx, cy, cz);
     gatherTile<T, N>(lds, F.field(k, R), k, F.n, cx, cy, cz, s0, s1 - s0 < PART ? s1 : s0 + PART, dep, cap, rowmap, out, P);
-  } else {
-    const int run = ((int)blockIdx.x + 1) * PART;
-    const double4 d = dep[run];
-    const int tile = Bins<N>::key(cellOf<N>(d.x, P.inv_dx) / Bins<N>::BS, cellOf<N>(d.y, P.inv_dx) / Bins<N>::BS,
-                                  cellOf<N>(d.z, P.inv_dx) / Bins<N>::BS) / GT::TSB;
-    const int first = start[tile * GT::TSB] + PART, last = end(tile);
-    const int s0 = first > run ? first : run, s1 = last < run + PART ? last : run + PART;
-    if (s0 >= s1) return;
-    Bins<N>::tileCell(tile, cx, cy, cz);
-    for (int k = 0; k < F.n; ++k) {
-      if (k) __syncthreads();            // the sums of the field before
-      gatherTile<T, N>(lds, F.field(k, R), k, F.n, cx, cy, cz, s0, s1, dep, cap, rowmap, out, P);
-    }
+    return;
+  }
+  const int run = (extra + 1) * PART;
+  const double4 d = dep[run];
+  const int tile = Bins<N>::key(cellOf<N>(d.x, P.inv_dx) / Bins<N>::BS, cellOf<N>(d.y, P.inv_dx) / Bins<N>::BS,
+                                cellOf<N>(d.z, P.inv_dx) / Bins<N>::BS) / GT::TSB;
+  const int first = start[tile * GT::TSB] + PART, last = end(tile);
+  const int s0 = first > run ? first : run, s1 = last < run + PART ? last : run + PART;
+  if (s0 >= s1) return;
+  Bins<N>::tileCell(tile, cx, cy, cz);
+#pragma unroll 1
+  for (int k = 0; k < F.n; ++k) {
+    if (k) __syncthreads();              // the sums of the field before
+    gatherTile<T, N>(lds, F.field(k, R), k, F.n, cx, cy, cz, s0, s1, dep, cap, rowmap, out, P);
   }
 }
 

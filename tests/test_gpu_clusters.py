@@ -144,3 +144,89 @@ def test_gather_of_a_cluster_is_not_serial(gpu):
         ms[side] = _ms(lambda: stb.interp_cosine(stb.coord, f))
         d.close()
     assert ms[0.05] < 5 * ms[1.0], ms
+
+
+def _cluster_rows(N, n, k, seed):
+    """n rows, k of them within one brick (16 cells, at its corner), the others uniform; unwrapped."""
+    rng = np.random.default_rng(seed)
+    rows = rng.uniform(0, 2 * np.pi, (n, 7))
+    dx = 2 * np.pi / N
+    rows[:k, :3] = 16 * dx + rng.uniform(-1.5, 14.5, (k, 3)) * dx
+    rows[:, :3] += 2 * np.pi * rng.integers(-1, 2, (n, 3))
+    rows[:, 6] = rng.uniform(0.05, 1.0, n) * 1e-3
+    return rows[rng.permutation(n)]
+
+
+# 8192 candidates stay with a brick's block; 64 shares at most (more than 64 x 8192 candidates in the last case)
+@pytest.mark.parametrize("N,n,k", [(32, 8192, 8192), (32, 8193, 8193), (64, 20000, 8000), (64, 20000, 8190),
+                                   (64, 40001, 30000), (64, 500_000, 450_000), (128, 700_000, 700_000)])
+def test_deposits_of_crowded_bricks(gpu, N, n, k, monkeypatch):
+    """Against one thread per row: positive FP64 terms, at most 10^6 a node in another order (1e-10 of the largest
+    value; FP32 fields: that sum rounded once).  A weight that is not finite reaches its own 64 nodes."""
+    import torch
+    rows = _cluster_rows(N, n, k, n + k)
+    w = torch.from_numpy(np.random.default_rng(n).uniform(0.1, 1.0, (n, 1))).to(gpu)
+    bad = w.clone()
+    bad[n // 2] = float("nan")
+    got = {}
+    for prec, line in (("f64", 1 << 40), ("f64", 0), ("f32", 0)):
+        monkeypatch.setenv("LD_ROW_SORT_MIN", str(line))
+        d, stb = _population(N, prec, rows)
+        c = d.zeros_real()
+        stb.exterpmat = bad
+        poison = torch.isnan(stb.exterp_cosine_scalar(stb.coord, torch.full_like(c, 3.0))).cpu().numpy()
+        stb.exterpmat = w
+        dep = stb.exterp_cosine_scalar(stb.coord, torch.full_like(c, 3.0)).double().cpu().numpy()
+        got[prec, line] = poison, dep
+        d.close()
+    p0, want = got["f64", 1 << 40]
+    top = np.max(want)
+    assert p0.any()
+    for key, rel in ((("f64", 0), 0.0), (("f32", 0), 2.0 ** -24)):
+        p, dep = got[key]
+        assert np.array_equal(p, p0)
+        assert np.all(np.abs(dep - want) <= 1e-10 * top + rel * np.abs(want)), key
+
+
+def test_steps_after_a_crowded_deposit(gpu, monkeypatch):
+    """The shares' scratch field is the fallback deposit's: it is zero again when RK4 uses it."""
+    import torch
+    from helpers import inputs
+    from lucky_droplets_amd.dns import ForcedDNS
+    from lucky_droplets_amd.particles import MPI_particles
+    monkeypatch.setenv("LD_ROW_SORT_MIN", "0")
+    n = 60_000
+    cfg = Config(N=64, precision="f64", nu=0.02, nshells=2, profile="k4", n_particles=n,
+                 st_dist=("uniform", 0.05, 1.0), gravity=True)
+    uk, nn, coord, _ = inputs(cfg, seed=3, n_noise=0.2)
+    crowd = torch.from_numpy(_cluster_rows(64, n, n, 1)).to(gpu)
+    rows = coord.copy()
+    rows[:, 3:6] *= 60.0                                  # most leave their bins: fallback deposit
+    out = []
+    for first in (False, True):
+        d = ForcedDNS(cfg)
+        stb = MPI_particles(None, cfg.L, cfg.N, n, cfg.sts, 0.05, cfg.g, cfg.nu_eff, cfg.tf, cfg.rhop, cfg.M0, dns=d,
+                            coord=rows)
+        if first:
+            stb.exterpmat = torch.ones((n, 1), dtype=torch.float64, device=gpu)
+            for _ in range(2):
+                stb.exterp_cosine_scalar(crowd, d.zeros_real())
+        t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).to(gpu)
+        r, u1, n1 = d.RK4(0.0, 0.01, stb, t(uk), t(nn))
+        out.append([x.cpu().numpy() for x in (r, u1, n1)])
+        d.close()
+    assert np.isfinite(out[0][2]).all()
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+
+
+def test_deposit_of_a_cluster_is_not_serial(gpu):
+    """10^6 rows at 128^3, uniform and in 1/20 of the box side."""
+    import torch
+    n, ms = 1_000_000, {}
+    for side in (1.0, 0.05):
+        d, stb = _population(128, "f32", _rows(n, side))
+        c = d.zeros_real()
+        stb.exterpmat = torch.rand((n, 1), dtype=torch.float64, device=gpu)
+        ms[side] = _ms(lambda: stb.exterp_cosine_scalar(stb.coord, c))
+        d.close()
+    assert ms[0.05] < 15 * ms[1.0], ms
