@@ -1005,9 +1005,7 @@ struct Engine final : EngineBase {
     hipLaunchKernelGGL(k_scan_local, dim3(NBS, 1, B), dim3(1024), 0, s, hist, NB, bsum, rs);
     LD_LAUNCHED();
     if (NBS == 1) return LD_OK;          // one block scanned them all
-    hipLaunchKernelGGL(k_scan_bsums, dim3(1, 1, B), dim3(1024), 0, s, bsum, NBS, rs);
-    LD_LAUNCHED();
-    hipLaunchKernelGGL(k_scan_add, dim3((NB + 255) / 256, 1, B), dim3(256), 0, s, hist, NB, (const int*)bsum, rs);
+    hipLaunchKernelGGL(k_scan_add, dim3(NBS, 1, B), dim3(1024), 0, s, hist, NB, (const int*)bsum, rs);
     LD_LAUNCHED();
     return LD_OK;
   }
@@ -1498,11 +1496,10 @@ struct Engine final : EngineBase {
     }
     hipLaunchKernelGGL(k_scan_local, dim3(nbs), dim3(1024), 0, st, chist, ncells, cbsum, (size_t)0);
     LD_LAUNCHED();
-    hipLaunchKernelGGL(k_scan_bsums, dim3(1), dim3(1024), 0, st, cbsum, nbs, (size_t)0);
-    LD_LAUNCHED();
-    hipLaunchKernelGGL(k_scan_add, dim3((ncells + 255) / 256), dim3(256), 0, st, chist, ncells, (const int*)cbsum,
-                       (size_t)0);
-    LD_LAUNCHED();
+    if (nbs > 1) {
+      hipLaunchKernelGGL(k_scan_add, dim3(nbs), dim3(1024), 0, st, chist, ncells, (const int*)cbsum, (size_t)0);
+      LD_LAUNCHED();
+    }
     hipLaunchKernelGGL(k_coll_scatter, dim3(pb), dim3(256), 0, st, rows, rad, (int)n_, p.L, (const int*)ckey,
                        (const int*)crank, (const int*)chist, corder, cpos, with_vel ? cvel : (double4*)nullptr);
     LD_LAUNCHED();
@@ -1664,7 +1661,13 @@ struct Engine final : EngineBase {
     LD_TRY(rows_begin());
     const unsigned pb = (unsigned)((n_ + 255) / 256);
     LD_TRY(fill<int>(st, hist, NB, 0));
-    hipLaunchKernelGGL((k_row_bin<N>), dim3(pb), dim3(256), 0, st, coord, (int)n_, p.L, dp.inv_dx, pkey, prank, hist);
+    auto bins = [&](auto nt) {
+      constexpr int NT = decltype(nt)::value;
+      hipLaunchKernelGGL((k_row_bin<N, NT>), dim3((unsigned)((n_ + NT - 1) / NT)), dim3(NT), 0, st, coord, (int)n_, p.L,
+                         dp.inv_dx, pkey, prank, hist);
+    };
+    if (n_ < 1 << 18) bins(std::integral_constant<int, 256>{});
+    else bins(std::integral_constant<int, 1024>{});
     LD_LAUNCHED();
     LD_TRY(scan_bins(st));
     hipLaunchKernelGGL((k_row_scatter<N>), dim3(pb), dim3(256), 0, st, coord, (int)n_, p.L, dp.inv_dx, w,
