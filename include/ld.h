@@ -142,15 +142,16 @@ int ld_status(ld_ctx* ctx, double* last_max, int32_t* blown_up);
 /* The same per realization: last_max and blown_up are host arrays of batch
  * entries.  No counterpart in the reference (one realization per job). */
 int ld_status_all(ld_ctx* ctx, double* last_max, int32_t* blown_up);
-/* The autotuner's choice: lines per block of the y passes (*ylines, host) and
- * the measured median times in microseconds of the candidates (us[3], host:
+/* Lines per block of the inverse y passes (*ylines, host; the forward passes
+ * run the same when the context was created with autotune, else M) and the
+ * autotuner's measured median times in microseconds of the candidates (us[3], host:
  * M, M/2 and 2M lines with M = 16 for FP32 and 8 for FP64; 0 for a candidate
  * not timed, all zeros when the context was created without autotune).  No
  * counterpart in the reference. */
 int ld_tuning(ld_ctx* ctx, int32_t* ylines, double* us);
 
-/* Every launch-geometry choice (host arrays): choice[7] = y-pass lines per
- * block, z-tile height of the u x omega pass and of the v pass, lines per
+/* Every launch-geometry choice (host arrays): choice[7] = lines per block
+ * of the inverse y passes (as ld_tuning), z-tile height of the u x omega pass and of the v pass, lines per
  * block of the u/omega, RHS and density x passes, and the threads per line N1
  * of the y passes' line split N = N1 N2; us[19] = the y-pass candidates'
  * median times (as ld_tuning), then per tuned kernel the times of its
@@ -174,7 +175,8 @@ int ld_tuning_all(ld_ctx* ctx, int32_t* choice, double* us);
 #define LD_K_ZVEL 5       /* z pass: v, n v */
 #define LD_K_XKN 6        /* x pass: density flux */
 #define LD_K_ZKN 7        /* z pass: kn, RK update of n */
-#define LD_K_DEPOSIT 8    /* droplet deposit: brick pass and fallback accumulate/fold */
+#define LD_K_DEPOSIT 8    /* droplet deposit: brick pass with the fallback slots' sums (the z pass of the
+                           * deposit field, in no class, adds those to it) */
 /* Start timing every launch of kernel class `kernel` (or stop, enable = 0). */
 int ld_profile(ld_ctx* ctx, int32_t kernel, int32_t enable);
 /* Synchronise, then report the summed duration (ms) and launch count since

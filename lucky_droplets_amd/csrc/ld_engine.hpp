@@ -321,7 +321,7 @@ struct Engine final : EngineBase {
   int tuning_all(int32_t* choice, double* us_out) override {
     const int32_t sizes[5][3] = {{P6, P6H, P6D}, {P3, P3H, P3D}, {M, MH, M}, {M3, M3H, M3}, {M, MH, M}};
     if (choice) {
-      choice[0] = my;
+      choice[0] = ylines_inv();
       for (int k = 0; k < 5; ++k) choice[1 + k] = sizes[k][vsel[k]];
       choice[6] = ysplit ? NQ : N1;
     }
@@ -334,7 +334,7 @@ struct Engine final : EngineBase {
     return LD_OK;
   }
   int tuning(int32_t* ylines, double* us) override {
-    if (ylines) *ylines = my;
+    if (ylines) *ylines = ylines_inv();
     if (us) { us[0] = tune_us[0]; us[1] = tune_us[1]; us[2] = tune_us[2]; }
     return LD_OK;
   }
@@ -479,6 +479,7 @@ struct Engine final : EngineBase {
   // us per pass, four steps 22.40 -> 22.21 ms; 512^3 518 -> 503 us; but 128^3
   // 10.3 -> 12.1 us, FP64 15.75 -> 16.25 us, and the forward passes are no faster)
   int myi = sizeof(T) == 4 && N >= 256 ? M2 : M;
+  int ylines_inv() const { return myi == M2 && (N / nslab) % M2 ? M : myi; }   // whole groups in a slab
   // ysplit = 1 (LD_YSPLIT=1): y passes split each line N = (N1/2) (2 N2)
   // instead of N1 N2.  Another factorisation rounds differently, so this is
   // a measurement switch, not an autotuner choice (the autotuner only chooses
@@ -494,7 +495,7 @@ struct Engine final : EngineBase {
     const int qoff = AXIS == 1 ? x0 * lw : 0, qend = AXIS == 1 ? (x0 + nx) * lw : 0;
     const int nl = nx * lw;
     LD_TRY(prof_mark(kid, s));
-    const int my = DIR < 0 ? this->my : myi == M2 && (N / nslab) % M2 ? M : myi;
+    const int my = DIR < 0 ? this->my : ylines_inv();
     if (AXIS == 1 && ysplit) {
       if (my == MH)
         hipLaunchKernelGGL((k_pass<T, N, MH, AXIS, DIR, NQ>), dim3((nl + MH - 1) / MH, nf, B), dim3(MH * NQ), 0, s,

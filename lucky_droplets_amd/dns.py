@@ -254,7 +254,7 @@ class ForcedDNS:
         _lib.check(self.lib.ld_advance(self.ctx, float(h), int(nsteps)))
 
     def tuning(self):
-        """(y-pass lines per block, [median us with M, M/2 and 2M lines])."""
+        """(lines per block of the inverse y passes, [median us with M, M/2 and 2M lines])."""
         yl = ctypes.c_int32()
         us = (ctypes.c_double * 3)()
         _lib.check(self.lib.ld_tuning(self.ctx, ctypes.byref(yl), us))
