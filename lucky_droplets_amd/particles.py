@@ -137,7 +137,7 @@ class MPI_particles:
         (Sundaram & Collins 1997).  Returns a dict of numpy arrays."""
         dns = self.dns
         coord, npart = dns._rows(self.coord)
-        buf = torch.empty((3, int(nbins)), dtype=torch.float64, device=dns.device)   # counts (int64), wsum, wneg
+        buf = torch.empty((3, nbins), dtype=torch.float64, device=dns.device)   # counts (int64), wsum, wneg
         dns._stream()
         _lib.check(dns.lib.ld_pair_stats(dns.ctx, _ptr(coord), npart, float(rmax), int(nbins), _ptr(buf[0]),
                                          _ptr(buf[1]), _ptr(buf[2])))
