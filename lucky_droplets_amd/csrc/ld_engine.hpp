@@ -108,6 +108,9 @@ struct Engine final : EngineBase {
   // queue a stage's density chain after the next flow x pass (measured at 256^3:
   // 8.18 vs 8.31 ms/step; the 64^3 ensemble is faster in the plain order)
   bool late_density = N >= 128;
+  // Lanes per droplet of the stage kernel (k_particles_stage); 0 = by density.
+  int lanes = 0;
+  bool eight_lanes() const { return 6 * np < (int64_t)RF; }
   // Dealiasing truncation: every mode with kz > N/3 is outside the mask
   // (kint >= kz), so the nonlinear term there is discarded and v_hat is zero.
   // The in-place y passes skip the kz > N/3 lines (kc = N/3; kc = N/2 runs
@@ -358,6 +361,7 @@ struct Engine final : EngineBase {
     if (const char* e = getenv("LD_SERIAL")) serial = atoi(e) != 0;
     if (const char* e = getenv("LD_YSPLIT")) ysplit = atoi(e) != 0;
     if (const char* e = getenv("LD_LATE_DENSITY")) late_density = atoi(e) != 0;
+    if (const char* e = getenv("LD_STAGE_LANES")) lanes = atoi(e);             // measurement, tests: 4 or 8
     if (const char* e = getenv("LD_ROW_TILE_MIN")) tile_rows_min = atoll(e);   // measurement, tests
     if (const char* e = getenv("LD_ROW_SORT_MIN")) api_sort_min = atoll(e);   // measurement, tests
     if (const char* e = getenv("LD_TRUNCATE")) kc = atoi(e) != 0 ? N / 3 : N / 2;
@@ -842,9 +846,9 @@ struct Engine final : EngineBase {
       };
       using L4 = std::integral_constant<int, 4>;
       using L8 = std::integral_constant<int, 8>;
-      const bool sparse = 6 * np < (int64_t)RF;       // lanes per droplet: see the kernel
-      if (B == 1) { if (sparse) stage(std::false_type{}, L8{}); else stage(std::false_type{}, L4{}); }
-      else { if (sparse) stage(std::true_type{}, L8{}); else stage(std::true_type{}, L4{}); }
+      const bool eight = lanes ? lanes == 8 : eight_lanes();
+      if (B == 1) { if (eight) stage(std::false_type{}, L8{}); else stage(std::false_type{}, L4{}); }
+      else { if (eight) stage(std::true_type{}, L8{}); else stage(std::true_type{}, L4{}); }
       LD_LAUNCHED();
       LD_TRY(prof_mark(LD_K_DROPLETS, st2));
       LD_TRY(prof_mark(LD_K_DEPOSIT, st2));

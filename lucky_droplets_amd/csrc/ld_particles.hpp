@@ -56,8 +56,10 @@ template <typename G> __device__ __forceinline__ void sincosGT(double th, G& s, 
 // arguments, whose code costs registers and scratch memory).
 template <typename G>
 __device__ __forceinline__ void sincosStencil(double x, int i0, double dx, double inv_dx, double pi_2dx, G& s, G& c) {
-  if constexpr (sizeof(G) == 4) sincosGT<G>((x - (double)i0 * dx) * pi_2dx, s, c);
-  else sincospi((x - (double)i0 * dx) * (0.5 * inv_dx), &s, &c);
+#pragma clang fp contract(off)
+  const double d = fma(-(double)i0, dx, x);
+  if constexpr (sizeof(G) == 4) sincosGT<G>(d * pi_2dx, s, c);
+  else sincospi(d * (0.5 * inv_dx), &s, &c);
 }
 
 // Periodic wrap of one coordinate, x mod L with numpy's sign convention
@@ -207,9 +209,10 @@ struct DropPhys {
 // interpolated components [u, v, n].
 __device__ __forceinline__ double dropletGrowth(const DropPhys& P, const double vp[3], double m, const double I[7],
                                                 double& W) {
+#pragma clang fp contract(off)
   const double st = pow(m / P.factor, 2.0 / 3.0);                          // :823
   const double d0 = vp[0] - I[3], d1 = vp[1] - I[4], d2 = vp[2] - I[5];
-  const double nrm = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+  const double nrm = sqrt(fma(d2, d2, fma(d1, d1, d0 * d0)));
   const double q = 1.0 + sqrt(P.st_s / st);
   W = P.growth * (q * q) * I[6] * nrm;                                      // :828
   return st * P.tau_eta;
@@ -229,16 +232,19 @@ __device__ __forceinline__ void dropletRhs(const DropPhys& P, const double vp[3]
 // are FP32 there); St from exp2(2/3 log2(m / factor)).
 __device__ __forceinline__ float dropletGrowth(const DropPhys& P, const float vp[3], float m, const float I[7],
                                                float& W) {
+#pragma clang fp contract(off)
   const float st = exp2f((2.0f / 3.0f) * log2f(m * (float)P.inv_factor));   // :823
   const float d0 = vp[0] - I[3], d1 = vp[1] - I[4], d2 = vp[2] - I[5];
-  const float nrm = sqrtf(d0 * d0 + d1 * d1 + d2 * d2);
+  const float nrm = sqrtf(fmaf(d2, d2, fmaf(d1, d1, d0 * d0)));
   const float q = 1.0f + sqrtf((float)P.st_s / st);
   W = (float)P.growth * (q * q) * I[6] * nrm;                                // :828
   return st * (float)P.tau_eta;
 }
 // x / den (FP32: by the reciprocal), less g
 __device__ __forceinline__ double dragTerm(double x, double den, double g) { return x / den - g; }
-__device__ __forceinline__ float dragTerm(float x, float den, float g) { return x * (1.0f / den) - g; }
+__device__ __forceinline__ float dragTerm(float x, float den, float g) { return fmaf(x, 1.0f / den, -g); }
+__device__ __forceinline__ double fmaG(double a, double b, double c) { return fma(a, b, c); }
+__device__ __forceinline__ float fmaG(float a, float b, float c) { return fmaf(a, b, c); }
 
 // ------------------------------------------------------------ lane quads
 // v of the lane L of the caller's quad of lanes (all four active), and of the
@@ -337,20 +343,22 @@ template <typename T, typename PT> struct PStage {
 // droplet's components instead of repeating each other: lane c forms axis c's
 // wrap, cell and sincos (lane 3 repeats z) and loads, updates and stores
 // component c of the position and of (velocity, mass); what all need moves by
-// DPP.  Every choice gives the same bits.
+// DPP.  Both give the same bits: products and sums are fused as written, not by
+// the compiler, which does it differently in the two.
 // Measured per launch (one lane forming everything, one slot for the largest W
 // -> 4 lanes -> 8 lanes): 10^6 droplets at 256^3 FP32 288 -> 300 -> 278 us (8
 // lanes, four blocks per CU: 267); 10^7 at 512^3 FP32 2470 -> 2562 -> 2358
 // (2262); 10^5 in each of 64 times 64^3 FP32 895 -> 871 -> 929 (4 lanes, four
 // blocks: 834); 10^5 at 64^3 FP32 26.2 -> 15.0 -> 17.7; 123457 at 128^3 FP64
 // 79.5 -> 83.7 -> 72.7.  Sparse droplets (each of the 28 lines of a stencil
-// serves few of them) are bound by the lines asked of L2, dense ones by
-// instructions: 8 lanes below one droplet in 6 cells, 4 above.
+// serves few of them) are bound by the lines, dense ones by instructions:
+// Engine::eight_lanes.
 // BAT: batched launch (blockIdx.z = realization); the single-realization
 // instantiation skips the pointer offsets and their registers.
 template <typename T, typename PT, int N, bool BAT, int NL>
 __global__ void __launch_bounds__(256)
 k_particles_stage(PStage<T, PT> A0) {
+#pragma clang fp contract(off)
   const PStage<T, PT> A = BAT ? A0.shifted() : A0;
   // XCD-aware mapping: the 8 XCDs take consecutive blocks round-robin; give
   // each XCD one contiguous range of (spatially sorted) droplets so its L2
@@ -374,7 +382,7 @@ k_particles_stage(PStage<T, PT> A0) {
   double kxc = 0.0;
   if (!s0) kxc = (double)A.kx[ax * cap + pp];
   const double L = A.P.L, dx = A.P.dx, pi_2dx = A.P.pi_2dx, invL = A.P.invL, inv_dx = A.P.inv_dx;
-  const double xw = wrapFast(x0c + ah * kxc, L, invL);
+  const double xw = wrapFast(fma(ah, kxc, x0c), L, invL);
   // one sincos per axis (cosW4); node i0 + a has weight (1 +- {cos, sin})/4.
   // The angles and the sincos are FP64; the weights and the gather sums are
   // kept in the field precision GT (FP32 fields: FP32 sums of 64 terms).
@@ -443,10 +451,10 @@ k_particles_stage(PStage<T, PT> A0) {
         for (int b = 0; b < 4; ++b) {
           const GT w = wy[b] * wx;
           const V4<T>& u = U[a * 4 + b];
-          Ig[0] += (GT)u.x * w;
-          Ig[1] += (GT)u.y * w;
-          Ig[2] += (GT)u.z * w;
-          Ig[3] += (GT)u.w * w;
+          Ig[0] = fmaG((GT)u.x, w, Ig[0]);
+          Ig[1] = fmaG((GT)u.y, w, Ig[1]);
+          Ig[2] = fmaG((GT)u.z, w, Ig[2]);
+          Ig[3] = fmaG((GT)u.w, w, Ig[3]);
         }
       }
     }
@@ -487,13 +495,13 @@ k_particles_stage(PStage<T, PT> A0) {
           const GT w = wy[b] * wx;
           const V4<T>& u = U[a * 4 + b];
           const V4<T>& v = V[a * 4 + b];
-          Ig[0] += (GT)u.x * w;
-          Ig[1] += (GT)u.y * w;
-          Ig[2] += (GT)u.z * w;
-          Ig[3] += (GT)v.x * w;
-          Ig[4] += (GT)v.y * w;
-          Ig[5] += (GT)v.z * w;
-          Ig[6] += (GT)v.w * w;
+          Ig[0] = fmaG((GT)u.x, w, Ig[0]);
+          Ig[1] = fmaG((GT)u.y, w, Ig[1]);
+          Ig[2] = fmaG((GT)u.z, w, Ig[2]);
+          Ig[3] = fmaG((GT)v.x, w, Ig[3]);
+          Ig[4] = fmaG((GT)v.y, w, Ig[4]);
+          Ig[5] = fmaG((GT)v.z, w, Ig[5]);
+          Ig[6] = fmaG((GT)v.w, w, Ig[6]);
         }
       }
     } else if (live) {
@@ -507,13 +515,13 @@ k_particles_stage(PStage<T, PT> A0) {
           const GT w = wy[b] * wx;
           const V4<T> U = ldRec<T, N>(A.gu, recU(o));
           const V4<T> V = ldRec<T, N>(A.gv, recV(o));
-          Ig[0] += (GT)U.x * w;
-          Ig[1] += (GT)U.y * w;
-          Ig[2] += (GT)U.z * w;
-          Ig[3] += (GT)V.x * w;
-          Ig[4] += (GT)V.y * w;
-          Ig[5] += (GT)V.z * w;
-          Ig[6] += (GT)V.w * w;
+          Ig[0] = fmaG((GT)U.x, w, Ig[0]);
+          Ig[1] = fmaG((GT)U.y, w, Ig[1]);
+          Ig[2] = fmaG((GT)U.z, w, Ig[2]);
+          Ig[3] = fmaG((GT)V.x, w, Ig[3]);
+          Ig[4] = fmaG((GT)V.y, w, Ig[4]);
+          Ig[5] = fmaG((GT)V.z, w, Ig[5]);
+          Ig[6] = fmaG((GT)V.w, w, Ig[6]);
         }
       }
     }
@@ -526,7 +534,7 @@ k_particles_stage(PStage<T, PT> A0) {
     }
   }
   // lane c's velocity component or, c == 3, the mass, and the droplet's four
-  const PT vc = v0c + (PT)ah * kvc;
+  const PT vc = fmaG((PT)ah, kvc, v0c);
   const PT vp[3] = {quadLane<0>(vc), quadLane<1>(vc), quadLane<2>(vc)};
   PT W = (PT)0;
   const PT den = dropletGrowth(A.P, vp, quadLane<3>(vc), I, W);
@@ -555,10 +563,10 @@ k_particles_stage(PStage<T, PT> A0) {
   // sump (forced-dns-sm.py:337, 342-358); the last stage writes the new state
   double* dxp = A.stage == 3 ? A.x0 : A.sx;
   PT* dvp = A.stage == 3 ? A.v0 : A.sv;
-  dvp[c * cap + p] = prv + (PT)A.wh * rc;
+  dvp[c * cap + p] = fmaG((PT)A.wh, rc, prv);
   if (A.stage < 3) A.kv[c * cap + p] = rc;
   if (c < 3) {
-    dxp[c * cap + p] = prx + A.wh * (double)vc;                            // :831
+    dxp[c * cap + p] = fma(A.wh, (double)vc, prx);                           // :831
     if (A.stage < 3) A.kx[c * cap + p] = vc;
   } else {
     // a fallback slot stores -W so the brick pass (which takes W > 0) skips it
