@@ -108,9 +108,27 @@ struct Engine final : EngineBase {
   // queue a stage's density chain after the next flow x pass (measured at 256^3:
   // 8.18 vs 8.31 ms/step; the 64^3 ensemble is faster in the plain order)
   bool late_density = N >= 128;
-  // Lanes per droplet of the stage kernel (k_particles_stage); 0 = by density.
+  // Lanes per droplet of the stage kernel (k_particles_stage); 0 = by the rule.
+  // 8 lanes ask for each line of a stencil once, at the price of instructions.
+  // They pay where the gather records of a realization come from memory (100 MB
+  // and more) and a line serves few droplets, and where the droplets are too few
+  // for 4 lanes to fill the chip (40000: of 256 CUs with 16 wavefronts each, 60 %).
+  // Us per launch, 4 / 8 lanes, at one droplet in so many cells:
+  //   256^3 FP32 (537 MB)      4.5 708/800  6 572/568  8 522/493  13 386/347  20 311/291
+  //   512^3 FP32 (4.3 GB)      5 5297/4907  8 3697/3441  13.4 2688/2341
+  //   128^3 FP64 (134 MB)      2.6 253/260  3.5 218/216  4.5 192/186  8 150/140  13 116/107
+  //   256^3 FP64 (1 GB)        2.6 1943/1954  3.5 1643/1589  4.5 1432/1403  8 1112/1020
+  //   128^3 FP32 (67 MB)       6 94/102  13 60/63  24 48/49  32 37/43  48 34/31 (43690 droplets)
+  //   64 x 64^3 FP32 (8 MB)    2.6 1491/1671  6 1161/1159  13 913/956  100 391/550  260 210/301
+  //   8 x 64^3 FP32            4 138/158  16 67/73  32 48/47 (65536)  64 42/35
+  //   64^3 FP32                4.5 13/17  6 11.6/12.9 (43690)  8 10.3/10.7  10 10.6/10.1  13 11.1/9.4
+  //   64^3 FP64 (17 MB)        4.5 25/26  6 22.5/23.3 (43690)  8 19.5/18.9  13 19.6/16.1
   int lanes = 0;
-  bool eight_lanes() const { return 6 * np < (int64_t)RF; }
+  bool eight_lanes() const {
+    if (np * B <= 40000) return true;
+    if (2 * RF * sizeof(V4<T>) < (size_t)100 << 20) return false;
+    return sizeof(T) == 8 ? 7 * np < 2 * (int64_t)RF : 6 * np < (int64_t)RF;
+  }
   // Dealiasing truncation: every mode with kz > N/3 is outside the mask
   // (kint >= kz), so the nonlinear term there is discarded and v_hat is zero.
   // The in-place y passes skip the kz > N/3 lines (kc = N/3; kc = N/2 runs
