@@ -109,16 +109,22 @@ def test_row_calls_on_several_streams(gpu, monkeypatch):
         return out
 
     jobs = [lambda r=r: row_calls(r) for r in rows] + [rk4, lambda: row_calls(rows[1]), steps, lambda: row_calls(rows[2]), rk4]
+    state = (rk4, steps)                 # calls on the context's state: their own order is the caller's
     alone = []
     for j in jobs:
         alone.append([x.clone() for x in j()])
         torch.cuda.synchronize()
     streams = [torch.cuda.Stream() for _ in range(3)]
     for turn in range(3):
-        got = []
+        got, last = [], None
         for k, j in enumerate(jobs):
             with torch.cuda.stream(streams[(k + turn) % 3]):
+                here = torch.cuda.current_stream()
+                if j in state and last is not None:
+                    here.wait_event(last)
                 got.append(j())
+                if j in state:
+                    last = here.record_event()
         torch.cuda.synchronize()
         for k, (a, b) in enumerate(zip(got, alone)):
             exact = len(a) if len(a) == 3 else 2
