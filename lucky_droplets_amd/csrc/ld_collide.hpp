@@ -21,36 +21,74 @@ __device__ __forceinline__ int collCell(double x, double cell, int nc) {
   return c < 0 ? 0 : (c >= nc ? nc - 1 : c);
 }
 
+// The cells per side: nc, or fine (if set) when the droplets crowd in the nc^3
+// cells (*same > many).  Read on the device, so that a call which has to choose
+// neither waits nor differs under capture.
+struct CellGrid {
+  int nc, fine;
+  unsigned long long *same, many;
+  __device__ __forceinline__ bool crowd() const { return same && *same > many; }
+  __device__ __forceinline__ int cells() const { return fine && crowd() ? fine : nc; }
+};
+
+// Count of the droplets per cell.  A droplet's rank is the number that its cell
+// held before it, so the ranks add up to the pairs of droplets that share a cell
+// (n / 2 of them for uniform droplets, one per cell).  *same += what they exceed
+// two per droplet by, block by block: nothing, and no atomic, where droplets
+// spread over the box (a pass of its own over 10^6 counts took 21 us).
+// again: the second count, in the fine cells if those are taken.
 static __global__ void __launch_bounds__(256)
-k_coll_count(const double* __restrict__ rows, int np, double L, double cell, int nc, int* __restrict__ key,
+k_coll_count(const double* __restrict__ rows, int np, double L, CellGrid G, bool again, int* __restrict__ key,
              int* __restrict__ rank, int* __restrict__ hist) {
+  __shared__ unsigned long long sh[4];
+  if (again && !G.crowd()) return;
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= np) return;
-  const double* r = rows + (size_t)p * 7;
-  const int cx = collCell(wrapL(r[0], L), cell, nc), cy = collCell(wrapL(r[1], L), cell, nc),
-            cz = collCell(wrapL(r[2], L), cell, nc);
-  const int k = (cx * nc + cy) * nc + cz;
-  key[p] = k;
-  rank[p] = atomicAdd(&hist[k], 1);
+  unsigned long long sum = 0;
+  if (p < np) {
+    const int nc = again ? G.fine : G.nc;
+    const double cell = L / nc;
+    const double* r = rows + (size_t)p * 7;
+    const int cx = collCell(wrapL(r[0], L), cell, nc), cy = collCell(wrapL(r[1], L), cell, nc),
+              cz = collCell(wrapL(r[2], L), cell, nc);
+    const int k = (cx * nc + cy) * nc + cz;
+    key[p] = k;
+    const int before = atomicAdd(&hist[k], 1);
+    rank[p] = before;
+    sum = (unsigned long long)before;
+  }
+  if (again || !G.same) return;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    sum = sh[0] + sh[1] + sh[2] + sh[3];
+    if (sum > 2 * 256) atomicAdd(G.same, sum - 2 * 256);
+  }
 }
 
-// *same += the pairs of droplets that share a cell, sum of c (c - 1) / 2 over the
-// counts: 16384 cells and one atomic (some 12 ns at one address) per block.
-static __global__ void __launch_bounds__(256)
-k_coll_same(const int* __restrict__ count, int ncells, unsigned long long* __restrict__ same) {
-  __shared__ unsigned long long sh[4];
-  unsigned long long s = 0;
-#pragma unroll 16
-  for (int k = 0; k < 64; ++k) {
-    const int i = (blockIdx.x * 64 + k) * 256 + threadIdx.x;
-    const unsigned long long c = i < ncells ? (unsigned long long)count[i] : 0ull;
-    s += c ? c * (c - 1) / 2 : 0ull;
+// The fine cells' counts cleared, if those are taken; then the scans over the
+// cells taken.  Their launches are of the size that the chip holds, whatever the
+// cells.
+static __global__ void __launch_bounds__(256) k_coll_clear(int* __restrict__ hist, CellGrid G) {
+  if (!G.crowd()) return;
+  const int n = G.fine * G.fine * G.fine;
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) hist[i] = 0;
+}
+static __global__ void __launch_bounds__(1024)
+k_coll_scan_local(int* __restrict__ hist, CellGrid G, int* __restrict__ bsum) {
+  __shared__ int sh[32];
+  const int nc = G.cells(), n = nc * nc * nc;
+  for (int c = blockIdx.x; c * 4096 < n; c += gridDim.x) scanChunk(hist, n, bsum, c, sh);
+}
+static __global__ void __launch_bounds__(1024)
+k_coll_scan_add(int* __restrict__ hist, CellGrid G, const int* __restrict__ bsum) {
+  __shared__ int sh[16];
+  const int nc = G.cells(), n = nc * nc * nc;
+  for (int c = blockIdx.x; c * 4096 < n; c += gridDim.x) {
+    if (c) scanAddChunk(hist, n, bsum, c, sh);
+    __syncthreads();                     // sh, before the next chunk's sums
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(same, sh[0] + sh[1] + sh[2] + sh[3]);
 }
 
 // Droplets in cell order: wrapped position and radius, input row, and (for the
@@ -119,15 +157,14 @@ __device__ __forceinline__ double separation(const double4& a, const double4& b,
 struct NearArgs {
   const double4 *pos, *vel;
   const int *order, *start;
-  int np, nc;
-  double L, cell;
+  int np;
+  CellGrid grid;                       // crowded without fine cells: nothing is done (the caller searches finer ones)
+  double L;
   unsigned long long *out, max_pairs, *count;                   // pairs
   double rmax, dr;                                               // statistics
   int nbins;
   unsigned long long* counts;
   double *wsum, *wneg;
-  const unsigned long long* same;      // set: nothing is done when *same > many (the caller searches finer cells)
-  unsigned long long many;
 };
 template <bool STATS> struct NearHist { unsigned long long c[512]; double w[512], n[512]; };
 template <> struct NearHist<false> {};
@@ -136,7 +173,10 @@ __global__ void __launch_bounds__(256) k_near(NearArgs A) {
 #pragma clang fp contract(off)
   __shared__ NearHist<STATS> H;
   __shared__ int2 queue[4][128];
-  if (A.same && *A.same > A.many) return;
+  const bool crowd = A.grid.crowd();
+  if (crowd && !A.grid.fine) return;
+  const int nc = crowd ? A.grid.fine : A.grid.nc, np = A.np;
+  const double cell = A.L / nc;
   if constexpr (STATS) {
     for (int k = threadIdx.x; k < A.nbins; k += 256) { H.c[k] = 0ull; H.w[k] = 0.0; H.n[k] = 0.0; }
     __syncthreads();
@@ -144,7 +184,6 @@ __global__ void __launch_bounds__(256) k_near(NearArgs A) {
   const int lane = threadIdx.x & 63;
   int2* q = queue[threadIdx.x >> 6];
   const int per = gridDim.x / 8, lb = (blockIdx.x % 8) * per + blockIdx.x / 8;   // XCD-aware: contiguous slots
-  const int nc = A.nc, np = A.np;
   const uint32_t slot = (uint32_t)lb * 256u + threadIdx.x;
   bool run = slot < (uint32_t)np;
   const int s = run ? (int)slot : 0;
@@ -152,7 +191,7 @@ __global__ void __launch_bounds__(256) k_near(NearArgs A) {
   int cx = 0, cy = 0, cz = 0, t = 0, e = 0;
   if (run) {
     me = A.pos[s];
-    cx = collCell(me.x, A.cell, nc); cy = collCell(me.y, A.cell, nc); cz = collCell(me.z, A.cell, nc);
+    cx = collCell(me.x, cell, nc); cy = collCell(me.y, cell, nc); cz = collCell(me.z, cell, nc);
     const int own = (cx * nc + cy) * nc + cz, last = (nc >= 3 && cz + 1 < nc) ? own + 1 : own;
     t = s + 1;
     e = last + 1 < nc * nc * nc ? A.start[last + 1] : np;

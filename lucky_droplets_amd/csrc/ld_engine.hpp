@@ -1430,7 +1430,7 @@ struct Engine final : EngineBase {
   // ------------------------------------------------------------ collisions
   int *ckey = nullptr, *crank = nullptr, *corder = nullptr, *chist = nullptr, *cbsum = nullptr, *cused = nullptr;
   double4 *cpos = nullptr, *cvel = nullptr;
-  unsigned long long *ckeys = nullptr, *ccount = nullptr;   // ccount: pairs found, pairs of droplets in one cell
+  unsigned long long *ckeys = nullptr, *ccount = nullptr;   // ccount: pairs found, crowding (CellGrid::same)
   unsigned long long* hcount = nullptr;                      // pinned host copy
   int *cnev = nullptr;
   int64_t ccap = 0, cvcap = 0, ckcap = 0;
@@ -1484,43 +1484,44 @@ struct Engine final : EngineBase {
   // than four cells per droplet, about one per droplet: 10^6 droplets whose pairs
   // reach 1/4000 of the box, pairs 505 us with 256^3 cells, whose counts and
   // scans cost more than the few candidates that 100^3 add, 337 us with 100^3.
-  // But droplets that cluster then share cells, so the caller has to ask for
-  // `same`, the pairs of droplets in one cell, and with more than 3 n of them
-  // (uniform droplets: n / 2) to search with `fit` cells instead: 10^5 droplets
-  // in a box of side L/2 (3.5 n) 250 us with 47^3 cells, 266 with 256^3; L/3
-  // (13 n) 377 / 269; L/20 16.6 ms / 0.74 ms.
-  static constexpr uint64_t CROWD = 3;
-  struct CellGrid { int nc, fit; };
+  // But droplets that cluster then share cells, so the pairs of droplets in one
+  // cell are counted (k_coll_count), and with more than 2.5 to 3 n of them (uniform
+  // droplets: n / 2) `fit` cells are searched instead (`fine`).  Us per call with
+  // n^(1/3) cells per side / with 256, reach a fifth of the spacing: 10^5 droplets
+  // in a box of side L/2 (3.5 n) 193 / 172, 0.35 L (10 n) 314 / 177, 0.15 L 1421 /
+  // 205; 1000 droplets 167 / 105, 269 / 103, 431 / 162.
   CellGrid cell_grid(int64_t n_, double reach) const {
     int most = 3;
     while (most < 256 && (int64_t)most * most * most < n_) ++most;
     int fit = (reach > 0.0 && p.L / reach < 256.0) ? (int)floor(p.L / reach) : 256;
     if (fit < 3) fit = 1;
-    return {fit <= most || (int64_t)fit * fit * fit <= 4 * n_ ? fit : most, fit};
+    if (fit <= most || (int64_t)fit * fit * fit <= 4 * n_) return {fit, 0, nullptr, 0};
+    return {most, fit, ccount + 1, (uint64_t)n_ / 2};
   }
   // Cell list of the droplet rows on st.  Cell starts in chist; positions, radii
   // and (with_vel) velocities in cell order in cpos and cvel, input rows in
-  // corder; same (device, may be null): += pairs of droplets in one cell.
-  int build_cells(const double* rows, const double* rad, int64_t n_, int nc, bool with_vel,
-                  unsigned long long* same) {
-    const double cell = p.L / nc;
-    const int ncells = nc * nc * nc;
+  // corder; g.same (device, may be null) counts how the droplets crowd.  g.fine set:
+  // the cells are those that the device then chooses.
+  int build_cells(const double* rows, const double* rad, int64_t n_, const CellGrid& g, bool with_vel) {
+    const int ncells = g.nc * g.nc * g.nc, most = g.fine ? g.fine * g.fine * g.fine : ncells;
     LD_TRY(coll_reserve(n_));
     if (with_vel) LD_TRY(coll_reserve_vel(n_));
-    LD_TRY(coll_reserve_cells(ncells));
+    LD_TRY(coll_reserve_cells(most));
     const unsigned pb = (unsigned)((n_ + 255) / 256);
     LD_TRY(fill<int>(st, chist, ncells, 0));
-    hipLaunchKernelGGL(k_coll_count, dim3(pb), dim3(256), 0, st, rows, (int)n_, p.L, cell, nc, ckey, crank, chist);
+    hipLaunchKernelGGL(k_coll_count, dim3(pb), dim3(256), 0, st, rows, (int)n_, p.L, g, false, ckey, crank, chist);
     LD_LAUNCHED();
-    const int nbs = (ncells + 4095) / 4096;
-    if (same) {
-      hipLaunchKernelGGL(k_coll_same, dim3((nbs + 3) / 4), dim3(256), 0, st, (const int*)chist, ncells, same);
+    if (g.fine) {
+      hipLaunchKernelGGL(k_coll_clear, dim3(1024), dim3(256), 0, st, chist, g);
+      LD_LAUNCHED();
+      hipLaunchKernelGGL(k_coll_count, dim3(pb), dim3(256), 0, st, rows, (int)n_, p.L, g, true, ckey, crank, chist);
       LD_LAUNCHED();
     }
-    hipLaunchKernelGGL(k_scan_local, dim3(nbs), dim3(1024), 0, st, chist, ncells, cbsum, (size_t)0);
+    const unsigned chunks = (unsigned)((most + 4095) / 4096), nbs = chunks < 512 ? chunks : 512;
+    hipLaunchKernelGGL(k_coll_scan_local, dim3(nbs), dim3(1024), 0, st, chist, g, cbsum);
     LD_LAUNCHED();
-    if (nbs > 1) {
-      hipLaunchKernelGGL(k_scan_add, dim3(nbs), dim3(1024), 0, st, chist, ncells, (const int*)cbsum, (size_t)0);
+    if (chunks > 1) {
+      hipLaunchKernelGGL(k_coll_scan_add, dim3(nbs), dim3(1024), 0, st, chist, g, (const int*)cbsum);
       LD_LAUNCHED();
     }
     hipLaunchKernelGGL(k_coll_scatter, dim3(pb), dim3(256), 0, st, rows, rad, (int)n_, p.L, (const int*)ckey,
@@ -1528,10 +1529,10 @@ struct Engine final : EngineBase {
     LD_LAUNCHED();
     return LD_OK;
   }
-  NearArgs near_args(int64_t n_, int nc) const {
+  NearArgs near_args(int64_t n_, const CellGrid& g) const {
     NearArgs a{};
     a.pos = cpos; a.vel = cvel; a.order = corder; a.start = chist;
-    a.np = (int)n_; a.nc = nc; a.L = p.L; a.cell = p.L / nc;
+    a.np = (int)n_; a.grid = g; a.L = p.L;
     return a;
   }
   static unsigned near_blocks(int64_t n_) { return (unsigned)(((n_ + 255) / 256 + 7) / 8 * 8); }
@@ -1546,31 +1547,19 @@ struct Engine final : EngineBase {
     LD_TRY(fill<double>(st, wsum, (size_t)nbins, 0.0));
     LD_TRY(fill<double>(st, wneg, (size_t)nbins, 0.0));
     if (n_ < 2) return LD_OK;
-    CellGrid g = cell_grid(n_, rmax);
-    if (g.nc < g.fit) {
-      // whether the droplets cluster is known on the device only: the call waits
-      // for it (10^6 uniform droplets, rmax 0.37 of their spacing, 338 -> 370
-      // us), unless the stream is under capture
-      bool cap_ = false;
-      LD_TRY(capturing(cap_));
-      if (cap_) g.fit = g.nc;
-    }
+    // whether the droplets cluster is known on the device only, and chosen there:
+    // the call does not wait (10^6 uniform droplets, rmax 0.37 of their spacing, 330
+    // us when it did, 306 now; 10^5 in a box of side L/2 217 -> 175)
     LD_TRY(coll_counters());
-    for (;;) {
-      const bool ask = g.nc < g.fit;
-      if (ask) LD_TRY(fill<unsigned long long>(st, ccount, 2, 0ull));
-      LD_TRY(build_cells(rows, nullptr, n_, g.nc, true, ask ? ccount + 1 : nullptr));
-      NearArgs a = near_args(n_, g.nc);
-      a.rmax = rmax; a.dr = rmax / nbins; a.nbins = nbins;
-      a.counts = (unsigned long long*)counts; a.wsum = wsum; a.wneg = wneg;
-      a.same = ask ? ccount + 1 : nullptr; a.many = CROWD * (uint64_t)n_;
-      hipLaunchKernelGGL((k_near<true>), dim3(near_blocks(n_)), dim3(256), 0, st, a);
-      LD_LAUNCHED();
-      if (!ask) return LD_OK;
-      LD_TRY(read_counters());
-      if (hcount[1] <= a.many) return LD_OK;
-      g.nc = g.fit;
-    }
+    const CellGrid g = cell_grid(n_, rmax);
+    if (g.same) LD_TRY(fill<unsigned long long>(st, ccount, 2, 0ull));
+    LD_TRY(build_cells(rows, nullptr, n_, g, true));
+    NearArgs a = near_args(n_, g);
+    a.rmax = rmax; a.dr = rmax / nbins; a.nbins = nbins;
+    a.counts = (unsigned long long*)counts; a.wsum = wsum; a.wneg = wneg;
+    hipLaunchKernelGGL((k_near<true>), dim3(near_blocks(n_)), dim3(256), 0, st, a);
+    LD_LAUNCHED();
+    return LD_OK;
   }
 
   int collide(const double* rows, const double* rad, int64_t n_, double rmax, int64_t* pairs, int64_t max_pairs,
@@ -1579,25 +1568,29 @@ struct Engine final : EngineBase {
     if (n_ < 2) return LD_OK;
     if (n_ > 0x7fffffff) { set_error("too many droplets"); return LD_ERR_ARG; }
     LD_TRY(join(st, st2, evB));
-    // cells of side >= 2 rmax (the largest pair distance)
-    CellGrid g = cell_grid(n_, 2.0 * rmax);
     const int64_t kc = pow2ceil(max_pairs > 2 ? max_pairs : 2);
     if (kc > ckcap) { LD_TRY(alloc(ckeys, kc)); ckcap = kc; }
     LD_TRY(coll_counters());
+    // cells of side >= 2 rmax (the largest pair distance); the call reads its count
+    // anyway, so the host takes the fine cells (and their memory) when it finds the
+    // droplets to crowd, from n rather than n / 2 on, because it then searches twice
+    // (10^5 droplets in a box of side L/2: 193 us coarse, 204 with the second search)
+    CellGrid g = cell_grid(n_, 2.0 * rmax);
+    const int fit = g.fine;
+    g.fine = 0;
+    g.many = (uint64_t)n_;
     unsigned long long cnt = 0;
     for (;;) {
-      const bool ask = g.nc < g.fit;
       LD_TRY(fill<unsigned long long>(st, ccount, 2, 0ull));
-      LD_TRY(build_cells(rows, rad, n_, g.nc, false, ask ? ccount + 1 : nullptr));
-      NearArgs a = near_args(n_, g.nc);
+      LD_TRY(build_cells(rows, rad, n_, g, false));
+      NearArgs a = near_args(n_, g);
       a.out = ckeys; a.max_pairs = (unsigned long long)max_pairs; a.count = ccount;
-      a.same = ask ? ccount + 1 : nullptr; a.many = CROWD * (uint64_t)n_;
       hipLaunchKernelGGL((k_near<false>), dim3(near_blocks(n_)), dim3(256), 0, st, a);
       LD_LAUNCHED();
       LD_TRY(read_counters());
       cnt = hcount[0];
-      if (!ask || hcount[1] <= a.many) break;
-      g.nc = g.fit;
+      if (!g.same || hcount[1] <= g.many) break;
+      g = {fit, 0, nullptr, 0};
     }
     *count = (int64_t)cnt;
     if ((int64_t)cnt > max_pairs) {

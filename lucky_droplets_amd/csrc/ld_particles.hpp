@@ -1410,12 +1410,9 @@ __device__ __forceinline__ int blockExclusiveScan1024(int v, int* sh, int& total
   return wpre + x - v;
 }
 
-static __global__ void __launch_bounds__(1024)
-k_scan_local(int* __restrict__ data0, int n, int* __restrict__ bsum0, size_t rs) {
-  int* __restrict__ data = rsel1(data0, rs);
-  int* __restrict__ bsum = rsel1(bsum0, rs);
-  __shared__ int sh[32];
-  const int base = blockIdx.x * 4096 + threadIdx.x * 4;
+// chunk number `chunk` of 4096 entries
+__device__ __forceinline__ void scanChunk(int* __restrict__ data, int n, int* __restrict__ bsum, int chunk, int* sh) {
+  const int base = chunk * 4096 + threadIdx.x * 4;
   int v[4], s = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) { v[i] = (base + i < n) ? data[base + i] : 0; s += v[i]; }
@@ -1426,23 +1423,25 @@ k_scan_local(int* __restrict__ data0, int n, int* __restrict__ bsum0, size_t rs)
     if (base + i < n) data[base + i] = pre;
     pre += v[i];
   }
-  if (threadIdx.x == 0) bsum[blockIdx.x] = total;
+  if (threadIdx.x == 0) bsum[chunk] = total;
+}
+static __global__ void __launch_bounds__(1024)
+k_scan_local(int* __restrict__ data, int n, int* __restrict__ bsum, size_t rs) {
+  __shared__ int sh[32];
+  scanChunk(rsel1(data, rs), n, rsel1(bsum, rs), blockIdx.x, sh);
 }
 
 // += the sums of the 4096-entry chunks before the block's, which each block adds
 // up itself (one launch of 5 us less than with a scan of the sums between the two).
-static __global__ void __launch_bounds__(1024)
-k_scan_add(int* __restrict__ data0, int n, const int* __restrict__ bsum0, size_t rs) {
-  int* __restrict__ data = rsel1(data0, rs) + (size_t)blockIdx.x * 4096;
-  const int* __restrict__ bsum = rsel1(bsum0, rs);
-  __shared__ int sh[16];
-  if (blockIdx.x == 0) return;
-  const int left = n - (int)blockIdx.x * 4096, tid = threadIdx.x;
+__device__ __forceinline__ void scanAddChunk(int* __restrict__ data, int n, const int* __restrict__ bsum, int chunk,
+                                             int* sh) {
+  data += (size_t)chunk * 4096;
+  const int left = n - chunk * 4096, tid = threadIdx.x;
   int v[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) v[k] = tid + k * 1024 < left ? data[tid + k * 1024] : 0;
   int s = 0;
-  for (int i = tid; i < (int)blockIdx.x; i += 1024) s += bsum[i];
+  for (int i = tid; i < chunk; i += 1024) s += bsum[i];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
   if ((tid & 63) == 0) sh[tid >> 6] = s;
@@ -1453,6 +1452,11 @@ k_scan_add(int* __restrict__ data0, int n, const int* __restrict__ bsum0, size_t
 #pragma unroll
   for (int k = 0; k < 4; ++k)
     if (tid + k * 1024 < left) data[tid + k * 1024] = v[k] + base;
+}
+static __global__ void __launch_bounds__(1024)
+k_scan_add(int* __restrict__ data, int n, const int* __restrict__ bsum, size_t rs) {
+  __shared__ int sh[16];
+  if (blockIdx.x) scanAddChunk(rsel1(data, rs), n, rsel1(bsum, rs), blockIdx.x, sh);
 }
 
 // Scatter the droplet state to its sorted slot.
